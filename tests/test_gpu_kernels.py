@@ -366,6 +366,69 @@ def test_top_k_ties_keep_index_order(ops):
     assert float((probs[0].double() - want).abs().max()) < 1e-6
 
 
+def vector_distribution(z, T, k, p):
+    """`plain.sample_distribution` in float64 without its loops over the vocabulary: ties at either threshold go by index."""
+    z = z.double() / T
+    V = z.numel()
+    if 0 < k < V:
+        order = torch.argsort(z, descending=True, stable=True)
+        z = z.clone()
+        z[order[k:]] = -float("inf")
+    q = torch.softmax(z, 0)
+    if 0.0 < p < 1.0:
+        order = torch.argsort(q, descending=True, stable=True)
+        cum = q[order].cumsum(0)
+        reached = (cum >= p).nonzero()
+        q = q.clone()
+        if len(reached):
+            q[order[int(reached[0]) + 1:]] = 0.0
+        q = q / q.sum()
+    return q
+
+
+@pytest.mark.parametrize("V,k,p", [(131072, 50, 0.95), (131072, 0, 0.9), (131071, 1023, 0.0), (131072, 1024, 0.3), (50001, 1025, 0.7),
+                                   (4099, 4098, 0.5), (1024, 1, 0.0), (5, 4, 0.9), (131072, 0, 0.0), (8193, 2000, 0.0)])
+def test_distribution_of_long_rows(ops, V, k, p):
+    """Both ways of the thresholds (a list of at most 1,024 kept, a histogram) on aligned rows and others.  A
+    probability has the error of its exponential and two divisions, a few 2^-24 of it; where the running sum of
+    sorted probabilities passes top_p within 1e-6, one more or less may be kept."""
+    logits = rnd(3, V, seed=31, scale=2.5)
+    logits[1] = (logits[1] * 2).round() / 2                  # many ties
+    logits[2, : V // 3] = -float("inf")                      # a masked vocabulary
+    counters = [[b, 5] for b in range(3)]
+    ids, probs = run_sample(ops, logits, 0.7, k, p, 17, counters)
+    for b in range(3):
+        want = vector_distribution(logits[b], torch.tensor(0.7).double(), k, p)
+        got = probs[b].double()
+        assert abs(float(got.sum()) - 1) < 1e-4
+        kept, expect = int((got > 0).sum()), int((want > 1e-38).sum())
+        assert abs(kept - expect) <= (1 if p else 0), (kept, expect)
+        assert float((got - want).abs().max()) < 2e-6 + (float(want[want > 0].min()) * 2 if kept != expect else 0)
+        r, cum = philox_uniform(17, 5, b), got.cumsum(0)
+        mine = int((cum >= r).nonzero()[0])
+        assert ids[b] == mine or abs(float(cum[min(ids[b], mine)]) - r) < 1e-6
+
+
+def test_rows_without_a_distribution(ops):
+    """Infinities and NaN among the logits: no draw, the last index; a row of one value: an even draw; -inf beside
+    one finite logit: that one."""
+    V = 3000
+    z = torch.zeros(5, V)
+    z[0, 7] = float("inf")
+    z[1, 7] = float("nan")
+    z[2] = -float("inf")
+    z[4] = -float("inf")
+    z[4, 11] = -3.0
+    for k, p in ((0, 0.0), (0, 0.9), (5, 0.0), (5, 0.9), (2000, 0.9)):
+        ids, probs = run_sample(ops, z, 1.0, k, p, 3)
+        assert ids[0] == ids[1] == ids[2] == V - 1, (k, p, ids)
+        kept = (probs[3] > 0).nonzero().flatten().tolist()
+        assert kept == list(range(len(kept))) and ids[3] in kept
+        n = min(k or V, V)
+        assert abs(len(kept) - (math.ceil(p * n - 1e-6) if p else n)) <= (1 if p else 0)
+        assert ids[4] == 11 and float(probs[4, 11]) == 1.0
+
+
 def test_draws_do_not_depend_on_batch_mates_and_follow_the_probabilities(ops):
     V = 8
     z = torch.tensor([[2.0, 1.0, 0.0, -1.0, 0.5, 1.5, -2.0, 0.2]])

@@ -36,186 +36,430 @@ __device__ inline float philox_uniform(uint32_t seed_lo, uint32_t seed_hi, uint3
   return (float)(c0 >> 8) * (1.0f / 16777216.0f);      // [0, 1)
 }
 
-__device__ __forceinline__ int block_sum_i(int v, int* sh) {
+// Four floats of a row from index i on (i a multiple of 4); `n` of them lie in the row.  VEC: rows are
+// aligned to 16 bytes and a multiple of 4 long.
+template <bool VEC> __device__ __forceinline__ int load4(const float* __restrict__ p, int i, int V, float v[4]) {
+  if (VEC) {
+    if (i >= V) return 0;
+    const f32x4 t = *(const f32x4*)(p + i);
+    v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
+    return 4;
+  }
+  const int n = max(0, min(4, V - i));
 #pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-  __syncthreads();
-  if (threadIdx.x % WAVE == 0) sh[threadIdx.x / WAVE] = v;
-  __syncthreads();
-  int r = 0;
+  for (int j = 0; j < 4; ++j) v[j] = j < n ? p[i + j] : 0.f;
+  return n;
+}
+template <bool VEC> __device__ __forceinline__ void store4(float* __restrict__ p, int i, int n, const float v[4]) {
+  if (VEC) {
+    if (n) *(f32x4*)(p + i) = f32x4{v[0], v[1], v[2], v[3]};
+    return;
+  }
 #pragma unroll
-  for (int i = 0; i < SNT / WAVE; ++i) r += sh[i];
-  return r;
+  for (int j = 0; j < 4; ++j)
+    if (j < n) p[i + j] = v[j];
 }
 
-// exclusive prefix over the threads of the block, in thread order
-template <typename V> __device__ __forceinline__ V block_excl_scan(V v, V* sh, V* total) {
-  __syncthreads();
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    V run = 0;
-    for (int i = 0; i < SNT; ++i) {
-      const V t = sh[i];
-      sh[i] = run;
-      run += t;
+// f(index, value) over a row, every thread on its own elements, in any order; `update` stores what f returns.
+// Eight loads of 16 bytes a thread are under way at a time: a row is read by one compute unit, whose way to
+// L2 (64 bytes a cycle) is what a pass over a long row takes.
+constexpr int ROW_LOADS = 8;
+template <bool VEC, typename F> __device__ __forceinline__ void visit(const float* __restrict__ p, int V, F f) {
+  for (int base = threadIdx.x * 4; base < V; base += SNT * 4 * ROW_LOADS) {
+    float v[ROW_LOADS][4];
+    int n[ROW_LOADS];
+#pragma unroll
+    for (int u = 0; u < ROW_LOADS; ++u) n[u] = load4<VEC>(p, base + u * SNT * 4, V, v[u]);
+#pragma unroll
+    for (int u = 0; u < ROW_LOADS; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < n[u]) f(base + u * SNT * 4 + j, v[u][j]);
+  }
+}
+template <bool VEC, typename F>
+__device__ __forceinline__ void update(const float* __restrict__ src, float* __restrict__ dst, int V, F f) {
+  for (int base = threadIdx.x * 4; base < V; base += SNT * 4 * ROW_LOADS) {
+    float v[ROW_LOADS][4];
+    int n[ROW_LOADS];
+#pragma unroll
+    for (int u = 0; u < ROW_LOADS; ++u) n[u] = load4<VEC>(src, base + u * SNT * 4, V, v[u]);
+#pragma unroll
+    for (int u = 0; u < ROW_LOADS; ++u) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < n[u]) v[u][j] = f(base + u * SNT * 4 + j, v[u][j]);
+      store4<VEC>(dst, base + u * SNT * 4, n[u], v[u]);
     }
-    sh[SNT] = run;
+  }
+}
+
+template <typename T> __device__ __forceinline__ T wave_incl_scan(T v) {
+  const int lane = threadIdx.x % WAVE;
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    const T t = __shfl_up(v, o, WAVE);
+    if (lane >= o) v += t;
+  }
+  return v;
+}
+// exclusive prefix over the threads of the block, in thread order; `sh` holds SNT / WAVE values
+template <typename T> __device__ __forceinline__ T block_excl_scan(T v, T* sh, T* total) {
+  const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const T incl = wave_incl_scan(v);
+  __syncthreads();
+  if (lane == WAVE - 1) sh[w] = incl;
+  __syncthreads();
+  T before = 0, all = 0;
+#pragma unroll
+  for (int i = 0; i < SNT / WAVE; ++i) {
+    if (i == w) before = all;
+    all += sh[i];
+  }
+  *total = all;
+  return before + incl - v;
+}
+
+// a probability as a whole number of 2^-60: sums of these are exact whatever their order
+constexpr double FIX = 1152921504606846976.0;
+__device__ __forceinline__ unsigned long long fixed60(float p) { return (unsigned long long)((double)p * FIX); }
+
+struct SampleShared {
+  unsigned long long hist[2048];
+  unsigned long long scan[SNT / WAVE];
+  unsigned long long above;
+  int digit;
+  int count;
+  int pick;
+  int wave_count[SNT / WAVE];
+  double wave_sum[SNT / WAVE];
+  float red[SNT / WAVE];
+};
+// the short lists of the way by candidates
+constexpr int CANDIDATES = 2048;
+constexpr int MOST_TOP_K = 1024;
+static_assert(MOST_TOP_K == SNT, "one kept candidate a thread");
+struct Lists {
+  float z[CANDIDATES];
+  int idx[CANDIDATES];
+  float top_z[MOST_TOP_K];
+  int top_i[MOST_TOP_K];
+};
+
+// The largest t with (weights of the keys >= t) >= target, digit by digit from the top (11, 11 and 10 bits) through
+// a histogram in LDS; 0 if no t reaches the target.  `above` returns the weights of the keys > t, `at` those of t.
+template <bool VEC, typename Key, typename Weight>
+__device__ __forceinline__ uint32_t select_key(const float* __restrict__ p, int V, unsigned long long target, Key key, Weight weight,
+                                               SampleShared& sh, unsigned long long* above, unsigned long long* at) {
+  uint32_t prefix = 0u;
+  unsigned long long over = 0;
+#pragma unroll 1
+  for (int round = 0; round < 3; ++round) {
+    const int shift = round == 0 ? 21 : (round == 1 ? 10 : 0);
+    const uint32_t bins = round == 2 ? 1024u : 2048u;
+    const uint32_t known = round == 0 ? 0u : (round == 1 ? 0xffe00000u : 0xfffffc00u);
+    __syncthreads();
+    sh.hist[threadIdx.x] = 0;
+    sh.hist[threadIdx.x + SNT] = 0;
+    if (threadIdx.x == 0) sh.digit = -1;
+    __syncthreads();
+    visit<VEC>(p, V, [&](int, float v) {
+      const uint32_t k = key(v);
+      if ((k & known) == prefix) atomicAdd(&sh.hist[(k >> shift) & (bins - 1u)], weight(v));
+    });
+    __syncthreads();
+    // thread t has the bins 2047 - 2 t and 2046 - 2 t, so that prefixes run from the largest key down
+    const int hi = 2047 - 2 * (int)threadIdx.x;
+    const unsigned long long wh = sh.hist[hi], wl = sh.hist[hi - 1];
+    unsigned long long total;
+    const unsigned long long before = over + block_excl_scan<unsigned long long>(wh + wl, sh.scan, &total);
+    if (before < target && before + wh + wl >= target) {
+      const bool first = before + wh >= target;
+      sh.digit = first ? hi : hi - 1;
+      sh.above = first ? before : before + wh;
+    }
+    __syncthreads();
+    if (sh.digit < 0) {                                  // all of them together do not reach the target
+      *above = total;                                    // (only the first digit can miss)
+      *at = 0;
+      return 0u;
+    }
+    over = sh.above;
+    *at = sh.hist[sh.digit];
+    prefix |= (uint32_t)sh.digit << shift;
+  }
+  *above = over;
+  return prefix;
+}
+
+// Keep the first `room` (in the order of the row) of the elements with key == thr, and those with a larger key:
+// the others become `gone`.  Waves take the row in equal runs, one after the other.
+template <bool VEC, typename Key, typename Kept>
+__device__ __forceinline__ void keep_ties(float* __restrict__ p, int V, uint32_t thr, int room, float gone, Key key, Kept kept, SampleShared& sh) {
+  const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int run = ((V + SNT / WAVE - 1) / (SNT / WAVE) + 255) / 256 * 256;
+  const int lo = min(V, w * run), hi = min(V, lo + run);
+  int c = 0;
+  for (int base = lo; base < hi; base += 256) {
+    float v[4];
+    const int n = load4<VEC>(p, base + lane * 4, V, v);
+    for (int j = 0; j < n; ++j) c += key(v[j]) == thr;
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) c += __shfl_xor(c, o, WAVE);
+  __syncthreads();
+  if (lane == 0) sh.wave_count[w] = c;
+  __syncthreads();
+  int rank = 0;
+  for (int i = 0; i < w; ++i) rank += sh.wave_count[i];
+  for (int base = lo; base < hi; base += 256) {
+    float v[4];
+    const int n = load4<VEC>(p, base + lane * 4, V, v);
+    int mine = 0;
+    for (int j = 0; j < n; ++j) mine += key(v[j]) == thr;
+    const int incl = wave_incl_scan(mine);
+    int at = rank + incl - mine;
+    for (int j = 0; j < n; ++j) {
+      const uint32_t k = key(v[j]);
+      if (k < thr || (k == thr && at++ >= room)) v[j] = gone;
+      else v[j] = kept(v[j]);
+    }
+    store4<VEC>(p, base + lane * 4, n, v);
+    rank += __shfl(incl, WAVE - 1, WAVE);
   }
   __syncthreads();
-  *total = sh[SNT];
-  return sh[threadIdx.x];
 }
 
+// The draw over a whole row of probabilities: the first index whose running sum reaches r, else the last.
+template <bool VEC> __device__ __forceinline__ void draw_row(const float* __restrict__ p, int V, float r, SampleShared& sh, int* __restrict__ out) {
+  const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int run = ((V + SNT / WAVE - 1) / (SNT / WAVE) + 255) / 256 * 256;
+  const int lo = min(V, w * run), hi = min(V, lo + run);
+  double s = 0.0;
+#pragma unroll 8
+  for (int base = lo; base < hi; base += 256) {
+    float v[4];
+    const int n = load4<VEC>(p, base + lane * 4, V, v);
+    for (int j = 0; j < n; ++j) s += (double)v[j];
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, WAVE);
+  __syncthreads();
+  if (lane == 0) sh.wave_sum[w] = s;
+  if (threadIdx.x == 0) sh.pick = V - 1;
+  __syncthreads();
+  double before = 0.0;
+  for (int i = 0; i < w; ++i) before += sh.wave_sum[i];
+  if (lo < hi && before < (double)r && before + s >= (double)r) {      // (one wave at most: sums only grow)
+    int pick = hi - 1;
+    double so_far = before;
+    for (int base = lo; base < hi; base += 256) {
+      float v[4];
+      const int n = load4<VEC>(p, base + lane * 4, V, v);
+      double mine = 0.0;
+      for (int j = 0; j < n; ++j) mine += (double)v[j];
+      const double incl = wave_incl_scan(mine);
+      const unsigned long long reached = __ballot(n > 0 && so_far + incl >= (double)r);
+      if (reached) {
+        const int first = __ffsll((long long)reached) - 1;
+        double t = so_far + incl - mine;
+        int at = base + lane * 4;
+        for (int j = 0; j < n; ++j) {
+          t += (double)v[j];
+          if (t >= (double)r) break;
+          if (j + 1 < n) ++at;
+        }
+        pick = __shfl(at, first, WAVE);
+        break;
+      }
+      so_far += __shfl(incl, WAVE - 1, WAVE);
+    }
+    if (lane == 0) sh.pick = pick;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *out = r > 0.f ? sh.pick : 0;   // (index 0's running sum reaches a draw of 0)
+}
+
+// One workgroup of 1,024 threads a row.  What bounds it is one compute unit's work on a row (131,072 logits are
+// 512 KB, 3.5 us a pass at 64 bytes a cycle from L2, and more where an element costs a division or an exponential)
+// times the number of passes, so passes are what was taken out:
+//   * top-k of at most 1,024 (two passes): the k-th largest of the threads' own maxima bounds the k-th largest of the
+//     row from below; what lies at or above it, little more than k elements, goes to a list in LDS, where a rank by
+//     comparison with all others sorts it; softmax, top-p and the draw run over the list.
+//   * everything else: thresholds by a histogram of the key's bits, three passes whatever the row holds, where
+//     bisection took one a bit.  top-p adds probabilities as whole numbers of 2^-60.
+// Microseconds, the kernel alone (by bisection, a bit a pass, before): 16 rows of 131,072 logits at T = 0.7 with top-k 50
+// and top-p 0.95 41 (1,612), top-p 0.9 alone 136 (840), neither 84 (166), top-k 2,000 135 (939), greedy 13 (24);
+// 64 rows of 32,000 30 (443), 46 (238), 27 (54), 45 (257), 8.5 (9.1).
+template <bool VEC>
 __global__ void __launch_bounds__(SNT)
 sample_kernel(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p,
               uint32_t seed_lo, uint32_t seed_hi, const int* __restrict__ counters,
               float* __restrict__ probs, int* __restrict__ out) {
-  __shared__ float shf[SNT + 1];
-  __shared__ int shi[SNT + 1];
-  __shared__ int sh_pick;
-  const int b = blockIdx.x, tid = threadIdx.x;
+  __shared__ SampleShared sh;
+  __shared__ Lists li;
+  const int b = blockIdx.x, tid = threadIdx.x, w = tid / WAVE, lane = tid % WAVE;
   const float* z_in = logits + (size_t)b * V;
   float* p = probs + (size_t)b * V;
 
-  if (!(temperature > 0.f)) {                           // greedy
+  if (!(temperature > 0.f)) {                           // greedy: of equal maxima the last index
     float best = -INFINITY;
     int bi = -1;
-    for (int i = tid; i < V; i += SNT) {
-      const float v = z_in[i];
+    visit<VEC>(z_in, V, [&](int i, float v) {
       if (bi < 0 || v >= best) { best = v; bi = i; }
+    });
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) {
+      const float v2 = __shfl_xor(best, o, WAVE);
+      const int i2 = __shfl_xor(bi, o, WAVE);
+      if (i2 >= 0 && (bi < 0 || v2 > best || (v2 == best && i2 > bi))) { best = v2; bi = i2; }
     }
-    shf[tid] = best;
-    shi[tid] = bi;
+    if (lane == 0) { sh.red[w] = best; sh.wave_count[w] = bi; }
     __syncthreads();
-    for (int o = SNT / 2; o > 0; o >>= 1) {
-      if (tid < o) {
-        const float v2 = shf[tid + o];
-        const int i2 = shi[tid + o];
-        if (i2 >= 0 && (shi[tid] < 0 || v2 > shf[tid] || (v2 == shf[tid] && i2 > shi[tid]))) {
-          shf[tid] = v2;
-          shi[tid] = i2;
-        }
+    if (tid == 0) {
+      for (int i = 1; i < SNT / WAVE; ++i) {
+        const float v2 = sh.red[i];
+        const int i2 = sh.wave_count[i];
+        if (i2 >= 0 && (bi < 0 || v2 > best || (v2 == best && i2 > bi))) { best = v2; bi = i2; }
       }
-      __syncthreads();
+      out[b] = bi;
     }
-    if (tid == 0) out[b] = shi[0];
     return;
   }
+  const float r = philox_uniform(seed_lo, seed_hi, (uint32_t)counters[2 * b + 1], (uint32_t)counters[2 * b]);
+  const auto order = [](float v) { return order_key(v); };
+  const auto bits = [](float v) { return __float_as_uint(v); };
 
-  // contiguous chunk of this thread, for the steps that go by index order
-  const int chunk = (V + SNT - 1) / SNT;
-  const int c0 = min(V, tid * chunk), c1 = min(V, c0 + chunk);
-
-  for (int i = tid; i < V; i += SNT) p[i] = z_in[i] / temperature;
-  __syncthreads();
-
-  if (top_k > 0 && top_k < V) {
-    // k-th largest by bisection on the ordered bit pattern
-    uint32_t thr = 0u;
-    for (int bit = 31; bit >= 0; --bit) {
-      const uint32_t cand = thr | (1u << bit);
-      int c = 0;
-      for (int i = tid; i < V; i += SNT) c += order_key(p[i]) >= cand;
-      if (block_sum_i(c, shi) >= top_k) thr = cand;
+  if (top_k > 0 && top_k < V && top_k <= MOST_TOP_K) {
+    uint32_t mine = 0u;
+    visit<VEC>(z_in, V, [&](int, float v) { mine = max(mine, order_key(v)); });
+    uint32_t bound = 0u;
+    for (int bit = 31; bit >= 12; --bit) {              // (a bound: its last bits may stay 0)
+      const uint32_t cand = bound | (1u << bit);
+      const int c = __popcll(__ballot(mine >= cand));
+      __syncthreads();
+      if (lane == 0) sh.wave_count[w] = c;
+      __syncthreads();
+      int all = 0;
+#pragma unroll
+      for (int i = 0; i < SNT / WAVE; ++i) all += sh.wave_count[i];
+      if (all >= top_k) bound = cand;
     }
-    int cge = 0, cgt = 0;
-    for (int i = c0; i < c1; ++i) {
-      const uint32_t k = order_key(p[i]);
-      cge += k >= thr;
-      cgt += k > thr;
-    }
-    const int n_ge = block_sum_i(cge, shi), n_gt = block_sum_i(cgt, shi);
-    if (n_ge <= top_k) {
-      for (int i = c0; i < c1; ++i)
-        if (order_key(p[i]) < thr) p[i] = -INFINITY;
-    } else {
-      int total;
-      int rank = block_excl_scan<int>(cge - cgt, shi, &total);   // ties before this chunk
-      const int keep_ties = top_k - n_gt;
-      for (int i = c0; i < c1; ++i) {
-        const uint32_t k = order_key(p[i]);
-        if (k < thr) p[i] = -INFINITY;
-        else if (k == thr) {
-          if (rank >= keep_ties) p[i] = -INFINITY;
-          ++rank;
+    // the passes go by the logits themselves (a division is 14 instructions, 12 us a pass over 131,072); two logits
+    // whose quotients round to one number lie within 2 units in the last place of each other, so 4 are a margin
+    bound = bound > 4u ? bound - 4u : 0u;
+    if (tid == 0) sh.count = 0;
+    __syncthreads();
+    update<VEC>(z_in, p, V, [&](int i, float v) {
+      if (order_key(v) >= bound) {
+        const int at = atomicAdd(&sh.count, 1);
+        if (at < CANDIDATES) { li.z[at] = v / temperature; li.idx[at] = i; }
+      }
+      return 0.f;
+    });
+    __syncthreads();
+    const int n = sh.count;
+    if (n <= CANDIDATES) {
+      // by value, of equal ones the smaller index first: the first k are kept
+      for (int c = tid; c < n; c += SNT) {
+        const uint32_t k = order_key(li.z[c]);
+        const int i = li.idx[c];
+        int rank = 0;
+        for (int o = 0; o < n; ++o) {
+          const uint32_t k2 = order_key(li.z[o]);
+          rank += k2 > k || (k2 == k && li.idx[o] < i);
         }
+        if (rank < top_k) { li.top_z[rank] = li.z[c]; li.top_i[rank] = i; }
+      }
+      __syncthreads();
+      const float mx = li.top_z[0], least = li.top_z[top_k - 1];
+      // (NaN fails the first; a last kept quotient among the denormals may be that of many logits)
+      if (mx < INFINITY && least > -INFINITY && fabsf(least) > 1e-30f) {
+        const bool have = tid < top_k;
+        const int my_i = have ? li.top_i[tid] : 0;
+        float e = have ? expf(li.top_z[tid] - mx) : 0.f;
+        const float sum = block_sum<SNT>(e, sh.red);
+        e = e / sum;
+        bool kept = have;
+        if (top_p > 0.f && top_p < 1.f) {
+          double total;
+          const double before = block_excl_scan<double>((double)e, sh.wave_sum, &total);
+          kept = have && before < (double)top_p;
+          const float new_sum = block_sum<SNT>(kept ? e : 0.f, sh.red);
+          e = kept ? e / new_sum : 0.f;
+        }
+        __syncthreads();
+        if (have) li.top_z[tid] = e;
+        if (tid == 0) sh.pick = V - 1;
+        __syncthreads();
+        if (kept) {
+          double run = 0.0;
+          for (int o = 0; o < top_k; ++o) run += li.top_i[o] <= my_i ? (double)li.top_z[o] : 0.0;
+          if (run >= (double)r) atomicMin(&sh.pick, my_i);
+          p[my_i] = e;                                  // (behind the zeros of the pass above: barriers lie between)
+        }
+        __syncthreads();
+        if (tid == 0) out[b] = r > 0.f ? sh.pick : 0;
+        return;
       }
     }
     __syncthreads();
+  }
+
+  update<VEC>(z_in, p, V, [&](int, float v) { return v / temperature; });
+  __syncthreads();
+  if (top_k > 0 && top_k < V) {
+    unsigned long long n_gt, n_at;
+    const uint32_t thr = select_key<VEC>(p, V, (unsigned long long)top_k, order, [](float) { return 1ull; }, sh, &n_gt, &n_at);
+    __syncthreads();
+    if (n_gt + n_at <= (unsigned long long)top_k) {
+      update<VEC>(p, p, V, [&](int, float v) { return order_key(v) < thr ? -INFINITY : v; });
+      __syncthreads();
+    } else {
+      keep_ties<VEC>(p, V, thr, top_k - (int)n_gt, -INFINITY, order, [](float v) { return v; }, sh);
+    }
   }
 
   // softmax
   float mx = -INFINITY;
-  for (int i = tid; i < V; i += SNT) mx = fmaxf(mx, p[i]);
-  mx = block_max<SNT>(mx, shf);
+  visit<VEC>(p, V, [&](int, float v) { mx = fmaxf(mx, v); });
+  mx = block_max<SNT>(mx, sh.red);
   float sum = 0.f;
-  for (int i = tid; i < V; i += SNT) {
-    const float e = expf(p[i] - mx);
-    p[i] = e;
+  update<VEC>(p, p, V, [&](int, float v) {
+    const float e = expf(v - mx);
     sum += e;
-  }
-  sum = block_sum<SNT>(sum, shf);
-  for (int i = tid; i < V; i += SNT) p[i] = p[i] / sum;
+    return e;
+  });
+  sum = block_sum<SNT>(sum, sh.red);
+  update<VEC>(p, p, V, [&](int, float v) { return v / sum; });
   __syncthreads();
+  if (!(sum > 0.f && sum < INFINITY)) {                 // infinities or NaN among the logits: no draw
+    if (tid == 0) out[b] = V - 1;
+    return;
+  }
 
   if (top_p > 0.f && top_p < 1.f) {
     // the largest t with sum(p_i >= t) >= top_p is the smallest kept probability
-    uint32_t thr = 0u;
-    for (int bit = 30; bit >= 0; --bit) {
-      const uint32_t cand = thr | (1u << bit);
-      float s = 0.f;
-      for (int i = tid; i < V; i += SNT) s += (__float_as_uint(p[i]) >= cand) ? p[i] : 0.f;
-      if (block_sum<SNT>(s, shf) >= top_p) thr = cand;
-    }
-    const float thr_f = __uint_as_float(thr);
-    float sgt = 0.f;
+    unsigned long long w_gt, w_at;
+    const uint32_t thr = select_key<VEC>(p, V, fixed60(top_p), bits, [](float v) { return fixed60(v); }, sh, &w_gt, &w_at);
+    const double thr_d = (double)__uint_as_float(thr), sum_gt = (double)w_gt / FIX;
     int ties = 0;
-    for (int i = c0; i < c1; ++i) {
-      const uint32_t k = __float_as_uint(p[i]);
-      if (k > thr) sgt += p[i];
-      ties += k == thr;
-    }
-    const float sum_gt = block_sum<SNT>(sgt, shf);
+    visit<VEC>(p, V, [&](int, float v) { ties += __float_as_uint(v) == thr; });
     int n_ties;
-    int rank = block_excl_scan<int>(ties, shi, &n_ties);
-    int keep_ties = (thr_f > 0.f) ? (int)ceilf((top_p - sum_gt) / thr_f) : n_ties;
-    keep_ties = max(1, min(keep_ties, n_ties));
-    const float new_sum = sum_gt + (float)keep_ties * thr_f;
-    for (int i = c0; i < c1; ++i) {
-      const uint32_t k = __float_as_uint(p[i]);
-      float v = p[i];
-      if (k < thr) v = 0.f;
-      else if (k == thr) {
-        if (rank >= keep_ties) v = 0.f;
-        ++rank;
-      }
-      p[i] = (new_sum > 0.f) ? v / new_sum : v;
-    }
-    __syncthreads();
-  }
-
-  // draw: first index whose running sum reaches r
-  const float r = philox_uniform(seed_lo, seed_hi, (uint32_t)counters[2 * b + 1],
-                                 (uint32_t)counters[2 * b]);
-  float local = 0.f;
-  for (int i = c0; i < c1; ++i) local += p[i];
-  float total;
-  const float before = block_excl_scan<float>(local, shf, &total);
-  if (tid == 0) sh_pick = V - 1;
-  __syncthreads();
-  if (c0 < c1 && before + local >= r) {
-    float run = before;
-    for (int i = c0; i < c1; ++i) {
-      run += p[i];
-      if (run >= r) {
-        atomicMin(&sh_pick, i);
-        break;
-      }
+    block_excl_scan<int>(ties, sh.wave_count, &n_ties);
+    int room = thr_d > 0.0 ? (int)fmin(ceil(((double)top_p - sum_gt) / thr_d), (double)n_ties) : n_ties;
+    room = max(1, min(room, n_ties));
+    const float new_sum = (float)(sum_gt + (double)room * thr_d);
+    const auto scaled = [&](float v) { return new_sum > 0.f ? v / new_sum : v; };
+    if (room >= n_ties) {
+      __syncthreads();
+      update<VEC>(p, p, V, [&](int, float v) { return __float_as_uint(v) < thr ? 0.f : scaled(v); });
+      __syncthreads();
+    } else {
+      keep_ties<VEC>(p, V, thr, room, 0.f, bits, scaled, sh);
     }
   }
-  __syncthreads();
-  if (tid == 0) out[b] = sh_pick;
+  draw_row<VEC>(p, V, r, sh, out + b);
 }
 
 }  // namespace tl
@@ -227,8 +471,10 @@ extern "C" int tl_sample(const float* logits, int B, int V, float temperature, i
                          hipStream_t st) {
   TL_REQUIRE(B >= 0 && V > 0, "sample: bad sizes B=%d V=%d", B, V);
   if (B == 0) return 0;
-  sample_kernel<<<B, SNT, 0, st>>>(logits, V, temperature, top_k, top_p, (uint32_t)(seed & 0xffffffffu),
-                                   (uint32_t)(seed >> 32), counters, probs, out);
+  const bool vec = V % 4 == 0 && ((uintptr_t)logits | (uintptr_t)probs) % 16 == 0;
+  const auto kernel = vec ? sample_kernel<true> : sample_kernel<false>;
+  kernel<<<B, SNT, 0, st>>>(logits, V, temperature, top_k, top_p, (uint32_t)(seed & 0xffffffffu),
+                            (uint32_t)(seed >> 32), counters, probs, out);
   TL_LAUNCH_CHECK("sample");
   return 0;
 }
