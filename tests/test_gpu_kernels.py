@@ -316,6 +316,32 @@ def test_philox_known_answer():
     assert int(philox_uniform(0, 0, 0) * 16777216) == 0x6627e8d5 >> 8
 
 
+@pytest.mark.parametrize("N,K", [(5, 36), (64, 2048), (250, 4100), (1030, 1024), (24, 8192), (70, 70)])
+def test_gemm_plain_adds_in_one_order(ops, N, K):
+    """The kernels for few rows, for a few tens and for many, and the one for operands whose rows are not aligned, give a
+    row the same bits; a sum of runs of L, groups and the whole has at most L + 16 roundings in a chain."""
+    a, w = rnd(200, K, seed=41).to(DEV), rnd(N, K, seed=42).to(DEV)
+    exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    L = (K + 1023) // 1024 * 16
+    base = torch.empty(200, N, device=DEV)
+    ops.gemm_plain(a, w, base)
+    assert float(((base.double() - exact).abs() / size).max()) < (L + 16) * 2.0 ** -24
+    for M in (1, 2, 3, 4, 7, 8, 9, 16, 17, 33, 64):
+        out = torch.empty(M, N, device=DEV)
+        ops.gemm_plain(a[:M].contiguous(), w, out)
+        assert torch.equal(out, base[:M]), M
+        ops.gemm_plain(a[:M].contiguous(), w, out, accumulate=True)
+        assert torch.equal(out, base[:M] + base[:M]), M
+    many = torch.empty(2600, N, device=DEV)                   # tiles of 64 x 64 where N is large enough
+    ops.gemm_plain(a.repeat(13, 1), w, many)
+    assert torch.equal(many, base.repeat(13, 1))
+    shifted = torch.empty(K * N + 1, device=DEV)[1:].view(N, K)
+    shifted.copy_(w)
+    out = torch.empty(9, N, device=DEV)
+    ops.gemm_plain(a[:9].contiguous(), shifted, out)          # not aligned: tiles of 64 x 64 whatever the size
+    assert torch.equal(out, base[:9])
+
+
 def run_sample(ops, logits, T, k=0, p=0.0, seed=0, counters=None):
     B, V = logits.shape
     counters = counters if counters is not None else [[b, 0] for b in range(B)]

@@ -2,82 +2,248 @@
 // product of the true 32-bit path, and the fallback for operand types that
 // the MFMA kernels do not take.  Weights are row-major [out, in] as the
 // checkpoint stores them (out[r] = sum_c W[r,c] x[c],
-// src/loader/parameters.rs:551-594 of the reference).  Each output element is
-// summed over k in ascending order whatever M is, so a row's result does not
-// depend on what else is in the batch.
+// src/loader/parameters.rs:551-594 of the reference).
+//
+// Every kernel here adds an output element in one order, which depends on K alone, so that a row's
+// result does not depend on what else is in the batch: K is cut into 8 groups of 8 runs of `run_length(K)`
+// channels; a run is summed over k in ascending order, a group over its runs, the result over its groups.
+// (The runs are what lets few rows spread over the chip: a chain of 8,192 additions in one thread is the
+// whole time of a product of one row.)
 #include "common.hpp"
 
 namespace tl {
 
-constexpr int BM = 64, BN = 64, BK = 16;
+constexpr int PG = 8, PR = 8;                     // groups of K, runs of a group
+constexpr int BK = 16;                            // runs are a multiple of this long
 
-template <typename TA, typename TW, bool ACCUMULATE>
-__global__ void __launch_bounds__(256)
-gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* __restrict__ C, int M,
-                  int N, int K, int lda, int ldw, int ldc) {
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Ws[BK][BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16, ty = tid / 16;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int lr = tid / 4, lk = (tid % 4) * 4;     // this thread loads row lr, 4 k's from lk
-  float acc[4][4];
+__host__ __device__ __forceinline__ int run_length(int K) { return (K + PG * PR * BK - 1) / (PG * PR * BK) * BK; }
+
+// Few rows of floats: a workgroup of 8 waves has 8 outputs' rows of W and up to MR rows of A.  A wave has a group
+// of K, its lanes the 64 pairs of an output and a run of the group; a lane's chain is one run long.  W comes in
+// coalesced pieces, 128 bytes of each of the 64 pairs at a time through the wave's own part of LDS, the next pieces
+// on their way in registers meanwhile.  Bound by the stream of W.  N / 8 workgroups fill the chip from N = 2,048 on;
+// tiles of 64 x 64 with a chain of all of K in a thread, which this replaced, made 32 workgroups there.
+// Microseconds at one row, tiles of 64 before: N x K = 2,048 x 8,192 19.4 and 525, 2,048 x 2,048 5.3 and 130,
+// 16,384 x 2,048 28.3 (4.7 TB/s) and 216.
+constexpr int CHUNK = 32;                         // channels of a pair that a wave brings in at a time
+template <int MR, bool ACCUMULATE>
+__global__ void __launch_bounds__(512)
+gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
+                       int K, int lda, int ldw, int ldc) {
+  __shared__ float stage[PG][64][CHUNK + 4];      // rows 144 bytes apart: 16-byte reads of 64 rows spread over the banks
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int n0 = blockIdx.x * 8, m0 = blockIdx.y * MR;
+  const int L = run_length(K);
+  const int run = lane / 8;                       // of this lane's pair: output lane % 8, run lane / 8
+  const int k0 = (wave * PR + run) * L;
+  const int rows = min(MR, M - m0);
+  float acc[MR];
+#pragma unroll
+  for (int m = 0; m < MR; ++m) acc[m] = 0.f;
+
+  // a load brings 128 bytes of 8 pairs: pair 8 i + lane / 8 (output lane / 8 of run i), 4 channels from 4 (lane % 8)
+  const int ln = n0 + lane / 8, lq = (lane % 8) * 4;
+  const float* wp = W + (size_t)min(ln, N - 1) * ldw;
+  f32x4 next[8];
+  const auto fetch = [&](int at) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int off = at + lq, k = (wave * PR + i) * L + off;
+      next[i] = (off < L && k < K && ln < N) ? *(const f32x4*)(wp + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  fetch(0);
+  for (int at = 0; at < L; at += CHUNK) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *(f32x4*)&stage[wave][i * 8 + lane / 8][lq] = next[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (at + CHUNK < L) fetch(at + CHUNK);
+    const int todo = min(CHUNK, L - at);          // (a multiple of 16)
+#pragma unroll 4
+    for (int q = 0; q < todo; q += 4) {
+      const f32x4 w = *(const f32x4*)&stage[wave][run * 8 + lane % 8][q];
+      const int k = k0 + at + q;
+      if (k < K) {                                // (K is a multiple of 4)
+        f32x4 a[MR];
+#pragma unroll
+        for (int m = 0; m < MR; ++m) a[m] = *(const f32x4*)(A + (size_t)(m0 + min(m, rows - 1)) * lda + k);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < MR; ++m) acc[m] = fmaf(a[m][j], w[j], acc[m]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  // the runs of a group in order, then the groups
+  __shared__ float sums[PG][MR][8];
+#pragma unroll
+  for (int m = 0; m < MR; ++m) {
+    float g = 0.f;
+#pragma unroll
+    for (int i = 0; i < PR; ++i) g += __shfl(acc[m], i * 8 + lane % 8, WAVE);
+    if (lane < 8) sums[wave][m][lane] = g;
+  }
+  __syncthreads();
+  const int m = threadIdx.x / 8, n = n0 + threadIdx.x % 8;
+  if (m < rows && n < N) {
+    float t = 0.f;
+#pragma unroll
+    for (int g = 0; g < PG; ++g) t += sums[g][m][threadIdx.x % 8];
+    float* c = C + (size_t)(m0 + m) * ldc + n;
+    *c = ACCUMULATE ? *c + t : t;
+  }
+}
+
+// 32 x 32 outputs a workgroup of 8 waves, each with a group of K and 4 x 4 outputs a lane, operands through the wave's
+// own part of LDS, the groups' sums through LDS at the end.  16 multiply-adds for two 16-byte reads of LDS a lane: the
+// vector pipes and LDS are about as busy as each other.  Eight times the waves of tiles of 64 x 64 with a thread's
+// chain over all of K for a product of the same size, and faster at every size measured, 1 to 1,024 rows:
+// N x K = 2,048 x 8,192 at 64 rows 76 us (563 with those), at 1,024 rows 575; 16,384 x 2,048 at 64 rows 78 (320).
+// VEC: rows of both operands may be read four channels at a time; else a channel a lane, 16 lanes along a row.
+template <typename T> __device__ __forceinline__ f32x4 four(const T* __restrict__ p) {
+  typedef __attribute__((ext_vector_type(4))) T T4;
+  const T4 t = *(const T4*)p;
+  return f32x4{to_f32(t[0]), to_f32(t[1]), to_f32(t[2]), to_f32(t[3])};
+}
+
+constexpr int GT = 32, GK = 16;
+template <typename TA, typename TW, bool VEC, bool ACCUMULATE>
+__global__ void __launch_bounds__(512)
+gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* __restrict__ C, int M, int N,
+                  int K, int lda, int ldw, int ldc) {
+  __shared__ float shared[PG * 2 * GK * (GT + 4)];
+  static_assert(PG * 2 * GK * (GT + 4) >= PG * GT * GT, "the sums of the groups take the operands' place");
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int tiles_n = (N + GT - 1) / GT;
+  const int m0 = (int)(blockIdx.x / tiles_n) * GT, n0 = (int)(blockIdx.x % tiles_n) * GT;
+  float (*As)[GT + 4] = (float (*)[GT + 4])(shared + wave * 2 * GK * (GT + 4));
+  float (*Ws)[GT + 4] = As + GK;
+  const int tx = lane % 8, ty = lane / 8;
+  const int L = run_length(K), first = wave * PR * L;
+  float group[4][4], acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-  const bool a_row = m0 + lr < M, w_row = n0 + lr < N;
-  const TA* ap = A + (size_t)(m0 + lr) * lda;
-  const TW* wp = W + (size_t)(n0 + lr) * ldw;
-  for (int k0 = 0; k0 < K; k0 += BK) {
+    for (int j = 0; j < 4; ++j) group[i][j] = acc[i][j] = 0.f;
+  // loads: rows lr, lr + RS, ..., VW channels from lk
+  constexpr int VW = VEC ? 4 : 1, RS = WAVE * VW / GK, LOADS = GT / RS;
+  const int lr = lane / (GK / VW), lk = lane % (GK / VW) * VW;
+  typedef __attribute__((ext_vector_type(VW))) float part;
+  part na[LOADS], nw[LOADS];
+  const auto fetch = [&](int k) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int kk = k0 + lk + i;
-      As[lk + i][lr] = (a_row && kk < K) ? to_f32(ap[kk]) : 0.f;
-      Ws[lk + i][lr] = (w_row && kk < K) ? to_f32(wp[kk]) : 0.f;
+    for (int h = 0; h < LOADS; ++h) {
+      const int m = m0 + lr + RS * h, n = n0 + lr + RS * h;
+      const TA* ap = A + (size_t)min(m, M - 1) * lda + k;
+      const TW* wp = W + (size_t)min(n, N - 1) * ldw + k;
+      if constexpr (VEC) {
+        na[h] = m < M && k < K ? four(ap) : f32x4{0.f, 0.f, 0.f, 0.f};
+        nw[h] = n < N && k < K ? four(wp) : f32x4{0.f, 0.f, 0.f, 0.f};
+      } else {
+        na[h] = m < M && k < K ? to_f32(*ap) : 0.f;
+        nw[h] = n < N && k < K ? to_f32(*wp) : 0.f;
+      }
     }
-    __syncthreads();
+  };
+  const int end = min(K, first + PR * L);
+  fetch(first + lk);
+  int in_run = 0;
+  for (int k0 = first; k0 < end; k0 += GK) {
 #pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      float a[4], b[4];
+    for (int h = 0; h < LOADS; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
+      for (int j = 0; j < VW; ++j) {
+        As[lk + j][lr + RS * h] = na[h][j];
+        Ws[lk + j][lr + RS * h] = nw[h][j];
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (k0 + GK < end) fetch(k0 + GK + lk);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Ws[kk][tx * 4 + j];
+    for (int kk = 0; kk < GK; ++kk) {
+      const f32x4 a = *(const f32x4*)&As[kk][ty * 4], b = *(const f32x4*)&Ws[kk][tx * 4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
     }
-    __syncthreads();
-  }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    in_run += GK;
+    if (in_run == L || k0 + GK >= end) {
+      in_run = 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float* c = C + (size_t)m * ldc + n;
-      *c = ACCUMULATE ? *c + acc[i][j] : acc[i][j];
+        for (int j = 0; j < 4; ++j) {
+          group[i][j] += acc[i][j];
+          acc[i][j] = 0.f;
+        }
     }
+  }
+  __syncthreads();
+  float* sums = shared + wave * GT * GT;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *(f32x4*)&sums[(ty * 4 + i) * GT + tx * 4] = f32x4{group[i][0], group[i][1], group[i][2], group[i][3]};
+  __syncthreads();
+  for (int e = threadIdx.x; e < GT * GT; e += 512) {
+    const int m = m0 + e / GT, n = n0 + e % GT;
+    if (m >= M || n >= N) continue;
+    float t = 0.f;
+#pragma unroll
+    for (int g = 0; g < PG; ++g) t += shared[g * GT * GT + e];
+    float* c = C + (size_t)m * ldc + n;
+    *c = ACCUMULATE ? *c + t : t;
   }
 }
 
-template <typename TA, typename TW>
-static int launch_plain(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldw,
-                        int ldc, int accumulate, hipStream_t st) {
-  dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+template <typename TA, typename TW, bool VEC>
+static int launch_tiles(const TA* A, const TW* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
+                        int accumulate, hipStream_t st) {
+  const long tiles = (long)((N + GT - 1) / GT) * ((M + GT - 1) / GT);
+  TL_REQUIRE(tiles < (1l << 31), "gemm: M=%d N=%d have more tiles than a grid holds", M, N);
   if (accumulate)
-    gemm_plain_kernel<TA, TW, true><<<grid, 256, 0, st>>>((const TA*)A, (const TW*)W, C, M, N, K, lda,
-                                                          ldw, ldc);
+    gemm_plain_kernel<TA, TW, VEC, true><<<(unsigned)tiles, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   else
-    gemm_plain_kernel<TA, TW, false><<<grid, 256, 0, st>>>((const TA*)A, (const TW*)W, C, M, N, K,
-                                                           lda, ldw, ldc);
+    gemm_plain_kernel<TA, TW, VEC, false><<<(unsigned)tiles, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   TL_LAUNCH_CHECK("gemm_plain");
   return 0;
+}
+
+template <int MR>
+static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
+                       int accumulate, hipStream_t st) {
+  dim3 grid((N + 7) / 8, (M + MR - 1) / MR);
+  if (accumulate)
+    gemm_plain_rows_kernel<MR, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+  else
+    gemm_plain_rows_kernel<MR, false><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+  TL_LAUNCH_CHECK("gemm_plain_rows");
+  return 0;
+}
+
+// The kernel for few rows reads W once for every 8 rows and has a thread's chain 64 times shorter than K; the tiles read
+// it once for 32.  Measured (rows / tiles, microseconds): N x K = 2,048 x 8,192 at 8 rows 32 / 65, at 16 52 / 68, at 32
+// 96 / 72; 3,072 x 2,048 at 8 14.4 / 18.6, at 16 21 / 19; 4,096 x 14,336 at 8 110 / 126, at 16 197 / 123; 16,384 x
+// 2,048 at 2 31 / 36, at 4 41 / 36; 32,000 x 2,048 at 2 58 / 65, at 4 76 / 65.
+static bool few_rows(int M, int N) { return M <= 2 || (M <= 16 && (long)M * N <= 32768); }
+
+template <typename TA, typename TW>
+static int launch_plain(const void* Av, const void* Wv, float* C, int M, int N, int K, int lda, int ldw,
+                        int ldc, int accumulate, hipStream_t st) {
+  const TA* A = (const TA*)Av;
+  const TW* W = (const TW*)Wv;
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 &&
+                   (uintptr_t)W % (4 * sizeof(TW)) == 0;
+  if (!vec) return launch_tiles<TA, TW, false>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+  if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4) {
+    if (few_rows(M, N)) {
+      if (M == 1) return launch_rows<1>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+      if (M == 2) return launch_rows<2>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+      if (M <= 4) return launch_rows<4>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+      return launch_rows<8>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+    }
+  }
+  return launch_tiles<TA, TW, true>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
 }
 
 }  // namespace tl
@@ -89,7 +255,7 @@ extern "C" int tl_gemm_plain(const void* A, int a_dt, const void* W, int w_dt, f
   TL_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
   TL_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: leading dimensions lda=%d ldw=%d ldc=%d too small "
              "for K=%d N=%d", lda, ldw, ldc, K, N);
-  TL_REQUIRE((M + BM - 1) / BM <= 65535, "gemm: M=%d has more row tiles than a grid holds", M);
+  TL_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d has more row tiles than a grid holds", M);
   if (M == 0) return 0;
   if (a_dt == DT_F32 && w_dt == DT_F32)
     return launch_plain<float, float>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
