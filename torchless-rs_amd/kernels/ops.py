@@ -1078,6 +1078,80 @@ def unary_act(u: torch.Tensor, activation: str, out: torch.Tensor, constants=Non
     _check(lib().tl_unary_act(_p(u), _code(u.dtype), ctypes.c_longlong(u.numel()), *code, _p(out), _code(out.dtype), _stream()))
 
 
+def grouped_experts_serve(y: torch.Tensor, up: torch.Tensor, down: torch.Tensor, ff: int, shared: int) -> bool:
+    """Do the products over each expert's own rows take these operands?  bfloat16, rows of whole 16-byte pieces."""
+    return (y.dtype == up.dtype == down.dtype == torch.bfloat16 and y.shape[1] % 8 == 0 and ff % 8 == 0 and shared % 8 == 0
+            and y.data_ptr() % 16 == 0 and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0)
+
+
+def group_pairs(chosen: torch.Tensor, E: int, offsets: torch.Tensor, order: torch.Tensor, place: torch.Tensor) -> None:
+    """The pairs n * top + k of `chosen` [n, top] sorted by expert, a row's place kept within one: `order` [n * top] the pair
+    at a position, `place` [n * top] a pair's position, `offsets` [E + 1] the experts' first positions; all int32."""
+    pairs = chosen.numel()
+    _req(chosen, "group_pairs.chosen", torch.int32)
+    _req(offsets, "group_pairs.offsets", torch.int32, (E + 1,))
+    _req(order, "group_pairs.order", torch.int32, (pairs,))
+    _req(place, "group_pairs.place", torch.int32, (pairs,))
+    _check(lib().tl_group_pairs(_p(chosen), pairs, int(E), _p(offsets), _p(order), _p(place), _stream()))
+
+
+MOST_SLICES = 8          # a shared expert runs along with the others in at most this many slices of an expert's size
+
+
+def shared_slices(ff: int, shared: int) -> int:
+    """Slices of at most `ff` channels of a shared expert (0: none, or too many to run along)."""
+    n = -(-shared // ff)
+    return n if n <= MOST_SLICES else 0
+
+
+def combine_pairs(z: torch.Tensor, place: torch.Tensor, out: torch.Tensor, accumulate: bool, slices: int = 0) -> None:
+    """out [n, H] (+)= the rows of z [n * (top + slices), H] that belong to the row's pairs, in the order of the slots, and those of
+    the shared expert's slices (float32)."""
+    n, H = out.shape
+    top = place.numel() // n
+    _req(z, "combine_pairs.z", torch.float32, (n * (top + slices), H))
+    _req(place, "combine_pairs.place", torch.int32, (n * top,))
+    _req(out, "combine_pairs.out", torch.float32)
+    _check(lib().tl_combine_pairs(_p(z), _p(place), n, top, int(slices), H, int(bool(accumulate)), _p(out), _stream()))
+
+
+def grouped_up(y: torch.Tensor, up: torch.Tensor, ff: int, shared: int, slices: int, offsets, order, top: int, weights, h: torch.Tensor,
+               activation=None, terms: Optional[GateTerms] = None, shared_weight=None) -> None:
+    """The experts' first halves over the rows that chose them: h [n * top, ff] at position p = the activation of row
+    y[order[p] // top] by its expert's rows of the stacked matrix `up`, with `weights` [n, E]; `activation` of
+    `EXPERT_ACTIVATIONS`, or `terms` for experts of [gate | up].  With `slices`: n positions more for each slice of the shared
+    expert (`shared_weight` [n] on its output)."""
+    n, H = y.shape
+    E, wide = weights.shape[1], 2 if terms is not None else 1
+    _req(y, "grouped_up.y", torch.bfloat16)
+    _req(up, "grouped_up.up", torch.bfloat16, (wide * (E * ff + shared), H))
+    _req(h, "grouped_up.h", torch.bfloat16, (n * (top + slices), ff))
+    _req(offsets, "grouped_up.offsets", torch.int32, (E + 1,))
+    _req(order, "grouped_up.order", torch.int32, (n * top,))
+    _req(weights, "grouped_up.weights", torch.float32, (n, E))
+    if activation in UNARY_CONSTANTS:
+        raise KernelError(f"grouped_up: {activation!r} takes learned numbers, which experts have none of")
+    code = 0 if terms is not None else _unary_args(activation, None)[0]
+    t = terms or GateTerms(1.0, 1.0, 0.0)
+    _check(lib().tl_gemm_grouped(_p(y), _p(up), _p(h), n, H, E, int(ff), int(shared), int(slices), int(top), _p(offsets), _p(order), _p(weights),
+                                 _shared_weight(shared_weight, n, "grouped_up"), 2 if terms is not None else 1, code, *t.args(), _stream()))
+
+
+def grouped_down(h: torch.Tensor, down: torch.Tensor, E: int, shared: int, slices: int, top: int, offsets: torch.Tensor, z: torch.Tensor) -> None:
+    """The experts' second halves: z float32 [positions, H] = h [positions, ff] by the position's expert's columns of the stacked
+    matrix `down` [H, E * ff + shared]; positions as in `grouped_up`."""
+    positions, ff = h.shape
+    H = down.shape[0]
+    n = positions // (top + slices)
+    _req(h, "grouped_down.h", torch.bfloat16, (n * (top + slices), ff))
+    _req(down, "grouped_down.down", torch.bfloat16, (H, E * ff + shared))
+    _req(offsets, "grouped_down.offsets", torch.int32, (E + 1,))
+    _req(z, "grouped_down.z", torch.float32, (positions, H))
+    t = GateTerms(1.0, 1.0, 0.0)
+    _check(lib().tl_gemm_grouped(_p(h), _p(down), _p(z), n, H, int(E), ff, int(shared), int(slices), int(top), _p(offsets), None, None, None, 0, 0,
+                                 *t.args(), _stream()))
+
+
 def expert_rows_up(y: torch.Tensor, up: torch.Tensor, chosen: torch.Tensor, weights: torch.Tensor, ff: int, shared: int,
                    activation: str, hs: torch.Tensor, constants=None, shared_weight: Optional[torch.Tensor] = None) -> None:
     """The chosen experts' first halves, row by row: hs[n, k*ff + j] = act(up[chosen[n,k]*ff + j] . y[n]) * weights[n, chosen[n,k]]

@@ -30,11 +30,11 @@ products of the framework's own kinds and no gather or scatter, whatever the tok
 reads every expert's weights in every step, as a step of many rows does anyway, and multiplies
 `n_experts / top` times what the chosen experts alone would.
 
-A step of many rows in bfloat16 (on average `GROUPED_ROWS_PER_EXPERT` rows an expert or more, more rows
-than the framework's own product kernels take, so that no graph holds the step) sorts the
-(row, chosen expert) pairs by expert and runs every expert's two products over its own rows
-(`_grouped`): the chosen experts' multiplications alone, at the price of one count per expert
-read back by the host.
+A step of more rows than the kernels for few rows take (`GROUPED_ROWS`, `GROUPED_SIZE`), in bfloat16, sorts
+the (row, chosen expert) pairs by expert and runs every expert's two products over its own rows
+(`_grouped`): the chosen experts' multiplications alone, in one launch for all experts, which finds
+its tiles on the device; the shared expert runs along as slices of an expert's size, or in steps of very
+many rows by the library's products.
 
 A step of few rows (rows * top <= n_experts: the rows cannot use every expert) runs the chosen
 experts alone: per row two products of its experts' matrices with a vector
@@ -55,7 +55,14 @@ from .base import FeedForward, flush_pending, register_part
 from .linear import Linear
 
 
-GROUPED_ROWS_PER_EXPERT = 128      # from this many rows an expert on average, experts run over their own rows
+# When experts run over their own rows.  Measured with both ways round (microseconds, grouped / side by side): 16 experts of
+# 3,584 channels, 4 a row, a shared one of 7,168: 16 rows 231 / 198, 24 rows 229 / 464, 64 rows 238 / 544, 128 rows 277 / 827,
+# 511 rows 367 / 758; gated ones of 1,792: 16 rows 216 / 166, 24 rows 221 / 337, 128 rows 294 / 568; 64 experts of 256, 2 a row:
+# 32 rows 62 / 51, 48 rows 63 / 140.
+GROUPED_ROWS = 16                  # up to here the kernels for few rows stream all experts' weights as fast as they come
+GROUPED_SIZE = 600000              # above, from this many rows times hidden channels of all experts
+GROUPED_ROWS_PER_EXPERT = 128      # or, above the own product kernels' rows, from this many rows an expert on average
+SLICED_ROWS = 512                  # up to here a shared expert runs along as slices (1,024 rows: 215 us against 140 by the library)
 
 
 class PlainFeedForward(FeedForward):
@@ -250,11 +257,51 @@ class RoutedExperts(FeedForward):
     def many_rows(self, ctx, y: torch.Tensor) -> bool:
         """Do the rows of `y` run expert by expert over each expert's own rows?"""
         n = y.shape[0]
-        return (y.dtype == torch.bfloat16 and self.up.weight.dtype == self.down.weight.dtype == torch.bfloat16
-                and n * self.top >= GROUPED_ROWS_PER_EXPERT * self.E and not self.up.own_kernels(n)
+        if not (y.dtype == self.up.weight.dtype == self.down.weight.dtype == torch.bfloat16):
+            return False
+        if self._serves(y):
+            if self.up.own_kernels(n):           # (a graph may hold the step: no product of the library's)
+                return (n > GROUPED_ROWS and n * self.total >= GROUPED_SIZE
+                        and (not self.shared or ops.shared_slices(self.ff, self.shared) > 0))
+            return n * self.top >= GROUPED_ROWS_PER_EXPERT * self.E or n * self.total >= GROUPED_SIZE
+        return (n * self.top >= GROUPED_ROWS_PER_EXPERT * self.E and not self.up.own_kernels(n)
                 and not ctx.host.get("fixed_launches"))
 
+    def _serves(self, y: torch.Tensor) -> bool:
+        return ops.grouped_experts_serve(y, self.up.weight, self.down.weight, self.ff, self.shared)
+
     def _grouped(self, ctx, y: torch.Tensor, out: torch.Tensor, accumulate: bool) -> None:
+        if not self._serves(y):
+            return self._grouped_library(ctx, y, out, accumulate)
+        n, E, top, ff, H = y.shape[0], self.E, self.top, self.ff, self.H
+        ws = ctx.workspace
+        weights, chosen, sw = self._route(ctx, y, True)
+        up_w, down_w = self.up.weight, self.down.weight
+        act = {"terms": self.gate_terms} if self.gated else {"activation": self.activation}
+        # the shared expert's slices write and read a row of float sums each, which the library's product of many rows does not
+        slices = ops.shared_slices(ff, self.shared) if self.shared and (n <= SLICED_ROWS or self.up.own_kernels(n)) else 0
+        offsets = ws.get("experts_offsets", (E + 1,), torch.int32)
+        order = ws.get("experts_order", (n * top,), torch.int32)
+        place = ws.get("experts_place", (n * top,), torch.int32)
+        ops.group_pairs(chosen, E, offsets, order, place)
+        h = ws.get("experts_gh", (n * (top + slices), ff), y.dtype)
+        ops.grouped_up(y, up_w, ff, self.shared, slices, offsets, order, top, weights, h, shared_weight=sw, **act)
+        z = ws.get("experts_gz", (n * (top + slices), H), torch.float32)
+        ops.grouped_down(h, down_w, E, self.shared, slices, top, offsets, z)
+        ops.combine_pairs(z, place, out, accumulate, slices)       # a row's experts in the order it chose them
+        if self.shared and not slices:
+            wide = 2 if self.gated else 1
+            us = ws.get("experts_su", (n, wide * self.shared), torch.float32)
+            ops.gemm(y, up_w[wide * E * ff:], us)
+            hs = ws.get("experts_sh", (n, self.shared), y.dtype)
+            if self.gated:
+                ops.expert_gated_act(us, None, 0, 0, self.shared, self.gate_terms, hs, sw)
+            else:
+                ops.expert_act(us, None, 0, self.shared, self.activation, hs, shared_weight=sw)
+            torch.addmm(out, hs, down_w[:, E * ff:].t(), out_dtype=torch.float32, out=out)
+
+    def _grouped_library(self, ctx, y: torch.Tensor, out: torch.Tensor, accumulate: bool) -> None:
+        """The same with the library's products, one expert after the other: sizes whose rows are no whole pieces of 16 bytes."""
         n, E, top, ff, H = y.shape[0], self.E, self.top, self.ff, self.H
         ws = ctx.workspace
         weights, chosen, sw = self._route(ctx, y, True)
