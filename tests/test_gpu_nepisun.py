@@ -800,3 +800,68 @@ def test_the_new_parts_serve_another_design(dtype):
     eng.free(s)
     close(torch.cat(got), want, dtype, "the same in portions of seven", margins[0])
     eng.close()
+
+
+def _recurrence_case(lens, heads, dv, N, G, seed, slow):
+    import math
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    n, B, inner = sum(lens), len(lens), heads * dv
+    C = inner + 2 * G * N
+    u = torch.nn.functional.silu(torch.randn(n, C, device="cuda", generator=g)).bfloat16()
+    proj = torch.randn(n, heads + 8, device="cuda", generator=g)
+    if slow:             # decays and steps as such layers are initialised: states that reach far back
+        A = torch.log(torch.empty(heads, device="cuda").uniform_(1.0, 16.0, generator=g))
+        bias = torch.log(torch.expm1(torch.exp(torch.empty(heads, device="cuda").uniform_(math.log(1e-3), math.log(1e-1), generator=g))))
+    else:
+        A, bias = 0.6 * torch.randn(heads, device="cuda", generator=g), 0.6 * torch.randn(heads, device="cuda", generator=g)
+    D = torch.randn(heads, device="cuda", generator=g)
+    state = torch.randn(B + 2, heads * N * dv + 24, device="cuda", generator=g)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device="cuda")
+    slots = torch.arange(B, 0, -1, dtype=torch.int32, device="cuda")
+    return u, proj, A, bias, D, state, cu, slots
+
+
+@pytest.mark.parametrize("lens, heads, dv, N, G", [([1], 2, 32, 32, 1), ([64, 1, 65], 4, 64, 128, 2), ([63, 200, 2, 128], 4, 32, 64, 4),
+                                                   ([130, 16, 17], 6, 96, 128, 3), ([7, 31, 33], 300, 64, 32, 1), ([321], 4, 64, 64, 1)])
+@pytest.mark.parametrize("slow", [True, False])
+def test_the_recurrence_by_chunks(lens, heads, dv, N, G, slow):
+    """Chunks of 64 rows on the matrix cores against float64, from a state that is not zero, with sequences in other slots than their
+    order: no further off than the row by row kernel is (both scatter; half as much again is the margin)."""
+    from torchless_rs_amd.kernels import ops
+    u, proj, A, bias, D, state, cu, slots = _recurrence_case(lens, heads, dv, N, G, sum(lens) + N, slow)
+    n, inner = u.shape[0], heads * dv
+    got = {}
+    for chunks in (False, True):
+        s, y = state.clone(), torch.full((n, inner), float("nan"), device="cuda")
+        ops.ssm_scan(u, proj, 8, G, N, heads, dv, bias, A, D, s, cu, slots, y, chunks=chunks)
+        got[chunks] = (y, s)
+    want_y, want_s = torch.empty(n, inner, dtype=torch.float64, device="cuda"), state.double()
+    for b, l in enumerate(lens):
+        r = slice(int(cu[b]), int(cu[b + 1]))
+        x = u[r, :inner].double().view(l, heads, dv)
+        Bm = u[r, inner:inner + G * N].double().view(l, G, N).repeat_interleave(heads // G, 1)
+        Cm = u[r, inner + G * N:].double().view(l, G, N).repeat_interleave(heads // G, 1)
+        dt = torch.nn.functional.softplus(proj[r, 8:].double() + bias.double(), threshold=1e9)
+        S = want_s[int(slots[b]), :heads * N * dv].view(heads, dv, N)
+        for i in range(l):
+            S *= torch.exp(-torch.exp(A.double()) * dt[i])[:, None, None]
+            S += (dt[i][:, None] * x[i])[:, :, None] * Bm[i][:, None, :]
+            want_y[int(cu[b]) + i] = ((S * Cm[i][:, None, :]).sum(-1) + D.double()[:, None] * x[i]).reshape(-1)
+    off = {c: [float((a.double() - w).norm() / w.norm()) for a, w in zip(got[c], (want_y, want_s))] for c in got}
+    assert all(a < 1.5 * b + 2.0 ** -24 for a, b in zip(off[True], off[False])), off
+    assert torch.equal(got[True][1][[0, len(lens) + 1]], state[[0, len(lens) + 1]])          # other slots
+    assert torch.equal(got[True][1][:, heads * N * dv:], state[:, heads * N * dv:])
+
+
+def test_which_recurrences_go_by_chunks():
+    """Sizes that the chunks do not take go row by row, and asking for chunks there is an error."""
+    from torchless_rs_amd.kernels import ops
+    for heads, dv, N, G, dtype in ((2, 32, 48, 1, torch.bfloat16), (2, 24, 32, 1, torch.bfloat16), (2, 32, 32, 1, torch.float32)):
+        u, proj, A, bias, D, state, cu, slots = _recurrence_case([40], heads, dv, N, G, 3, False)
+        y = torch.empty(40, heads * dv, device="cuda")
+        a, b = state.clone(), state.clone()
+        ops.ssm_scan(u.to(dtype), proj, 8, G, N, heads, dv, bias, A, D, a, cu, slots, y)
+        ops.ssm_scan(u.to(dtype), proj, 8, G, N, heads, dv, bias, A, D, b, cu, slots, y, chunks=False)
+        assert torch.equal(a, b)
+        with pytest.raises(ops.KernelError):
+            ops.ssm_scan(u.to(dtype), proj, 8, G, N, heads, dv, bias, A, D, a, cu, slots, y, chunks=True)

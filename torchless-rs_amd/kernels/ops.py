@@ -919,12 +919,21 @@ def ssm_conv(proj: torch.Tensor, off: int, C: int, w: torch.Tensor, bias, conv_s
                              _p(out), _code(out.dtype), _stream()))
 
 
+# Rows a sequence from which a step's recurrence goes by chunks: a chunk takes 8 us whatever its rows, a row by itself 0.6.
+# 128 heads of 128 x 64, microseconds, row by row / by chunks: 8 sequences of 4 rows 24 / 37, of 16 rows 45 / 37; one of 9 rows
+# 14.5 / 14, of 2,048 rows 1,215 / 255; four of 128 to 1,024 rows 838 / 165; one of 100 rows beside 63 of one 150 / 244.
+SSM_CHUNK_ROWS = 12
+
+
 def ssm_scan(u: torch.Tensor, proj: torch.Tensor, dt_off: int, G: int, N: int, heads: int, dv: int, dt_bias, A_log, D,
-             state: torch.Tensor, cu_seqlens, slots, y: torch.Tensor) -> None:
+             state: torch.Tensor, cu_seqlens, slots, y: torch.Tensor, chunks: Optional[bool] = None) -> None:
     """The recurrence of a state-space mixer over the rows of a step, sequence by sequence: u [n, heads*dv + 2*G*N]
     = [x | B | C] (after the convolution), dt at the columns dt_off .. of proj (float32 [n, width]);
     dt' = softplus(dt + dt_bias[h]), S <- exp(-exp(A_log[h]) dt') S + dt' B x^T, y = S^T C + D[h] x; `state`
-    float32 [slots, >= heads*N*dv] is read and left updated; y float32 [n, heads*dv]."""
+    float32 [slots, >= heads*N*dv] is read and left updated; y float32 [n, heads*dv].
+
+    bfloat16 steps of `SSM_CHUNK_ROWS` rows a sequence on average go by chunks of 64 rows on the matrix cores where the
+    sizes allow (`chunks`: the caller's choice; True is an error where they do not)."""
     n, C = u.shape
     B = slots.shape[0]
     _req(u, "ssm_scan.u")
@@ -938,6 +947,15 @@ def ssm_scan(u: torch.Tensor, proj: torch.Tensor, dt_off: int, G: int, N: int, h
     _req(cu_seqlens, "ssm_scan.cu_seqlens", torch.int32, (B + 1,))
     _req(slots, "ssm_scan.slots", torch.int32)
     _req(y, "ssm_scan.y", torch.float32, (n, heads * dv))
+    if chunks is None:
+        chunks = n >= SSM_CHUNK_ROWS * B and bool(lib().tl_ssm_chunks_serve(_code(u.dtype), C, G, N, heads, dv, _p(u), _p(state),
+                                                                            ctypes.c_longlong(state.stride(0))))
+    if chunks:
+        if u.dtype != torch.bfloat16:
+            raise KernelError("ssm_scan: chunks take bfloat16 rows")
+        _check(lib().tl_ssm_chunks(_p(u), C, G, N, heads, dv, _p(proj), proj.shape[1], int(dt_off), _p(dt_bias), _p(A_log), _p(D), _p(state),
+                                   ctypes.c_longlong(state.stride(0)), _p(cu_seqlens), _p(slots), n, B, _p(y), _stream()))
+        return
     _check(lib().tl_ssm_scan(_p(u), _code(u.dtype), C, G, N, heads, dv, _p(proj), proj.shape[1], int(dt_off), _p(dt_bias),
                              _p(A_log), _p(D), _p(state), ctypes.c_longlong(state.stride(0)), _p(cu_seqlens), _p(slots), n, B,
                              _p(y), _stream()))
