@@ -865,3 +865,44 @@ def test_which_recurrences_go_by_chunks():
         assert torch.equal(a, b)
         with pytest.raises(ops.KernelError):
             ops.ssm_scan(u.to(dtype), proj, 8, G, N, heads, dv, bias, A, D, a, cu, slots, y, chunks=True)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("taps", [1, 2, 4, 8])
+@pytest.mark.parametrize("C,off", [(8, 4), (1028, 0), (771, 0), (260, 3)])
+def test_convolution_of_rows_together_and_one_by_one(dtype, taps, C, off):
+    """Runs of rows (starts of sequences within and at the edge of a workgroup's rows) against the kernel of one row a
+    sequence, which keeps the same order of sums: the same bits, and the same block behind them."""
+    from torchless_rs_amd.kernels import ops
+    lens = [8, 29, 1, 5, 16, 3]
+    n, B, width = sum(lens), len(lens), off + C + (4 - (off + C) % 4) % 4
+    g = torch.Generator().manual_seed(C + taps)
+    proj, w, bias = (dev(torch.randn(*s, generator=g)) for s in ((n, width), (C, taps), (C,)))
+    first = dev(torch.randn(B + 2, taps * C, generator=g))
+    slots = [4, 0, 6, 2, 5, 1]
+    starts = [sum(lens[:b]) for b in range(B)]
+    out, one = (torch.empty(n, C, dtype=TORCH[dtype], device="cuda") for _ in range(2))
+    block, step = first.clone(), first.clone()
+    ops.ssm_conv(proj, off, C, w, bias, block, i32([b for b, t in enumerate(lens) for _ in range(t)]), i32(starts + [n]), i32(slots), out)
+    for b, t in enumerate(lens):
+        for r in range(starts[b], starts[b] + t):
+            ops.ssm_conv(proj[r:r + 1], off, C, w, bias, step, i32([0]), i32([0, 1]), i32([slots[b]]), one[r:r + 1], single=True)
+    assert torch.equal(out, one) and torch.equal(block, step)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("P,extra", [(4, 0), (30, 2), (1024, 4), (1028, 0), (1028, 1), (2052, 4), (4100, 0), (8192, 4), (8196, 0)])
+def test_gated_norm_of_parts_of_any_length(dtype, P, extra):
+    """Each share of a part a thread can have, and lengths and widths that rule out wide loads.  Float: P terms summed by 256
+    threads, a chain of at most 33, and a logistic function, a root and three products of a few units of 2^-24 each: within
+    4e-6 of the value; bfloat16: a rounding to 8 bits, 2^-8, on top."""
+    from torchless_rs_amd.kernels import ops
+    n, parts = 3, 2
+    inner = parts * P
+    g = torch.Generator().manual_seed(P)
+    y, proj, w = torch.randn(n, inner, generator=g), torch.randn(n, inner + extra, generator=g), torch.randn(inner, generator=g)
+    out = torch.empty(n, inner, dtype=TORCH[dtype], device="cuda")
+    ops.ssm_gate_norm(dev(y), dev(proj), parts, dev(w), 1e-5, out)
+    want = plain.gated_group_norm(y.double(), proj[:, :inner].double(), parts, 1e-5, w.double())
+    bound = (4e-6 if dtype == "float32" else 2.0 ** -8 + 4e-6) * want.abs() + 1e-7
+    assert bool(((out.double().cpu() - want).abs() <= bound).all())

@@ -28,26 +28,85 @@ __device__ __forceinline__ float softplus_f(float a) { return fmaxf(a, 0.f) + lo
 
 // out[n, c] = silu(bias[c] + sum_j w[c, j] * u[row - (taps-1-j), c]); rows before the step come
 // from the sequence's block, rows before the sequence are zeros (the block is zero then).
-template <typename T>
+//
+// Memory: every input read once and every output written once are 6 bytes an element (bfloat16 out), and the
+// logistic function is as much work again.  So a thread takes CV neighbouring channels (one load of 16 bytes)
+// down SSM_CONV_ROWS rows, all of whose inputs are asked for before the first is used; an input is read from
+// memory 11/8 times instead of `taps` times, and the filter once per 8 rows.  2,312 rows of 10,240 channels,
+// 4 taps: 116 -> 35 us (142 MB), the
+// same bits.  Rows at the start of a sequence, whose inputs come from two places, go one by one.
+constexpr int SSM_CONV_ROWS = 8;
+
+template <typename T, int CV, int TAPS>
 __global__ void __launch_bounds__(256)
 ssm_conv_kernel(const float* __restrict__ proj, int width, int off, int C, const float* __restrict__ w,
-                const float* __restrict__ bias, int taps, const float* __restrict__ conv_state, long long stride,
-                const int* __restrict__ row_seq, const int* __restrict__ cu_seqlens, const int* __restrict__ slots,
+                const float* __restrict__ bias, const float* __restrict__ conv_state, long long stride,
+                const int* __restrict__ row_seq, const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int n,
                 T* __restrict__ out) {
-  const int n = blockIdx.x;
-  const int c = blockIdx.y * 256 + threadIdx.x;
+  constexpr int RB = SSM_CONV_ROWS;
+  typedef float vec __attribute__((ext_vector_type(CV)));
+  const int n0 = blockIdx.x * RB, rows = min(RB, n - n0);
+  const int c = (blockIdx.y * 256 + threadIdx.x) * CV;
   if (c >= C) return;
-  const int b = row_seq[n];
-  const int i = n - cu_seqlens[b];
-  const float* old = conv_state + (long long)slots[b] * stride;
-  float acc = bias ? bias[c] : 0.f;
-  for (int j = 0; j < taps; ++j) {
-    const int back = taps - 1 - j;
-    const int src = i - back;
-    const float u = src >= 0 ? proj[(size_t)(n - back) * width + off + c] : old[(size_t)(taps - 1 + src) * C + c];
-    acc = fmaf(w[(size_t)c * taps + j], u, acc);
+  float wv[CV][TAPS], bv[CV];
+#pragma unroll
+  for (int e = 0; e < CV; ++e) {
+    bv[e] = bias ? bias[c + e] : 0.f;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) wv[e][j] = w[(size_t)(c + e) * TAPS + j];
   }
-  out[(size_t)n * C + c] = from_f32<T>(silu_f(acc));
+  const auto put = [&](int row, const vec (&u)[TAPS]) {
+    T r[CV];
+#pragma unroll
+    for (int e = 0; e < CV; ++e) {
+      float acc = bv[e];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) acc = fmaf(wv[e][j], u[j][e], acc);
+      r[e] = from_f32<T>(silu_f(acc));
+    }
+    T* o = out + (size_t)row * C + c;
+    if constexpr (CV == 4 && sizeof(T) == 2) {
+      bf16x4 v;
+#pragma unroll
+      for (int e = 0; e < CV; ++e) v[e] = r[e];
+      *reinterpret_cast<bf16x4*>(o) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < CV; ++e) o[e] = r[e];
+    }
+  };
+  const int b0 = row_seq[n0];
+  if (rows == RB && row_seq[n0 + RB - 1] == b0 && n0 - cu_seqlens[b0] >= TAPS - 1) {
+    const float* src = proj + (size_t)(n0 - (TAPS - 1)) * width + off + c;
+    vec u[RB + TAPS - 1];
+#pragma unroll
+    for (int r = 0; r < RB + TAPS - 1; ++r) u[r] = *reinterpret_cast<const vec*>(src + (size_t)r * width);
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      vec x[TAPS];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) x[j] = u[r + j];
+      put(n0 + r, x);
+    }
+    return;
+  }
+#pragma unroll 4
+  for (int r = 0; r < rows; ++r) {
+    const int row = n0 + r, b = row_seq[row], i = row - cu_seqlens[b];
+    const float* old = conv_state + (long long)slots[b] * stride;
+    vec x[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      const int from = i - (TAPS - 1 - j);
+      if (from >= 0) {
+        x[j] = *reinterpret_cast<const vec*>(proj + (size_t)(row - (TAPS - 1 - j)) * width + off + c);
+      } else {
+#pragma unroll
+        for (int e = 0; e < CV; ++e) x[j][e] = old[(size_t)(TAPS - 1 + from) * C + c + e];
+      }
+    }
+    put(row, x);
+  }
 }
 
 // The block's last taps-1 inputs after the step: from the step's rows, or shifted within the block.
@@ -247,7 +306,13 @@ ssm_scan_kernel(const T* __restrict__ u, int C, int inner, int G, int N, int hea
 }
 
 // out[n, part] = rms(y * silu(z)) * w over each of `parts` equal parts of the row.
-template <typename T>
+//
+// Memory: y and z once and the result, 10 bytes an element.  VL > 0 (the part's length, width and pointers allow
+// loads of 16 bytes and a thread's share of a part is at most VL of them): the gated values stay in registers
+// between the sum of squares and its use, so that nothing is read and no logistic function worked out twice; a
+// thread's terms of the sum are those neighbours.  VL == 0: any length.  2,312 rows of 8 parts of 1,024:
+// 50 -> 33 us (190 MB).
+template <typename T, int VL>
 __global__ void __launch_bounds__(256)
 ssm_gate_norm_kernel(const float* __restrict__ y, const float* __restrict__ proj, int width, int inner, int parts,
                      const float* __restrict__ w, float eps, T* __restrict__ out) {
@@ -256,22 +321,99 @@ ssm_gate_norm_kernel(const float* __restrict__ y, const float* __restrict__ proj
   const int P = inner / parts;
   const float* yr = y + (size_t)n * inner + part * P;
   const float* zr = proj + (size_t)n * width + part * P;
+  T* o = out + (size_t)n * inner + part * P;
   float ss = 0.f;
-  for (int i = threadIdx.x; i < P; i += 256) {
-    const float a = yr[i] * silu_f(zr[i]);
-    ss += a * a;
-  }
-  ss = block_sum<256>(ss, sh);
-  const float f = 1.0f / sqrtf(ss / (float)P + eps);
-  for (int i = threadIdx.x; i < P; i += 256) {
-    const float a = yr[i] * silu_f(zr[i]);
-    out[(size_t)n * inner + part * P + i] = from_f32<T>(a * f * w[part * P + i]);
+  if constexpr (VL > 0) {
+    f32x4 a[VL], z[VL];
+#pragma unroll
+    for (int k = 0; k < VL; ++k) {
+      const int i = (threadIdx.x + 256 * k) * 4;
+      a[k] = z[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (i < P) {
+        a[k] = *reinterpret_cast<const f32x4*>(yr + i);
+        z[k] = *reinterpret_cast<const f32x4*>(zr + i);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < VL; ++k) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a[k][e] *= silu_f(z[k][e]);
+        ss += a[k][e] * a[k][e];
+      }
+    }
+    ss = block_sum<256>(ss, sh);
+    const float f = 1.0f / sqrtf(ss / (float)P + eps);
+#pragma unroll
+    for (int k = 0; k < VL; ++k) {
+      const int i = (threadIdx.x + 256 * k) * 4;
+      if (i >= P) continue;
+      const f32x4 wv = *reinterpret_cast<const f32x4*>(w + part * P + i);
+      if constexpr (sizeof(T) == 2) {
+        bf16x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = (bf16)(a[k][e] * f * wv[e]);
+        *reinterpret_cast<bf16x4*>(o + i) = r;
+      } else {
+        f32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = a[k][e] * f * wv[e];
+        *reinterpret_cast<f32x4*>(o + i) = r;
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < P; i += 256) {
+      const float a = yr[i] * silu_f(zr[i]);
+      ss += a * a;
+    }
+    ss = block_sum<256>(ss, sh);
+    const float f = 1.0f / sqrtf(ss / (float)P + eps);
+    for (int i = threadIdx.x; i < P; i += 256) {
+      const float a = yr[i] * silu_f(zr[i]);
+      o[i] = from_f32<T>(a * f * w[part * P + i]);
+    }
   }
 }
 
 }  // namespace tl
 
 using namespace tl;
+
+template <typename T, int CV>
+static void conv_launch(const float* proj, int width, int off, int C, const float* w, const float* bias, int taps, const float* conv_state,
+                        long long stride, const int* row_seq, const int* cu_seqlens, const int* slots, int n, T* out, hipStream_t st) {
+  const dim3 grid((n + SSM_CONV_ROWS - 1) / SSM_CONV_ROWS, (C + 256 * CV - 1) / (256 * CV));
+#define TL_CONV(TAPS)                                                                                                                    \
+  case TAPS:                                                                                                                             \
+    ssm_conv_kernel<T, CV, TAPS><<<grid, 256, 0, st>>>(proj, width, off, C, w, bias, conv_state, stride, row_seq, cu_seqlens, slots, n, out); \
+    break
+  switch (taps) {
+    TL_CONV(1);
+    TL_CONV(2);
+    TL_CONV(3);
+    TL_CONV(4);
+    TL_CONV(5);
+    TL_CONV(6);
+    TL_CONV(7);
+    TL_CONV(8);
+  }
+#undef TL_CONV
+}
+
+template <typename T>
+static void gate_norm_launch(const float* y, const float* proj, int width, int inner, int parts, const float* w, float eps, int n, T* out,
+                             hipStream_t st) {
+  const int P = inner / parts;
+  const bool vec = P % 4 == 0 && width % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)proj % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const dim3 grid(n, parts);
+#define TL_GATE(VL) ssm_gate_norm_kernel<T, VL><<<grid, 256, 0, st>>>(y, proj, width, inner, parts, w, eps, out)
+  if (!vec || P > 8192) TL_GATE(0);
+  else if (P <= 1024) TL_GATE(1);
+  else if (P <= 2048) TL_GATE(2);
+  else if (P <= 4096) TL_GATE(4);
+  else TL_GATE(8);
+#undef TL_GATE
+}
 
 // How a head's dv columns are cut over workgroups and a workgroup's 256 lanes over its columns: lanes take DC = 4
 // columns each where dv allows it, a workgroup the largest part of dv of at most `most` columns (a multiple of DC).
@@ -353,13 +495,14 @@ int tl_ssm_conv(const float* proj, int width, int off, int C, const float* w, co
     TL_LAUNCH_CHECK("ssm_conv_single");
     return 0;
   }
-  const dim3 grid(n, (C + 255) / 256);
-  if (dt == DT_F32)
-    ssm_conv_kernel<float><<<grid, 256, 0, st>>>(proj, width, off, C, w, bias, taps, conv_state, stride, row_seq, cu_seqlens,
-                                                 slots, (float*)out);
-  else
-    ssm_conv_kernel<bf16><<<grid, 256, 0, st>>>(proj, width, off, C, w, bias, taps, conv_state, stride, row_seq, cu_seqlens,
-                                                slots, (bf16*)out);
+  const bool vec = C % 4 == 0 && width % 4 == 0 && off % 4 == 0 && (uintptr_t)proj % 16 == 0 && (uintptr_t)out % 16 == 0;
+  if (dt == DT_F32) {
+    if (vec) conv_launch<float, 4>(proj, width, off, C, w, bias, taps, conv_state, stride, row_seq, cu_seqlens, slots, n, (float*)out, st);
+    else conv_launch<float, 1>(proj, width, off, C, w, bias, taps, conv_state, stride, row_seq, cu_seqlens, slots, n, (float*)out, st);
+  } else {
+    if (vec) conv_launch<bf16, 4>(proj, width, off, C, w, bias, taps, conv_state, stride, row_seq, cu_seqlens, slots, n, (bf16*)out, st);
+    else conv_launch<bf16, 1>(proj, width, off, C, w, bias, taps, conv_state, stride, row_seq, cu_seqlens, slots, n, (bf16*)out, st);
+  }
   TL_LAUNCH_CHECK("ssm_conv");
   if (taps > 1) {
     ssm_conv_carry_kernel<<<dim3(B, (C + 255) / 256), 256, 0, st>>>(proj, width, off, C, taps, conv_state, stride, cu_seqlens,
@@ -422,11 +565,8 @@ int tl_ssm_gate_norm(const float* y, const float* proj, int width, int inner, in
   TL_REQUIRE(y && proj && w && out, "ssm_gate_norm: a buffer is missing");
   TL_REQUIRE(dt == DT_F32 || dt == DT_BF16, "ssm_gate_norm: unknown dtype code %d", dt);
   if (n == 0) return 0;
-  const dim3 grid(n, parts);
-  if (dt == DT_F32)
-    ssm_gate_norm_kernel<float><<<grid, 256, 0, st>>>(y, proj, width, inner, parts, w, eps, (float*)out);
-  else
-    ssm_gate_norm_kernel<bf16><<<grid, 256, 0, st>>>(y, proj, width, inner, parts, w, eps, (bf16*)out);
+  if (dt == DT_F32) gate_norm_launch(y, proj, width, inner, parts, w, eps, n, (float*)out, st);
+  else gate_norm_launch(y, proj, width, inner, parts, w, eps, n, (bf16*)out, st);
   TL_LAUNCH_CHECK("ssm_gate_norm");
   return 0;
 }
