@@ -1383,3 +1383,49 @@ def test_rotations_that_cannot_be_are_refused(ops):
         ops.rope_split(qkv, pos, ops.Rotation(inv[:3].contiguous(), 7), 2, 1, 16, q, k, v)    # odd
     with pytest.raises(ops.KernelError, match="inv_freq"):
         ops.rope_split(qkv, pos, ops.Rotation(inv, 8), 2, 1, 16, q, k, v)            # 9 frequencies for 4 pairs
+
+
+@pytest.mark.parametrize("M", [129, 192, 193, 256])
+@pytest.mark.parametrize("N,K", [(64, 768), (192, 832), (4096, 1024), (640, 4160), (4096, 14336)])
+def test_wide_products_in_slices_of_K(M, N, K):
+    """The slices' sums against float64.  A sum of K products kept in 32 bits, in any order, lies within K 2^-24 of the sum of
+    the products' sizes; the worst of M N chains is a few dozen standard errors of a walk, sqrt(K) 2^-24 of it, below 8."""
+    from torchless_rs_amd.kernels import ops
+    stages = K // 64
+    S = -(-stages // -(-stages // min(stages // 4, 16)))
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = (torch.randn(r, K, device="cuda", generator=g).bfloat16() for r in (M, N))
+    a[-1, -64:] *= 16
+    w[-1, :64] *= 16
+    parts = torch.full((S, M, N), float("nan"), device="cuda")
+    ops.gemm_wide_bf16(a, w, parts, S)
+    x = torch.randn(M, N, device="cuda", generator=g)
+    want = x.double() + a.double() @ w.double().t()
+    size = x.double().abs() + a.double().abs() @ w.double().abs().t()
+    ops.add_partials(x, parts)
+    assert bool(((x.double() - want).abs() <= 8 * K ** 0.5 * 2.0 ** -24 * size).all())
+
+
+def test_wide_products_are_refused_where_they_do_not_fit():
+    from torchless_rs_amd.kernels import ops
+    for M, N, K in ((128, 4096, 4096), (257, 4096, 4096), (192, 4100, 4096), (192, 4096, 4104), (192, 28672, 4096), (192, 4096, 512), (256, 4096, 4096)):
+        assert ops.wide_splits(M, N, K, 256) == 1
+    assert [ops.wide_splits(192, N, K, 256) for N, K in ((4096, 14336), (6144, 4096), (4096, 4096), (7168, 5120))] == [8, 5, 8, 4]
+    a, w = torch.zeros(192, 512, dtype=torch.bfloat16, device="cuda"), torch.zeros(96, 512, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(ops.KernelError, match="multiples of 64"):
+        ops.gemm_wide_bf16(a, w, torch.zeros(2, 192, 96, device="cuda"), 2)
+    w = torch.zeros(64, 512, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(ops.KernelError, match="without a stage"):
+        ops.gemm_wide_bf16(a, w, torch.zeros(5, 192, 64, device="cuda"), 5)
+
+
+@pytest.mark.parametrize("n,H,S", [(1, 1, 1), (3, 5, 2), (129, 64, 8), (2, 6, 3), (1, 4, 17)])
+def test_add_partials_in_order(n, H, S):
+    from torchless_rs_amd.kernels import ops
+    g = torch.Generator(device="cuda").manual_seed(n + H)
+    x, parts = torch.randn(n, H, device="cuda", generator=g), torch.randn(S + 1, n, H, device="cuda", generator=g)
+    want = x.clone()
+    for s in range(1, S + 1):
+        want += parts[s]
+    ops.add_partials(x, parts[1:])          # (an odd size: a base that no wide load may take)
+    assert torch.equal(x, want)

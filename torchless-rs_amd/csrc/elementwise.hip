@@ -216,12 +216,15 @@ add_rmsnorm_reg_kernel(float* __restrict__ x, const float* __restrict__ parts, i
   }
 }
 
-__global__ void add_partials_kernel(float* __restrict__ x, const float* __restrict__ parts, int n_parts,
-                                    size_t part_stride, size_t total) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// (V: f32x4 where the pointers and the count allow it: 8 parts of 192 x 4,096 in 6.4 us, by floats 7.7)
+template <typename V>
+__global__ void __launch_bounds__(256)
+add_partials_kernel(V* __restrict__ x, const V* __restrict__ parts, int n_parts, size_t total) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
-  float a = x[i];
-  for (int s = 0; s < n_parts; ++s) a += parts[s * part_stride + i];
+  V a = x[i];
+#pragma unroll 8
+  for (int s = 0; s < n_parts; ++s) a += parts[s * total + i];
   x[i] = a;
 }
 
@@ -911,7 +914,10 @@ int tl_add_partials(float* x, const float* parts, int n_parts, int n, int H, hip
   TL_REQUIRE(n >= 0 && H > 0 && n_parts >= 0, "add_partials: bad sizes n=%d H=%d parts=%d", n, H, n_parts);
   if (n == 0 || n_parts == 0) return 0;
   const size_t total = (size_t)n * H;
-  add_partials_kernel<<<(unsigned)((total + 255) / 256), 256, 0, st>>>(x, parts, n_parts, total, total);
+  if (total % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)parts % 16 == 0)
+    add_partials_kernel<f32x4><<<(unsigned)((total / 4 + 255) / 256), 256, 0, st>>>((f32x4*)x, (const f32x4*)parts, n_parts, total / 4);
+  else
+    add_partials_kernel<float><<<(unsigned)((total + 255) / 256), 256, 0, st>>>(x, parts, n_parts, total);
   TL_LAUNCH_CHECK("add_partials");
   return 0;
 }

@@ -1962,6 +1962,36 @@ def gemm_mid_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: 
     _check(lib().tl_gemm_mid_bf16(_p(a), _p(w), _p(out), M, N, K, int(n_split), epi, _stream()))
 
 
+WIDE_ROWS = 256      # most rows of the kernel that cuts a product of more than MID_ROWS rows along K
+
+
+def wide_splits(M: int, N: int, K: int, units: int) -> int:
+    """For MID_ROWS + 1 .. WIDE_ROWS rows: into how many slices `gemm_wide_bf16` cuts K, as many as make one round of
+    workgroups of 128 channels over the `units` compute units, each with four stages of 64 k at least; 1 where the BLAS
+    library's product is to be taken: sizes that are no multiples of 64, and two slices or fewer, where the
+    channels come near to filling the units by themselves (192 rows, with the partial sums added / the library's, microseconds:
+    16,384 x 4,096 in 2 slices 51 / 48, 12,288 x 2,048 in 2 30 / 27, 10,240 x 8,192 in 3 61 / 77, 7,168 x 5,120 in 4 34 / 43);
+    and partial sums, written and read, of more than one and a half times the weights' bytes (4,096 x 4,096 in 8, 192 rows
+    23 / 34, 256 rows 27 / 24; 8,192 x 1,024 in 4, 192 rows 24 / 21)."""
+    if not (MID_ROWS < M <= WIDE_ROWS and N % 64 == 0 and K % 64 == 0):
+        return 1
+    stages = K // 64
+    S = min(units // -(-N // 128), stages // 4, 16)
+    if S < 3 or 8 * S * M > 3 * K:
+        return 1
+    return -(-stages // -(-stages // S))            # (as many as have a stage)
+
+
+def gemm_wide_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int) -> None:
+    """Partial sums out float32 [n_split, M, N] of the product of up to WIDE_ROWS rows, N and K multiples of 64."""
+    M, K = a.shape
+    N = w.shape[0]
+    _req(a, "gemm.a", torch.bfloat16)
+    _req(w, "gemm.w", torch.bfloat16, (N, K))
+    _req(out, "gemm.out", torch.float32, (n_split, M, N))
+    _check(lib().tl_gemm_wide_bf16(_p(a), _p(w), _p(out), M, N, K, int(n_split), _stream()))
+
+
 def gemm_ring_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int = 1, accumulate: bool = False,
                    silu_pair: bool = False, waves: int = 4, kc: int = 128, pair_act: str = "silu") -> None:
     """`gemm_mid_bf16` through the kernel that brings both operands into a ring of stages in LDS

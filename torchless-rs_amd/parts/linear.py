@@ -69,14 +69,17 @@ class Linear:
 
     def partial(self, a: torch.Tensor, ctx, name: str):
         """The product as partial sums [S, M, N] (float32) for a reader that adds
-        them up, where that pays (17..MID_ROWS rows and K worth cutting); else None."""
-        if not self.mid(a):
-            return None
-        S = ops.mid_splits(a.shape[0], self.out_features, self.in_features, ops.compute_units(a.device))
+        them up, where that pays (17..WIDE_ROWS rows and K worth cutting); else None."""
+        M, N, K = a.shape[0], self.out_features, self.in_features
+        wide = M > ops.MID_ROWS
+        if wide:
+            S = ops.wide_splits(M, N, K, ops.compute_units(a.device)) if ops.bf16_gemm_ok(a, self.weight) else 1
+        else:
+            S = ops.mid_splits(M, N, K, ops.compute_units(a.device)) if self.mid(a) else 1
         if S == 1:
             return None
-        parts = ctx.workspace.get(name, (S, a.shape[0], self.out_features), torch.float32)
-        ops.gemm_mid_bf16(a, self.weight, parts, S)
+        parts = ctx.workspace.get(name, (S, M, N), torch.float32)
+        (ops.gemm_wide_bf16 if wide else ops.gemm_mid_bf16)(a, self.weight, parts, S)
         return parts
 
     def add_into(self, a: torch.Tensor, x: torch.Tensor, ctx, name: str) -> None:
