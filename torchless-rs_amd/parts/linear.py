@@ -69,17 +69,27 @@ class Linear:
 
     def partial(self, a: torch.Tensor, ctx, name: str):
         """The product as partial sums [S, M, N] (float32) for a reader that adds
-        them up, where that pays (17..WIDE_ROWS rows and K worth cutting); else None."""
+        them up, where that pays (17..MID_ROWS rows and K worth cutting); else None."""
+        if not self.mid(a):
+            return None
+        S = ops.mid_splits(a.shape[0], self.out_features, self.in_features, ops.compute_units(a.device))
+        if S == 1:
+            return None
+        parts = ctx.workspace.get(name, (S, a.shape[0], self.out_features), torch.float32)
+        ops.gemm_mid_bf16(a, self.weight, parts, S)
+        return parts
+
+    def wide_partial(self, a: torch.Tensor, ctx, name: str):
+        """The same for MID_ROWS + 1..WIDE_ROWS rows, where the sums go to the stream: the next norm adds them as it reads.
+        (q|k|v of a prompt would need a pass of its own for that: 24 + 6 us for 226 rows of 6,144 x 4,096, the library's 26.)"""
         M, N, K = a.shape[0], self.out_features, self.in_features
-        wide = M > ops.MID_ROWS
-        if wide:
-            S = ops.wide_splits(M, N, K, ops.compute_units(a.device)) if ops.bf16_gemm_ok(a, self.weight) else 1
-        else:
-            S = ops.mid_splits(M, N, K, ops.compute_units(a.device)) if self.mid(a) else 1
+        if not (ops.MID_ROWS < M <= ops.WIDE_ROWS and ops.bf16_gemm_ok(a, self.weight)):
+            return None
+        S = ops.wide_splits(M, N, K, ops.compute_units(a.device))
         if S == 1:
             return None
         parts = ctx.workspace.get(name, (S, M, N), torch.float32)
-        (ops.gemm_wide_bf16 if wide else ops.gemm_mid_bf16)(a, self.weight, parts, S)
+        ops.gemm_wide_bf16(a, self.weight, parts, S)
         return parts
 
     def add_into(self, a: torch.Tensor, x: torch.Tensor, ctx, name: str) -> None:
@@ -98,6 +108,8 @@ class Linear:
             ctx.prenormed = (norm, xt, ops.RowFactor(ssq, groups, form.size, form.eps))
             return
         parts = self.partial(a, ctx, name)
+        if parts is None:
+            parts = self.wide_partial(a, ctx, name)
         if parts is None:
             self(a, x, accumulate=True)
         else:
