@@ -1429,3 +1429,21 @@ def test_add_partials_in_order(n, H, S):
         want += parts[s]
     ops.add_partials(x, parts[1:])          # (an odd size: a base that no wide load may take)
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("M,N,K,sliced", [(128, 4096, 4096, True), (130, 4096, 4096, True), (256, 4096, 14336, True), (256, 4096, 4096, False), (257, 4096, 14336, False)])
+def test_products_into_the_stream_around_the_wide_rows(M, N, K, sliced):
+    """`add_into` at the edges of the rule: pending sums or the product at once, the same stream (bound as above)."""
+    from types import SimpleNamespace
+    from torchless_rs_amd.parts.base import flush_pending
+    from torchless_rs_amd.parts.linear import Linear
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a, w = (torch.randn(r, K, device="cuda", generator=g).bfloat16() for r in (M, N))
+    x = torch.randn(M, N, device="cuda", generator=g)
+    want = x.double() + a.double() @ w.double().t()
+    size = x.double().abs() + a.double().abs() @ w.double().abs().t()
+    ctx = SimpleNamespace(pending=None, norm_ahead=None, workspace=SimpleNamespace(get=lambda name, shape, dtype: torch.empty(shape, dtype=dtype, device="cuda")))
+    Linear(w).add_into(a, x, ctx, "parts")
+    assert (ctx.pending is not None) == sliced
+    flush_pending(ctx, x)
+    assert bool(((x.double() - want).abs() <= 8 * K ** 0.5 * 2.0 ** -24 * size).all())

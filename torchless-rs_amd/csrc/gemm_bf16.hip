@@ -17,8 +17,10 @@
 //    single-token steps, with rotation and the write into the cache's pages.
 //  * gemm_mid: 17..128 rows.  The activations of a k-step are shared by the four
 //    waves through LDS; K may be cut over workgroups into partial sums.
-// Products with more rows (prefill, large decode batches) are the BLAS library's, as the
-// reference hands its products to the vendor's library.
+//  * gemm_ring: the same rows where K is a multiple of 128, both operands through a ring in LDS.
+//  * gemm_wide: 129..256 rows into the stream where the channels leave compute units idle.
+// Products with more rows (prefill, large decode batches) and those that gemm_wide does not serve are the BLAS
+// library's, as the reference hands its products to the vendor's library.
 //
 // All need K % 8 == 0 and 16-byte aligned rows; callers fall back to the
 // plain kernel otherwise.

@@ -1895,8 +1895,8 @@ LIBRARY_ROWS = 64   # where K is no such multiple, the BLAS library's product be
 
 
 def own_rows(K: int) -> int:
-    """The most rows for which a bfloat16 product over K runs in this package's own kernels (more
-    go to the BLAS library)."""
+    """The most rows for which a bfloat16 product over K always runs in this package's own kernels (of more, those that
+    `wide_splits` takes do; the others go to the BLAS library)."""
     return MID_ROWS if K % RING_K == 0 else LIBRARY_ROWS
 
 
