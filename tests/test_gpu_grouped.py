@@ -171,3 +171,62 @@ def test_a_graph_of_a_routed_step(n):
         want = h @ part.down.weight.double().T
         # the hidden channels are rounded to bfloat16: a thousand and more of them, so far below 2^-8 of a result's size
         assert float((out[sure].double() - want[sure]).norm() / want[sure].norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("E,top,groups,keep,options", [
+    (16, 4, 0, 0, {}), (16, 4, 4, 2, {}), (130, 3, 0, 0, {"logistic": True}), (24, 6, 4, 2, {"logistic": True, "correction": True, "two_largest": True}),
+    (8, 8, 0, 0, {"normalise_eps": 0.0}), (5, 2, 0, 0, {"correction": True})])
+@pytest.mark.parametrize("n", [9, 70])
+def test_rows_whose_scores_are_not_numbers_choose_experts(ops, n, E, top, groups, keep, options):
+    """NaN and infinite rows among others: every slot holds an expert and no expert twice, the row's NaN stays in its weights,
+    and the other rows have the bits they have without them."""
+    W = 64
+    g = torch.Generator(device=DEV).manual_seed(n + E)
+    y, router = (torch.randn(r, W, generator=g, device=DEV) for r in (n, E))
+    if options.get("correction"):
+        options = dict(options, correction=torch.randn(E, generator=g, device=DEV))
+    bad = {1: float("nan"), 3: float("inf"), n - 1: -float("inf")}
+    spoilt = y.clone()
+    for row, value in bad.items():
+        spoilt[row, row % W] = value
+    spoilt[1] = float("nan")
+    results = []
+    for rows in (y, spoilt):
+        weights, chosen = torch.empty(n, E, device=DEV), torch.full((n, top), -1, dtype=torch.int32, device=DEV)
+        ops.route(rows, router, groups, keep, top, weights, chosen, **options)
+        assert int(chosen.min()) >= 0 and int(chosen.max()) < E
+        assert bool((chosen.sort(dim=1).values.diff(dim=1) > 0).all()) or top == 1
+        results.append((weights, chosen))
+    (weights, chosen), (w_spoilt, c_spoilt) = results
+    well = [r for r in range(n) if r not in bad]
+    assert torch.equal(weights[well], w_spoilt[well]) and torch.equal(chosen[well], c_spoilt[well])
+    assert bool(w_spoilt[1][c_spoilt[1].long()].isnan().all())
+
+
+@pytest.mark.parametrize("n", [20, 64, 200])
+def test_a_routed_step_with_rows_that_are_not_numbers(n):
+    """The rows beside one of NaN keep their bits; its own result is NaN."""
+    from types import SimpleNamespace
+    from torchless_rs_amd.parts import ffn_routed
+    from torchless_rs_amd.parts.base import Workspace
+    H, E, top, ff = 64, 16, 4, 3000
+    part = ffn_routed.RoutedExperts(H, E, top, ff, shared_size=64, activation="relu2")
+    g = torch.Generator(device=DEV).manual_seed(n)
+    part.load({k: (torch.randn(v.shape, generator=g, device=DEV) * v.shape[-1] ** -0.5).bfloat16() for k, v in part.weight_specs().items()},
+              torch.bfloat16)
+    y = torch.randn(n, H, generator=g, device=DEV).bfloat16()
+    spoilt = y.clone()
+    spoilt[[2, n - 1]] = float("nan")
+    out = []
+    for rows in (y, spoilt):
+        ctx = SimpleNamespace(workspace=Workspace(torch.device(DEV)), dtype=torch.bfloat16, host={}, pending=None)
+        assert part.many_rows(ctx, rows)
+        ctx.workspace.get("experts_chosen", (n, top), torch.int32).fill_(-1)
+        ctx.workspace.get("experts_place", (n * top,), torch.int32).fill_(0)
+        x = torch.empty(n, H, device=DEV)
+        part._grouped(ctx, rows, x, False)
+        out.append(x)
+    well = [r for r in range(n) if r not in (2, n - 1)]
+    # (which rows share a tile may change with the choices of two, which changes no row's order of sums)
+    assert torch.equal(out[0][well], out[1][well])
+    assert bool(out[1][[2, n - 1]].isnan().all())

@@ -7,7 +7,9 @@
 // chosen (groups == 0: every expert can).  Of those the `top` with the largest c are chosen; their
 // weights are their s, as they are or divided by (their sum + normalise_eps) (`normalise`).  Of equal
 // scores the one with the smaller index goes first.  A shared expert may have a weight of its own, the
-// logistic function of one more row of the router's matrix (`shared_weight`).
+// logistic function of one more row of the router's matrix (`shared_weight`).  A score that is not a number goes
+// first in the choice: its expert is chosen with its NaN, which so stays in the row's result, and a row has `top`
+// different experts whatever its scores.
 //
 // `route` leaves the weights as a row of E floats, zero for an expert that was not chosen.
 // The experts run as ONE wide feed-forward: the rows of all up projections stacked (the shared
@@ -30,6 +32,9 @@ struct RouteTerms {
   float* shared_weight;      // [n] or null; with it the router's matrix has a row E
   const float* bias;         // [E] on the products, or null
 };
+
+// what the choice goes by: numbers that compare
+__device__ __forceinline__ float ranked(float c) { return isnan(c) ? INFINITY : c; }
 
 template <typename T, int NT>
 __global__ void __launch_bounds__(NT)
@@ -86,7 +91,7 @@ route_kernel(const T* __restrict__ h, int W, const float* __restrict__ wr, int E
     for (int e = t; e < E; e += NT) s_s[e] = expf(s_s[e] - m) / sum;
   }
   __syncthreads();
-  for (int e = t; e < E; e += NT) c_s[e] = s_s[e] + (k.correction ? k.correction[e] : 0.f);
+  for (int e = t; e < E; e += NT) c_s[e] = ranked(s_s[e] + (k.correction ? k.correction[e] : 0.f));
   __syncthreads();
   if (groups > 0) {
     const int per = E / groups;
@@ -97,7 +102,7 @@ route_kernel(const T* __restrict__ h, int W, const float* __restrict__ wr, int E
         second = fmaxf(second, fminf(best, c));
         best = fmaxf(best, c);
       }
-      g_s[g] = k.two_largest && per > 1 ? best + second : best;
+      g_s[g] = ranked(k.two_largest && per > 1 ? best + second : best);
     }
     __syncthreads();
     for (int g = t; g < groups; g += NT) {
