@@ -44,6 +44,18 @@ def test_group_pairs(ops, n, E, top, crowded):
     assert torch.equal(off.long(), torch.cat([torch.zeros(1, dtype=torch.long, device=DEV), torch.bincount(flat, minlength=E).cumsum(0)]))
 
 
+def test_pairs_of_numbers_that_are_no_experts_have_places(ops):
+    """What goes by `order` and `place` stays in its buffers whatever the choice holds."""
+    chosen = choose(300, 6, 3, 5, False)
+    chosen[7, 1], chosen[8, 0], chosen[299, 2], chosen[0, 0] = -1, 6, 2 ** 31 - 1, -2 ** 31
+    off, order, place = (torch.full((s,), -9, dtype=torch.int32, device=DEV) for s in (7, 900, 900))
+    ops.group_pairs(chosen, 6, off, order, place)
+    flat = chosen.clamp(0, 5).view(-1).long()
+    want = torch.argsort(flat, stable=True)
+    assert torch.equal(order.long(), want) and torch.equal(place.long()[want], torch.arange(900, device=DEV))
+    assert off.tolist() == [0] + flat.bincount(minlength=6).cumsum(0).tolist()
+
+
 CASES = [  # n, H, E, top, ff, shared, gated, on_input, crowded
     (1, 64, 4, 2, 64, 64, False, False, False), (33, 72, 6, 2, 40, 24, True, False, True), (160, 128, 2, 1, 256, 512, False, False, False),
     (161, 200, 3, 2, 264, 600, True, True, True), (320, 8, 5, 4, 8, 64, False, False, True), (700, 256, 16, 4, 136, 0, True, True, False),

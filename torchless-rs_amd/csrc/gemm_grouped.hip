@@ -21,7 +21,9 @@ namespace tl {
 // chosen [n_pairs] expert numbers -> offsets [E + 1], order [n_pairs]: position -> pair, place [n_pairs]: pair ->
 // position.  A workgroup an expert: it counts the pairs of smaller experts and its own (every workgroup reads all
 // of `chosen`, a few tens of KB from L2), then deals its pairs their positions, wave after wave.  6 us for 9,248 pairs
-// of 16 experts, where a sort, a count and their index kernels took 80.
+// of 16 experts, where a sort, a count and their index kernels took 80.  A number that is no expert's counts as the
+// nearest expert's, so that `order` and `place` are a permutation, and what goes by them stays in its buffers, whatever
+// `chosen` holds.
 constexpr int GP_WAVES = 16;
 __global__ void __launch_bounds__(GP_WAVES * WAVE)
 group_pairs_kernel(const int* __restrict__ chosen, int n_pairs, int E, int* __restrict__ offsets, int* __restrict__ order,
@@ -34,7 +36,7 @@ group_pairs_kernel(const int* __restrict__ chosen, int n_pairs, int E, int* __re
   int less = 0, mine = 0;
 #pragma unroll 4
   for (int i = lo + lane; i < hi; i += WAVE) {
-    const int c = chosen[i];
+    const int c = min(max(chosen[i], 0), E - 1);
     less += c < e;
     mine += c == e;
   }
@@ -59,7 +61,7 @@ group_pairs_kernel(const int* __restrict__ chosen, int n_pairs, int E, int* __re
   int at = first + before;
   for (int base = lo; base < hi; base += WAVE) {
     const int i = base + lane;
-    const bool hit = i < hi && chosen[i] == e;
+    const bool hit = i < hi && min(max(chosen[i], 0), E - 1) == e;
     const unsigned long long hits = __ballot(hit);
     if (hit) {
       const int pos = at + __popcll(hits & ((1ull << lane) - 1ull));

@@ -1104,7 +1104,8 @@ def grouped_experts_serve(y: torch.Tensor, up: torch.Tensor, down: torch.Tensor,
 
 def group_pairs(chosen: torch.Tensor, E: int, offsets: torch.Tensor, order: torch.Tensor, place: torch.Tensor) -> None:
     """The pairs n * top + k of `chosen` [n, top] sorted by expert, a row's place kept within one: `order` [n * top] the pair
-    at a position, `place` [n * top] a pair's position, `offsets` [E + 1] the experts' first positions; all int32."""
+    at a position, `place` [n * top] a pair's position, `offsets` [E + 1] the experts' first positions; all int32.  A number
+    outside 0..E-1 counts as the nearest expert's."""
     pairs = chosen.numel()
     _req(chosen, "group_pairs.chosen", torch.int32)
     _req(offsets, "group_pairs.offsets", torch.int32, (E + 1,))
