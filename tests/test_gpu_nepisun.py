@@ -853,6 +853,41 @@ def test_the_recurrence_by_chunks(lens, heads, dv, N, G, slow):
     assert torch.equal(got[True][1][:, heads * N * dv:], state[:, heads * N * dv:])
 
 
+@pytest.mark.parametrize("heads, dv, N, G", [(2, 32, 32, 1), (2, 32, 64, 2), (130, 64, 64, 1), (4, 32, 128, 2), (130, 64, 128, 2)])
+@pytest.mark.parametrize("row", [0, 70, 149])
+@pytest.mark.parametrize("what, value", [("x", "nan"), ("x", "inf"), ("B", "-inf"), ("C", "nan"), ("C", "inf"), ("dt", "nan"), ("dt", "inf"),
+                                         ("state", "inf"), ("state", "nan"), ("A", "nan")])
+def test_a_chunk_with_a_number_that_is_none(heads, dv, N, G, row, what, value):
+    """A NaN or infinity in the first, a middle or the last row of a sequence reaches what it reaches row by row, and nothing else:
+    no row before its own, no other column, head or sequence."""
+    from torchless_rs_amd.kernels import ops
+    lens = [90, 150, 64]
+    u, proj, A, bias, D, state, cu, slots = _recurrence_case(lens, heads, dv, N, G, N + row, True)
+    n, inner, at, bad = sum(lens), heads * dv, 90 + row, float(value)
+    u = u.clone()
+    if what == "x":
+        u[at, inner - 3] = bad
+    elif what in "BC":
+        u[at, inner + (G * N if what == "C" else 0) + N // 2 + 1] = bad
+    elif what == "dt":
+        proj[at, 8 + heads - 1] = bad
+    elif what == "state":
+        state[int(slots[1]), 5 * N + 7] = bad
+    else:
+        A[heads - 1] = bad
+    got = []
+    for chunks in (False, True):
+        s, y = state.clone(), torch.empty(n, inner, device="cuda")
+        ops.ssm_scan(u, proj, 8, G, N, heads, dv, bias, A, D, s, cu, slots, y, chunks=chunks)
+        got.append((y, s))
+    assert not bool(got[0][0].isfinite().all())
+    for a, b in zip(*got):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+        assert torch.equal(a[a.isinf()], b[b.isinf()])
+        ok = a.isfinite()
+        assert float((a[ok].double() - b[ok].double()).norm() / a[ok].double().norm()) < 2e-6
+
+
 def test_which_recurrences_go_by_chunks():
     """Sizes that the chunks do not take go row by row, and asking for chunks there is an error."""
     from torchless_rs_amd.kernels import ops

@@ -13,6 +13,11 @@
 // A workgroup has 16 columns of one head of one sequence a wave and goes through the sequence's chunks, the state in its
 // accumulators: lane (li, kg) of a wave holds S[n][d] for d = li and n = 16 t + 4 kg + r.  Two such tiles are, as they lie,
 // an operand of the first product, whose 32 terms a lane may name in any order as long as C's operand follows it.
+//
+// The products give every row of a chunk a term of every other, with weight 0 where there is none, and take floats apart
+// into terms: a NaN or an infinity spreads to rows before its own, and an infinite state becomes NaN.  Whatever x, B, C, dt
+// or state holds one, some y of the chunk is not finite then (each has its term in one, be it with weight 0).  The workgroup
+// leaves the chunks there and goes on row by row from the state before that one.
 // What bounds it: a chunk's way of phases (rows to LDS, weights, products), each short and behind the one before: 8 us a
 // chunk, where its 130 products of 16 cycles a wave take 0.9, its splits about as long and its traffic in LDS 0.8; a
 // second workgroup on the compute unit fills gaps (5 us a chunk).
@@ -58,11 +63,13 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
   __shared__ __attribute__((aligned(16))) bf16 Cs[SC * N], Bs[SC * N], Bt[N * SC], xT[16 * WV * SC];
   __shared__ __attribute__((aligned(16))) bf16 Ms[3][6 * 512];         // blocks of 16 rows x 32 places of the lower triangle
   __shared__ __attribute__((aligned(16))) Decays decays[2];            // of this chunk and of the next
+  __shared__ int spoilt;                                               // a chunk's y were not all finite
   const int h = blockIdx.x, b = blockIdx.y, t = threadIdx.x, wave = t / WAVE, lane = t % WAVE, li = lane % 16, kg = lane / 16;
   const int d0 = blockIdx.z * (16 * WV), g = h / (heads / G);
   const int row0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - row0;
   if (n_new <= 0) return;
-  const double rate = -(double)expf(A_log[h]) * 1.4426950408889634;
+  const float neg_rate = -expf(A_log[h]);
+  const double rate = (double)neg_rate * 1.4426950408889634;
   const float bias = dt_bias[h], skip = Dw[h];
 
   // the state: this lane's column and rows
@@ -101,8 +108,9 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
     const bool row = i0 + lane < n_new;
     const float dt = row ? sc_softplus(raw + bias) : 0.f;
     load_dt(i0 + SC);
-    // (a decay this small is 0 in a float: the cut keeps differences of sums finite)
-    double c = row ? fmax(rate * (double)dt, -1e6) : 0.0;
+    // (a decay this small is 0 in a float: the cut keeps differences of sums finite; NaN stays)
+    double c = row ? rate * (double)dt : 0.0;
+    c = c < -1e6 ? -1e6 : c;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
       const double p = __shfl_up(c, o, WAVE);
@@ -117,6 +125,8 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
     out.weight[lane] = exp2f((float)(all - c)) * dt;
   };
   typedef __attribute__((ext_vector_type(2))) __bf16 pair;
+  int from = n_new;                                      // the first row that this wave takes by itself
+  if (t == 0) spoilt = 0;
   load(0);
   if (wave == WV - 1) {
     load_dt(0);
@@ -131,14 +141,21 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
     const Decays& dec = decays[i0 / SC % 2];
     const int rows = min(SC, n_new - i0);
     __syncthreads();                                     // the last chunk has been read
+    const int leave = spoilt;
+    // where registers are too few to keep the places in LDS over all chunks (eight waves a unit, states of 128 rows: 44 spilled), the
+    // thread's number is opaque and the places are worked out anew: 64 sequences of 13 rows 173 us, with spills 293; where they are
+    // not, that costs a tenth (one of 2,048 rows 279 against 255)
+    int tl = t;
+    if constexpr (NT == 8 && WV == 4) asm volatile("" : "+v"(tl));
+    const int li = tl % 16, kg = tl / 16 % 4;
 #pragma unroll
     for (int k = 0; k < CL; ++k) {
-      const int e = t + THREADS * k, r = e / NC, c = e % NC;
+      const int e = tl + THREADS * k, r = e / NC, c = e % NC;
       *reinterpret_cast<bf16x8*>(Cs + r * N + ((c ^ r) & (NC - 1)) * 8) = cr[k];
     }
 #pragma unroll
     for (int k = 0; k < BP; ++k) {
-      const int e = t + THREADS * k, r = e / NC * 2, c = e % NC;
+      const int e = tl + THREADS * k, r = e / NC * 2, c = e % NC;
       *reinterpret_cast<bf16x8*>(Bs + r * N + ((c ^ r) & (NC - 1)) * 8) = br[2 * k];
       *reinterpret_cast<bf16x8*>(Bs + (r + 1) * N + ((c ^ (r + 1)) & (NC - 1)) * 8) = br[2 * k + 1];
 #pragma unroll
@@ -148,12 +165,16 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
       }
     }
     {
-      const int r = t / (2 * WV) * 2, c = t % (2 * WV);
+      const int r = tl / (2 * WV) * 2, c = tl % (2 * WV);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int d = c * 8 + q;
         *reinterpret_cast<pair*>(xT + d * SC + ((r / 8) ^ sc_key(d)) * 8 + r % 8) = pair{xr[0][q], xr[1][q]};
       }
+    }
+    if (leave) {
+      from = min(from, i0);
+      break;
     }
     __syncthreads();
     if (i0 + SC < n_new) load(i0 + SC);
@@ -202,6 +223,7 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
     __syncthreads();
 
     const int d = wave * 16 + li;
+    float finite = 0.f;                                  // NaN once a y was not
     bf16x8 xf[2];                                        // x^T of column d, places 32 ks + 8 kg
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) xf[ks] = *reinterpret_cast<const bf16x8*>(xT + d * SC + ((4 * ks + kg) ^ sc_key(d)) * 8);
@@ -231,8 +253,16 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
       // o[r]: row i4 + r, column d
       const bf16x4 xv = *reinterpret_cast<const bf16x4*>(xT + d * SC + ((i4 / 8) ^ sc_key(d)) * 8 + i4 % 8);
 #pragma unroll
+      for (int r = 0; r < 4; ++r) finite = fmaf(o[r], 0.f, finite);
+#pragma unroll
       for (int r = 0; r < 4; ++r)
         if (i4 + r < rows) y[(size_t)(row0 + i0 + i4 + r) * inner + h * dv + d0 + d] = fmaf(skip, (float)xv[r], o[r]);
+    }
+
+    if (__any(isnan(finite))) {
+      from = i0;
+      spoilt = 1;                                        // (read behind the next barrier)
+      continue;
     }
 
     // the state behind the chunk
@@ -257,6 +287,30 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
 #pragma unroll
         for (int q = 2; q >= 0; --q) S[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf, xw[q][ks], S[nt], 0, 0, 0);
       }
+    }
+  }
+  if (from < n_new) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the y that these rows' go over have arrived
+    const int col = h * dv + d0 + wave * 16 + li;
+    for (int i = from; i < n_new; ++i) {
+      const bf16* row = u + (size_t)(row0 + i) * C;
+      const bf16 *Br = row + inner + g * N + 4 * kg, *Cr = Br + G * N;
+      const float dt = sc_softplus(proj[(size_t)(row0 + i) * width + dt_off + h] + bias), a = expf(neg_rate * dt);
+      const float x = (float)row[col], dtx = dt * x;
+      f32x4 sums = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const bf16x4 bv = *reinterpret_cast<const bf16x4*>(Br + 16 * n), cv = *reinterpret_cast<const bf16x4*>(Cr + 16 * n);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[n][r] = fmaf(a, S[n][r], (float)bv[r] * dtx);
+          sums[r] = fmaf(S[n][r], (float)cv[r], sums[r]);
+        }
+      }
+      float sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+      sum += __shfl_xor(sum, 16, WAVE);
+      sum += __shfl_xor(sum, 32, WAVE);
+      if (kg == 0) y[(size_t)(row0 + i) * inner + col] = fmaf(skip, x, sum);
     }
   }
 #pragma unroll
