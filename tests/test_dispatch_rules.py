@@ -120,3 +120,19 @@ def test_prefill_layout_cuts_long_blocks_of_small_launches_into_runs():
             (1, 4, 32), (8, 256, 1024)):
         before = (before * len(n_new))[:len(n_new)]
         check(n_new, before, window, nq, units)
+
+
+def test_which_sequences_of_a_step_go_by_chunks():
+    """The choice belongs to the sequence: long ones by chunks beside short ones row by row, whatever the step's average."""
+    def of(lens, heads=128, N=128, dv=64, known=True):
+        return ops.ssm_chunks_from(sum(lens), len(lens), heads, N, dv, (min(lens), max(lens)) if known else None)
+
+    assert of([512] + [1] * 64) == 12 and of([512] + [1] * 64, N=64) == 16
+    assert of([90] * 8 + [1] * 56) == 12
+    assert of([1] * 64) == of([11] * 64) == of([11]) == of([15, 15], heads=8) == 0
+    assert of([64]) == of([2048, 100]) == of([13] * 64) == 1
+    assert of([100] + [1] * 7) == 1 and of([40, 1], heads=8) == 1          # room for the short ones beside the long one
+    assert of([15] + [1] * 63) == 0 and of([31] * 60 + [1] * 4) == 12      # one launch more for a few rows, and for many
+    # without the host's numbers: nothing where no sequence can be long, else the device looks at each
+    assert of([1] * 64, known=False) == of([11], known=False) == 0
+    assert of([11] * 64, known=False) == of([512] + [1] * 64, known=False) == 12 and of([64], known=False) == 1

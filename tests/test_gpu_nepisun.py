@@ -888,6 +888,26 @@ def test_a_chunk_with_a_number_that_is_none(heads, dv, N, G, row, what, value):
         assert float((a[ok].double() - b[ok].double()).norm() / a[ok].double().norm()) < 2e-6
 
 
+@pytest.mark.parametrize("lens, heads, dv, N, span", [([40] + [1] * 17, 128, 64, 128, (1, 40)), ([40, 1, 11, 64, 12], 130, 32, 128, None),
+                                                      ([1, 16, 15, 90], 4, 64, 64, None), ([2, 33, 1], 6, 96, 32, (1, 33)), ([3, 1, 2], 4, 32, 32, None)])
+def test_long_and_short_sequences_of_a_step(lens, heads, dv, N, span):
+    """Every sequence has the bits of the kernel it belongs to, and no other sequence's rows or state are touched."""
+    from torchless_rs_amd.kernels import ops
+    u, proj, A, bias, D, state, cu, slots = _recurrence_case(lens, heads, dv, N, 2, sum(lens), True)
+    n, inner = sum(lens), heads * dv
+    got = {}
+    for chunks in (None, False, True):
+        s, y = state.clone(), torch.full((n, inner), float("nan"), device="cuda")
+        ops.ssm_scan(u, proj, 8, 2, N, heads, dv, bias, A, D, s, cu, slots, y, chunks=chunks, span=span if chunks is None else None)
+        got[chunks] = (y, s)
+    least = ops.ssm_chunks_from(n, len(lens), heads, N, dv, span)
+    for b, l in enumerate(lens):
+        want = got[bool(least) and l >= least]
+        rows, slot = slice(int(cu[b]), int(cu[b + 1])), int(slots[b])
+        assert torch.equal(got[None][0][rows], want[0][rows]) and torch.equal(got[None][1][slot], want[1][slot]), (b, l, least)
+    assert torch.equal(got[None][1][[0, len(lens) + 1]], state[[0, len(lens) + 1]])
+
+
 def test_which_recurrences_go_by_chunks():
     """Sizes that the chunks do not take go row by row, and asking for chunks there is an error."""
     from torchless_rs_amd.kernels import ops

@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(256)
 ssm_scan_kernel(const T* __restrict__ u, int C, int inner, int G, int N, int heads, int dv, int dvb, int nsl, int NP,
                 const float* __restrict__ proj, int width, int dt_off, const float* __restrict__ dt_bias,
                 const float* __restrict__ A_log, const float* __restrict__ Dw, float* __restrict__ state, long long stride,
-                const int* __restrict__ cu_seqlens, const int* __restrict__ slots, float* __restrict__ y) {
+                const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int most, float* __restrict__ y) {
   extern __shared__ __attribute__((aligned(16))) float ssm_lds[];
   float* xs = ssm_lds;                 // [SSM_TB][dvb]
   float* Bs = xs + SSM_TB * dvb;       // [SSM_TB][NP]: NP = R * nsl >= N, zeros behind the N rows, so that the
@@ -187,6 +187,7 @@ ssm_scan_kernel(const T* __restrict__ u, int C, int inner, int G, int N, int hea
   const int c0 = active ? cg * DC : 0;                // this lane's first column among the workgroup's
   const int PW = dvb * nsl;
   const int row0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - row0;
+  if (n_new > most) return;
   float* S_g = state + (long long)slots[b] * stride + (size_t)h * N * dv + (size_t)(d0 + c0) * N;
   float S[R][DC];
 #pragma unroll
@@ -451,10 +452,10 @@ static ScanShape scan_shape(int N, int dv, int units) {
 template <typename T>
 static int scan_launch(const ScanShape& z, dim3 grid, size_t lds, hipStream_t st, const T* u, int C, int inner, int G, int N,
                        int heads, int dv, const float* proj, int width, int dt_off, const float* dt_bias, const float* A_log,
-                       const float* D, float* state, long long stride, const int* cu, const int* slots, float* y) {
+                       const float* D, float* state, long long stride, const int* cu, const int* slots, int most, float* y) {
 #define TL_SCAN(RR, DD)                                                                                                      \
   ssm_scan_kernel<T, RR, DD><<<grid, 256, lds, st>>>(u, C, inner, G, N, heads, dv, z.dvb, z.nsl, RR * z.nsl, proj, width, dt_off, dt_bias, \
-                                                     A_log, D, state, stride, cu, slots, y)
+                                                     A_log, D, state, stride, cu, slots, most, y)
   if (z.DC == 4) {
     if (z.R <= 1) TL_SCAN(1, 4);
     else if (z.R <= 2) TL_SCAN(2, 4);
@@ -526,10 +527,11 @@ int tl_conv_carry(const float* proj, int width, int off, int C, int taps, float*
   return 0;
 }
 
-// u [n, C] = [x | B | C] after the convolution; proj [n, width] holds dt at column dt_off + h.
+// u [n, C] = [x | B | C] after the convolution; proj [n, width] holds dt at column dt_off + h.  Sequences of more than
+// `most` rows are left alone.
 int tl_ssm_scan(const void* u, int dt, int C, int G, int N, int heads, int dv, const float* proj, int width, int dt_off,
                 const float* dt_bias, const float* A_log, const float* D, float* state, long long stride,
-                const int* cu_seqlens, const int* slots, int n, int B, float* y, hipStream_t st) {
+                const int* cu_seqlens, const int* slots, int n, int B, int most, float* y, hipStream_t st) {
   TL_REQUIRE(n >= 0 && B >= 0 && heads > 0 && G > 0 && heads % G == 0 && N > 0 && dv > 0, "ssm_scan: bad sizes heads=%d G=%d N=%d dv=%d",
              heads, G, N, dv);
   TL_REQUIRE(N <= SSM_MAX_N && dv <= SSM_MAX_DV, "ssm_scan: a state of %d x %d is not served (up to %d x %d)", N, dv, SSM_MAX_N,
@@ -549,10 +551,10 @@ int tl_ssm_scan(const void* u, int dt, int C, int G, int N, int heads, int dv, c
   const size_t lds = sizeof(float) * ((size_t)SSM_TB * (z.dvb + 2 * Rt * z.nsl) + 2 * SSM_TB + (size_t)SSM_TB * z.dvb * z.nsl);
   if (dt == DT_F32)
     scan_launch<float>(z, grid, lds, st, (const float*)u, C, inner, G, N, heads, dv, proj, width, dt_off, dt_bias, A_log, D, state, stride,
-                       cu_seqlens, slots, y);
+                       cu_seqlens, slots, most, y);
   else
     scan_launch<bf16>(z, grid, lds, st, (const bf16*)u, C, inner, G, N, heads, dv, proj, width, dt_off, dt_bias, A_log, D, state, stride,
-                      cu_seqlens, slots, y);
+                      cu_seqlens, slots, most, y);
   TL_LAUNCH_CHECK("ssm_scan");
   return 0;
 }

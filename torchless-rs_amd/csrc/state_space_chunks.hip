@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(WV * WAVE, WV / 2)
 ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads, int dv, const float* __restrict__ proj, int width,
                   int dt_off, const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dw,
                   float* __restrict__ state, long long stride, const int* __restrict__ cu_seqlens, const int* __restrict__ slots,
-                  float* __restrict__ y) {
+                  int least, float* __restrict__ y) {
   constexpr int N = 16 * NT, NC = N / 8, THREADS = WV * WAVE;          // NC: chunks of 8 of a row of B or C
   constexpr int CL = SC * NC / THREADS, BP = CL / 2;                   // loads of C, pairs of rows of B a thread
   static_assert(NT >= 2 && NT % 2 == 0 && CL % 2 == 0 && CL > 0, "whole pairs of rows a thread");
@@ -67,7 +67,7 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
   const int h = blockIdx.x, b = blockIdx.y, t = threadIdx.x, wave = t / WAVE, lane = t % WAVE, li = lane % 16, kg = lane / 16;
   const int d0 = blockIdx.z * (16 * WV), g = h / (heads / G);
   const int row0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - row0;
-  if (n_new <= 0) return;
+  if (n_new < least) return;
   const float neg_rate = -expf(A_log[h]);
   const double rate = (double)neg_rate * 1.4426950408889634;
   const float bias = dt_bias[h], skip = Dw[h];
@@ -320,9 +320,9 @@ ssm_chunks_kernel(const bf16* __restrict__ u, int C, int inner, int G, int heads
 template <int NT, int WV>
 static int launch_chunks(const bf16* u, int C, int inner, int G, int heads, int dv, const float* proj, int width, int dt_off,
                          const float* dt_bias, const float* A_log, const float* D, float* state, long long stride, const int* cu,
-                         const int* slots, int B, float* y, hipStream_t st) {
+                         const int* slots, int B, int least, float* y, hipStream_t st) {
   ssm_chunks_kernel<NT, WV><<<dim3(heads, B, dv / (16 * WV)), WV * WAVE, 0, st>>>(u, C, inner, G, heads, dv, proj, width, dt_off, dt_bias, A_log, D,
-                                                                                  state, stride, cu, slots, y);
+                                                                                  state, stride, cu, slots, least, y);
   TL_LAUNCH_CHECK("ssm_chunks");
   return 0;
 }
@@ -340,11 +340,12 @@ int tl_ssm_chunks_serve(int dt, int C, int G, int N, int heads, int dv, const vo
          stride % 4 == 0 && ((uintptr_t)u | (uintptr_t)state) % 16 == 0;
 }
 
-// as tl_ssm_scan, for buffers that tl_ssm_chunks_serve takes
+// as tl_ssm_scan, for buffers that tl_ssm_chunks_serve takes and the sequences of `least` rows or more (at least one); the
+// others are left alone
 int tl_ssm_chunks(const void* u, int C, int G, int N, int heads, int dv, const float* proj, int width, int dt_off, const float* dt_bias,
                   const float* A_log, const float* D, float* state, long long stride, const int* cu_seqlens, const int* slots, int n, int B,
-                  float* y, hipStream_t st) {
-  TL_REQUIRE(n >= 0 && B >= 0 && heads > 0 && G > 0 && dv > 0, "ssm_chunks: bad sizes heads=%d G=%d N=%d dv=%d", heads, G, N, dv);
+                  int least, float* y, hipStream_t st) {
+  TL_REQUIRE(n >= 0 && B >= 0 && heads > 0 && G > 0 && dv > 0 && least > 0, "ssm_chunks: bad sizes heads=%d G=%d N=%d dv=%d least=%d", heads, G, N, dv, least);
   TL_REQUIRE(tl_ssm_chunks_serve(DT_BF16, C, G, N, heads, dv, u, state, stride), "ssm_chunks: C=%d G=%d N=%d heads=%d dv=%d stride=%lld are not served", C,
              G, N, heads, dv, stride);
   TL_REQUIRE(dt_off >= 0 && dt_off + heads <= width && stride >= (long long)heads * N * dv, "ssm_chunks: bad sizes dt_off=%d width=%d stride=%lld", dt_off,
@@ -354,7 +355,7 @@ int tl_ssm_chunks(const void* u, int C, int G, int N, int heads, int dv, const f
   // 64 columns a workgroup share the weights' work; 32 where there would be fewer than one workgroup a compute unit
   const bool four = dv % 64 == 0 && (long)heads * B * (dv / 64) >= 256;
 #define TL_CHUNKS(NN, WW) \
-  return launch_chunks<NN, WW>((const bf16*)u, C, heads * dv, G, heads, dv, proj, width, dt_off, dt_bias, A_log, D, state, stride, cu_seqlens, slots, B, y, st)
+  return launch_chunks<NN, WW>((const bf16*)u, C, heads * dv, G, heads, dv, proj, width, dt_off, dt_bias, A_log, D, state, stride, cu_seqlens, slots, B, least, y, st)
   if (N == 32) {
     TL_CHUNKS(2, 2);
   } else if (N == 64) {

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -919,21 +919,43 @@ def ssm_conv(proj: torch.Tensor, off: int, C: int, w: torch.Tensor, bias, conv_s
                              _p(out), _code(out.dtype), _stream()))
 
 
-# Rows a sequence from which a step's recurrence goes by chunks: a chunk takes 8 us whatever its rows, a row by itself 0.6.
-# 128 heads of 128 x 64, microseconds, row by row / by chunks: 8 sequences of 4 rows 24 / 37, of 16 rows 45 / 37; one of 9 rows
-# 14.5 / 14, of 2,048 rows 1,215 / 255; four of 128 to 1,024 rows 838 / 165; one of 100 rows beside 63 of one 150 / 244.
-SSM_CHUNK_ROWS = 12
+# Short sequences beside long ones.  Up to SSM_CHUNK_UNITS workgroups of 64 columns the short ones find room beside the long ones;
+# above, a launch for each.  One of 512 rows beside 64 single ones, 128 heads of 128 x 64: row by row 480, both 180; 8 of 90
+# beside 56 287 (by chunks alone 195) / 163; one of 100 beside 7 (1,024 workgroups) 88, by chunks alone 32.  A second launch for
+# sequences of fewer rows than SSM_CHUNK_ALONE pays only where there are many (one of 15 beside 63: 122 / 130).
+SSM_CHUNK_UNITS = 1024
+SSM_CHUNK_ALONE = 32
+
+
+def ssm_chunks_from(n: int, B: int, heads: int, N: int, dv: int, span: Optional[Tuple[int, int]]) -> int:
+    """The rows from which a sequence of a step of n rows and B sequences goes by chunks (1: all of them, 0: none); `span`: the
+    fewest and the most rows of a sequence, or None where only the device knows.
+
+    A chunk takes much the same whatever its rows and N, a row by itself the longer the larger N is and the fuller the chip: 16 rows,
+    or 12.  Row by row / by chunks, microseconds: 128 heads of 128 x 64, one sequence of 12 rows 11.8 / 13.0, of 16 13.0 / 13.0, 8 of
+    12 36 / 28, 64 of 13 300 / 173; 8 such heads, 8 of 12 11.5 / 12.8, 64 of 13 19.5 / 17.0; 64 heads of 32 x 64, 64 of 13 65 / 68."""
+    least = 12 if N == 128 and heads * B >= 512 else 16
+    shortest, longest = n if B == 1 else 1, n - B + 1
+    if longest >= least and span is not None:
+        shortest, longest = span
+    if longest < least:
+        return 0
+    if shortest >= least or (span is not None and heads * B * -(-dv // 64) <= SSM_CHUNK_UNITS):
+        return 1
+    return 0 if longest < SSM_CHUNK_ALONE and n < least * B else least
 
 
 def ssm_scan(u: torch.Tensor, proj: torch.Tensor, dt_off: int, G: int, N: int, heads: int, dv: int, dt_bias, A_log, D,
-             state: torch.Tensor, cu_seqlens, slots, y: torch.Tensor, chunks: Optional[bool] = None) -> None:
+             state: torch.Tensor, cu_seqlens, slots, y: torch.Tensor, chunks: Optional[bool] = None,
+             span: Optional[Tuple[int, int]] = None) -> None:
     """The recurrence of a state-space mixer over the rows of a step, sequence by sequence: u [n, heads*dv + 2*G*N]
     = [x | B | C] (after the convolution), dt at the columns dt_off .. of proj (float32 [n, width]);
     dt' = softplus(dt + dt_bias[h]), S <- exp(-exp(A_log[h]) dt') S + dt' B x^T, y = S^T C + D[h] x; `state`
     float32 [slots, >= heads*N*dv] is read and left updated; y float32 [n, heads*dv].
 
-    bfloat16 steps of `SSM_CHUNK_ROWS` rows a sequence on average go by chunks of 64 rows on the matrix cores where the
-    sizes allow (`chunks`: the caller's choice; True is an error where they do not)."""
+    bfloat16 sequences of many rows go by chunks of 64 rows on the matrix cores where the sizes allow, the others row by row
+    (`ssm_chunks_from`; `chunks`: the caller's choice for all of them, True is an error where the sizes do not allow it).  `span`:
+    the fewest and the most rows of a sequence, if the host knows them; otherwise each sequence is looked at on the device."""
     n, C = u.shape
     B = slots.shape[0]
     _req(u, "ssm_scan.u")
@@ -947,18 +969,21 @@ def ssm_scan(u: torch.Tensor, proj: torch.Tensor, dt_off: int, G: int, N: int, h
     _req(cu_seqlens, "ssm_scan.cu_seqlens", torch.int32, (B + 1,))
     _req(slots, "ssm_scan.slots", torch.int32)
     _req(y, "ssm_scan.y", torch.float32, (n, heads * dv))
+    least, serve = 1, chunks
     if chunks is None:
-        chunks = n >= SSM_CHUNK_ROWS * B and bool(lib().tl_ssm_chunks_serve(_code(u.dtype), C, G, N, heads, dv, _p(u), _p(state),
-                                                                            ctypes.c_longlong(state.stride(0))))
-    if chunks:
-        if u.dtype != torch.bfloat16:
-            raise KernelError("ssm_scan: chunks take bfloat16 rows")
+        least = ssm_chunks_from(n, B, heads, N, dv, span)
+        serve = least > 0 and bool(lib().tl_ssm_chunks_serve(_code(u.dtype), C, G, N, heads, dv, _p(u), _p(state),
+                                                             ctypes.c_longlong(state.stride(0))))
+    if serve and u.dtype != torch.bfloat16:
+        raise KernelError("ssm_scan: chunks take bfloat16 rows")
+    if serve:
         _check(lib().tl_ssm_chunks(_p(u), C, G, N, heads, dv, _p(proj), proj.shape[1], int(dt_off), _p(dt_bias), _p(A_log), _p(D), _p(state),
-                                   ctypes.c_longlong(state.stride(0)), _p(cu_seqlens), _p(slots), n, B, _p(y), _stream()))
-        return
+                                   ctypes.c_longlong(state.stride(0)), _p(cu_seqlens), _p(slots), n, B, least, _p(y), _stream()))
+        if least == 1:
+            return
     _check(lib().tl_ssm_scan(_p(u), _code(u.dtype), C, G, N, heads, dv, _p(proj), proj.shape[1], int(dt_off), _p(dt_bias),
                              _p(A_log), _p(D), _p(state), ctypes.c_longlong(state.stride(0)), _p(cu_seqlens), _p(slots), n, B,
-                             _p(y), _stream()))
+                             least - 1 if serve else 2 ** 31 - 1, _p(y), _stream()))
 
 
 def ssm_gate_norm(y: torch.Tensor, proj: torch.Tensor, parts: int, w: torch.Tensor, eps: float, out: torch.Tensor) -> None:

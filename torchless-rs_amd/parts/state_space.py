@@ -96,8 +96,11 @@ class StateSpaceMixer(Mixer):
         ops.ssm_conv(proj, self.inner, self.C, self.conv_w, self.conv_b, block, ctx.row_seq, ctx.cu_seqlens, ctx.slots, u,
                      single=ctx.all_single)
         yy = ws.get("ssm_y", (n, self.inner), torch.float32)
+        span = ctx.host.get("row_span")
+        if span is None and "n_new" in ctx.host:         # the same for every layer
+            span = ctx.host["row_span"] = (int(min(ctx.host["n_new"])), int(max(ctx.host["n_new"])))
         ops.ssm_scan(u, proj, self.inner + self.C, self.G, self.N, self.heads, self.dv, self.dt_bias, self.A_log, self.D,
-                     block[:, self.conv_elems:], ctx.cu_seqlens, ctx.slots, yy)
+                     block[:, self.conv_elems:], ctx.cu_seqlens, ctx.slots, yy, span=span)
         g = ws.get("ssm_g", (n, self.inner), ctx.dtype)
         ops.ssm_gate_norm(yy, proj, self.parts, self.norm_w, self.eps, g)
         self.o.add_into(g, x, ctx, "ssm_o_parts")
