@@ -435,6 +435,20 @@ def test_distribution_of_long_rows(ops, V, k, p):
         assert ids[b] == mine or abs(float(cum[min(ids[b], mine)]) - r) < 1e-6
 
 
+def test_top_p_goes_by_probability_however_the_row_is_cut(ops):
+    """Logits that differ by a unit in the last place and less than a probability can show, the larger ones behind: top-p keeps the
+    first of them in the row, from the list of candidates as from a whole row."""
+    unit = 2.0 ** -27                                        # of a float below 0.125
+    z = torch.full((1, 5000), -60.0)
+    at = [700, 1300, 2100, 4400]
+    for j, i in enumerate(at):
+        z[0, i] = torch.tensor(0.1).item() + j * unit
+    assert len(set(z[0, at].tolist())) == 4 and len(set(torch.exp(z[0, at] - z.max()).tolist())) == 1
+    for k in (0, 4, 10, 1024, 2000):
+        _, probs = run_sample(ops, z, 1.0, k, 0.45, 3)
+        assert (probs[0] > 0).nonzero().flatten().tolist() == at[:2], k
+
+
 def test_rows_without_a_distribution(ops):
     """Infinities and NaN among the logits: no draw, the last index; a row of one value: an even draw; -inf beside
     one finite logit: that one."""

@@ -382,8 +382,20 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
         e = e / sum;
         bool kept = have;
         if (top_p > 0.f && top_p < 1.f) {
-          double total;
-          const double before = block_excl_scan<double>((double)e, sh.wave_sum, &total);
+          // by probability, of equal ones the smaller index first: the list's order unless quotients that differ have
+          // exponentials that do not
+          __syncthreads();
+          if (have) li.top_z[tid] = e;
+          __syncthreads();
+          const float e_next = have && tid + 1 < top_k ? li.top_z[tid + 1] : -1.f;
+          const bool turned = e_next > e || (e_next == e && li.top_i[tid + 1] < my_i);
+          double before = 0.0, total;
+          if (__syncthreads_or(turned)) {
+            for (int o = 0; o < top_k; ++o)
+              before += li.top_z[o] > e || (li.top_z[o] == e && li.top_i[o] < my_i) ? (double)li.top_z[o] : 0.0;
+          } else {
+            before = block_excl_scan<double>((double)e, sh.wave_sum, &total);
+          }
           kept = have && before < (double)top_p;
           const float new_sum = block_sum<SNT>(kept ? e : 0.f, sh.red);
           e = kept ? e / new_sum : 0.f;
