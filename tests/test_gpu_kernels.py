@@ -435,6 +435,20 @@ def test_distribution_of_long_rows(ops, V, k, p):
         assert ids[b] == mine or abs(float(cum[min(ids[b], mine)]) - r) < 1e-6
 
 
+@pytest.mark.parametrize("V", [2, 64, 255, 256, 257, 512, 513, 1300, 2048, 2049, 3001])
+@pytest.mark.parametrize("k", [1, 7, 255, 257, 1023])
+def test_the_largest_of_rows_of_ties(ops, V, k):
+    """Rows of one value and of a few: the larger values, and of the smallest kept one the first in the row."""
+    z = torch.zeros(3, V)
+    z[1] = torch.arange(V) % 3
+    z[2] = -(torch.arange(V) // 5).float() / 64
+    _, probs = run_sample(ops, z, 1.0, k, 0.0, 3)
+    for b in range(3):
+        want = torch.argsort(z[b], descending=True, stable=True)[:k].sort().values
+        assert torch.equal((probs[b] > 0).nonzero().flatten().cpu(), want), b
+        assert float((probs[b].double().cpu()[want] - torch.softmax(z[b][want].double(), 0)).abs().max()) < 1e-6
+
+
 def test_top_p_goes_by_probability_however_the_row_is_cut(ops):
     """Logits that differ by a unit in the last place and less than a probability can show, the larger ones behind: top-p keeps the
     first of them in the row, from the list of candidates as from a whole row."""
