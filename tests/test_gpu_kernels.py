@@ -449,6 +449,29 @@ def test_the_largest_of_rows_of_ties(ops, V, k):
         assert float((probs[b].double().cpu()[want] - torch.softmax(z[b][want].double(), 0)).abs().max()) < 1e-6
 
 
+@pytest.mark.parametrize("V", [1, 2, 3, 5, 7, 4095, 4097, 32770, 65539])
+def test_rows_of_any_length_and_place(ops, V):
+    """Rows that start at every multiple of 4 bytes and end within a load of 16: greedy, a plain draw, nothing written beside them."""
+    z = rnd(5, V, seed=V, scale=2.0)
+    z[3, V // 2:] = z[3].max()
+    z[4, V - 1] = z[4].max() + 1
+    ids, _ = run_sample(ops, z, 0.0)
+    assert ids == [V - 1 if b == 3 else int((z[b] == z[b].max()).nonzero().max()) for b in range(5)]
+    flat, kept = torch.full((5 * V + 9,), 7.0, device=DEV), torch.full((5 * V + 9,), 7.0, device=DEV)
+    logits, probs = flat[3: 3 + 5 * V].view(5, V), kept[5: 5 + 5 * V].view(5, V)
+    logits.copy_(z)
+    counters, out = torch.tensor([[b, 2] for b in range(5)], dtype=torch.int32, device=DEV), torch.empty(5, dtype=torch.int32, device=DEV)
+    ops.sample(logits, 0.8, 0, 0.0, 11, counters, probs, out)
+    want = torch.softmax(z.double() / torch.tensor(0.8).double(), -1)
+    assert float((probs.double().cpu() - want).abs().max()) < 2e-6
+    assert bool((kept[:5] == 7.0).all()) and bool((kept[5 + 5 * V:] == 7.0).all())
+    cum = probs.double().cpu().cumsum(-1)
+    for b, i in enumerate(out.tolist()):
+        r = philox_uniform(11, 2, b)
+        mine = int((cum[b] >= r).nonzero()[0])
+        assert i == mine or abs(float(cum[b, min(i, mine)]) - r) < 1e-6
+
+
 def test_top_p_goes_by_probability_however_the_row_is_cut(ops):
     """Logits that differ by a unit in the last place and less than a probability can show, the larger ones behind: top-p keeps the
     first of them in the row, from the list of candidates as from a whole row."""
