@@ -136,3 +136,25 @@ def test_which_sequences_of_a_step_go_by_chunks():
     # without the host's numbers: nothing where no sequence can be long, else the device looks at each
     assert of([1] * 64, known=False) == of([11], known=False) == 0
     assert of([11] * 64, known=False) == of([512] + [1] * 64, known=False) == 12 and of([64], known=False) == 1
+
+
+def test_when_experts_run_over_their_own_rows():
+    """Against the wide form by the library: where all experts together are wide beside a row, and not where tiles would be empty."""
+    from types import SimpleNamespace
+
+    import torch
+    from torchless_rs_amd.parts.ffn_routed import RoutedExperts
+
+    def grouped(n, H, E, top, ff, shared=0, gated=False):
+        part = RoutedExperts(H, E, top, ff, shared_size=shared or None, gated=gated, activation="silu" if gated else "relu2")
+        weight = torch.empty(part.total, H, dtype=torch.bfloat16, device="meta")
+        part.up = part.down = SimpleNamespace(weight=weight, own_kernels=lambda rows: rows <= ops.own_rows(H))
+        return part.many_rows(SimpleNamespace(host={}), torch.empty(n, H, dtype=torch.bfloat16, device="meta"))
+
+    assert not any(grouped(n, 4096, 16, 4, 256, 256) for n in (129, 200, 511)) and grouped(512, 4096, 16, 4, 256, 256)
+    assert not grouped(400, 8192, 16, 4, 512) and grouped(200, 8192, 16, 4, 2048)
+    assert not grouped(400, 2048, 64, 8, 32) and grouped(200, 2048, 128, 8, 128)
+    assert not grouped(300, 1024, 512, 8, 32) and grouped(1000, 1024, 512, 8, 32)
+    assert grouped(300, 4096, 16, 4, 3584, 7168) and grouped(200, 7168, 64, 8, 256, 256, gated=True) and grouped(200, 512, 16, 4, 512)
+    # rows that a graph may hold: by their number and size alone
+    assert grouped(128, 2048, 64, 8, 128) and not grouped(128, 2048, 64, 8, 32) and not grouped(16, 4096, 16, 4, 3584)

@@ -62,6 +62,15 @@ from .linear import Linear
 GROUPED_ROWS = 16                  # up to here the kernels for few rows stream all experts' weights as fast as they come
 GROUPED_SIZE = 600000              # above, from this many rows times hidden channels of all experts
 GROUPED_ROWS_PER_EXPERT = 128      # or, above the own product kernels' rows, from this many rows an expert on average
+# Above the own product kernels' rows the wide form is the library's, whose time goes with the channels of all experts, where a tile of
+# an expert's rows goes through all of a row's channels in a chain: the experts' own rows pay from GROUPED_WIDTH channels (a gated
+# one counts twice) a channel of the row.  And an expert of few channels leaves its tile of 256 empty: below GROUPED_FF it takes
+# GROUPED_FEW rows an expert.  Microseconds, wide / grouped, 16 experts, 4 a row, 4,096 channels a row: experts of 256, 200 rows
+# 65 / 114, 400 rows 77 / 134; of 512 79 / 92, 103 / 123; of 1,024 and a shared one 209 / 140; 8,192 a row and experts of 512
+# 129 / 166, of 1,024 230 / 227, of 2,048 479 / 280; 512 a row and experts of 512 63 / 42.  512 experts of 32, 8 a row, 1,024 a row:
+# 200 rows 254 / 279, 511 rows 286 / 283, 800 rows 353 / 320; 128 experts of 128 132 / 107 at 200 rows.
+GROUPED_WIDTH = 2.5
+GROUPED_FF, GROUPED_FEW = 64, 8
 SLICED_ROWS = 512                  # up to here a shared expert runs along as slices (1,024 rows: 215 us against 140 by the library)
 
 
@@ -263,7 +272,9 @@ class RoutedExperts(FeedForward):
             if self.up.own_kernels(n):           # (a graph may hold the step: no product of the library's)
                 return (n > GROUPED_ROWS and n * self.total >= GROUPED_SIZE
                         and (not self.shared or ops.shared_slices(self.ff, self.shared) > 0))
-            return n * self.top >= GROUPED_ROWS_PER_EXPERT * self.E or n * self.total >= GROUPED_SIZE
+            return n * self.top >= GROUPED_ROWS_PER_EXPERT * self.E or (
+                n * self.total >= GROUPED_SIZE and (2 if self.gated else 1) * self.total >= GROUPED_WIDTH * self.H
+                and (self.ff >= GROUPED_FF or n * self.top >= GROUPED_FEW * self.E))
         return (n * self.top >= GROUPED_ROWS_PER_EXPERT * self.E and not self.up.own_kernels(n)
                 and not ctx.host.get("fixed_launches"))
 
