@@ -342,6 +342,17 @@ def test_gemm_plain_adds_in_one_order(ops, N, K):
     assert torch.equal(out, base[:9])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 40, 71), (33, 65, 68), (70, 130, 1026), (200, 33, 2049)])
+@pytest.mark.parametrize("a_type,w_type", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "bfloat16")])
+def test_gemm_plain_of_16_bit_operands(ops, M, N, K, a_type, w_type):
+    """Rows that may be read four channels at a time and others: a product of 16-bit operands is the one of their values in 32."""
+    a, w = rnd(M, K, seed=43).to(DEV, DT[a_type]), rnd(N, K, seed=44).to(DEV, DT[w_type])
+    out, want = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    ops.gemm_plain(a, w, out)
+    ops.gemm_plain(a.float(), w.float(), want)
+    assert torch.equal(out, want)
+
+
 def run_sample(ops, logits, T, k=0, p=0.0, seed=0, counters=None):
     B, V = logits.shape
     counters = counters if counters is not None else [[b, 0] for b in range(B)]

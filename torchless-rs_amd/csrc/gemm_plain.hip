@@ -98,15 +98,10 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
 // 32 x 32 outputs a workgroup of 8 waves, each with a group of K and 4 x 4 outputs a lane, operands through the wave's
 // own part of LDS, the groups' sums through LDS at the end.  16 multiply-adds for two 16-byte reads of LDS a lane: the
 // vector pipes and LDS are about as busy as each other.  Eight times the waves of tiles of 64 x 64 with a thread's
-// chain over all of K for a product of the same size, and faster at every size measured, 1 to 1,024 rows:
-// N x K = 2,048 x 8,192 at 64 rows 76 us (563 with those), at 1,024 rows 575; 16,384 x 2,048 at 64 rows 78 (320).
+// chain over all of K for a product of the same size, and faster at every size measured, 1 to 8,192 rows:
+// N x K = 2,048 x 8,192 at 64 rows 76 us (563 with those), at 1,024 rows 582 (1,259), at 2,048 1,040 (1,790); 16,384 x
+// 2,048 at 64 rows 78 (320), at 2,048 2,210 (3,600); bfloat16 4,096 x 4,097 at 2,048 rows 1,175 (1,373).
 // VEC: rows of both operands may be read four channels at a time; else a channel a lane, 16 lanes along a row.
-template <typename T> __device__ __forceinline__ f32x4 four(const T* __restrict__ p) {
-  typedef __attribute__((ext_vector_type(4))) T T4;
-  const T4 t = *(const T4*)p;
-  return f32x4{to_f32(t[0]), to_f32(t[1]), to_f32(t[2]), to_f32(t[3])};
-}
-
 constexpr int GT = 32, GK = 16;
 template <typename TA, typename TW, bool VEC, bool ACCUMULATE>
 __global__ void __launch_bounds__(512)
@@ -129,21 +124,16 @@ gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* __r
   // loads: rows lr, lr + RS, ..., VW channels from lk
   constexpr int VW = VEC ? 4 : 1, RS = WAVE * VW / GK, LOADS = GT / RS;
   const int lr = lane / (GK / VW), lk = lane % (GK / VW) * VW;
-  typedef __attribute__((ext_vector_type(VW))) float part;
-  part na[LOADS], nw[LOADS];
+  typedef __attribute__((ext_vector_type(VW))) TA part_a;
+  typedef __attribute__((ext_vector_type(VW))) TW part_w;
+  part_a na[LOADS];                                // as they come: a conversion here would wait for the load
+  part_w nw[LOADS];
   const auto fetch = [&](int k) {
 #pragma unroll
     for (int h = 0; h < LOADS; ++h) {
       const int m = m0 + lr + RS * h, n = n0 + lr + RS * h;
-      const TA* ap = A + (size_t)min(m, M - 1) * lda + k;
-      const TW* wp = W + (size_t)min(n, N - 1) * ldw + k;
-      if constexpr (VEC) {
-        na[h] = m < M && k < K ? four(ap) : f32x4{0.f, 0.f, 0.f, 0.f};
-        nw[h] = n < N && k < K ? four(wp) : f32x4{0.f, 0.f, 0.f, 0.f};
-      } else {
-        na[h] = m < M && k < K ? to_f32(*ap) : 0.f;
-        nw[h] = n < N && k < K ? to_f32(*wp) : 0.f;
-      }
+      na[h] = m < M && k < K ? *(const part_a*)(A + (size_t)min(m, M - 1) * lda + k) : part_a{};
+      nw[h] = n < N && k < K ? *(const part_w*)(W + (size_t)min(n, N - 1) * ldw + k) : part_w{};
     }
   };
   const int end = min(K, first + PR * L);
@@ -154,8 +144,8 @@ gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* __r
     for (int h = 0; h < LOADS; ++h)
 #pragma unroll
       for (int j = 0; j < VW; ++j) {
-        As[lk + j][lr + RS * h] = na[h][j];
-        Ws[lk + j][lr + RS * h] = nw[h][j];
+        As[lk + j][lr + RS * h] = to_f32((TA)na[h][j]);
+        Ws[lk + j][lr + RS * h] = to_f32((TW)nw[h][j]);
       }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (k0 + GK < end) fetch(k0 + GK + lk);
