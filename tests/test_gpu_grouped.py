@@ -127,6 +127,45 @@ def test_experts_over_their_own_rows(ops, n, H, E, top, ff, shared, gated, on_in
     assert torch.equal(out, total)
 
 
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_experts_of_sizes_that_are_no_multiples_of_eight(gated, accumulate):
+    """Very many rows, an expert after the other by the library's products.  The hidden channels are rounded to bfloat16 once, the
+    rest are sums of 32 bits."""
+    from types import SimpleNamespace
+    from torchless_rs_amd.parts import ffn_routed
+    from torchless_rs_amd.parts.base import Workspace
+    H, E, top, ff, shared, n = 64, 3, 2, 12, 10, 200
+    part = ffn_routed.RoutedExperts(H, E, top, ff, shared_size=shared, gated=gated, activation="silu" if gated else "relu2")
+    g = torch.Generator(device=DEV).manual_seed(7 + gated)
+    part.load({k: (torch.randn(v.shape, generator=g, device=DEV) * v.shape[-1] ** -0.5).bfloat16() for k, v in part.weight_specs().items()},
+              torch.bfloat16)
+    ctx = SimpleNamespace(workspace=Workspace(torch.device(DEV)), dtype=torch.bfloat16, host={}, pending=None)
+    y, x = torch.randn(n, H, generator=g, device=DEV).bfloat16(), torch.randn(n, H, generator=g, device=DEV)
+    assert not part._serves(y) and part.many_rows(ctx, y)
+    score = torch.softmax(y.double() @ part.router.double().T, dim=-1)
+    picked = score.topk(top + 1)
+    sure = picked.values[:, top - 1] > picked.values[:, top] * (1 + 1e-4)
+    wt = torch.zeros_like(score).scatter_(1, picked.indices[:, :top], picked.values[:, :top])
+    want = x.double().clone() if accumulate else torch.zeros(n, H, dtype=torch.float64, device=DEV)
+    size = want.abs()
+    up, down, at, wide = part.up.weight.double(), part.down.weight.double(), 0, 2 if gated else 1
+    for e in range(E + 1):
+        m = ff if e < E else shared
+        z = y.double() @ up[wide * at: wide * (at + m)].T
+        h = torch.nn.functional.silu(z[:, :m]) * z[:, m:] if gated else torch.relu(z) ** 2
+        h = h * (wt[:, e: e + 1] if e < E else 1.0)
+        want += h @ down[:, at: at + m].T
+        size += h.abs() @ down[:, at: at + m].abs().T
+        at += m
+    if accumulate:
+        part.forward(ctx, y, x)
+    else:
+        part.produce(ctx, y, x)
+    # a hidden channel off by half a unit of its 8 bits, at most 2^-8 of itself, and the sums of 32 bits before and behind it
+    assert bool(((x.double() - want).abs() <= (2.0 ** -8 + (H + 64) * 2.0 ** -24) * size + 1e-5)[sure].all())
+
+
 def test_refused(ops):
     """Operands that the kernel does not take are an error, not a wrong result."""
     y = torch.zeros(4, 64, dtype=torch.bfloat16, device=DEV)

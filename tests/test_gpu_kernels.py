@@ -332,13 +332,13 @@ def test_gemm_plain_adds_in_one_order(ops, N, K):
         assert torch.equal(out, base[:M]), M
         ops.gemm_plain(a[:M].contiguous(), w, out, accumulate=True)
         assert torch.equal(out, base[:M] + base[:M]), M
-    many = torch.empty(2600, N, device=DEV)                   # tiles of 64 x 64 where N is large enough
+    many = torch.empty(2600, N, device=DEV)                   # many tiles of 32 x 32
     ops.gemm_plain(a.repeat(13, 1), w, many)
     assert torch.equal(many, base.repeat(13, 1))
     shifted = torch.empty(K * N + 1, device=DEV)[1:].view(N, K)
     shifted.copy_(w)
     out = torch.empty(9, N, device=DEV)
-    ops.gemm_plain(a[:9].contiguous(), shifted, out)          # not aligned: tiles of 64 x 64 whatever the size
+    ops.gemm_plain(a[:9].contiguous(), shifted, out)          # not aligned: tiles of 32 x 32, a channel a load
     assert torch.equal(out, base[:9])
 
 

@@ -240,12 +240,14 @@ static int launch_plain(const void* Av, const void* Wv, float* C, int M, int N, 
 
 using namespace tl;
 
+constexpr int MOST_ROWS = 65535 * 64;      // what callers have always been held to; the tiles' own limit is `launch_tiles`'
+
 extern "C" int tl_gemm_plain(const void* A, int a_dt, const void* W, int w_dt, float* C, int M, int N,
                              int K, int lda, int ldw, int ldc, int accumulate, hipStream_t st) {
   TL_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
   TL_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: leading dimensions lda=%d ldw=%d ldc=%d too small "
              "for K=%d N=%d", lda, ldw, ldc, K, N);
-  TL_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d has more row tiles than a grid holds", M);
+  TL_REQUIRE(M <= MOST_ROWS, "gemm: M=%d, products have at most %d rows", M, MOST_ROWS);
   if (M == 0) return 0;
   if (a_dt == DT_F32 && w_dt == DT_F32)
     return launch_plain<float, float>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
