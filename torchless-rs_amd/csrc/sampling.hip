@@ -322,8 +322,8 @@ template <bool VEC> __device__ __forceinline__ void draw_row(const float* __rest
 //   * everything else: thresholds by a histogram of the key's bits, three passes whatever the row holds, where
 //     bisection took one a bit.  top-p adds probabilities as whole numbers of 2^-60.
 // Microseconds, the kernel alone (by bisection, a bit a pass, before): 16 rows of 131,072 logits at T = 0.7 with top-k 50
-// and top-p 0.95 41 (1,612), top-p 0.9 alone 136 (840), neither 84 (166), top-k 2,000 135 (939), greedy 13 (24);
-// 64 rows of 32,000 30 (443), 46 (238), 27 (54), 45 (257), 8.5 (9.1).
+// and top-p 0.95 36 (1,612), top-p 0.9 alone 135 (840), neither 81 (166), top-k 2,000 134 (939), greedy 12 (24);
+// 64 rows of 32,000 25 (443), 46 (238), 27 (54), 44 (257), 7 (9.1).
 template <bool VEC>
 __global__ void __launch_bounds__(SNT)
 sample_kernel(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p,

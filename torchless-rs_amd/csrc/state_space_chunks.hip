@@ -21,8 +21,8 @@
 // What bounds it: a chunk's way of phases (rows to LDS, weights, products), each short and behind the one before: 8 us a
 // chunk, where its 130 products of 16 cycles a wave take 0.9, its splits about as long and its traffic in LDS 0.8; a
 // second workgroup on the compute unit fills gaps (5 us a chunk).
-// 128 heads of 128 x 64, microseconds, row by row before: one sequence of 2,048 rows 257 (1,215), four of 128 to 1,024 rows 165
-// (838), one of 8,192 1,010 (5,580).  Relative error against float64 (2,000 rows): y 1.2e-7 (5.7e-7), state 1.0e-7 (3.3e-7).
+// 128 heads of 128 x 64, microseconds, row by row before: one sequence of 2,048 rows 258 (1,215), four of 128 to 1,024 rows 117
+// (838), one of 8,192 1,020 (5,580).  Relative error against float64 (2,000 rows): y 1.2e-7 (5.7e-7), state 1.0e-7 (3.3e-7).
 #include "common.hpp"
 
 namespace tl {
