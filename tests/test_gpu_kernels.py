@@ -342,6 +342,18 @@ def test_gemm_plain_adds_in_one_order(ops, N, K):
     assert torch.equal(out, base[:9])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 70_000_000, 4), (2, 70_000_001, 3), (4_190_000, 2080, 4)])
+def test_gemm_plain_of_more_tiles_than_a_grid_is_wide(ops, M, N, K):
+    """One launch has fewer than 2^32 threads along x: what lies behind them is there too."""
+    a, w, out = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV), torch.empty(M, N, device=DEV)
+    out[-1, -1] = out[M // 2, N // 2] = float("nan")
+    ops.gemm_plain(a, w, out)
+    for m, n in ((0, 0), (M - 1, N - 1), (M // 2, N // 2), (M - 33 if M > 33 else 0, 0)):
+        rows, cols = slice(max(0, m - 40), m + 40), slice(max(0, n - 40), n + 40)
+        want = a[rows].double() @ w[cols].double().T
+        assert float((out[rows, cols].double() - want).abs().max()) < 2e-6 * K * float(a[rows].abs().max() * w[cols].abs().max())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 40, 71), (33, 65, 68), (70, 130, 1026), (200, 33, 2049)])
 @pytest.mark.parametrize("a_type,w_type", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "bfloat16")])
 def test_gemm_plain_of_16_bit_operands(ops, M, N, K, a_type, w_type):

@@ -16,6 +16,10 @@ namespace tl {
 constexpr int PG = 8, PR = 8;                     // groups of K, runs of a group
 constexpr int BK = 16;                            // runs are a multiple of this long
 
+// A launch has fewer than 2^32 threads along x (more are not refused: some are left out), here 512 a workgroup; what has more
+// workgroups goes on along another dimension.
+constexpr long GRID_X = 1l << 22;
+
 __host__ __device__ __forceinline__ int run_length(int K) { return (K + PG * PR * BK - 1) / (PG * PR * BK) * BK; }
 
 // Few rows of floats: a workgroup of 8 waves has 8 outputs' rows of W and up to MR rows of A.  A wave has a group
@@ -32,7 +36,9 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
                        int K, int lda, int ldw, int ldc) {
   __shared__ float stage[PG][64][CHUNK + 4];      // rows 144 bytes apart: 16-byte reads of 64 rows spread over the banks
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int n0 = blockIdx.x * 8, m0 = blockIdx.y * MR;
+  const long first_n = ((long)blockIdx.z * gridDim.x + blockIdx.x) * 8;
+  if (first_n >= N) return;
+  const int n0 = (int)first_n, m0 = blockIdx.y * MR;
   const int L = run_length(K);
   const int run = lane / 8;                       // of this lane's pair: output lane % 8, run lane / 8
   const int k0 = (wave * PR + run) * L;
@@ -110,8 +116,9 @@ gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* __r
   __shared__ float shared[PG * 2 * GK * (GT + 4)];
   static_assert(PG * 2 * GK * (GT + 4) >= PG * GT * GT, "the sums of the groups take the operands' place");
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int tiles_n = (N + GT - 1) / GT;
-  const int m0 = (int)(blockIdx.x / tiles_n) * GT, n0 = (int)(blockIdx.x % tiles_n) * GT;
+  const unsigned tiles_n = (N + GT - 1) / GT, tile = blockIdx.y * gridDim.x + blockIdx.x;
+  if (tile >= tiles_n * ((M + GT - 1) / GT)) return;
+  const int m0 = (int)(tile / tiles_n) * GT, n0 = (int)(tile % tiles_n) * GT;
   float (*As)[GT + 4] = (float (*)[GT + 4])(shared + wave * 2 * GK * (GT + 4));
   float (*Ws)[GT + 4] = As + GK;
   const int tx = lane % 8, ty = lane / 8;
@@ -191,10 +198,11 @@ static int launch_tiles(const TA* A, const TW* W, float* C, int M, int N, int K,
                         int accumulate, hipStream_t st) {
   const long tiles = (long)((N + GT - 1) / GT) * ((M + GT - 1) / GT);
   TL_REQUIRE(tiles < (1l << 31), "gemm: M=%d N=%d have more tiles than a grid holds", M, N);
+  const dim3 grid((unsigned)(tiles < GRID_X ? tiles : GRID_X), (unsigned)((tiles + GRID_X - 1) / GRID_X));
   if (accumulate)
-    gemm_plain_kernel<TA, TW, VEC, true><<<(unsigned)tiles, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+    gemm_plain_kernel<TA, TW, VEC, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   else
-    gemm_plain_kernel<TA, TW, VEC, false><<<(unsigned)tiles, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+    gemm_plain_kernel<TA, TW, VEC, false><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   TL_LAUNCH_CHECK("gemm_plain");
   return 0;
 }
@@ -202,7 +210,8 @@ static int launch_tiles(const TA* A, const TW* W, float* C, int M, int N, int K,
 template <int MR>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                        int accumulate, hipStream_t st) {
-  dim3 grid((N + 7) / 8, (M + MR - 1) / MR);
+  const long groups = ((long)N + 7) / 8;
+  const dim3 grid((unsigned)(groups < GRID_X ? groups : GRID_X), (M + MR - 1) / MR, (unsigned)((groups + GRID_X - 1) / GRID_X));
   if (accumulate)
     gemm_plain_rows_kernel<MR, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   else
