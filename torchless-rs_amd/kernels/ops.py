@@ -1031,7 +1031,7 @@ def route(h: torch.Tensor, router: torch.Tensor, groups: int, keep: int, top: in
     of the `keep` groups (of `groups` equal groups of neighbours; 0: no groups) whose best c is largest
     (`two_largest`: the sum of whose two best is), the `top` experts with the largest c; `weights` float32
     [n, E] receives s for those (with `normalise_eps`: divided by (their sum + normalise_eps)) and 0 for the
-    others, `chosen` (int32 [n, top], or None) their indices, the best first.  With `shared_weight` (float32
+    others, `chosen` (int32 [n, top], or None) their indices, the best first (a c that is NaN counts as the largest).  With `shared_weight` (float32
     [n]) the router has one row more, whose product's logistic function goes there."""
     n, W = h.shape
     E = weights.shape[1]
