@@ -853,9 +853,15 @@ gemm_ring_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, float* 
               ((place ^ key(r)) * 16);
     adst[x] = q < A_INSTR ? q * 1024 : -1;
   }
-  auto issue = [&](int i) {                                 // stage i of this split into its place in the ring
+  // Where K is not cut, workgroups of other channels begin with other stages and go round: rows of W are all the same power
+  // of two (or nearly) apart, so that workgroups in step would ask a few of the memory's channels at a time.  gate|up of the
+  // 7B shape at 24 / 64 / 128 rows 50 / 52 / 67 us in step, 41 / 44 / 64 like this (5.3 TB/s at 64 rows; a read of rows 8 KB
+  // apart alone: 4.9 TB/s in step, 6.9 not), the head of 32,000 channels 55 / 57 / 66 and 45 / 47 / 64.  Slices of K begin
+  // in different places already: o, down and q|k|v take what they took.
+  const int first = gridDim.y == 1 ? blockIdx.x % n_t : 0;
+  auto issue = [&](int i) {                                 // the stage with which turn i is concerned into its place in the ring
     unsigned char* slot = ring_smem + (i % NS) * STAGE;
-    const size_t off = (size_t)i * ROWB;
+    const size_t off = (size_t)(i + first < n_t ? i + first : i + first - n_t) * ROWB;
 #pragma unroll
     for (int x = 0; x < A_PER; ++x) {
       unsigned char* dst = adst[x] >= 0 ? slot + adst[x] : ring_smem + SPARE;
