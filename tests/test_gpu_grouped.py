@@ -281,3 +281,40 @@ def test_a_routed_step_with_rows_that_are_not_numbers(n):
     # (which rows share a tile may change with the choices of two, which changes no row's order of sums)
     assert torch.equal(out[0][well], out[1][well])
     assert bool(out[1][[2, n - 1]].isnan().all())
+
+
+@pytest.mark.parametrize("positions", [1, 31, 32, 33, 95, 97, 159, 161, 191, 193, 223, 224, 225, 449])
+@pytest.mark.parametrize("H,ff", [(64, 256), (136, 264), (320, 24)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_tiles_of_every_height(ops, positions, H, ff, gated):
+    """An expert of `positions` rows between one of none and one of a single row: a tile is up to 224 positions high, in steps
+    of 32, and K's end may lie inside a stage of 64 (136, 264, 24) or be the first stage's (64, 24).  The bounds are those
+    of `test_experts_over_their_own_rows`."""
+    E, n, wide = 3, positions + 1, 2 if gated else 1
+    g = torch.Generator(device=DEV).manual_seed(positions + H)
+    up = (torch.randn(wide * E * ff, H, generator=g, device=DEV) * H ** -0.5).bfloat16()
+    down = (torch.randn(H, E * ff, generator=g, device=DEV) * ff ** -0.5).bfloat16()
+    y = torch.randn(n, H, generator=g, device=DEV).bfloat16()
+    chosen = torch.full((n, 1), 1, dtype=torch.int32, device=DEV)
+    chosen[n // 2] = 2
+    weights = torch.rand(n, E, generator=g, device=DEV) + 0.1
+    off, order, place = grouped(ops, chosen, E)
+    h = torch.empty(n, ff, dtype=torch.bfloat16, device=DEV)
+    act = {"terms": ops.GateTerms(1.5, 1.702, 1.0, 0.75, True)} if gated else {"activation": "relu2"}
+    ops.grouped_up(y, up, ff, 0, 0, off, order, 1, weights, h, **act)
+    want, z_want, z_size = (torch.zeros(n, c, dtype=torch.float64, device=DEV) for c in (ff, H, H))
+    for e, at in ((1, slice(0, positions)), (2, slice(positions, n))):
+        rows = order[at].long()
+        s = weights[rows, e: e + 1].double()
+        p = y[rows].double() @ up[wide * e * ff: wide * (e + 1) * ff].double().T
+        if gated:
+            a, u = (p[:, :ff] * s).clamp(max=1.5), (p[:, ff:] * s).clamp(-1.5, 1.5)
+            want[at] = a * torch.sigmoid(1.702 * a) * (u + 1.0)
+        else:
+            want[at] = torch.relu(p) ** 2 * s
+        d = down[:, e * ff: (e + 1) * ff].double()
+        z_want[at], z_size[at] = h[at].double() @ d.T, h[at].double().abs() @ d.abs().T
+    assert float(((h.double() - want).abs() - want.abs() * 2.0 ** -8).max()) < 1e-4 * float(want.abs().max())
+    z = torch.empty(n, H, device=DEV)
+    ops.grouped_down(h, down, E, 0, 0, 1, off, z)
+    assert bool(((z.double() - z_want).abs() <= (ff + 8) * 2.0 ** -24 * z_size + 1e-30).all())

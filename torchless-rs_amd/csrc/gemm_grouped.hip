@@ -3,7 +3,7 @@
 // the host knowing how many there are.
 //
 //  * group_pairs: the (row, chosen expert) pairs in the order of their experts, a row's place kept within one.
-//  * gemm_grouped: tiles of up to 160 positions of one group by 256 of its channels.  What a tile does with its sums is the
+//  * gemm_grouped: tiles of up to 224 positions of one group by 256 of its channels.  What a tile does with its sums is the
 //    kernel's template: an expert's activation times the row's weight into bfloat16, gated or not, or the sums as
 //    they are.
 //  * combine_pairs: a row's results from its experts added up in the order in which it chose them.
@@ -11,11 +11,9 @@
 // A shared expert, which every row uses, can run along as slices of at most an expert's size: groups E, E + 1, ... of all
 // rows each, at the positions behind the pairs', whose results are added behind the chosen experts'.
 #include "experts.hpp"
+#include "tile_loop.hpp"
 
 namespace tl {
-
-#define TL_AS1 __attribute__((address_space(1)))      // global memory and LDS, as global_load_lds takes them
-#define TL_AS3 __attribute__((address_space(3)))
 
 // ---- the order of the pairs --------------------------------------------------------------------------------
 // chosen [n_pairs] expert numbers -> offsets [E + 1], order [n_pairs]: position -> pair, place [n_pairs]: pair ->
@@ -118,155 +116,98 @@ __device__ __forceinline__ int group_first(const Grouped& g, int x) {
 }
 __device__ __forceinline__ int group_size(const Grouped& g, int x) { return x < g.E ? g.offsets[x + 1] - g.offsets[x] : g.rows; }
 
-constexpr int GG_BM = 160, GG_BN = 256, GG_BK = 64, GG_NS = 3, GG_WAVES = 4;
-constexpr int GG_ROWB = GG_BK * 2, GG_STAGE = (GG_BM + GG_BN) * GG_ROWB, GG_LDS = GG_NS * GG_STAGE;
+constexpr int GG_BM = 224, GG_BN = 256, GG_WN = 4, GG_NA = 2, GG_NW = 3;
+constexpr int GG_LDS = tile_lds<GG_WN, GG_BM / 32, GG_NA, GG_NW>();
 static_assert(GG_LDS <= 160 * 1024, "a compute unit's LDS");
 
-// Where the operands of a tile come from, and its place.
+// A tile and its place.
 struct Tile {
-  const bf16* asrc[GG_BM / 32];      // this lane's sources: of the 8 rows wave + 4 x of A's, and of the wave's 64 rows of W
-  const bf16* wsrc[8];
   int e, m0, m_rows, n0;
   int K, N;                          // of its group
   int row0;                          // what a position of a slice lies past its row
   int first;                         // the stage of K it begins with
 };
 
-// All of K for 16 MU rows of A (MU: an even number of 16-row blocks, those that hold positions) by the wave's 64 rows of W.
+// All of K for 32 MU rows of A (those that hold positions, and up to 31 more) by 256 rows of W.
 template <int EPI, int MU>
 __device__ __forceinline__ void gg_tile(const Grouped& g, const Tile& t, unsigned char* smem) {
-  constexpr int AI = MU / 2, LPS = AI + 8;                     // loads of a wave a stage: A's, and all
-  constexpr int EARLY = MU < 4 ? MU : 4;                       // blocks of A that are in registers before their turn
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, li = lane % 16, kg = lane / 16;
-  const int stages = (t.K + GG_BK - 1) / GG_BK;
-  const int chunk = (lane % 8) ^ ((lane / 16) & 3);            // of an 8-row load's even half of 16 rows; the odd half's differs in bit 2
-  const auto issue = [&](int i) {
-    unsigned char* slot = smem + (i % GG_NS) * GG_STAGE;
-    int k = i + t.first;
-    if (k >= stages) k -= stages;
-    k *= GG_BK;
-    // (past the end of a row its last chunk again, see `cut`)
-    const int even = min(k + chunk * 8, t.K - 8), odd = min(k + (chunk ^ 4) * 8, t.K - 8), mine = wave % 2 ? odd : even;
+  using S = TileShape<GG_WN, MU>;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, li = lane % 16, kg = lane / 16;
+  const int wm = wave / GG_WN, wn = wave % GG_WN, sub = lane / 8;
+  const bool slice = t.e >= g.E;
+  const char* asrc[S::A_PER];
 #pragma unroll
-    for (int x = 0; x < 8; ++x)
-      __builtin_amdgcn_global_load_lds((const TL_AS1 void*)(t.wsrc[x] + (x % 2 ? odd : even)),
-                                       (TL_AS3 void*)(slot + GG_BM * GG_ROWB + (wave * 8 + x) * 1024), 16, 0, 0);
+  for (int x = 0; x < S::A_PER; ++x) {
+    const int pos = t.m0 + min(tile_load<S::A_LOADS>(wave, x) * 8 + sub, t.m_rows - 1);
+    const int row = !g.order ? pos : slice ? pos - t.row0 : g.order[pos] / g.top;
+    asrc[x] = reinterpret_cast<const char*>(g.A + (size_t)row * g.lda);
+  }
+  const bool apart = EPI == GG_GATED && slice;
+  const bf16* We = apart ? g.gated_slices + (size_t)(t.e - g.E) * g.N * g.ldw : g.W + (size_t)t.e * g.w_step;
+  const size_t up_at = EPI == GG_GATED ? (apart ? (size_t)g.up_step : (size_t)g.N * g.ldw) : 0;
+  const char* wsrc[S::W_PER];
 #pragma unroll
-    for (int x = 0; x < AI; ++x)
-      __builtin_amdgcn_global_load_lds((const TL_AS1 void*)(t.asrc[x] + mine), (TL_AS3 void*)(slot + (wave + 4 * x) * 1024), 16, 0, 0);
-  };
+  for (int x = 0; x < S::W_PER; ++x) {
+    const int r = (wave + TILE_WAVES * x) * 8 + sub;           // row of the tile
+    if (EPI == GG_GATED)                                       // 16 gate rows and their 16 up rows in turn
+      wsrc[x] = reinterpret_cast<const char*>(We + (size_t)min(t.n0 + r / 32 * 16 + r % 16, t.N - 1) * g.ldw + (r / 16 % 2 ? up_at : 0));
+    else
+      wsrc[x] = reinterpret_cast<const char*>(We + (size_t)min(t.n0 + r, t.N - 1) * g.ldw);
+  }
   f32x4 acc[MU][4];
 #pragma unroll
   for (int u = 0; u < MU; ++u)
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[u][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // chunk c of row r of a stage lies at place c ^ (r / 2 % 8) of its 128 bytes
-  const int row_at = li * GG_ROWB, place[2] = {(kg ^ (li / 2)) * 16, ((4 + kg) ^ (li / 2)) * 16};
-  const auto fetch_w = [&](int i, int half, bf16x8 (&w)[4]) {
-    const unsigned char* slot = smem + (i % GG_NS) * GG_STAGE + GG_BM * GG_ROWB + wave * 8192 + row_at + place[half];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) w[v] = *reinterpret_cast<const bf16x8*>(slot + v * 2048);
-  };
-  const auto fetch_a = [&](int i, int half, int u) {
-    return *reinterpret_cast<const bf16x8*>(smem + (i % GG_NS) * GG_STAGE + row_at + place[half] + u * 2048);
-  };
-  // half a stage (32 k): the operands of its first products are in registers; the others come from LDS between the products (a
-  // wave is alone on its SIMD, and a row of reads would let the matrix core idle), and behind them the next half's first
-  const auto multiply = [&](int i, int half, bool more, bool cut, const bf16x8 (&a)[EARLY], const bf16x8 (&w)[4], bf16x8 (&an)[EARLY], bf16x8 (&wn)[4]) {
-    bf16x8 b[MU];
-#pragma unroll
-    for (int u = 0; u < EARLY; ++u) b[u] = a[u];
-#pragma unroll
-    for (int u = EARLY; u < MU; ++u) b[u] = fetch_a(i, half, u);
-    if (more) {
-      fetch_w(i + half, 1 - half, wn);
-#pragma unroll
-      for (int u = 0; u < EARLY; ++u) an[u] = fetch_a(i + half, 1 - half, u);
-    }
-    if (cut && (stages - 1) * GG_BK + (half * 4 + kg) * 8 >= t.K) {      // what lies past the end of K (a multiple of 8)
-#pragma unroll
-      for (int u = 0; u < MU; ++u)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[u][j] = (bf16)0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < MU; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[v], b[u], acc[u][v], 0, 0, 0);
-    constexpr int READS = MU + 4, EACH = MU * 4 / READS;
-#pragma unroll
-    for (int r = 0; r < READS; ++r) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // this wave's reads have returned, before the next barrier
-  };
-  issue(0);
-  if (stages > 1) {
-    issue(1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPS) : "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  __builtin_amdgcn_s_barrier();
-  bf16x8 a0[EARLY], a1[EARLY], w0[4], w1[4];
-  fetch_w(0, 0, w0);
-#pragma unroll
-  for (int u = 0; u < EARLY; ++u) a0[u] = fetch_a(0, 0, u);
-  for (int i = 0; i + 1 < stages; ++i) {
-    __builtin_amdgcn_s_barrier();                              // everyone has left stage i - 1
-    if (i + 2 < stages) issue(i + 2);                          // into its place
-    multiply(i, 0, true, false, a0, w0, a1, w1);
-    // stage i + 1 is here when only the loads behind it are under way
-    if (i + 2 < stages) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    multiply(i, 1, true, false, a1, w1, a0, w0);
-  }
-  const bool cut = t.K % GG_BK != 0;
-  multiply(stages - 1, 0, true, cut, a0, w0, a1, w1);
-  multiply(stages - 1, 1, false, cut, a1, w1, a0, w0);
+  tile_loop<GG_WN, MU, GG_NA, GG_NW, 0>(smem, [&](int x) { return asrc[x]; }, [&](int x) { return wsrc[x]; }, t.K, 0,
+                                        (t.K + TILE_K - 1) / TILE_K, t.first, acc);
 
-  // acc[u][v][r]: position 16 u + li of the tile, row 64 wave + 16 v + 4 kg + r of W's tile
+  // acc[u][v][r]: position 16 (wm MU + u) + li of the tile, row 64 wn + 16 v + 4 kg + r of W's tile
+  float s[MU], after[MU];
+  if constexpr (EPI != GG_STORE) {
+#pragma unroll
+    for (int u = 0; u < MU; ++u) {
+      const int pos = t.m0 + min((wm * MU + u) * 16 + li, t.m_rows - 1);
+      const int row = slice ? pos - t.row0 : g.order[pos] / g.top;
+      s[u] = slice ? 1.f : g.weights[(size_t)row * g.E + t.e];
+      after[u] = slice && g.row_weight ? g.row_weight[row] : 1.f;
+    }
+  }
 #pragma unroll
   for (int u = 0; u < MU; ++u) {
-    const int m = u * 16 + li;
+    const int m = (wm * MU + u) * 16 + li;
     if (m >= t.m_rows) continue;
     const int pos = t.m0 + m;
     if constexpr (EPI == GG_STORE) {
       float* out = (float*)g.C + (size_t)pos * g.N;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int n = t.n0 + wave * 64 + v * 16 + kg * 4;
+        const int n = t.n0 + wn * 64 + v * 16 + kg * 4;
         if (n < t.N) *reinterpret_cast<f32x4*>(out + n) = acc[u][v];
       }
     } else {
-      const bool slice = t.e >= g.E;
-      const int row = slice ? pos - t.row0 : g.order[pos] / g.top;
-      const float s = slice ? 1.f : g.weights[(size_t)row * g.E + t.e];
-      const float after = slice && g.row_weight ? g.row_weight[row] : 1.f;
       bf16* out = (bf16*)g.C + (size_t)pos * g.N;
       if constexpr (EPI == GG_UNARY) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int n = t.n0 + wave * 64 + v * 16 + kg * 4;
+          const int n = t.n0 + wn * 64 + v * 16 + kg * 4;
           if (n >= t.N) continue;
           bf16x4 h;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float z = fmaxf(acc[u][v][r], 0.f);
-            h[r] = (bf16)((g.squared ? z * z : z) * s * after);
+            h[r] = (bf16)((g.squared ? z * z : z) * s[u] * after[u]);
           }
           *reinterpret_cast<bf16x4*>(out + n) = h;
         }
       } else {
 #pragma unroll
         for (int v = 0; v < 4; v += 2) {
-          const int n = t.n0 + wave * 32 + v * 8 + kg * 4;
+          const int n = t.n0 + wn * 32 + v * 8 + kg * 4;
           if (n >= t.N) continue;
           bf16x4 h;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) h[r] = (bf16)(gated_value(acc[u][v][r], acc[u][v + 1][r], s, slice ? g.gate.limit_shared : g.gate.limit, g.gate) * after);
+          for (int r = 0; r < 4; ++r) h[r] = (bf16)(gated_value(acc[u][v][r], acc[u][v + 1][r], s[u], slice ? g.gate.limit_shared : g.gate.limit, g.gate) * after[u]);
           *reinterpret_cast<bf16x4*>(out + n) = h;
         }
       }
@@ -274,23 +215,19 @@ __device__ __forceinline__ void gg_tile(const Grouped& g, const Tile& t, unsigne
   }
 }
 
-// A workgroup of 4 waves, one to a SIMD, has a tile of up to 160 positions of a group x 256 rows of W; a wave has all of the
-// positions and 64 of the rows (160 sums a lane), so that a tile with fewer positions costs the matrix cores that much
-// less, in steps of 32.  A group's positions are dealt to its tiles evenly.  Stages of 64 k (52 KB, whole lines of 128 bytes:
-// halves of 64 were fetched twice) go from memory straight into a ring of three in LDS.  Chunk c of row r of a stage lies at
-// place c ^ (r / 2 % 8): 16 lanes that read one chunk of 16 rows fall on all banks once.  Rows of A come from where the
-// pair's row lies (a lane gives its own address).
-// What bounds it: the products of a stage are 1,280 cycles of the matrix cores, the reads and writes of LDS 1,310, and they
-// overlap in part only: a stage takes 1.5 us with the chip full, 1.26 with the loads taken out, 0.9 with the products.
-// Other tiles measured (2,312 rows, 16 experts of 3,584 channels, 4 a row, up / down, microseconds; this one 444 / 361):
-// 128 x 256 with stages of 32 k and two workgroups a unit 461 / 407, 256 x 256 with 4 waves 462 / 450, with 8 waves 438 / 383
-// (1,024 rows: 256 / 224 against 189 / 164 here, since 257 rows take two of its tiles), W from memory into registers 472 / 442.
+// A workgroup of 8 waves has a tile of up to 224 positions of a group x 256 rows of W (see tile_loop.hpp; 256 positions would
+// spill); a tile with fewer positions costs the matrix cores that much less, in steps of 32.  A group's positions are dealt to its
+// tiles evenly.  Rows of A come from where the pair's row lies (a lane gives its own address).
+// Bound by the products' rate with the chip full, and with few positions an expert by the weights (5.7 TB/s at 130 rows).  16
+// experts, 4 a row, microseconds, up / down, before with four waves of 160 x 64, a wave alone on its SIMD: 3,584 channels at 600 rows
+// 125 / 188 and 110 / 113 now, 2,312 rows 381 / 325 and 287 / 272 (0.95 and 1.0 PFLOP/s), 8,192 rows 1,144 / 1,081 and 862 / 891
+// (1.1); 1,792 gated ones at 2,312 rows 386 / 183 and 280 / 142; 130 and 300 rows as they were.
 template <int EPI>
-__global__ void __launch_bounds__(GG_WAVES * WAVE, 1)
+__global__ void __launch_bounds__(TILE_WAVES * WAVE)
 gemm_grouped_kernel(Grouped g) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gg_smem[];
   constexpr int CT = EPI == GG_GATED ? GG_BN / 2 : GG_BN;      // channels of C a tile
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int lane = threadIdx.x % WAVE;
   const int nt = (g.N + CT - 1) / CT;
 
   // which tile: an expert's tiles follow each other, of its tiles those of the same channels; each of the 8 XCDs
@@ -340,32 +277,16 @@ gemm_grouped_kernel(Grouped g) {
   t.K = last && g.slice_k ? g.last : g.K;
   t.N = last && !g.slice_k ? g.last : g.N;
   if (t.n0 >= t.N) return;                                     // (the last slice may have fewer channels)
-  t.first = g.stagger ? (int)((long)t.first * ((t.K + GG_BK - 1) / GG_BK) / nt) : 0;
+  t.first = g.stagger ? (int)((long)t.first * ((t.K + TILE_K - 1) / TILE_K) / nt) : 0;
 
-  const int sub = lane / 8;                                    // a load takes 8 rows of 128 bytes
-#pragma unroll
-  for (int x = 0; x < GG_BM / 32; ++x) {
-    const int pos = t.m0 + min((wave + 4 * x) * 8 + sub, t.m_rows - 1);
-    const int row = !g.order ? pos : slice ? pos - t.row0 : g.order[pos] / g.top;
-    t.asrc[x] = g.A + (size_t)row * g.lda;
-  }
-  const bool apart = EPI == GG_GATED && slice;
-  const bf16* We = apart ? g.gated_slices + (size_t)(t.e - g.E) * g.N * g.ldw : g.W + (size_t)t.e * g.w_step;
-  const size_t up_at = EPI == GG_GATED ? (apart ? (size_t)g.up_step : (size_t)g.N * g.ldw) : 0;
-#pragma unroll
-  for (int x = 0; x < 8; ++x) {
-    const int r16 = wave * 4 + x / 2, r = x % 2 * 8 + sub;     // row r of 16 rows of the tile
-    if (EPI == GG_GATED)                                       // gate and up in turn
-      t.wsrc[x] = We + (size_t)min(t.n0 + r16 / 2 * 16 + r, t.N - 1) * g.ldw + (r16 % 2 ? up_at : 0);
-    else
-      t.wsrc[x] = We + (size_t)min(t.n0 + r16 * 16 + r, t.N - 1) * g.ldw;
-  }
   switch ((t.m_rows + 31) / 32) {
-    case 1: gg_tile<EPI, 2>(g, t, gg_smem); break;
-    case 2: gg_tile<EPI, 4>(g, t, gg_smem); break;
-    case 3: gg_tile<EPI, 6>(g, t, gg_smem); break;
-    case 4: gg_tile<EPI, 8>(g, t, gg_smem); break;
-    default: gg_tile<EPI, 10>(g, t, gg_smem); break;
+    case 1: gg_tile<EPI, 1>(g, t, gg_smem); break;
+    case 2: gg_tile<EPI, 2>(g, t, gg_smem); break;
+    case 3: gg_tile<EPI, 3>(g, t, gg_smem); break;
+    case 4: gg_tile<EPI, 4>(g, t, gg_smem); break;
+    case 5: gg_tile<EPI, 5>(g, t, gg_smem); break;
+    case 6: gg_tile<EPI, 6>(g, t, gg_smem); break;
+    default: gg_tile<EPI, 7>(g, t, gg_smem); break;
   }
 }
 
@@ -384,7 +305,7 @@ template <int EPI> static int launch_grouped(const Grouped& g, hipStream_t st) {
   const long most = nt * (pairs / GG_BM + (g.E < pairs ? g.E : pairs) + (long)g.slices * ((g.rows + GG_BM - 1) / GG_BM));
   const long grid = (most + 7) / 8 * 8;
   TL_REQUIRE(grid < (1l << 31), "gemm_grouped: rows=%d N=%d have more tiles than a grid holds", g.rows, g.N);
-  gemm_grouped_kernel<EPI><<<(unsigned)grid, GG_WAVES * WAVE, GG_LDS, st>>>(g);
+  gemm_grouped_kernel<EPI><<<(unsigned)grid, TILE_WAVES * WAVE, GG_LDS, st>>>(g);
   TL_LAUNCH_CHECK("gemm_grouped");
   return 0;
 }
@@ -444,7 +365,7 @@ int tl_gemm_grouped(const void* A, const void* W, void* C, int n, int H, int E, 
   g.gated_slices = g.W + (long long)2 * E * ff * H;
   // where an expert has few positions the weights come from memory, row after row at one distance: workgroups that go along K
   // in step would ask the same channels of the memory at a time (130 rows of 16 experts: 113 to 86 us; K's tail has to be the last stage)
-  g.stagger = g.K % GG_BK == 0 && (!down || slices == 0 || g.last % GG_BK == 0) && (long)n * top <= (long)E * GG_BM;
+  g.stagger = g.K % TILE_K == 0 && (!down || slices == 0 || g.last % TILE_K == 0) && (long)n * top <= (long)E * GG_BM;
   g.weights = weights; g.row_weight = row_weight;
   g.squared = act_code == 0;
   g.gate = GateTerms{limit, limit_shared, alpha, shift, on_input};
