@@ -1,0 +1,116 @@
+"""Products of more than 128 rows in tiles of the package's own (csrc/gemm_tall.hip, csrc/tile_loop.hpp) against float64, at the
+edges of tiles, of K's stages and slices, and of the rule that chooses them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TILES = [(256, 256), (224, 256), (192, 256), (160, 256), (256, 128), (192, 128), (128, 128)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from torchless_rs_amd.kernels import ops as o
+    o.lib()
+    return o
+
+
+def operands(M, N, K, apart=0):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), torch.randn(N, K + apart, generator=g, device=DEV).bfloat16()[:, :K]
+    return a, w, a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+
+
+def bound(K, size):
+    """A sum of K products in 32 bits, in any order, lies within K 2^-24 of the sum of the products' sizes; the worst of M N
+    chains is a few dozen standard errors of a walk, sqrt(K) 2^-24 of it, below 8."""
+    return 8 * K ** 0.5 * 2.0 ** -24 * size + 1e-30
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K,apart", [(1, 4, 8, 0), (129, 64, 64, 8), (257, 772, 136, 0), (300, 260, 640, 0), (513, 128, 1096, 16)])
+def test_tiles_and_slices(ops, tile, M, N, K, apart):
+    a, w, want, size = operands(M, N, K, apart)
+    stages = -(-K // 64)
+    for S in (1, 2, 3, 5):
+        if (S - 1) * -(-stages // S) >= stages:
+            continue
+        plan = ops.TallPlan(*tile, S, stagger=S == 1 and K % 64 == 0)
+        out = torch.full((S, M, N), float("nan"), device=DEV)
+        ops.gemm_tall_bf16(a, w, out if S > 1 else out[0], plan)
+        assert bool(((out.double().sum(0) - want).abs() <= bound(K, size)).all())
+    x = torch.randn(M, N, device=DEV)
+    total = x.double() + want
+    ops.gemm_tall_bf16(a, w, x, ops.TallPlan(*tile), accumulate=True)
+    assert bool(((x.double() - total).abs() <= bound(K, size) + 2.0 ** -23 * total.abs()).all())
+
+
+@pytest.mark.parametrize("tile", [t for t in TILES if t[1] == 256])
+@pytest.mark.parametrize("parts", [2, 4])
+@pytest.mark.parametrize("M,N", [(17, 4100), (257, 2176), (1000, 772), (1025, 640)])
+def test_last_tiles_in_parts(ops, tile, parts, M, N):
+    """Whole tiles and parts write every sum once: halves by channels, quarters by rows too, the last of either cut short."""
+    K = 192
+    a, w, want, size = operands(M, N, K)
+    tiles = -(-M // tile[0]) * -(-N // 256)
+    for whole in (0, 8, tiles // 8 * 8):
+        if whole <= tiles:
+            x = torch.ones(M, N, device=DEV)
+            ops.gemm_tall_bf16(a, w, x, ops.TallPlan(*tile, whole=whole, parts=parts), accumulate=True)
+            assert bool(((x.double() - 1.0 - want).abs() <= bound(K, size) + 2.0 ** -23 * (want.abs() + 1.0)).all()), whole
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu", ("swish_clamped", {"alpha": 1.702, "limit": 7.0, "shift": 1.0})])
+@pytest.mark.parametrize("M,I,K,plan", [(129, 32, 64, (192, 128)), (300, 96, 264, (160, 256)), (520, 672, 128, (256, 256, 1, False, 8, 2)),
+                                        (520, 672, 128, (192, 256, 1, False, 8, 4))])
+def test_paired(ops, act, M, I, K, plan):
+    """act(gate) * up of the sums, rounded to bfloat16 once (2^-9 of itself); the sums' error and the exponential's, 2^-20, pass
+    through functions whose slope is near 1 or below, times the other factor: 1e-5 of the sums' sizes covers both."""
+    a, w, p, size = operands(M, 2 * I, K)
+    a, p, size = a * K ** -0.5, p * K ** -0.5, size * K ** -0.5
+    p = a.double() @ w.double().t()
+    gate, up = p.view(M, I // 32, 2, 32).unbind(2)
+    gate, up = gate.reshape(M, I), up.reshape(M, I)
+    name = act if isinstance(act, str) else act[0]
+    if name == "silu":
+        want = torch.nn.functional.silu(gate) * up
+    elif name == "gelu_tanh":
+        want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+    elif name == "relu":
+        want = torch.relu(gate) * up
+    else:
+        gate = gate.clamp(max=7.0)
+        want = gate * torch.sigmoid(1.702 * gate) * (up.clamp(-7.0, 7.0) + 1.0)
+    out = torch.full((M, I), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.gemm_tall_bf16(a, w, out, ops.TallPlan(*plan), silu_pair=True, pair_act=act)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + size.max())).all())
+
+
+def test_plans_fit_what_they_are_for(ops):
+    """Every plan of the rule can be launched: K's slices all have stages, whole tiles are rounds of workgroups, partial sums are
+    made only where they are welcome, nothing is planned up to MID_ROWS rows or for sizes the tiles do not take."""
+    for N, K in ((28672, 4096), (4096, 14336), (5120, 14336), (18560, 4096), (64, 64), (12288, 4104), (4096, 4096), (2048, 8192)):
+        for M in list(range(129, 700, 37)) + [1024, 1999, 2048, 4097, 16384]:
+            for kind, sums in (("store", False), ("add", False), ("add", True), ("pair", False)):
+                p = ops.tall_plan(M, N, K, 256, kind, sums)
+                if p is None:
+                    continue
+                stages = -(-K // 64)
+                assert (p.rows, p.channels) in TILES and (p.n_split == 1 or (sums and kind == "add"))
+                assert (p.n_split - 1) * -(-stages // p.n_split) < stages and not (p.stagger and (K % 64 or p.n_split > 1 or p.parts))
+                assert p.parts in (0, 2, 4) and p.whole % 256 == 0 and (p.parts or not p.whole)
+    assert ops.tall_plan(128, 28672, 4096, 256, "pair") is None and ops.tall_plan(2048, 28672, 4100, 256, "pair") is None
+    assert ops.tall_plan(2048, 28704, 4096, 256, "pair") is None and ops.tall_plan(2048, 4098, 4096, 256, "add") is None
+
+
+def test_what_the_tiles_do_not_take_is_refused(ops):
+    a, w = torch.zeros(200, 128, dtype=torch.bfloat16, device=DEV), torch.zeros(256, 128, dtype=torch.bfloat16, device=DEV)
+    out = torch.zeros(200, 256, device=DEV)
+    with pytest.raises(ops.KernelError, match="no tiles"):
+        ops.gemm_tall_bf16(a, w, out, ops.TallPlan(64, 256))
+    with pytest.raises(ops.KernelError, match="without a stage"):
+        ops.gemm_tall_bf16(a, w, torch.zeros(3, 200, 256, device=DEV), ops.TallPlan(256, 256, 3))
+    with pytest.raises(ops.KernelError, match="multiple of 8"):
+        ops.gemm_tall_bf16(a, w, out, ops.TallPlan(256, 256, whole=1, parts=2))
+    with pytest.raises(ops.KernelError, match="bfloat16 rows"):
+        ops.gemm_tall_bf16(a, torch.zeros(128, 256, dtype=torch.bfloat16, device=DEV).t(), out, ops.TallPlan(256, 256))

@@ -18,15 +18,15 @@
 //  * gemm_mid: 17..128 rows.  The activations of a k-step are shared by the four
 //    waves through LDS; K may be cut over workgroups into partial sums.
 //  * gemm_ring: the same rows where K is a multiple of 128, both operands through a ring in LDS.
-//  * gemm_wide: 129..256 rows into the stream where the channels leave compute units idle.
-// Products with more rows (prefill, large decode batches) and those that gemm_wide does not serve are the BLAS
-// library's, as the reference hands its products to the vendor's library.
+// Products with more rows (prefill, large decode batches) are gemm_tall.hip's or the BLAS library's, as the reference hands its
+// products to the vendor's library.
 //
 // All need K % 8 == 0 and 16-byte aligned rows; callers fall back to the
 // plain kernel otherwise.
 #include <type_traits>
 
 #include "common.hpp"
+#include "epilogues.hpp"
 
 namespace tl {
 
@@ -45,40 +45,6 @@ __device__ __forceinline__ bf16x8 zero8() {
 #pragma unroll
   for (int i = 0; i < 8; ++i) z[i] = (bf16)0.f;
   return z;
-}
-
-// what happens to the product
-constexpr int EPI_STORE = 0;        // C = product (float)
-constexpr int EPI_ACCUMULATE = 1;   // C += product (float; the residual stream)
-constexpr int EPI_SILU_PAIR = 2;    // W's rows come in groups of 64 (32 gate rows, their 32 up rows):
-                                    // C is bfloat16 [M, N/2] = silu(gate) * up
-constexpr int EPI_GELU_PAIR = 3;    // the same pairs with the tanh form of gelu on the gate:
-                                    // 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3)))
-constexpr int EPI_SWISH_CLAMPED_PAIR = 4;   // the same pairs with g' = min(g, limit), u' = clamp(u, -limit, limit):
-                                            // g' / (1 + exp(-alpha g')) * (u' + shift)
-constexpr int EPI_RELU_PAIR = 5;    // the same pairs with max(g, 0) on the gate
-__host__ __device__ __forceinline__ bool is_pair(int epilogue) {
-  return epilogue == EPI_SILU_PAIR || epilogue == EPI_GELU_PAIR || epilogue == EPI_SWISH_CLAMPED_PAIR ||
-         epilogue == EPI_RELU_PAIR;
-}
-// What happens to the product as the kernels take it: the code, and the constants of a paired epilogue
-// whose function has some.  It reads as its code wherever a plain number is asked for.
-struct Epi {
-  int code;
-  float alpha, limit, shift;
-  __host__ __device__ Epi(int c = EPI_STORE, float a = 1.f, float l = 0.f, float s = 0.f) : code(c), alpha(a), limit(l), shift(s) {}
-  __host__ __device__ __forceinline__ operator int() const { return code; }
-};
-// act(gate) * up of a paired epilogue, on the float sums
-__device__ __forceinline__ float pair_value(float g, float u, const Epi& e) {
-  if (e.code == EPI_SWISH_CLAMPED_PAIR) {
-    g = fminf(g, e.limit);
-    u = fminf(fmaxf(u, -e.limit), e.limit);
-    return (g / (1.0f + expf(-e.alpha * g))) * (u + e.shift);
-  }
-  if (e.code == EPI_RELU_PAIR) return fmaxf(g, 0.f) * u;
-  if (e.code == EPI_GELU_PAIR) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
-  return (g / (1.0f + expf(-g))) * u;
 }
 
 // An RMSNorm cut in two around a product of at most 16 rows, so that the norm needs no
@@ -853,12 +819,12 @@ gemm_ring_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, float* 
               ((place ^ key(r)) * 16);
     adst[x] = q < A_INSTR ? q * 1024 : -1;
   }
-  // Where K is not cut, workgroups of other channels begin with other stages and go round: rows of W are all the same power
-  // of two (or nearly) apart, so that workgroups in step would ask a few of the memory's channels at a time.  gate|up of the
-  // 7B shape at 24 / 64 / 128 rows 50 / 52 / 67 us in step, 41 / 44 / 64 like this (5.3 TB/s at 64 rows; a read of rows 8 KB
-  // apart alone: 4.9 TB/s in step, 6.9 not), the head of 32,000 channels 55 / 57 / 66 and 45 / 47 / 64.  Slices of K begin
-  // in different places already: o, down and q|k|v take what they took.
-  const int first = gridDim.y == 1 ? blockIdx.x % n_t : 0;
+  // Where K is not cut and rows of W are multiples of 4 KB apart, workgroups of other channels begin with other stages and go
+  // round: in step they would ask a few of the memory's channels at a time.  28,672 channels at 24 / 64 rows, in step and
+  // like this, us: K = 4,096 46 / 47 and 40 / 43, 6,144 73 / 78 and 58 / 63, 8,192 104 / 102 and 74 / 78; 32,768 x 14,336 148 / 157
+  // and 144 / 151; other distances spread by themselves (3,584 35 / 39 either way; 5,120 at 24 rows 49.6 and 50.3).  Slices of K begin in
+  // different places already: o, down and q|k|v take what they took.
+  const int first = gridDim.y == 1 && K % 2048 == 0 ? blockIdx.x % n_t : 0;
   auto issue = [&](int i) {                                 // the stage with which turn i is concerned into its place in the ring
     unsigned char* slot = ring_smem + (i % NS) * STAGE;
     const size_t off = (size_t)(i + first < n_t ? i + first : i + first - n_t) * ROWB;
@@ -987,129 +953,6 @@ static int launch_ring_rows(const bf16* A, const bf16* W, float* C, int M, int N
   return launch_ring<8, WAVES, KC>(A, W, C, M, N, K, n_split, epilogue, st);
 }
 
-// ------------------------------------------------------------------ wide ----
-// 129..256 rows, N and K multiples of 64: a workgroup has all of the rows and 128 channels, so that the weights are read once,
-// and the few tiles are cut along K instead of along the rows: partial sums, which the next kernel adds up.
-// Both operands go into a ring of three or four stages of 64 k in LDS, as in gemm_ring.  There a wave reads every row of A for
-// its 16 channels, which at 192 rows would keep LDS busier than memory; here a wave has 32 channels and one half of a
-// stage's k: eight waves, two on a SIMD, of which one reads while the other multiplies.  The halves' sums meet at the end.
-// What bounds it: a compute unit's loads, 40 or 48 KB a stage of which 16 KB come from memory: 1.1 us (a fourth
-// stage under way takes nothing off).  So a product whose channels alone fill the units is as fast in the BLAS library
-// (28,672 x 4,096, 192 rows: 72 us here, 66 there); one that has few tiles is not.  With the partial sums added, the library's in
-// brackets, 192 rows: 4,096 x 14,336 42 us (103), 6,144 x 4,096 29 (34), 4,096 x 4,096 23 (34); 5,120 x 27,648 88 (212).
-constexpr int WIDE_ROWS = 256;
-constexpr int WIDE_KC = 64, WIDE_CH = 128;
-
-constexpr int wide_stages(int MU) { return MU <= 12 ? 4 : 3; }      // of 40 KB, or 48
-
-template <int MU>
-__global__ void __launch_bounds__(512)
-gemm_wide_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, float* __restrict__ C, int M, int N, int K,
-                 int stages_per_split) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char wide_smem[];
-  constexpr int ROWB = WIDE_KC * 2, A_BYTES = MU * 16 * ROWB, STAGE = A_BYTES + WIDE_CH * ROWB, NS = wide_stages(MU);
-  constexpr int A_PER = MU / 4, LPS = A_PER + 2;            // loads a wave issues for a stage: of A's 2 MU, and 2 of W's 16
-  static_assert(MU % 4 == 0, "the rows' loads go evenly over eight waves");
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 16, kg = lane / 16;
-  const int half = wave / 4, w4 = wave % 4;
-  const int n0 = blockIdx.x * WIDE_CH;
-  const int t_begin = blockIdx.y * stages_per_split;
-  const int n_t = min(K / WIDE_KC, t_begin + stages_per_split) - t_begin;
-  // a load takes 8 rows of 128 bytes; chunk c of row r lies at place c ^ (r / 2 % 8)
-  const int sub = lane / 8;
-  const char* asrc[A_PER];
-  const char* wsrc[2];
-#pragma unroll
-  for (int x = 0; x < A_PER; ++x) {
-    const int r = 8 * (wave + 8 * x) + sub;
-    asrc[x] = reinterpret_cast<const char*>(A + (size_t)min(r, M - 1) * K) + (size_t)t_begin * ROWB + (((lane % 8) ^ (r / 2 % 8)) * 16);
-  }
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    const int r = 8 * (wave * 2 + x) + sub;
-    wsrc[x] = reinterpret_cast<const char*>(W + (size_t)min(n0 + r, N - 1) * K) + (size_t)t_begin * ROWB + (((lane % 8) ^ (r / 2 % 8)) * 16);
-  }
-  const auto issue = [&](int i) {
-    unsigned char* slot = wide_smem + (i % NS) * STAGE;
-    const size_t off = (size_t)i * ROWB;
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-      __builtin_amdgcn_global_load_lds((const TL_AS1 void*)(wsrc[x] + off), (TL_AS3 void*)(slot + A_BYTES + (wave * 2 + x) * 1024), 16, 0,
-                                       0);
-#pragma unroll
-    for (int x = 0; x < A_PER; ++x)
-      __builtin_amdgcn_global_load_lds((const TL_AS1 void*)(asrc[x] + off), (TL_AS3 void*)(slot + (wave + 8 * x) * 1024), 16, 0, 0);
-  };
-  f32x4 acc[MU][2];
-#pragma unroll
-  for (int u = 0; u < MU; ++u) acc[u][0] = acc[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int at = li * ROWB + (((half * 4 + kg) ^ (li / 2)) * 16);      // of a block of 16 rows: this lane's chunk of its row
-  const int wat = A_BYTES + w4 * 32 * ROWB + at;
-#pragma unroll
-  for (int i = 0; i < NS - 1; ++i)
-    if (i < n_t) issue(i);
-  for (int i = 0; i < n_t; ++i) {
-    if (n_t - 1 - i >= NS - 2) wait_loads_but<(NS - 2) * LPS>();
-    else wait_loads_but<0>();
-    __builtin_amdgcn_s_barrier();                           // stage i is here for all; everyone has left stage i - 1
-    if (i + NS - 1 < n_t) issue(i + NS - 1);
-    const unsigned char* slot = wide_smem + (i % NS) * STAGE;
-    bf16x8 w[2], a[MU];
-#pragma unroll
-    for (int v = 0; v < 2; ++v) w[v] = *reinterpret_cast<const bf16x8*>(slot + wat + v * 16 * ROWB);
-#pragma unroll
-    for (int u = 0; u < MU; ++u) a[u] = *reinterpret_cast<const bf16x8*>(slot + u * 16 * ROWB + at);
-#pragma unroll
-    for (int u = 0; u < MU; ++u)
-#pragma unroll
-      for (int v = 0; v < 2; ++v) acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[v], a[u], acc[u][v], 0, 0, 0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this wave's reads have returned, before the next barrier
-  }
-  // the halves' sums: each wave gives half of its rows' to the wave of the other half and finishes the rest
-  __syncthreads();
-  f32x4* ex = reinterpret_cast<f32x4*>(wide_smem) + (size_t)wave * MU * 64 + lane;      // [wave][MU][64 lanes]: MU KB a wave
-  const f32x4* got = reinterpret_cast<const f32x4*>(wide_smem) + (size_t)(wave ^ 4) * MU * 64 + lane;
-  const auto give = [&](auto first) {
-#pragma unroll
-    for (int u = 0; u < MU / 2; ++u)
-#pragma unroll
-      for (int v = 0; v < 2; ++v) ex[(u * 2 + v) * 64] = acc[first + u][v];
-  };
-  if (half) give(std::integral_constant<int, 0>{});
-  else give(std::integral_constant<int, MU / 2>{});
-  __syncthreads();
-  const auto finish = [&](auto first) {
-#pragma unroll
-    for (int u = 0; u < MU / 2; ++u) {
-      const int m = (first + u) * 16 + li;
-      if (m >= M) continue;
-      float* c = C + ((size_t)blockIdx.y * M + m) * N;
-#pragma unroll
-      for (int v = 0; v < 2; ++v) {
-        const int n = n0 + w4 * 32 + v * 16 + kg * 4;
-        if (n < N) *reinterpret_cast<f32x4*>(c + n) = acc[first + u][v] + got[(u * 2 + v) * 64];
-      }
-    }
-  };
-  if (half) finish(std::integral_constant<int, MU / 2>{});
-  else finish(std::integral_constant<int, 0>{});
-}
-
-template <int MU>
-static int launch_wide(const bf16* A, const bf16* W, float* C, int M, int N, int K, int n_split, hipStream_t st) {
-  constexpr int LDS = wide_stages(MU) * (MU * 16 + WIDE_CH) * WIDE_KC * 2;
-  static_assert(LDS <= 160 * 1024 && LDS >= 8 * MU * 1024, "the ring, and at the end the halves' sums, fit a unit's LDS");
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<MU>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  if (e != hipSuccess) {
-    set_error("gemm_wide: cannot have %d bytes of LDS: %s", LDS, hipGetErrorString(e));
-    return 2;
-  }
-  const int stages = K / WIDE_KC, per = (stages + n_split - 1) / n_split;
-  gemm_wide_kernel<MU><<<dim3((N + WIDE_CH - 1) / WIDE_CH, n_split), 512, LDS, st>>>(A, W, C, M, N, K, per);
-  TL_LAUNCH_CHECK("gemm_wide");
-  return 0;
-}
-
 }  // namespace tl
 
 using namespace tl;
@@ -1122,9 +965,11 @@ extern "C" int tl_pair_constants(float alpha, float limit, float shift) {
   g_pair_alpha = alpha; g_pair_limit = limit; g_pair_shift = shift;
   return 0;
 }
-static Epi epi_of(int epilogue) {
+namespace tl {
+Epi epi_of(int epilogue) {
   return epilogue == EPI_SWISH_CLAMPED_PAIR ? Epi(epilogue, g_pair_alpha, g_pair_limit, g_pair_shift) : Epi(epilogue);
 }
+}  // namespace tl
 
 // epilogue: 0 store float, 1 accumulate into float, 2 silu(gate) * up into bfloat16 [M, N/2]
 // (W's rows in groups of 64: 32 gate rows and their 32 up rows; N a multiple of 64).
@@ -1258,20 +1103,6 @@ extern "C" int tl_gemm_ring_bf16(const void* A, const void* W, void* C, int M, i
   TL_RING(8);
 #undef TL_RING
   TL_REQUIRE(false, "gemm_ring: %d waves a workgroup (4, 7 or 8)", waves);
-}
-
-// Up to 256 rows, N and K multiples of 64: C float [n_split][M][N] receives partial sums.  Every split has one stage of 64 k
-// at least.
-extern "C" int tl_gemm_wide_bf16(const void* A, const void* W, void* C, int M, int N, int K, int n_split, hipStream_t st) {
-  TL_REQUIRE(M > 0 && M <= WIDE_ROWS && N > 0 && N % 64 == 0 && K > 0 && K % WIDE_KC == 0,
-             "gemm_wide: bad sizes M=%d N=%d K=%d (M at most %d, N and K multiples of 64)", M, N, K, WIDE_ROWS);
-  TL_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)C % 16 == 0, "gemm_wide: operands must be 16-byte aligned");
-  const int stages = K / WIDE_KC;
-  TL_REQUIRE(n_split >= 1 && n_split <= stages && n_split <= 65535, "gemm_wide: %d splits do not fit K=%d", n_split, K);
-  const int per = (stages + n_split - 1) / n_split;
-  TL_REQUIRE((n_split - 1) * per < stages, "gemm_wide: %d splits of K=%d would leave one without a stage", n_split, K);
-  if (M <= 192) return launch_wide<12>((const bf16*)A, (const bf16*)W, (float*)C, M, N, K, n_split, st);
-  return launch_wide<16>((const bf16*)A, (const bf16*)W, (float*)C, M, N, K, n_split, st);
 }
 
 // q|k|v of a step with one token a sequence (row m is sequence m, at position row_pos[m]):

@@ -159,7 +159,7 @@ __device__ __forceinline__ void gg_tile(const Grouped& g, const Tile& t, unsigne
   for (int u = 0; u < MU; ++u)
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[u][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  tile_loop<GG_WN, MU, GG_NA, GG_NW, 0>(smem, [&](int x) { return asrc[x]; }, [&](int x) { return wsrc[x]; }, t.K, 0,
+  tile_loop<GG_WN, MU, GG_NA, GG_NW, 0>(smem, [&](int x, unsigned at) { return asrc[x] + at; }, [&](int x, unsigned at) { return wsrc[x] + at; }, t.K, 0,
                                         (t.K + TILE_K - 1) / TILE_K, t.first, acc);
 
   // acc[u][v][r]: position 16 (wm MU + u) + li of the tile, row 64 wn + 16 v + 4 kg + r of W's tile

@@ -44,7 +44,8 @@ template <int LOADS> __device__ __forceinline__ int tile_load(int wave, int x) {
 }
 
 // acc[u][v][r] += the sum over stages t0 .. t0 + n_t - 1 for row wm * 16 MU + 16 u + lane % 16 of A's tile and row
-// wn * 64 + 16 v + 4 (lane / 16) + r of W's.  a_at(x), w_at(x): this lane's row of load x (row lane / 8 of the eight of `tile_load`), at k = 0.
+// wn * 64 + 16 v + 4 (lane / 16) + r of W's.  a_at(x, at), w_at(x, at): byte `at` of this lane's row of load x (row
+// lane / 8 of the eight of `tile_load`).
 // first: the stage (from t0 on) it begins with, going round.  K: whole rows' length, a multiple of 8; the stage that holds K's
 // end, if that is no multiple of 64, has to come last (first = 0).  n_t >= 1.
 template <int WN, int MU, int NA, int NW, int W_AUX, typename AAt, typename WAt>
@@ -60,43 +61,53 @@ __device__ __forceinline__ void tile_loop(unsigned char* smem, AAt a_at, WAt w_a
   const int wm = wave / WN, wn = wave % WN;
   const int chunk = ((lane % 8) ^ (4 * wave + lane / 16) % 8) * 16;      // this lane's chunk of its rows, in bytes: the same for every load
   const int most = K * 2 - 16 - chunk;                                   // (past the end of a row its last chunk again, see `cut`)
-  const auto bytes_at = [&](int i) { return min((t0 + (i + first < n_t ? i + first : i + first - n_t)) * TILE_ROW, most) + chunk; };
-  const auto load_a = [&](int i, int x, int at) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a_at(x) + at),
-                                     (__attribute__((address_space(3))) void*)(smem + (i % NA) * S::A_SLOT + tile_load<S::A_LOADS>(wave, x) * 1024), 16, 0, 0);
+  const auto bytes_at = [&](int i) { return (unsigned)(min((t0 + (i + first < n_t ? i + first : i + first - n_t)) * TILE_ROW, most) + chunk); };
+  // places in the rings, in bytes: where a stage's operands lie, and where the next stage's do
+  struct Place { int a, w; };
+  const auto behind_of = [](Place p) {
+    return Place{p.a + S::A_SLOT < NA * S::A_SLOT ? p.a + S::A_SLOT : 0, p.w + S::W_SLOT < NW * S::W_SLOT ? p.w + S::W_SLOT : 0};
   };
-  const auto load_w = [&](int i, int x, int at) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(w_at(x) + at),
-                                     (__attribute__((address_space(3))) void*)(smem + W_RING + (i % NW) * S::W_SLOT + (wave + TILE_WAVES * x) * 1024), 16, 0, W_AUX);
+  const auto load_a = [&](int place, int x, unsigned at) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)a_at(x, at),
+                                     (__attribute__((address_space(3))) void*)(smem + place + tile_load<S::A_LOADS>(wave, x) * 1024), 16, 0, 0);
+  };
+  const auto load_w = [&](int place, int x, unsigned at) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)w_at(x, at),
+                                     (__attribute__((address_space(3))) void*)(smem + W_RING + place + (wave + TILE_WAVES * x) * 1024), 16, 0, W_AUX);
   };
   const int a_row = (wm * MU * 16 + li) * TILE_ROW, w_row = W_RING + (wn * 64 + li) * TILE_ROW;
   // read r of a half's MU + 4, W's first
-  const auto read = [&](int i, int half, int r, bf16x8 (&a)[MU], bf16x8 (&w)[4]) {
-    const int place = ((half * 4 + kg) ^ (li / 2)) * 16;
-    if (r < 4) w[r] = *reinterpret_cast<const bf16x8*>(smem + (i % NW) * S::W_SLOT + w_row + place + r * 16 * TILE_ROW);
-    else a[r - 4] = *reinterpret_cast<const bf16x8*>(smem + (i % NA) * S::A_SLOT + a_row + place + (r - 4) * 16 * TILE_ROW);
+  const auto read = [&](Place p, int half, int r, bf16x8 (&a)[MU], bf16x8 (&w)[4]) {
+    const int c = ((half * 4 + kg) ^ (li / 2)) * 16;
+    if (r < 4) w[r] = *reinterpret_cast<const bf16x8*>(smem + p.w + w_row + c + r * 16 * TILE_ROW);
+    else a[r - 4] = *reinterpret_cast<const bf16x8*>(smem + p.a + a_row + c + (r - 4) * 16 * TILE_ROW);
   };
   constexpr int READS = MU + 4, PART = MU > 3 ? MU - 2 : 1;              // the last products cover the reads' way
   constexpr int READS_EACH = (READS + PART - 1) / PART, LOADS_EACH = (LOADS + MU - 1) / MU;
-  // The products of a half; between them, if `more`, the reads of half rh of stage ri, and with `la`, `lw` the loads of turn i.
-  const auto half = [&](const bf16x8 (&a)[MU], const bf16x8 (&w)[4], bool more, int ri, int rh, bf16x8 (&an)[MU], bf16x8 (&wn_)[4], bool la, bool lw, int i) {
-    const int at_a = la ? bytes_at(i + NA) : 0, at_w = lw ? bytes_at(i + NW) : 0;
+  // The products of a half; between them, if `more`, the reads of half rh at `from`, and with `la`, `lw` the loads of turn i into
+  // `into`.
+  const auto half = [&](const bf16x8 (&a)[MU], const bf16x8 (&w)[4], bool more, Place from, int rh, bf16x8 (&an)[MU], bf16x8 (&wn_)[4], bool la, bool lw,
+                        int i, Place into) {
+    const unsigned at_a = la ? bytes_at(i + NA) : 0, at_w = lw ? bytes_at(i + NW) : 0;
 #pragma unroll
     for (int u = 0; u < MU; ++u) {
       if (more) {
 #pragma unroll
-        for (int r = u * READS_EACH; r < (u + 1) * READS_EACH && r < READS; ++r) read(ri, rh, r, an, wn_);
+        for (int r = u * READS_EACH; r < (u + 1) * READS_EACH && r < READS; ++r) read(from, rh, r, an, wn_);
       }
 #pragma unroll
       for (int q = u * LOADS_EACH; q < (u + 1) * LOADS_EACH && q < LOADS; ++q) {
         if (A_FIRST ? q < S::A_PER : q >= S::W_PER) {
-          if (la) load_a(i + NA, A_FIRST ? q : q - S::W_PER, at_a);
+          if (la) load_a(into.a, A_FIRST ? q : q - S::W_PER, at_a);
         } else if (lw) {
-          load_w(i + NW, A_FIRST ? q - S::A_PER : q, at_w);
+          load_w(into.w, A_FIRST ? q - S::A_PER : q, at_w);
         }
       }
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[v], a[u], acc[u][v], 0, 0, 0);
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int v = u % 2 ? 3 - i4 : i4;
+        acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[v], a[u], acc[u][v], 0, 0, 0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -114,16 +125,16 @@ __device__ __forceinline__ void tile_loop(unsigned char* smem, AAt a_at, WAt w_a
   for (int e = -DEEP; e < 0; ++e) {                            // the turns before the first: stages 0 .. of both rings
     const auto fill_a = [&]() {
       if (e + NA >= 0 && e + NA < n_t) {
-        const int at = bytes_at(e + NA);
+        const unsigned at = bytes_at(e + NA);
 #pragma unroll
-        for (int x = 0; x < S::A_PER; ++x) load_a(e + NA, x, at);
+        for (int x = 0; x < S::A_PER; ++x) load_a((e + NA) * S::A_SLOT, x, at);
       }
     };
     if (A_FIRST) fill_a();
     if (e + NW >= 0 && e + NW < n_t) {
-      const int at = bytes_at(e + NW);
+      const unsigned at = bytes_at(e + NW);
 #pragma unroll
-      for (int x = 0; x < S::W_PER; ++x) load_w(e + NW, x, at);
+      for (int x = 0; x < S::W_PER; ++x) load_w((e + NW) * S::W_SLOT, x, at);
     }
     if (!A_FIRST) fill_a();
   }
@@ -131,25 +142,30 @@ __device__ __forceinline__ void tile_loop(unsigned char* smem, AAt a_at, WAt w_a
   if (n_t >= DEEP) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD + LOADS) : "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   meet();
+  Place here{0, 0};
 #pragma unroll
-  for (int r = 0; r < READS; ++r) read(0, 0, r, a0, w0);
+  for (int r = 0; r < READS; ++r) read(here, 0, r, a0, w0);
   reads_back();
   int i = 0;
   for (; i + DEEP < n_t; ++i) {
-    half(a0, w0, true, i, 1, a1, w1, false, false, i);
+    const Place next = behind_of(here);
+    half(a0, w0, true, here, 1, a1, w1, false, false, i, here);
     reads_back();
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");         // stage i + 1 is here
     meet();
-    half(a1, w1, true, i + 1, 0, a0, w0, true, true, i);
+    half(a1, w1, true, next, 0, a0, w0, true, true, i, here);
     reads_back();
+    here = next;
   }
   for (; i + 1 < n_t; ++i) {
-    half(a0, w0, true, i, 1, a1, w1, false, false, i);
+    const Place next = behind_of(here);
+    half(a0, w0, true, here, 1, a1, w1, false, false, i, here);
     reads_back();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     meet();
-    half(a1, w1, true, i + 1, 0, a0, w0, i + NA < n_t, i + NW < n_t, i);
+    half(a1, w1, true, next, 0, a0, w0, i + NA < n_t, i + NW < n_t, i, here);
     reads_back();
+    here = next;
   }
   const int behind = (t0 + n_t) * TILE_K - K;                  // > 0: what lies past the end of K (a multiple of 8) counts as 0
   const auto cut = [&](int h, bf16x8 (&a)[MU]) {
@@ -161,10 +177,10 @@ __device__ __forceinline__ void tile_loop(unsigned char* smem, AAt a_at, WAt w_a
     }
   };
   cut(0, a0);
-  half(a0, w0, true, n_t - 1, 1, a1, w1, false, false, i);
+  half(a0, w0, true, here, 1, a1, w1, false, false, i, here);
   reads_back();
   cut(1, a1);
-  half(a1, w1, false, 0, 0, a0, w0, false, false, i);
+  half(a1, w1, false, here, 0, a0, w0, false, false, i, here);
 }
 
 }  // namespace tl

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+from dataclasses import dataclass
 from typing import Optional, Tuple
 
 import torch
@@ -2009,13 +2010,120 @@ def wide_splits(M: int, N: int, K: int, units: int) -> int:
 
 
 def gemm_wide_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int) -> None:
-    """Partial sums out float32 [n_split, M, N] of the product of up to WIDE_ROWS rows, N and K multiples of 64."""
+    """Partial sums out float32 [n_split, M, N] of the product of up to WIDE_ROWS rows, N and K multiples of 64, in tiles of all of
+    the rows by 128 channels.  192 rows in 8 slices: 4,096 x 14,336 37 us, in 256 rows 40; 4,096 x 4,096 17."""
+    M, K = a.shape
+    N = w.shape[0]
+    if not (0 < M <= WIDE_ROWS and N % 64 == 0 and K % 64 == 0):
+        raise KernelError(f"gemm_wide: bad sizes M={M} N={N} K={K} (M at most {WIDE_ROWS}, N and K multiples of 64)")
+    gemm_tall_bf16(a, w, out, TallPlan(192 if M <= 192 else 256, 128, int(n_split)))
+
+
+@dataclass(frozen=True)
+class TallPlan:
+    """How `gemm_tall_bf16` is to do a product: tiles of `rows` x `channels`, K in `n_split` slices, tiles of other channels
+    beginning with other stages of K (`stagger`), and the tiles behind the first `whole` in `parts` each."""
+    rows: int
+    channels: int
+    n_split: int = 1
+    stagger: bool = False
+    whole: int = 0
+    parts: int = 0
+
+
+# microseconds that a stage of 64 k takes with every compute unit at work on tiles of so many rows and channels
+TALL_STAGE = {(256, 256): 1.45, (224, 256): 1.32, (192, 256): 1.15, (160, 256): 1.0, (256, 128): 0.93, (192, 128): 0.80, (128, 128): 0.68}
+TALL_ROUND, TALL_LAUNCH = 8.0, 4.0        # a round of workgroups besides its stages (first loads, results), and the launch
+TALL_SHARED = 4 << 20                     # bytes of A that an XCD's L2 holds: up to there tiles may go through K out of step
+
+
+@functools.lru_cache(maxsize=4096)
+def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False) -> Optional[TallPlan]:
+    """How the product of more than MID_ROWS rows, [M, K] by [N, K], goes in tiles of this package's own, or None where the BLAS
+    library's product is to be taken.  `kind`: "store" (float32), "add" (to float32) or "pair" (the activation of a paired
+    product, which the library's needs a kernel of its own for).  `sums`: partial sums over slices of K are welcome (the
+    next norm adds them).
+
+    The time of every way is reckoned from what was measured: rounds of workgroups over the compute units, each a few microseconds
+    and its stages of K (`TALL_STAGE`); what does not fill a last round goes in halves or quarters of tiles.  Reckoned and
+    measured, microseconds: 28,672 x 4,096 paired 2,048 rows 375 / 368 (halves), 3,000 561 / 552 (quarters), 600 148 / 139;
+    18,560 x 4,096 1,536 rows 189 / 191; 4,096 x 14,336 in slices 1,024 rows 101 / 101, 2,048 182 / 184.  The library's:
+    with the activation's kernel about 1.15 PFLOP/s, or 0.95 up to 640 rows, and no faster than 3.2 TB/s of weights (28,672 x
+    4,096 at 226 rows 73, here 67; 2,048 381; 3,000 579; 28,672 x 5,120 at 1,024 283, here 241, at 2,048 519 and 459); added
+    to the stream 3 us + 3.65 ns K + 1.5 PFLOP/s (4,096 x 14,336 at 512 rows 93, here 62 and 5 to 8 more in the norm; at
+    1,024 133, here 101 and 10; 4,096 x 4,096 at 2,048 65, here 62 and 12: the library's); more rows,
+    or stored, up to 1.43 PFLOP/s where both sizes are multiples of 256, less where rows are not, 0.9 where channels are not
+    (12,288 x 4,096 at 1,024 rows 82, here 89: the library's; at 6,000 584, here 476; 18,560 x 4,096 at 2,312 rows 386, here
+    305; 5,120 x 14,336 at 2,500 456, here 302)."""
+    if M <= MID_ROWS or K % 8 or N % (64 if kind == "pair" else 4) or max(M, N) >= 1 << 24 or K >= 1 << 22:
+        return None
+    stages = -(-K // 64)
+    best, plan = float("inf"), None
+
+    def fill(workgroups):                     # a stage's time in a round that leaves units idle: their power goes to the others
+        return 0.75 + 0.25 * max(0.0, 2.0 * workgroups / units - 1.0)
+
+    for (rows, channels), stage in TALL_STAGE.items():
+        mt, nt = -(-M // rows), -(-N // channels)
+        if mt == 1 and channels > 128:                               # more workgroups with 128 channels stream the weights faster:
+            continue                                                 # 28,672 x 4,096 paired at 150 rows 70 us in 160 x 256, 53 in 192 x 128
+        tiles = mt * nt
+        stagger = K % 64 == 0 and M * K * 2 <= TALL_SHARED
+        # K in slices, one round of workgroups
+        for S in range(2, min(units // tiles, stages // 4, 16) + 1) if sums and kind == "add" else ():
+            per = -(-stages // S)
+            if (S - 1) * per >= stages:
+                continue
+            size = 4.0 * M * N                                       # of a partial sum, in bytes; the norm reads all, and writes one
+            t = TALL_LAUNCH + 2.0 + per * stage * fill(tiles * S) + S * size / 8e6 + max(1.0, ((S + 1) * size - 30e6) / 5e6)
+            if t < best:
+                best, plan = t, TallPlan(rows, channels, S)
+        full, rest = divmod(tiles, units)
+        t = TALL_LAUNCH + full * (TALL_ROUND + stages * stage)
+        whole = parts = 0
+        if rest:
+            cut = [(stage * fill(rest), 0)]
+            if full and channels == 256 and units % 8 == 0:
+                if 2 * rest <= units:
+                    cut.append((TALL_STAGE[256, 128] * fill(2 * rest), 2))
+                if 4 * rest <= units:
+                    cut.append((TALL_STAGE[128, 128] * fill(4 * rest), 4))
+            last, parts = min(cut)
+            t += TALL_ROUND + stages * last
+            whole = full * units if parts else 0
+        if t < best:
+            best, plan = t, TallPlan(rows, channels, 1, stagger and not parts, whole, parts)
+    flops, weights = 2.0 * M * N * K, 2.0 * N * K
+    if kind == "pair":
+        library = max(weights / 3.2e6, flops / (0.95e9 if M <= 640 else 1.15e9))
+    else:
+        library = flops / (1.0e9 if N % 256 else 1.2e9 if M % 256 else 1.5e9)
+        if kind == "add" and M <= 2048:
+            library = 0.9 * (3.0 + 3.65e-3 * K + flops / 1.5e9)      # (what both ways take besides is not in it)
+    return plan if best < library else None
+
+
+def gemm_tall_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, plan: TallPlan, accumulate: bool = False, silu_pair: bool = False,
+                   pair_act: str = "silu") -> None:
+    """The product in tiles as `plan` says (`tall_plan`); out as in `gemm_mid_bf16`.  `w` [N, K] may be columns of a wider matrix."""
     M, K = a.shape
     N = w.shape[0]
     _req(a, "gemm.a", torch.bfloat16)
-    _req(w, "gemm.w", torch.bfloat16, (N, K))
-    _req(out, "gemm.out", torch.float32, (n_split, M, N))
-    _check(lib().tl_gemm_wide_bf16(_p(a), _p(w), _p(out), M, N, K, int(n_split), _stream()))
+    if not w.is_cuda or w.dtype != torch.bfloat16 or tuple(w.shape) != (N, K) or w.stride(1) != 1:
+        raise KernelError(f"gemm_tall.w: {w.dtype} {tuple(w.shape)} with strides {w.stride()}, kernel needs bfloat16 rows of {K} on the GPU")
+    if plan.n_split > 1:
+        if accumulate or silu_pair:
+            raise KernelError("gemm_tall: partial sums cannot be accumulated or paired")
+        _req(out, "gemm.out", torch.float32, (plan.n_split, M, N))
+        epi = EPI_STORE
+    elif silu_pair:
+        _req(out, "gemm.out", torch.bfloat16, (M, N // 2))
+        epi = _pair_epilogue(pair_act)
+    else:
+        _req(out, "gemm.out", torch.float32, (M, N))
+        epi = EPI_ACCUMULATE if accumulate else EPI_STORE
+    _check(lib().tl_gemm_tall(_p(a), K, _p(w), w.stride(0), _p(out), M, N, K, plan.rows, plan.channels, plan.n_split,
+                              int(M <= plan.rows and not plan.parts), int(plan.stagger), plan.whole, plan.parts, epi, _stream()))
 
 
 def gemm_ring_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int = 1, accumulate: bool = False,
@@ -2098,7 +2206,11 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     with float32 in it to the plain FMA kernel.  `tiles`: see `gemm_bf16`."""
     if bf16_gemm_ok(a, w):
         if a.shape[0] > own_rows(a.shape[1]):
-            gemm_library(a, w, out, accumulate)
+            plan = tall_plan(a.shape[0], w.shape[0], a.shape[1], compute_units(a.device), "add" if accumulate else "store")
+            if plan is not None and out.data_ptr() % 16 == 0:
+                gemm_tall_bf16(a, w, out, plan, accumulate)
+            else:
+                gemm_library(a, w, out, accumulate)
         elif a.shape[0] > LIBRARY_ROWS:
             gemm_mid_bf16(a, w, out, 1, accumulate)
         else:

@@ -91,7 +91,10 @@ class SwiGLU(FeedForward):
         elif self.paired and self.gate_up.mid(y):
             ops.gemm_mid_bf16(y, self.gate_up.weight, h, 1, silu_pair=True, pair_act=self.pair)
         elif self.paired and ops.bf16_gemm_ok(y, self.gate_up.weight):
-            if n > ops.LIBRARY_ROWS:
+            plan = ops.tall_plan(n, 2 * self.I, self.H, ops.compute_units(y.device), "pair")
+            if plan is not None and h.data_ptr() % 16 == 0:
+                ops.gemm_tall_bf16(y, self.gate_up.weight, h, plan, silu_pair=True, pair_act=self.pair)
+            elif n > ops.LIBRARY_ROWS:
                 gu = ctx.workspace.get("ffn_gu16", (n, 2 * self.I), torch.bfloat16)
                 ops.gemm_library(y, self.gate_up.weight, gu)
                 ops.silu_mul_pairs(gu, h, self.activation, self.constants)

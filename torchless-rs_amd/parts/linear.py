@@ -92,6 +92,19 @@ class Linear:
         ops.gemm_wide_bf16(a, self.weight, parts, S)
         return parts
 
+    def tall_partial(self, a: torch.Tensor, ctx, name: str):
+        """The same for more rows than that, or fewer slices, where a norm that adds such sums is announced as the stream's next
+        reader (without one they would take a pass of their own)."""
+        norm = ctx.norm_ahead
+        if a.shape[0] <= ops.MID_ROWS or norm is None or not getattr(norm, "takes_pending", False) or not ops.bf16_gemm_ok(a, self.weight):
+            return None
+        plan = ops.tall_plan(a.shape[0], self.out_features, self.in_features, ops.compute_units(a.device), "add", True)
+        if plan is None or plan.n_split == 1:
+            return None
+        parts = ctx.workspace.get(name, (plan.n_split, a.shape[0], self.out_features), torch.float32)
+        ops.gemm_tall_bf16(a, self.weight, parts, plan)
+        return parts
+
     def add_into(self, a: torch.Tensor, x: torch.Tensor, ctx, name: str) -> None:
         """x += a @ W^T, now or as partial sums left in `ctx.pending`."""
         from .base import flush_pending
@@ -110,6 +123,8 @@ class Linear:
         parts = self.partial(a, ctx, name)
         if parts is None:
             parts = self.wide_partial(a, ctx, name)
+        if parts is None:
+            parts = self.tall_partial(a, ctx, name)
         if parts is None:
             self(a, x, accumulate=True)
         else:
