@@ -2051,10 +2051,10 @@ def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False)
     with the activation's kernel about 1.15 PFLOP/s, or 0.95 up to 640 rows, and no faster than 3.2 TB/s of weights (28,672 x
     4,096 at 226 rows 73, here 67; 2,048 381; 3,000 579; 28,672 x 5,120 at 1,024 283, here 241, at 2,048 519 and 459); added
     to the stream 3 us + 3.65 ns K + 1.5 PFLOP/s (4,096 x 14,336 at 512 rows 93, here 62 and 5 to 8 more in the norm; at
-    1,024 133, here 101 and 10; 4,096 x 4,096 at 2,048 65, here 62 and 12: the library's); more rows,
-    or stored, up to 1.43 PFLOP/s where both sizes are multiples of 256, less where rows are not, 0.9 where channels are not
-    (12,288 x 4,096 at 1,024 rows 82, here 89: the library's; at 6,000 584, here 476; 18,560 x 4,096 at 2,312 rows 386, here
-    305; 5,120 x 14,336 at 2,500 456, here 302)."""
+    1,024 133, here 101 and 10; 4,096 x 4,096 at 2,048 65, here 62 and 12: the library's); more rows, or stored, up to 1.43 PFLOP/s
+    where both sizes are multiples of 256, less where rows are not, the least where channels are not (12,288 x 4,096 at 1,024
+    rows 82, here 89: the library's; 6,144 x 4,096 at 2,034 85, here 97: the library's; 14,336 x 4,096 at 3,220 432, here
+    314; 18,560 x 4,096 at 2,312 386, here 305; 5,120 x 14,336 at 2,500 456, here 302)."""
     if M <= MID_ROWS or K % 8 or N % (64 if kind == "pair" else 4) or max(M, N) >= 1 << 24 or K >= 1 << 22:
         return None
     stages = -(-K // 64)
@@ -2097,7 +2097,8 @@ def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False)
     if kind == "pair":
         library = max(weights / 3.2e6, flops / (0.95e9 if M <= 640 else 1.15e9))
     else:
-        library = flops / (1.0e9 if N % 256 else 1.2e9 if M % 256 else 1.5e9)
+        one_round = -(-M // plan.rows) * -(-N // plan.channels) <= units
+        library = flops / (1.0e9 if N % 256 else 1.5e9 if M % 256 == 0 else 1.2e9 if M <= 1536 or one_round else 1.08e9)
         if kind == "add" and M <= 2048:
             library = 0.9 * (3.0 + 3.65e-3 * K + flops / 1.5e9)      # (what both ways take besides is not in it)
     return plan if best < library else None
