@@ -678,13 +678,27 @@ __global__ void cast_rows_kernel(const float* __restrict__ x, size_t total, bf16
   if (i < total) out[i] = (bf16)x[i];
 }
 
-// h = act(gate) * up from gu[n, 2I] = [gate | up]
+// h = act(gate) * up from gu[n, 2I] = [gate | up].  A row is shared by as many workgroups as it has runs of 1,024 channels (up to
+// the grid's limit, then round again), four channels a thread: with one workgroup a row a step of two rows of 8,192 took 10.1 us,
+// 32 loads a thread one after the other, and takes 2.2 so; 2,048 rows 32.5 and 30.4.  `vec`: rows and buffers are aligned for
+// loads of four.
 template <typename TO>
-__global__ void act_mul_kernel(const float* __restrict__ gu, int I, int act, ActConstants k, TO* __restrict__ out) {
+__global__ void __launch_bounds__(256)
+act_mul_kernel(const float* __restrict__ gu, int I, int act, ActConstants k, bool vec, TO* __restrict__ out) {
   const int n = blockIdx.x;
   const float* row = gu + (size_t)n * 2 * I;
-  for (int i = threadIdx.x; i < I; i += blockDim.x)
-    out[(size_t)n * I + i] = from_f32<TO>(gate_times_up(row[i], row[I + i], act, k));
+  TO* o = out + (size_t)n * I;
+  for (long i = (blockIdx.y * 256 + threadIdx.x) * 4; i < I; i += gridDim.y * 1024) {
+    if (vec) {
+      const f32x4 g = *reinterpret_cast<const f32x4*>(row + i), u = *reinterpret_cast<const f32x4*>(row + I + i);
+      __attribute__((ext_vector_type(4))) TO h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = from_f32<TO>(gate_times_up(g[e], u[e], act, k));
+      *reinterpret_cast<decltype(h)*>(o + i) = h;
+    } else {
+      for (int e = 0; e < 4 && i + e < I; ++e) o[i + e] = from_f32<TO>(gate_times_up(row[i + e], row[I + i + e], act, k));
+    }
+  }
 }
 
 // ---- an RMS norm of a sublayer's OUTPUT, added to the stream ---------------------------------
@@ -1163,10 +1177,12 @@ int tl_act_mul(const float* gu, int n, int I, int act, float alpha, float limit,
   TL_REQUIRE(act != ACT_SWISH_CLAMPED || limit > 0.f, "act_mul: the clamp needs a positive limit");
   if (n == 0) return 0;
   const ActConstants k{alpha, limit, shift};
+  const bool vec = I % 4 == 0 && (uintptr_t)gu % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const dim3 grid(n, (unsigned)min(((long)I + 1023) / 1024, 1024l));
   if (out_dt == DT_F32)
-    act_mul_kernel<float><<<n, 256, 0, st>>>(gu, I, act, k, (float*)out);
+    act_mul_kernel<float><<<grid, 256, 0, st>>>(gu, I, act, k, vec, (float*)out);
   else if (out_dt == DT_BF16)
-    act_mul_kernel<bf16><<<n, 256, 0, st>>>(gu, I, act, k, (bf16*)out);
+    act_mul_kernel<bf16><<<grid, 256, 0, st>>>(gu, I, act, k, vec, (bf16*)out);
   else
     TL_REQUIRE(false, "act_mul: unknown dtype code %d", out_dt);
   TL_LAUNCH_CHECK("act_mul");
