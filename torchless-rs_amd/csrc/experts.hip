@@ -140,6 +140,116 @@ route_kernel(const T* __restrict__ h, int W, const float* __restrict__ wr, int E
   }
 }
 
+// The same bits for steps of many rows and 16 to 64 experts.  What bounds `route_kernel` there is the router's matrix, which every
+// row's workgroup reads whole from L2 (2,348 rows x 16 experts x 4,096 channels: 600 MB).  Here a workgroup has four rows: a wave
+// takes four experts at a time for all of them, so that a load of the matrix serves four rows and one of a row four experts, the
+// sums of a dot in the same order.  Then every wave chooses for one row, an expert a lane, with no barrier.
+// 16 experts, before and now: 1,024 rows 20.8 / 16.4 us, 2,348 42.0 / 21.6, 8,192 121 / 67; 64 experts 68 / 54, 153 / 69, 469 / 230.
+// A workgroup's chain of loads takes 14 us, so that the line lies where the other kernel does (512 rows 13.2 and 15.8).  With 5
+// experts, where most of the waves have none, it is the slower (8,192 rows 27.5 and 34).  Two experts a wave and eight waves a
+// workgroup: 13.9 us at 1,024 rows, but 26 at 2,348.
+constexpr int RR_FROM = 768, RR_MIN_E = 16, RR_MAX_E = WAVE;
+constexpr int RR_ROWS = 4, RR_EXPERTS = 4;
+
+// lane o's value, o the same in all lanes
+__device__ __forceinline__ float lane_value(float v, int o) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), o)); }
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+route_rows_kernel(const T* __restrict__ h, int n_rows, int W, const float* __restrict__ wr, int E, int groups, int keep, int top,
+                  int logistic, RouteTerms k, float* __restrict__ weights, int* __restrict__ chosen) {
+  __shared__ float s_s[RR_ROWS][RR_MAX_E + 1];
+  const int n0 = blockIdx.x * RR_ROWS;
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int rows = E + (k.shared_weight ? 1 : 0);
+  const T* row[RR_ROWS];
+#pragma unroll
+  for (int r = 0; r < RR_ROWS; ++r) row[r] = h + (size_t)min(n0 + r, n_rows - 1) * W;
+  for (int e0 = wave * RR_EXPERTS; e0 < rows; e0 += 4 * RR_EXPERTS) {
+    const float* w[RR_EXPERTS];
+#pragma unroll
+    for (int e = 0; e < RR_EXPERTS; ++e) w[e] = wr + (size_t)min(e0 + e, rows - 1) * W;
+    f32x4 d[RR_ROWS][RR_EXPERTS];
+#pragma unroll
+    for (int r = 0; r < RR_ROWS; ++r)
+#pragma unroll
+      for (int e = 0; e < RR_EXPERTS; ++e) d[r][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int c = lane * 4; c + 3 < W; c += WAVE * 4) {
+      f32x4 wv[RR_EXPERTS], rv[RR_ROWS];
+#pragma unroll
+      for (int e = 0; e < RR_EXPERTS; ++e) wv[e] = *reinterpret_cast<const f32x4*>(w[e] + c);
+#pragma unroll
+      for (int r = 0; r < RR_ROWS; ++r) {
+        if constexpr (sizeof(T) == 2) {
+          const bf16x4 b = *reinterpret_cast<const bf16x4*>(row[r] + c);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rv[r][i] = (float)b[i];
+        } else {
+          rv[r] = *reinterpret_cast<const f32x4*>(row[r] + c);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RR_ROWS; ++r)
+#pragma unroll
+        for (int e = 0; e < RR_EXPERTS; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) d[r][e][i] = fmaf(wv[e][i], rv[r][i], d[r][e][i]);
+    }
+#pragma unroll
+    for (int r = 0; r < RR_ROWS; ++r)
+#pragma unroll
+      for (int e = 0; e < RR_EXPERTS; ++e) {
+        const float dot = wave_sum((d[r][e][0] + d[r][e][1]) + (d[r][e][2] + d[r][e][3]));
+        if (lane == 0 && e0 + e < rows) s_s[r][e0 + e] = dot + (k.bias && e0 + e < E ? k.bias[e0 + e] : 0.f);
+      }
+  }
+  __syncthreads();
+  const int n = n0 + wave;
+  if (n >= n_rows) return;
+  if (k.shared_weight && lane == 0) k.shared_weight[n] = 1.0f / (1.0f + expf(-s_s[wave][E]));
+  const bool mine_ok = lane < E;
+  float s = mine_ok ? s_s[wave][lane] : -INFINITY;
+  if (logistic) {
+    s = 1.0f / (1.0f + expf(-s));
+  } else {
+    const float m = wave_max(s);
+    const float x = mine_ok ? expf(s - m) : 0.f;
+    s = x / wave_sum(x);
+  }
+  const float c = mine_ok ? ranked(s + (k.correction ? k.correction[lane] : 0.f)) : -INFINITY;
+  bool ok = mine_ok;
+  if (groups > 0) {
+    const int per = E / groups, g0 = mine_ok ? lane / per * per : 0;
+    float best = __shfl(c, g0), second = -INFINITY;
+    for (int i = 1; i < per; ++i) {
+      const float o = __shfl(c, g0 + i);
+      second = fmaxf(second, fminf(best, o));
+      best = fmaxf(best, o);
+    }
+    const float score = ranked(k.two_largest && per > 1 ? best + second : best);
+    int ahead = 0;
+    for (int o = 0; o < E; o += per) {
+      const float other = lane_value(score, o);
+      ahead += (other > score || (other == score && o < g0)) ? 1 : 0;
+    }
+    ok = mine_ok && ahead < keep;
+  }
+  int ahead = 0;
+  const unsigned long long oks = __ballot(ok);
+  for (int o = 0; o < E; ++o) {
+    const float other = lane_value(c, o);
+    ahead += ((oks >> o & 1) && (other > c || (other == c && o < lane))) ? 1 : 0;
+  }
+  float wgt = 0.f;
+  if (ok && ahead < top) {
+    wgt = s;
+    if (chosen) chosen[(size_t)n * top + ahead] = lane;
+  }
+  if (k.normalise) wgt /= wave_sum(wgt) + k.normalise_eps;
+  if (mine_ok) weights[(size_t)n * E + lane] = wgt;
+}
+
 // out[n, j] = act(u[n, j]) * (j < E * ff ? weights[n, j / ff] : shared_w ? shared_w[n] : 1)
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -356,6 +466,15 @@ int tl_route(const void* h, int dt, int n, int W, const float* wr, int E, int gr
   TL_REQUIRE(dt == DT_F32 || dt == DT_BF16, "route: unknown dtype code %d", dt);
   const RouteTerms k{correction, two_largest, normalise, normalise_eps, shared_weight, bias};
   const bool few = n <= 64 && E > 4;             // fewer rows than compute units: more waves a row
+  if (n >= RR_FROM && E >= RR_MIN_E && E <= RR_MAX_E && vec) {
+    const unsigned grid = ((unsigned)n + RR_ROWS - 1) / RR_ROWS;
+    if (dt == DT_F32)
+      route_rows_kernel<float><<<grid, 256, 0, st>>>((const float*)h, n, W, wr, E, groups, keep, top, logistic, k, weights, chosen);
+    else
+      route_rows_kernel<bf16><<<grid, 256, 0, st>>>((const bf16*)h, n, W, wr, E, groups, keep, top, logistic, k, weights, chosen);
+    TL_LAUNCH_CHECK("route");
+    return 0;
+  }
   if (dt == DT_F32 && few)
     route_kernel<float, 1024><<<n, 1024, 0, st>>>((const float*)h, W, wr, E, groups, keep, top, logistic, k, weights, chosen, vec);
   else if (dt == DT_F32)
