@@ -43,6 +43,46 @@ def test_a_step_of_many_rows_routes_as_its_rows_do_in_small_steps(ops, dtype, E,
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk,dv,rotary", [(64, 64, 64), (65, 40, 24), (128, 128, 64), (128, 96, 128), (200, 64, 130), (256, 256, 256), (96, 32, 0)])
+def test_heads_of_many_rows_are_those_of_few(ops, dtype, dk, dv, rotary):
+    """A wave that goes from head to head leaves what a wave a head leaves, against 64 bits and bit by bit."""
+    nq, nkv, ng, n = 3, 2, 300, 2100
+    g = torch.Generator(device=DEV).manual_seed(dk + rotary)
+    width = nq * dk + nkv * (dk + dv) + ng
+    proj = torch.randn(n, width, generator=g, device=DEV)
+    pos = torch.randint(0, 5000, (n,), generator=g, device=DEV, dtype=torch.int32)
+    inv = 10000.0 ** (-2.0 * torch.arange(rotary // 2, device=DEV) / max(rotary, 1)) if rotary else None
+    qn, kn = (1.0 + 0.1 * torch.randn(dk, generator=g, device=DEV) for _ in range(2))
+    bias = torch.randn(width, generator=g, device=DEV)
+    for kw in ({}, {"q_norm": qn, "k_norm": kn, "bias": bias}, {"unit_norm": True, "v_factor": 0.5}):
+        def run(rows, at):
+            m = rows.shape[0]
+            q, k, v = (torch.empty(m, h, d, dtype=dtype, device=DEV) for h, d in ((nq, dk), (nkv, dk), (nkv, dv)))
+            gate = torch.empty(m, ng, device=DEV)
+            ops.head_prepare(rows, at, ops.Rotation(inv, rotary), ops.HeadTerms(eps=1e-5, **kw), nq, nkv, dk, dv, ng, q, k, v, gate)
+            return q, k, v, gate
+        many = run(proj, pos)
+        few = [torch.cat(t) for t in zip(*(run(proj[i:i + 30], pos[i:i + 30]) for i in range(0, 90, 30)))]
+        for a, b in zip(many, few):
+            assert torch.equal(a[:90], b)
+        t = proj.double() + (kw["bias"].double() if "bias" in kw else 0.0)
+        x = t[:, :(nq + nkv) * dk].view(n, nq + nkv, dk)
+        if "q_norm" in kw:
+            x = x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+            x = torch.cat([x[:, :nq] * qn.double(), x[:, nq:] * kn.double()], 1)
+        half = rotary // 2
+        if half:
+            angle = (pos.float()[:, None] * inv).double()[:, None]
+            u, w = x[..., :half], x[..., half:rotary]
+            x = torch.cat([u * angle.cos() - w * angle.sin(), u * angle.sin() + w * angle.cos(), x[..., rotary:]], -1)
+        if kw.get("unit_norm"):
+            x = x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+        # float32: a few roundings of 2^-24 of the two products of a rotated channel; bfloat16: one of 2^-9 of the result
+        tol = 4e-6 * (1.0 + x.abs().amax(-1, keepdim=True)) + (2.0 ** -8 * x.abs() if dtype == torch.bfloat16 else 0.0)
+        assert bool(((torch.cat(many[:2], 1).double() - x).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,I", [(1, 1), (2, 1023), (2, 1024), (3, 1028), (2, 8192), (1, 1048580), (129, 2050)])
 def test_the_activation_of_a_stored_product(ops, dtype, n, I):
     gu = torch.randn(n, 2 * I, generator=torch.Generator(device=DEV).manual_seed(I), device=DEV)
