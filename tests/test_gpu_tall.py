@@ -114,3 +114,35 @@ def test_what_the_tiles_do_not_take_is_refused(ops):
         ops.gemm_tall_bf16(a, w, out, ops.TallPlan(256, 256, whole=1, parts=2))
     with pytest.raises(ops.KernelError, match="bfloat16 rows"):
         ops.gemm_tall_bf16(a, torch.zeros(128, 256, dtype=torch.bfloat16, device=DEV).t(), out, ops.TallPlan(256, 256))
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("act", ["relu2", "relu", "xielu", "gated", "plain_gated"])
+@pytest.mark.parametrize("M,I,K,plan", [(129, 32, 64, (192, 128)), (300, 160, 264, (160, 256)), (520, 672, 128, (256, 256, 1, False, 8, 2)),
+                                        (520, 672, 128, (192, 256, 1, False, 8, 4)), (257, 96, 128, (256, 128, 1, True))])
+def test_an_experts_activation(ops, act, M, I, K, plan, weighted):
+    """The activation on the sums, rounded to bfloat16 once, as in `test_paired`; gate and up rows lie apart.  The square's slope is twice
+    its root: 1e-5 of the sums' sizes times the largest of them covers it."""
+    gated = "gated" in act
+    a, w, p, size = operands(M, 2 * I if gated else I, K)
+    a = a * K ** -0.5
+    p = a.double() @ w.double().t()
+    top = float(p.abs().max())
+    factor = torch.rand(M, device=DEV) if weighted else None
+    kw = {}
+    if gated:
+        limit, alpha, shift = (0.75, 1.702, 1.0) if act == "gated" else (float("inf"), 1.0, 0.0)
+        kw["terms"] = ops.GateTerms(3.0, alpha, shift, limit, True)
+        g, u = p[:, :I].clamp(max=limit), p[:, I:].clamp(-limit, limit)
+        want = g * torch.sigmoid(alpha * g) * (u + shift)
+    else:
+        kw["activation"] = act
+        want = torch.relu(p) ** 2 if act == "relu2" else torch.relu(p)
+        if act == "xielu":
+            kw["constants"] = {"a": 0.8, "b": 0.9}
+            want = torch.where(p > 0, 0.8 * p * p + 0.5 * p, 0.9 * (torch.expm1(p) - p) + 0.5 * p)
+    if weighted:
+        want = want * factor.double()[:, None]
+    out = torch.full((M, I), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.gemm_tall_act(a, w, out, ops.TallPlan(*plan), row_weight=factor, **kw)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + top) * (1.0 + top)).all())

@@ -2,6 +2,7 @@
 // library's (ops.tall_plan): tiles of 128 to 256 rows by 128 or 256 channels (tile_loop.hpp), K cut over workgroups into
 // partial sums where the tiles are too few for the chip, the activation of a paired product in the epilogue.
 #include "epilogues.hpp"
+#include "experts.hpp"
 #include "tile_loop.hpp"
 
 namespace tl {
@@ -17,7 +18,13 @@ struct Tall {
   int stagger;                 // tiles of other channels begin with other stages
   int whole, parts;            // the tiles behind the first `whole` ones are cut in `parts` (2 or 4); 0: none is
   Epi epi;
+  // TALL_UNARY, TALL_GATED: the activation of an expert on the sums, times a factor of the row (null: 1); C is bfloat16
+  UnaryAct unary;              // [M, N]
+  GateTerms gate;              // [M, N / 2]; W is [gate | up] by rows, paired as the tile is loaded: channels in groups of 64,
+                               // 32 of gate and the 32 rows N / 2 further
+  const float* row_weight;
 };
+constexpr int TALL_UNARY = 6, TALL_GATED = 7;   // epilogues beside those of `Epi`
 
 constexpr int TALL_GROUP = 8;  // tiles of rows that go side by side through the channels
 
@@ -30,12 +37,16 @@ __device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int
   const int t0 = blockIdx.y * g.stages, n_t = min((g.K + TILE_K - 1) / TILE_K - t0, g.stages);
   // a lane's rows as distances from the tile's first: at most 256 rows of K
   const char* A0 = reinterpret_cast<const char*>(g.A + (size_t)m0 * g.lda);
-  const char* W0 = reinterpret_cast<const char*>(g.W + (size_t)n0 * g.ldw);
+  const bool apart = g.epi == TALL_GATED;
+  const char* W0 = reinterpret_cast<const char*>(g.W + (size_t)(apart ? n0 / 2 : n0) * g.ldw);
   unsigned aoff[S::A_PER], woff[S::W_PER];
 #pragma unroll
   for (int x = 0; x < S::A_PER; ++x) aoff[x] = (unsigned)min(tile_load<S::A_LOADS>(wave, x) * 8 + sub, m_rows - 1) * (unsigned)g.lda * 2u;
 #pragma unroll
-  for (int x = 0; x < S::W_PER; ++x) woff[x] = (unsigned)min((wave + TILE_WAVES * x) * 8 + sub, g.N - 1 - n0) * (unsigned)g.ldw * 2u;
+  for (int x = 0; x < S::W_PER; ++x) {
+    const int c = min((wave + TILE_WAVES * x) * 8 + sub, g.N - 1 - n0);
+    woff[x] = (unsigned)(apart ? c / 64 * 32 + c % 32 + (c & 32 ? g.N / 2 : 0) : c) * (unsigned)g.ldw * 2u;
+  }
 
   f32x4 acc[MU][4];
 #pragma unroll
@@ -47,20 +58,41 @@ __device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int
 
   // acc[u][v][r]: row 16 (wm MU + u) + li of the tile, channel 64 wn + 16 v + 4 kg + r
   const int c0 = n0 + wn * 64 + kg * 4;
-  if (is_pair(g.epi)) {                        // a wave's 64 channels are 32 gate rows and their 32 up rows
+  if (apart || is_pair(g.epi)) {               // a wave's 64 channels are 32 gate rows and their 32 up rows
 #pragma unroll
     for (int u = 0; u < MU; ++u) {
       const int m = (wm * MU + u) * 16 + li;
       if (m >= m_rows) continue;
       bf16* out = reinterpret_cast<bf16*>(g.C) + (size_t)(m0 + m) * (g.N / 2);
+      const float after = g.row_weight ? g.row_weight[m0 + m] : 1.f;
 #pragma unroll
       for (int v = 0; v < 2; ++v) {
         const int n = (n0 + wn * 64) / 2 + v * 16 + kg * 4;
         if (n >= g.N / 2) continue;
         bf16x4 h;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) h[r] = (bf16)pair_value_near(acc[u][v][r], acc[u][v + 2][r], g.epi);
+        for (int r = 0; r < 4; ++r)
+          h[r] = (bf16)(apart ? gated_value_near(acc[u][v][r], acc[u][v + 2][r], 1.f, g.gate.limit_shared, g.gate) * after
+                              : pair_value_near(acc[u][v][r], acc[u][v + 2][r], g.epi));
         *reinterpret_cast<bf16x4*>(out + n) = h;
+      }
+    }
+    return;
+  }
+  if (g.epi == TALL_UNARY) {
+#pragma unroll
+    for (int u = 0; u < MU; ++u) {
+      const int m = (wm * MU + u) * 16 + li;
+      if (m >= m_rows) continue;
+      bf16* out = reinterpret_cast<bf16*>(g.C) + (size_t)(m0 + m) * g.N;
+      const float after = g.row_weight ? g.row_weight[m0 + m] : 1.f;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (c0 + v * 16 >= g.N) continue;
+        bf16x4 h;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[r] = (bf16)(unary_act(acc[u][v][r], g.unary) * after);
+        *reinterpret_cast<bf16x4*>(out + c0 + v * 16) = h;
       }
     }
     return;
@@ -156,20 +188,22 @@ using namespace tl;
 // one tile of rows only (its loads are marked non-temporal); stagger: tiles of other channels begin with other stages of K
 // (K a multiple of 64, not cut).  parts: 0, or 2 or 4 (tiles of 256 channels, K not cut): the tiles behind the first `whole`, a
 // multiple of 8, are cut into so many.
-extern "C" int tl_gemm_tall(const void* A, int lda, const void* W, int ldw, void* C, int M, int N, int K, int rows, int channels, int n_split,
-                            int once, int stagger, int whole, int parts, int epilogue, hipStream_t st) {
+static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipStream_t st) {
+  const int M = g.M, N = g.N, K = g.K, lda = g.lda, ldw = g.ldw, stagger = g.stagger, whole = g.whole, parts = g.parts, epilogue = g.epi;
+  const void *A = g.A, *W = g.W, *C = g.C;
   TL_REQUIRE(M > 0 && N > 0 && K > 0 && K % 8 == 0 && N % 4 == 0, "gemm_tall: bad sizes M=%d N=%d K=%d (K a multiple of 8, N of 4)", M, N, K);
   TL_REQUIRE(lda >= K && ldw >= K && lda % 8 == 0 && ldw % 8 == 0 && lda < (1 << 22) && ldw < (1 << 22),
              "gemm_tall: rows %d and %d apart for K=%d (multiples of 8 below 2^22)", lda, ldw, K);
   TL_REQUIRE(A && W && C && ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 == 0, "gemm_tall: operands must be 16-byte aligned");
-  TL_REQUIRE(epilogue >= 0 && epilogue <= 5 && (n_split == 1 || epilogue == EPI_STORE), "gemm_tall: epilogue %d cannot go with %d splits", epilogue, n_split);
-  TL_REQUIRE(!is_pair(epilogue) || N % 64 == 0, "gemm_tall: the paired epilogue needs N=%d to be a multiple of 64", N);
+  TL_REQUIRE(epilogue >= 0 && epilogue <= TALL_GATED && (n_split == 1 || epilogue == EPI_STORE), "gemm_tall: epilogue %d cannot go with %d splits", epilogue, n_split);
+  TL_REQUIRE(!(is_pair(epilogue) || epilogue == TALL_GATED) || N % 64 == 0, "gemm_tall: the paired epilogue needs N=%d to be a multiple of 64", N);
   const int stages = (K + TILE_K - 1) / TILE_K, per = (stages + n_split - 1) / (n_split > 0 ? n_split : 1);
   TL_REQUIRE(n_split >= 1 && n_split <= 65535 && (long)(n_split - 1) * per < stages, "gemm_tall: %d splits of K=%d would leave one without a stage", n_split, K);
   TL_REQUIRE(!stagger || (n_split == 1 && K % TILE_K == 0), "gemm_tall: stages in turn need K=%d uncut and a multiple of %d", K, TILE_K);
   TL_REQUIRE(parts == 0 || ((parts == 2 || parts == 4) && n_split == 1 && channels == 256 && !once && !stagger && whole >= 0),
              "gemm_tall: tiles in %d parts (2 or 4, of 256 channels, K not cut)", parts);
-  Tall g{(const bf16*)A, (const bf16*)W, (float*)C, M, N, K, lda, ldw, 0, 0, 0, per, stagger, whole, parts, epi_of(epilogue)};
+  TL_REQUIRE(epilogue != TALL_GATED || (long)N * ldw < (1l << 30), "gemm_tall: gate and up rows of %d x %d lie too far apart", N, ldw);
+  g.stages = per;
 #define TL_TALL(R, CH, WN, MU, NA, NW)                                                         \
   if (rows == R && channels == CH) {                                                           \
     if (parts) return launch_tall<4, MU, 2, 3, 0, true>(g, n_split, st);                       \
@@ -188,4 +222,32 @@ extern "C" int tl_gemm_tall(const void* A, int lda, const void* W, int ldw, void
   TL_TALL(128, 2, 5, 5)
 #undef TL_TALL
   TL_REQUIRE(false, "gemm_tall: no tiles of %d x %d", rows, channels);
+}
+
+extern "C" int tl_gemm_tall(const void* A, int lda, const void* W, int ldw, void* C, int M, int N, int K, int rows, int channels, int n_split,
+                            int once, int stagger, int whole, int parts, int epilogue, hipStream_t st) {
+  TL_REQUIRE(epilogue >= 0 && epilogue <= 5, "gemm_tall: unknown epilogue %d", epilogue);
+  Tall g{};
+  g.A = (const bf16*)A; g.W = (const bf16*)W; g.C = (float*)C;
+  g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldw = ldw;
+  g.stagger = stagger; g.whole = whole; g.parts = parts;
+  g.epi = epi_of(epilogue);
+  return run_tall(g, rows, channels, n_split, once, st);
+}
+
+// The same with an expert's activation on the sums, times row_weight[m] (or null): gated == 0: C bfloat16 [M, N] = act(product) (codes
+// of `UnaryAct`); gated == 1: W [gate | up], N / 2 rows each, C bfloat16 [M, N / 2] = act(gate, up) (`gated_value`; N a multiple of 64).
+extern "C" int tl_gemm_tall_act(const void* A, int lda, const void* W, int ldw, void* C, int M, int N, int K, int rows, int channels, int once,
+                                int stagger, int whole, int parts, int gated, int act_code, float act_a, float act_b, float limit, float alpha,
+                                float shift, const float* row_weight, hipStream_t st) {
+  TL_REQUIRE(act_code >= 0 && act_code <= 2, "gemm_tall_act: unknown activation %d", act_code);
+  Tall g{};
+  g.A = (const bf16*)A; g.W = (const bf16*)W; g.C = (float*)C;
+  g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldw = ldw;
+  g.stagger = stagger; g.whole = whole; g.parts = parts;
+  g.epi = Epi(gated ? TALL_GATED : TALL_UNARY);
+  g.unary = UnaryAct{act_code, act_a, act_b};
+  g.gate = GateTerms{limit, limit, alpha, shift, 0};
+  g.row_weight = row_weight;
+  return run_tall(g, rows, channels, 1, once, st);
 }

@@ -2041,7 +2041,9 @@ TALL_SHARED = 4 << 20                     # bytes of A that an XCD's L2 holds: u
 def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False) -> Optional[TallPlan]:
     """How the product of more than MID_ROWS rows, [M, K] by [N, K], goes in tiles of this package's own, or None where the BLAS
     library's product is to be taken.  `kind`: "store" (float32), "add" (to float32) or "pair" (the activation of a paired
-    product, which the library's needs a kernel of its own for).  `sums`: partial sums over slices of K are welcome (the
+    product, which the library's needs a kernel of its own for), "act" (the activation of an expert, for which a stored product's
+    float sums are written and read once more: 14,336 x 4,096 gated at 2,348 rows 302, here 238; at 1,024
+    115 and 98; 7,168 x 4,096 of one argument at 2,348 161 and 134, at 512 45, here 81: the library's).  `sums`: partial sums over slices of K are welcome (the
     next norm adds them).
 
     The time of every way is reckoned from what was measured: rounds of workgroups over the compute units, each a few microseconds
@@ -2099,6 +2101,8 @@ def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False)
     else:
         one_round = -(-M // plan.rows) * -(-N // plan.channels) <= units
         library = flops / (1.0e9 if N % 256 else 1.5e9 if M % 256 == 0 else 1.2e9 if M <= 1536 or one_round else 1.08e9)
+        if kind == "act":
+            library += 3.0 + 5.0 * M * N / 4.5e6
         if kind == "add" and M <= 2048:
             library = 0.9 * (3.0 + 3.65e-3 * K + flops / 1.5e9)      # (what both ways take besides is not in it)
     return plan if best < library else None
@@ -2125,6 +2129,24 @@ def gemm_tall_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, plan: Ta
         epi = EPI_ACCUMULATE if accumulate else EPI_STORE
     _check(lib().tl_gemm_tall(_p(a), K, _p(w), w.stride(0), _p(out), M, N, K, plan.rows, plan.channels, plan.n_split,
                               int(M <= plan.rows and not plan.parts), int(plan.stagger), plan.whole, plan.parts, epi, _stream()))
+
+
+def gemm_tall_act(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, plan: TallPlan, terms: Optional[GateTerms] = None,
+                  activation: str = "relu2", constants=None, row_weight: Optional[torch.Tensor] = None) -> None:
+    """An expert's first half in tiles as `plan` says: out bfloat16 = act(a w^T) (`activation`), or with `terms` act(gate, up) for w
+    [gate | up] by rows (limit: the shared expert's), times `row_weight` (float32 [M])."""
+    M, K = a.shape
+    N = w.shape[0]
+    _req(a, "gemm_tall_act.a", torch.bfloat16)
+    _req(w, "gemm_tall_act.w", torch.bfloat16, (N, K))
+    _req(out, "gemm_tall_act.out", torch.bfloat16, (M, N // 2 if terms is not None else N))
+    if plan.n_split != 1:
+        raise KernelError("gemm_tall_act: partial sums have no activation")
+    code = (0, ctypes.c_float(0.0), ctypes.c_float(0.0)) if terms is not None else _unary_args(activation, constants)
+    t = terms or GateTerms(1.0, 1.0, 0.0)
+    _check(lib().tl_gemm_tall_act(_p(a), K, _p(w), K, _p(out), M, N, K, plan.rows, plan.channels, int(M <= plan.rows and not plan.parts),
+                                  int(plan.stagger), plan.whole, plan.parts, int(terms is not None), *code, ctypes.c_float(t.limit_shared),
+                                  ctypes.c_float(t.alpha), ctypes.c_float(t.shift), _shared_weight(row_weight, M, "gemm_tall_act"), _stream()))
 
 
 def gemm_ring_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int = 1, accumulate: bool = False,

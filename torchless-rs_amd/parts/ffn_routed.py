@@ -302,13 +302,20 @@ class RoutedExperts(FeedForward):
         ops.combine_pairs(z, place, out, accumulate, slices)       # a row's experts in the order it chose them
         if self.shared and not slices:
             wide = 2 if self.gated else 1
-            us = ws.get("experts_su", (n, wide * self.shared), torch.float32)
-            ops.gemm(y, up_w[wide * E * ff:], us)
             hs = ws.get("experts_sh", (n, self.shared), y.dtype)
-            if self.gated:
-                ops.expert_gated_act(us, None, 0, 0, self.shared, self.gate_terms, hs, sw)
+            shared_w = up_w[wide * E * ff:]
+            plan = None
+            if not self.gated or self.shared % 32 == 0:
+                plan = ops.tall_plan(n, wide * self.shared, H, ops.compute_units(y.device), "act")
+            if plan is not None and hs.data_ptr() % 16 == 0 and shared_w.data_ptr() % 16 == 0:
+                ops.gemm_tall_act(y, shared_w, hs, plan, row_weight=sw, **act)
             else:
-                ops.expert_act(us, None, 0, self.shared, self.activation, hs, shared_weight=sw)
+                us = ws.get("experts_su", (n, wide * self.shared), torch.float32)
+                ops.gemm(y, shared_w, us)
+                if self.gated:
+                    ops.expert_gated_act(us, None, 0, 0, self.shared, self.gate_terms, hs, sw)
+                else:
+                    ops.expert_act(us, None, 0, self.shared, self.activation, hs, shared_weight=sw)
             torch.addmm(out, hs, down_w[:, E * ff:].t(), out_dtype=torch.float32, out=out)
 
     def _grouped_library(self, ctx, y: torch.Tensor, out: torch.Tensor, accumulate: bool) -> None:
