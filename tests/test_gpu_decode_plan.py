@@ -1,0 +1,156 @@
+"""A single-token step's keys in parts by the lengths of its sequences (attn_decode_plan_kernel, csrc/attention_bf16.hip): the plan
+against its rule, and attention through it against float64."""
+import types
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+PAGE = 64
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from torchless_rs_amd.kernels import ops as o
+    o.lib()
+    return o
+
+
+def n_pages(p, window, keep, chunk):
+    lo = max(0, p - window + 1) if window else 0
+    if chunk:
+        lo = max(lo, p // chunk * chunk)
+    kept = min(-(-keep // PAGE), lo // PAGE) if window else 0
+    return p // PAGE - lo // PAGE + 1 + kept
+
+
+def part_pages(n, round_, rounds):
+    """The rule: over the counts of rounds that hold every sequence, the smallest parts that fit, the count with the least rounds x
+    pages (the fewest rounds of equal ones), at least as many pages as the merge of a part more is worth."""
+    best = None
+    least = next(q for q in range(1, 10 ** 6) if 20 * q * q >= 3 * max(n))
+    for k in range(1, rounds + 1):
+        if k * round_ < len(n):
+            continue
+        q = next(q for q in range(1, max(n) + 1) if sum(-(-x // q) for x in n) <= k * round_)
+        q = max(q, least)
+        if best is None or k * q < best[0]:
+            best = (k * q, q)
+    return best[1]
+
+
+@pytest.mark.parametrize("lengths,round_,rounds", [([1, 1], 2, 1), ([64, 65, 130], 16, 1), ([1062, 1125, 1319, 1323, 2297, 2604, 3832, 8192], 64, 1),
+                                                   ([4096] * 20, 64, 1), ([4096] * 22, 64, 3), ([131072, 1], 512, 1), (list(range(1, 6400, 100)), 64, 3),
+                                                   ([17] * 512, 512, 1), ([9000] + [30] * 99, 100, 3), ([5000] * 65, 512, 2)])
+@pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (300, 0, 0), (4096, 100, 0), (0, 0, 256)])
+def test_a_plan_covers_every_page_once_in_the_smallest_parts(ops, lengths, round_, rounds, window, keep, chunk):
+    B, places = len(lengths), round_ * rounds
+    pos = [x - 1 for x in lengths]
+    plan = torch.full((places + 8, 4), -7, dtype=torch.int32, device=DEV)
+    seqs = torch.full((B, 2), -7, dtype=torch.int32, device=DEV)
+    row_pos = torch.tensor(pos, dtype=torch.int32, device=DEV)
+    ops._check(ops.lib().tl_attn_decode_plan(ops._p(row_pos), B, window, keep, chunk, round_, rounds, ops._p(plan), ops._p(seqs), ops._stream()))
+    plan, seqs = plan.tolist(), seqs.tolist()
+    n = [n_pages(p, window, keep, chunk) for p in pos]
+    Q = part_pages(n, round_, rounds)
+    at = 0
+    for b in range(B):
+        parts = -(-n[b] // Q)
+        assert seqs[b] == [at, parts]
+        cuts = [s * n[b] // parts for s in range(parts + 1)]
+        assert plan[at:at + parts] == [[4 * b + 2 * (s == 0) + (parts == 1), cuts[s], cuts[s + 1], pos[b]] for s in range(parts)]
+        at += parts
+    assert at <= places and all(e[0] == -1 for e in plan[at:places]) and plan[places:] == [[-7] * 4] * 8
+
+
+def step(ops, lengths, nq, nkv, d, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    width = -(-max(lengths) // PAGE) + 1
+    pages = torch.randn(len(lengths) * width, 2, nkv, PAGE, d, generator=g, device=DEV).bfloat16()
+    table = torch.randperm(len(lengths) * width, generator=g, device=DEV).view(len(lengths), width).int()
+    q = torch.randn(len(lengths), nq, d, generator=g, device=DEV).bfloat16()
+    from torchless_rs_amd.parts.base import Workspace
+    ctx = types.SimpleNamespace(n_rows=len(lengths), device=torch.device(DEV), host={}, workspace=Workspace(torch.device(DEV)), all_single=True,
+                                row_pos=torch.tensor([x - 1 for x in lengths], dtype=torch.int32, device=DEV))
+    return q, pages, table, ctx
+
+
+def want(q, pages, table, lengths, scale, window=0, keep=0, chunk=0, logistic=False, bias=None, sinks=None, gate=None):
+    B, nq, d = q.shape
+    nkv = pages.shape[2]
+    out, size = torch.empty(B, nq, d, dtype=torch.float64, device=DEV), torch.empty(B, nq, d, dtype=torch.float64, device=DEV)
+    for b, L in enumerate(lengths):
+        mine = pages[table[b].long()].double()
+        k = mine[:, 0].transpose(0, 1).reshape(nkv, -1, d)[:, :L].repeat_interleave(nq // nkv, 0)
+        v = mine[:, 1].reshape(-1, nkv, d, PAGE).permute(1, 0, 3, 2).reshape(nkv, -1, d)[:, :L].repeat_interleave(nq // nkv, 0)
+        s = (k * q[b].double()[:, None]).sum(-1) * scale
+        j, p = torch.arange(L, device=DEV), L - 1
+        ok = torch.ones(L, dtype=torch.bool, device=DEV)
+        if window:
+            ok &= (p - j < window) | (j < keep)
+        if chunk:
+            ok &= j // chunk == p // chunk
+        if logistic:
+            w = torch.sigmoid(s + bias.double()[:, None]) * ok
+        else:
+            s = s.masked_fill(~ok, float("-inf"))
+            if sinks is not None:
+                s = torch.cat([s, sinks.double()[:, None]], 1)
+            w = torch.softmax(s, -1)[:, :L]
+        if gate is not None:
+            w = w * gate[b].double()[:, None]
+        out[b], size[b] = (w[..., None] * v).sum(1), (w[..., None] * v.abs()).sum(1)
+    return out, size
+
+
+LENGTHS = [[1, 700], [64, 65, 1, 1500, 129], [2048] + [130] * 30, [3000, 1, 500, 2999] * 7]
+
+
+@pytest.mark.parametrize("lengths", LENGTHS)
+@pytest.mark.parametrize("nq,nkv,d", [(8, 2, 128), (32, 8, 64), (12, 3, 128), (4, 1, 256), (40, 2, 64)])
+@pytest.mark.parametrize("window", [None, 300])
+def test_attention_in_planned_parts(ops, lengths, nq, nkv, d, window):
+    """The weights go to the second product with 8 bits and so does the result: 2^-9 of the sum of sizes and of itself; twice that."""
+    q, pages, table, ctx = step(ops, lengths, nq, nkv, d)
+    out = torch.full_like(q, float("nan"))
+    planned = ops.decode_plan(ctx, nq, nkv, d, table.shape[1], window)
+    if planned is None:                              # 28 or 31 sequences of these heads are more than half a round
+        assert len(lengths) > 5
+    assert planned is None or ops.decode_plan(ctx, nq, nkv, d, table.shape[1], window)[0] is planned[0]
+    ops.attention(q, None, None, pages, table, table.shape[1], ctx, None, window, d ** -0.5, out)
+    ref, size = want(q, pages, table, lengths, d ** -0.5, window or 0)
+    assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs()) + 1e-5).all())
+
+
+@pytest.mark.parametrize("lengths", LENGTHS[:3])
+@pytest.mark.parametrize("kind", ["sinks", "logistic", "kept", "chunk"])
+def test_attention_with_terms_in_planned_parts(ops, lengths, kind):
+    nq, nkv, d = 8, 2, 128
+    q, pages, table, ctx = step(ops, lengths, nq, nkv, d, 1)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    kw, ref_kw = {"sinks": ({"sinks": torch.randn(nq, generator=g, device=DEV)},) * 2,
+                  "logistic": ({"logistic": True, "score_bias": torch.randn(nq, generator=g, device=DEV) - 4.0},) * 2,
+                  "kept": ({"window": 200, "keep_first": 70},) * 2, "chunk": ({"chunk": 192},) * 2}[kind]
+    ref_kw = {{"score_bias": "bias", "keep_first": "keep"}.get(k, k): v for k, v in ref_kw.items()}
+    gate = torch.rand(len(lengths), nq, generator=g, device=DEV) if kind in ("sinks", "logistic") else None
+    out = torch.full_like(q, float("nan"))
+    ring = 1 << 20 if kind == "kept" else table.shape[1]
+    ops.attention_scored(q, None, None, pages, nkv, d, table, ring, ctx, None, ops.ScoreTerms(d ** -0.5, **kw), gate, out)
+    assert "decode_plans" in ctx.host
+    ref, size = want(q, pages, table, lengths, d ** -0.5, gate=gate, **ref_kw)
+    assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs()) + 1e-5).all())
+
+
+def test_who_goes_without_a_plan(ops):
+    assert ops.decode_rounds(1, 32, 8, 256, 128) is None and ops.decode_rounds(33, 32, 8, 256, 128) is None
+    assert ops.decode_rounds(8, 32, 8, 256, 128) == (64, 1) and ops.decode_rounds(22, 32, 8, 256, 128) == (64, 3)
+    assert ops.decode_rounds(513, 4, 1, 2048, 128) is None and ops.decode_rounds(4, 32, 32, 256, 256) == (8, 3)
+    assert ops.decode_rounds(32, 32, 8, 256, 128) == (64, 3)
+    q, pages, table, ctx = step(ops, [100, 70], 4, 2, 96)
+    assert ops.decode_plan(ctx, 4, 2, 96, table.shape[1], None) is None and ops.decode_plan(ctx, 4, 2, 64, 2049, None) is None
+    was = ops.decode_through_lds(False)
+    try:
+        assert ops.decode_plan(ctx, 4, 2, 64, 8, None) is None
+    finally:
+        ops.decode_through_lds(was)

@@ -806,13 +806,95 @@ template <int N> __device__ __forceinline__ void wait_page_loads_but() {     // 
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// The parts of a step whose sequences have unequal lengths, made once a step for all of its layers (the lengths are the device's: a
+// captured step is replayed with others).  With as many parts for every sequence, a step waits for the longest sequence's parts:
+// 8 sequences of 1,062 to 8,192 keys in 8 parts each had 16 pages a workgroup where 6 are an equal share.  Here parts of at most Q
+// pages are dealt to `round` places, as many workgroups (over heads) as the device holds at a time, or two or three such rounds:
+// for each count of rounds the smallest Q whose parts fit, and of these the one with the least rounds x Q; but not so small that
+// the merge costs more (Q^2 >= 0.15 pages of the longest, the merge's share of a part).  Those 8 sequences (89 MB a layer): 27 us a
+// layer before and 20.4 now, a step 3,842 and 3,639; 8 of equal lengths as before, and the plan's 5 us a step.
+//   plan[place] = {4 sequence + 2 (its first part) + (its only part), first page, end, position}, {-1, ..} where a place is empty
+//   seqs[sequence] = {first place, parts}
+constexpr int DP_EACH = 8, DP_MAX_SEQS = DP_EACH * WAVE;
+
+__global__ void __launch_bounds__(WAVE)
+attn_decode_plan_kernel(const int* __restrict__ row_pos, int B, int window, int keep_first, int chunk, int round, int rounds,
+                        int4* __restrict__ plan, int2* __restrict__ seqs) {
+  const int lane = threadIdx.x;
+  const auto sum = [](int v) {
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+    return v;
+  };
+  int n[DP_EACH], pos[DP_EACH], total = 0, longest = 0;
+#pragma unroll
+  for (int j = 0; j < DP_EACH; ++j) {
+    const int b = j * WAVE + lane;
+    pos[j] = b < B ? row_pos[b] : 0;
+    int lo = (window > 0 && pos[j] - window + 1 > 0) ? pos[j] - window + 1 : 0;
+    if (chunk > 0) lo = max(lo, (pos[j] / chunk) * chunk);
+    n[j] = b < B ? PageSpan(lo, pos[j], window > 0 ? keep_first : 0).n : 0;
+    total += n[j];
+    longest = max(longest, n[j]);
+  }
+  total = sum(total);
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) longest = max(longest, __shfl_xor(longest, o, WAVE));
+  const auto parts = [&](int q) {
+    int v = 0;
+#pragma unroll
+    for (int j = 0; j < DP_EACH; ++j) v += (n[j] + q - 1) / q;
+    return sum(v);
+  };
+  int least = 1;
+  while (20 * least * least < 3 * longest) ++least;
+  int Q = longest, cost = 0x7fffffff;
+  for (int k = 1; k <= rounds; ++k) {
+    const int places = k * round;
+    if (places < B) continue;
+    int lo = max(1, (total + places - 1) / places), hi = longest;      // parts(hi) <= places throughout
+    if (places > B) hi = min(hi, max(lo, (total + places - B - 1) / (places - B)));
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (parts(mid) <= places) hi = mid;
+      else lo = mid + 1;
+    }
+    const int q = max(hi, least);
+    if (k * q < cost) {
+      cost = k * q;
+      Q = q;
+    }
+  }
+  int at = 0;
+#pragma unroll
+  for (int j = 0; j < DP_EACH; ++j) {
+    if (j * WAVE >= B) break;
+    const int b = j * WAVE + lane, mine = (n[j] + Q - 1) / Q;
+    int before = mine;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const int v = __shfl_up(before, o, WAVE);
+      if (lane >= o) before += v;
+    }
+    const int all = __shfl(before, WAVE - 1, WAVE), first = at + before - mine;
+    if (b < B) {
+      seqs[b] = make_int2(first, mine);
+      for (int s = 0; s < mine; ++s)
+        plan[first + s] = make_int4(4 * b + (s == 0 ? 2 : 0) + (mine == 1 ? 1 : 0), (int)((long long)s * n[j] / mine),
+                                    (int)((long long)(s + 1) * n[j] / mine), pos[j]);
+    }
+    at += all;
+  }
+  for (int place = at + lane; place < rounds * round; place += WAVE) plan[place] = make_int4(-1, 0, 0, 0);
+}
+
 template <int D, int NS, bool TERMS = false, bool LOGI = false>
 __global__ void __launch_bounds__(DC_WAVES * 64)
 attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pages,
                         const int* __restrict__ table, int table_stride, int ring_pages,
                         const int* __restrict__ row_pos, int nq, int nkv, int window, float scale,
                         int n_splits, int head_groups, float* __restrict__ part, bf16* __restrict__ out,
-                        MoreTerms terms) {
+                        MoreTerms terms, const int4* __restrict__ plan = nullptr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char dr_smem[];
   constexpr int KB = D / 32, VB = D / 16;
   constexpr int K_BYTES = PAGE * D * 2, STAGE = 2 * K_BYTES;   // keys, then values, as many bytes each
@@ -825,18 +907,21 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
   const int g = nq / nkv;
   const int hg = blockIdx.x % head_groups;
   const int kvh = (blockIdx.x / head_groups) % nkv;
-  const int b = blockIdx.x / (head_groups * nkv);
-  const int split = blockIdx.y;
+  const int place = blockIdx.x / (head_groups * nkv);
+  const int4 part_of = plan != nullptr ? plan[place] : make_int4(0, 0, 0, 0);
+  if (part_of.x < 0) return;
+  const int b = plan != nullptr ? part_of.x / 4 : place;
+  const bool first_part = plan != nullptr ? part_of.x & 2 : blockIdx.y == 0, alone = plan != nullptr ? part_of.x & 1 : n_splits == 1;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 16, kg = lane / 16;
   const int hl = hg * 16 + li;
   const int h = kvh * g + min(hl, g - 1);
-  const int p = row_pos[b];
+  const int p = plan != nullptr ? part_of.w : row_pos[b];
   int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
   if (TERMS && terms.chunk > 0) lo = max(lo, (p / terms.chunk) * terms.chunk);
   const int keep = (TERMS && window > 0) ? terms.keep_first : 0;
   const PageSpan span(lo, p, keep);
-  const int my_lo = (int)((long long)split * span.n / n_splits);
-  const int my_hi = (int)((long long)(split + 1) * span.n / n_splits);
+  const int my_lo = plan != nullptr ? part_of.y : (int)((long long)blockIdx.y * span.n / n_splits);
+  const int my_hi = plan != nullptr ? part_of.z : (int)((long long)(blockIdx.y + 1) * span.n / n_splits);
   const int n_st = my_hi - my_lo;                     // this split's pages: the stages
   const size_t head_elems = (size_t)PAGE * D, page_elems = 2 * (size_t)nkv * head_elems;
   auto kkey = [](int r) { return K_CPR >= 16 ? r % 16 : (r / 2) % 8; };   // swizzle of a key's row
@@ -1004,7 +1089,7 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
     for (int w = 1; w < DC_WAVES; ++w) osum += red_o[w * (VB * 4 * 64) + idx];
     const size_t bh = (size_t)b * nq + kvh * g + hg * 16 + hd;
     if constexpr (TERMS) {
-      if (terms.sinks != nullptr && split == 0) {     // the sink counts once: with the first split
+      if (terms.sinks != nullptr && first_part) {     // the sink counts once: with the first split
         const float sk = terms.sinks[kvh * g + hg * 16 + hd];
         const float ms = fmaxf(mh, sk);
         const float fs = (mh == -INFINITY) ? 0.f : __expf(mh - ms);
@@ -1013,15 +1098,15 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
         mh = ms;
       }
     }
-    if constexpr (LOGI) ll = split == 0 ? 1.f : 0.f;  // the sum is a 1, once for a row
-    if (n_splits == 1) {
+    if constexpr (LOGI) ll = first_part ? 1.f : 0.f;  // the sum is a 1, once for a row
+    if (alone) {
       float res = osum / ll;
       if constexpr (TERMS)
         if (terms.gate != nullptr) res *= terms.gate[bh];
       out[bh * D + dv] = (bf16)res;
       continue;
     }
-    float* dst = part + (bh * n_splits + split) * (D + 2);
+    float* dst = part + (plan != nullptr ? (size_t)place * nq + kvh * g + hg * 16 + hd : bh * n_splits + blockIdx.y) * (D + 2);
     dst[2 + dv] = osum;
     if (dv == 0) {
       dst[0] = mh;
@@ -1041,12 +1126,19 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
 // chunks merge by the running-maximum rule.
 __global__ void __launch_bounds__(64)
 attn_decode_combine_kernel(const float* __restrict__ part, int n_splits, int d, bf16* __restrict__ out,
-                           const float* __restrict__ gate = nullptr) {
+                           const float* __restrict__ gate = nullptr, const int2* __restrict__ seqs = nullptr, int nq = 1) {
   constexpr int CH = 8, MAXV = 4;                      // d <= 256: at most 4 elements a lane
   const size_t bh = blockIdx.x;
   const float* src = part + bh * n_splits * (d + 2);
   const int lane = threadIdx.x;
-  const size_t stride = d + 2;
+  size_t stride = d + 2;
+  if (seqs != nullptr) {                               // a planned step: a sequence has parts of its own, place after place
+    const int2 mine = seqs[bh / nq];
+    if (mine.y == 1) return;                           // (its only part has written the result)
+    n_splits = mine.y;
+    src = part + ((size_t)mine.x * nq + bh % nq) * (d + 2);
+    stride *= nq;
+  }
   float mm = -INFINITY, ll = 0.f, acc[MAXV];
 #pragma unroll
   for (int v = 0; v < MAXV; ++v) acc[v] = 0.f;
@@ -1197,10 +1289,18 @@ static bool decode_through_lds = true;
 constexpr int DR_MAX_PAGES = 2048;      // most pages of a sequence that the kernel through LDS keeps the ids of (8 KB)
 
 // single-token steps with more terms on the scores; LOGI: logistic weights
+// a step's parts as attn_decode_plan_kernel made them (null: n_splits for every sequence), over `places` places
+struct DecodePlan {
+  const int4* plan = nullptr;
+  const int2* seqs = nullptr;
+  int places = 0;
+};
+
 template <int DPAD, bool LOGI>
 static int launch_decode_terms(const bf16* q, const bf16* pages, const int* table, int table_stride,
                                int ring_pages, const int* row_pos, int B, int nq, int nkv, int d, int window,
-                               float scale, int n_splits, float* part, bf16* out, hipStream_t st, const MoreTerms* terms) {
+                               float scale, int n_splits, float* part, bf16* out, hipStream_t st, const MoreTerms* terms,
+                         const DecodePlan& plan) {
   const int g = nq / nkv, head_groups = (g + 15) / 16;
   dim3 grid(B * nkv * head_groups, n_splits);
   if constexpr (DPAD == 64 || DPAD == 128 || DPAD == 256) {
@@ -1217,12 +1317,13 @@ static int launch_decode_terms(const bf16* q, const bf16* pages, const int* tabl
         }
         raised_terms = true;
       }
+      if (plan.plan != nullptr) grid = dim3(plan.places * nkv * head_groups, 1);
       attn_decode_ring_kernel<DPAD, NS, true, LOGI><<<grid, DC_WAVES * 64, LDS, st>>>(q, pages, table, table_stride, ring_pages,
                                                                                       row_pos, nq, nkv, window, scale, n_splits,
-                                                                                      head_groups, part, out, *terms);
+                                                                                      head_groups, part, out, *terms, plan.plan);
       TL_LAUNCH_CHECK("attn_decode_ring with terms");
-      if (n_splits > 1) {
-        attn_decode_combine_kernel<<<B * nq, 64, 0, st>>>(part, n_splits, d, out, terms->gate);
+      if (n_splits > 1 || plan.plan != nullptr) {
+        attn_decode_combine_kernel<<<B * nq, 64, 0, st>>>(part, n_splits, d, out, terms->gate, plan.seqs, nq);
         TL_LAUNCH_CHECK("attn_decode_combine");
       }
       return 0;
@@ -1248,15 +1349,16 @@ static int launch_decode_terms(const bf16* q, const bf16* pages, const int* tabl
 template <int DPAD>
 static int launch_decode(const bf16* q, const bf16* pages, const int* table, int table_stride,
                          int ring_pages, const int* row_pos, int B, int nq, int nkv, int d, int window,
-                         float scale, int n_splits, float* part, bf16* out, hipStream_t st, const MoreTerms* terms) {
+                         float scale, int n_splits, float* part, bf16* out, hipStream_t st, const MoreTerms* terms,
+                         const DecodePlan& plan) {
   const int g = nq / nkv, head_groups = (g + 15) / 16;
   dim3 grid(B * nkv * head_groups, n_splits);
   if (terms != nullptr && terms->logistic)
     return launch_decode_terms<DPAD, true>(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale,
-                                           n_splits, part, out, st, terms);
+                                           n_splits, part, out, st, terms, plan);
   if (terms != nullptr)
     return launch_decode_terms<DPAD, false>(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale,
-                                            n_splits, part, out, st, terms);
+                                            n_splits, part, out, st, terms, plan);
   if constexpr (DPAD == 64 || DPAD == 128 || DPAD == 256) {
     if (d == DPAD && decode_through_lds && table_stride <= DR_MAX_PAGES) {
       constexpr int NS = DPAD == 64 ? 4 : 2;         // 64 KB of LDS, two workgroups a compute unit; heads of 256: 128 KB, one
@@ -1271,12 +1373,13 @@ static int launch_decode(const bf16* q, const bf16* pages, const int* table, int
         }
         raised = true;
       }
+      if (plan.plan != nullptr) grid = dim3(plan.places * nkv * head_groups, 1);
       attn_decode_ring_kernel<DPAD, NS><<<grid, DC_WAVES * 64, LDS, st>>>(q, pages, table, table_stride, ring_pages,
                                                                           row_pos, nq, nkv, window, scale, n_splits,
-                                                                          head_groups, part, out, MoreTerms{});
+                                                                          head_groups, part, out, MoreTerms{}, plan.plan);
       TL_LAUNCH_CHECK("attn_decode_ring");
-      if (n_splits > 1) {
-        attn_decode_combine_kernel<<<B * nq, 64, 0, st>>>(part, n_splits, d, out);
+      if (n_splits > 1 || plan.plan != nullptr) {
+        attn_decode_combine_kernel<<<B * nq, 64, 0, st>>>(part, n_splits, d, out, nullptr, plan.seqs, nq);
         TL_LAUNCH_CHECK("attn_decode_combine");
       }
       return 0;
@@ -1439,7 +1542,7 @@ extern "C" int tl_attn_decode_through_lds(int on) {
 static int attn_decode_entry(const void* q, const void* pages, const int* table, int table_stride,
                                    int ring_pages, const int* row_pos, int B, int nq, int nkv, int d,
                                    int window, float scale, int n_splits, float* part, void* out,
-                                   hipStream_t st, const MoreTerms* terms) {
+                                   hipStream_t st, const MoreTerms* terms, const DecodePlan& plan = DecodePlan{}) {
   TL_REQUIRE(B > 0 && nq > 0 && nkv > 0 && nq % nkv == 0, "attn_decode: bad sizes B=%d nq=%d nkv=%d", B,
              nq, nkv);
   TL_REQUIRE(d >= 16 && d <= 256 && d % 16 == 0, "attn_decode: head size %d is not served "
@@ -1448,7 +1551,7 @@ static int attn_decode_entry(const void* q, const void* pages, const int* table,
              "attn_decode: bad geometry ring_pages=%d table_stride=%d window=%d splits=%d", ring_pages,
              table_stride, window, n_splits);
   TL_BY_DPAD(launch_decode, (const bf16*)q, (const bf16*)pages, table, table_stride, ring_pages, row_pos,
-             B, nq, nkv, d, window, scale, n_splits, part, (bf16*)out, st, terms);
+             B, nq, nkv, d, window, scale, n_splits, part, (bf16*)out, st, terms, plan);
   return 1;
 }
 
@@ -1473,6 +1576,46 @@ extern "C" int tl_attn_decode_terms_bf16(const void* q, const void* pages, const
   const MoreTerms terms{slopes, sinks, gate, window > 0 ? keep_first : 0, chunk, logistic, score_bias};
   return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, n_splits,
                            part, out, st, &terms);
+}
+
+// Do single-token steps with heads of d and page tables of this width go through the kernel that stages the pages in LDS (the one
+// that takes a plan)?
+extern "C" int tl_attn_decode_takes_plan(int d, int table_stride) {
+  return (d == 64 || d == 128 || d == 256) && decode_through_lds && table_stride <= DR_MAX_PAGES ? 1 : 0;
+}
+
+// plan int [rounds * round][4], seqs int [B][2] for a step's sequences (see attn_decode_plan_kernel); every layer with this window,
+// these kept first positions and this chunk can use them
+extern "C" int tl_attn_decode_plan(const int* row_pos, int B, int window, int keep_first, int chunk, int round, int rounds, int* plan,
+                                   int* seqs, hipStream_t st) {
+  TL_REQUIRE(B > 0 && B <= DP_MAX_SEQS && round > 0 && rounds > 0 && rounds <= 16 && (long)round * rounds >= B && (long)round * rounds < (1l << 20),
+             "attn_decode_plan: %d sequences in %d x %d places", B, rounds, round);
+  TL_REQUIRE(window >= 0 && keep_first >= 0 && chunk >= 0, "attn_decode_plan: bad window %d, %d kept, chunk %d", window, keep_first, chunk);
+  TL_REQUIRE(row_pos && plan && seqs && (uintptr_t)plan % 16 == 0 && (uintptr_t)seqs % 8 == 0, "attn_decode_plan: a buffer is missing or not aligned");
+  attn_decode_plan_kernel<<<1, WAVE, 0, st>>>(row_pos, B, window, keep_first, chunk, round, rounds, (int4*)plan, (int2*)seqs);
+  TL_LAUNCH_CHECK("attn_decode_plan");
+  return 0;
+}
+
+// tl_attn_decode_bf16, or with `more` tl_attn_decode_terms_bf16, with the parts of a plan over `places` places; part: float scratch of
+// places * nq * (d + 2) elements
+extern "C" int tl_attn_decode_planned_bf16(const void* q, const void* pages, const int* table, int table_stride, int ring_pages,
+                                           const int* row_pos, int B, int nq, int nkv, int d, int window, float scale, const int* plan,
+                                           const int* seqs, int places, int more, int keep_first, int chunk, const float* slopes,
+                                           const float* sinks, const float* gate, int logistic, const float* score_bias, float* part,
+                                           void* out, hipStream_t st) {
+  TL_REQUIRE(tl_attn_decode_takes_plan(d, table_stride), "attn_decode_planned: heads of %d with %d pages go without a plan", d, table_stride);
+  TL_REQUIRE(plan && seqs && part && places >= B && (uintptr_t)plan % 16 == 0 && (uintptr_t)seqs % 8 == 0 &&
+             nq > 0 && nkv > 0 && (long)places * nkv * ((nq / nkv + 15) / 16) * DC_WAVES * 64 < (1l << 31),
+             "attn_decode_planned: %d places for %d sequences", places, B);
+  const DecodePlan dp{(const int4*)plan, (const int2*)seqs, places};
+  if (!more) return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, 1, part, out, st, nullptr, dp);
+  TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || window == 0 || (long long)ring_pages * PAGE >= (1LL << 24)),
+             "attn_decode: first positions that stay visible beside a window need a cache that keeps every position");
+  TL_REQUIRE(chunk >= 0 && (!logistic || sinks == nullptr) && (logistic || score_bias == nullptr),
+             "attn_decode: %d positions a chunk; logistic weights have no sink, a softmax no bias on the score", chunk);
+  const MoreTerms terms{slopes, sinks, gate, window > 0 ? keep_first : 0, chunk, logistic, score_bias};
+  return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, 1, part, out, st, &terms, dp);
 }
 
 // ---- the entry point that allocates nothing (declared in no_alloc.h) --------

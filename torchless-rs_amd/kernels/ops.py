@@ -644,6 +644,10 @@ def attention_scored(q, k_new, v_new, pages, nkv: int, dv: int, table, ring_page
             most_pages = min(most_pages, -(-terms.window // PAGE) + 1 + -(-int(terms.keep_first or 0) // PAGE))
         if terms.chunk:
             most_pages = min(most_pages, -(-terms.chunk // PAGE) + 1)
+        plan = decode_plan(ctx, nq, nkv, dk, table.shape[1], terms.window, int(terms.keep_first or 0), terms.chunk)
+        if plan is not None:
+            attn_decode_planned(q, pages, table, ring_pages, ctx, plan, terms.window, terms.scale, out, terms, gate)
+            return
         splits = decode_splits(n, nq, nkv, most_pages, compute_units(q.device), dk)
         part = ctx.workspace.get("attn_part", (n * nq * splits * (dk + 2),), torch.float32)
         _decode_args(q, pages, table, ctx.row_pos, part, out, splits)
@@ -2549,6 +2553,59 @@ def decode_splits(B: int, nq: int, nkv: int, max_pages: int, units: int, head_di
     return _decode_splits(decode_groups(B, nq, nkv), int(max_pages), int(units) * decode_workgroups_per_unit(head_dim))
 
 
+PLAN_SEQS = 512             # most sequences that a plan is made for
+
+
+def decode_rounds(B: int, nq: int, nkv: int, units: int, head_dim: int):
+    """(places, rounds) of the plan of a decode step's parts, or None where it goes without one: `decode_splits` then gives every
+    sequence as many parts.  A place is one workgroup for each KV head (16 query heads of its group), a round as many places as the
+    units hold at a time.  One sequence has nothing to balance, and where more than half of a round are sequences the uniform parts
+    are so many that the units even out what they have by themselves (64 sequences of 140 to 2,048 keys: 60.5 us and 4.9 for the merge,
+    65.1 without parts; a step the same).  From a third of a round on, two or three rounds of smaller parts may divide better (20
+    sequences of one length in 64 places: 3 parts each, 60; 22: 2 parts each, or 5 each in two rounds)."""
+    places = units * decode_workgroups_per_unit(head_dim) // decode_groups(1, nq, nkv)
+    if not (2 <= B <= min(places // 2, PLAN_SEQS)):
+        return None
+    return places, (1 if 3 * B <= places else 3)
+
+
+def decode_plan(ctx, nq: int, nkv: int, d: int, table_width: int, window: Optional[int], keep_first: int = 0, chunk: int = 0):
+    """The plan of a single-token step's parts for layers of these sizes, made by the first of them (one small kernel, 4 us) and kept
+    while the step runs: (plan int32 [places, 4], seqs int32 [B, 2]), or None."""
+    B = ctx.row_pos.shape[0]
+    shape = decode_rounds(B, nq, nkv, compute_units(ctx.row_pos.device), d)
+    if shape is None or not lib().tl_attn_decode_takes_plan(d, int(table_width)):
+        return None
+    key = (shape, int(window or 0), int(keep_first) if window else 0, int(chunk or 0))
+    plans = ctx.host.setdefault("decode_plans", {})
+    if key not in plans:
+        name = "attn_plan_" + "_".join(map(str, shape + key[1:]))
+        plan = ctx.workspace.get(name, (shape[0] * shape[1], 4), torch.int32)
+        seqs = ctx.workspace.get(name + "_seqs", (B, 2), torch.int32)
+        _req(ctx.row_pos, "attn_decode_plan.row_pos", torch.int32, (B,))
+        _check(lib().tl_attn_decode_plan(_p(ctx.row_pos), B, *key[1:], *shape, _p(plan), _p(seqs), _stream()))
+        plans[key] = plan, seqs
+    return plans[key]
+
+
+def attn_decode_planned(q, pages, table, ring_pages: int, ctx, plan, window: Optional[int], scale: float, out,
+                        terms: Optional[ScoreTerms] = None, gate=None) -> None:
+    """`attn_decode_bf16`, or with `terms` its variant with those, in the parts of `decode_plan`."""
+    B, nq, d = q.shape
+    nkv = pages.shape[2]
+    places, seqs = plan
+    _req(places, "attn_decode_planned.plan", torch.int32)
+    _req(seqs, "attn_decode_planned.seqs", torch.int32, (B, 2))
+    part = ctx.workspace.get("attn_part", (places.shape[0] * nq * (d + 2),), torch.float32)
+    _decode_args(q, pages, table, ctx.row_pos, part, out, 1)
+    slopes, sinks, gt = _terms_args(terms, gate, B, nq) if terms is not None else (None, None, None)
+    more = (1, int(terms.keep_first or 0), terms.chunk) if terms is not None else (0, 0, 0)
+    _check(lib().tl_attn_decode_planned_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(ctx.row_pos), B, nq, nkv, d,
+                                             int(window or 0), ctypes.c_float(scale), _p(places), _p(seqs), places.shape[0], *more, slopes,
+                                             sinks, gt, int(terms.logistic) if terms is not None else 0,
+                                             _p(terms.score_bias) if terms is not None else None, _p(part), _p(out), _stream()))
+
+
 def uses_transposed_values(dtype: torch.dtype, d: int, all_single: bool) -> bool:
     """Does `attention` take this step's values transposed (`vt_new`)?"""
     return dtype == torch.bfloat16 and d % 16 == 0 and 16 <= d <= 256 and not all_single
@@ -2566,6 +2623,10 @@ def attention(q, k_new, v_new, pages, table, ring_pages: int, ctx, n_cached, win
     fast = q.dtype == torch.bfloat16 and d % 16 == 0 and 16 <= d <= 256
     if fast and k_new is None and ctx.all_single:
         nkv = pages.shape[2]
+        plan = decode_plan(ctx, nq, nkv, d, table.shape[1], window)
+        if plan is not None:
+            attn_decode_planned(q, pages, table, ring_pages, ctx, plan, window, scale, out)
+            return
         splits = decode_splits(n, nq, nkv, table.shape[1], compute_units(q.device), d)   # by the table's width: fixed while a graph lives
         part = ctx.workspace.get("attn_part", (n * nq * splits * (d + 2),), torch.float32)
         attn_decode_bf16(q, pages, table, ring_pages, ctx.row_pos, window, scale, splits, part, out)
