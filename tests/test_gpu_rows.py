@@ -92,3 +92,35 @@ def test_the_activation_of_a_stored_product(ops, dtype, n, I):
     want = gate / (1.0 + torch.exp(-gate)) * up
     # the exponential, the division and two products: a few units of 2^-24; bfloat16 rounds the result once
     assert bool(((out.double() - want).abs() <= want.abs() * (1e-6 if dtype == torch.float32 else 2.0 ** -8) + 1e-30).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nq,nkv,d", [(1, 1, 8), (3, 1, 64), (32, 8, 128), (5, 5, 200), (40, 8, 256)])
+def test_pairs_by_fours_are_those_one_by_one(ops, dtype, nq, nkv, d):
+    """Rotation four pairs a thread, values four channels and their commit 16 bytes at a time leave the bits that buffers off 16 bytes get,
+    for 70 sequences, of which some begin inside a page and end inside one."""
+    g = torch.Generator(device=DEV).manual_seed(d)
+    new = [1 + (7 * b) % 131 for b in range(70)]
+    cached = [(29 * b) % 200 for b in range(70)]
+    n, i32 = sum(new), lambda l: torch.tensor(l, dtype=torch.int32, device=DEV)
+    off, cols = ops.aligned_columns(cached, new)
+    seq = i32([b for b in range(70) for _ in range(new[b])])
+    pos = i32([cached[b] + i for b in range(70) for i in range(new[b])])
+    cu, after = i32([sum(new[:b]) for b in range(71)]), i32([c + m for c, m in zip(cached, new)])
+    inv = 10000.0 ** (-2.0 * torch.arange(d // 2, device=DEV) / d)
+    data = torch.randn(n, (nq + 2 * nkv) * d, generator=g, device=DEV)
+    table = torch.randperm(70 * 6, generator=g, device=DEV).view(70, 6).int()
+
+    def run(shift):
+        def buf(fill, *shape, dt=dtype):
+            size = 1
+            for s in shape:
+                size *= s
+            return torch.full((size + shift,), fill, dtype=dt, device=DEV)[shift:].view(shape)
+        qkv = buf(0.0, *data.shape, dt=torch.float32).copy_(data)
+        q, k, vt, pages = buf(3.0, n, nq, d), buf(3.0, n, nkv, d), buf(7.0, nkv, d, cols), buf(5.0, 420, 2, nkv, 64, d)
+        ops.rope_v_tiles(qkv, pos, inv, nq, nkv, d, q, k, vt, cu, i32(off), i32(cached), after)
+        ops.kv_commit_tiles(k, vt, seq, pos, i32(off), i32(cached), after, table, 1 << 24, pages)
+        return q, k, vt, pages
+    for a, b in zip(run(0), run(1)):
+        assert torch.equal(a, b)
