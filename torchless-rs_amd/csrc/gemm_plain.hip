@@ -28,9 +28,10 @@ __host__ __device__ __forceinline__ int run_length(int K) { return (K + PG * PR 
 // on their way in registers meanwhile.  Bound by the stream of W.  N / 8 workgroups fill the chip from N = 2,048 on;
 // tiles of 64 x 64 with a chain of all of K in a thread, which this replaced, made 32 workgroups there.
 // Microseconds at one row, tiles of 64 before: N x K = 2,048 x 8,192 19.4 and 525, 2,048 x 2,048 5.3 and 130,
-// 16,384 x 2,048 28.3 (4.7 TB/s) and 216.
+// 16,384 x 2,048 28.3 (4.7 TB/s; 24.5 by the kernel below) and 216.
+// LINES: W's loads take whole lines, each once, and are marked non-temporal (2,048 x 8,192 at 2 rows 20.0 us without, 18.2 with).
 constexpr int CHUNK = 32;                         // channels of a pair that a wave brings in at a time
-template <int MR, bool ACCUMULATE>
+template <int MR, bool ACCUMULATE, bool LINES>
 __global__ void __launch_bounds__(512)
 gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc) {
@@ -55,7 +56,8 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int off = at + lq, k = (wave * PR + i) * L + off;
-      next[i] = (off < L && k < K && ln < N) ? *(const f32x4*)(wp + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+      next[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (off < L && k < K && ln < N) next[i] = LINES ? __builtin_nontemporal_load((const f32x4*)(wp + k)) : *(const f32x4*)(wp + k);
     }
   };
   fetch(0);
@@ -98,6 +100,82 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
     for (int g = 0; g < PG; ++g) t += sums[g][m][threadIdx.x % 8];
     float* c = C + (size_t)(m0 + m) * ldc + n;
     *c = ACCUMULATE ? *c + t : t;
+  }
+}
+
+// The same bits for one or two rows, K up to 2,048 and many outputs: a workgroup goes through a run of eights of outputs, the next
+// eight's pieces under way while it sums the last's, and a lane keeps its run of A, one piece long, in registers.  With an
+// eight a workgroup every workgroup waited for memory once and did nothing meanwhile, and read A from L1 for each.  One / two rows,
+// before and now: 16,384 x 2,048 28.5 / 32.8 and 24.5 / 25.9 us, 32,000 x 2,048 52.2 / 60.0 and 42.9 / 44.0 (5.95 TB/s).  With fewer
+// eights than workgroups there is nothing to go on to (3,072 x 2,048 9.0 us at two rows, 10.1 so).
+constexpr int ROWS_WORKGROUPS = 512;              // two a compute unit (74 KB of LDS each), so that all run at once
+template <int MR, bool ACCUMULATE, bool LINES>
+__global__ void __launch_bounds__(512)
+gemm_plain_short_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int N, int K, int lda, int ldw,
+                        int ldc) {
+  __shared__ float stage[PG][64][CHUNK + 4];      // rows 144 bytes apart: 16-byte reads of 64 rows spread over the banks
+  __shared__ float sums[2][PG][MR][8];            // of this eight, and of the one before, which others may still read
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const long eights = (N - 1) / 8 + 1;
+  const int from = (int)(blockIdx.x * eights / gridDim.x), to = (int)((blockIdx.x + 1) * eights / gridDim.x);
+  const int L = run_length(K);                    // at most CHUNK
+  const int run = lane / 8;                       // of this lane's pair: output lane % 8, run lane / 8
+  const int k0 = (wave * PR + run) * L;
+  // a load brings 128 bytes of 8 pairs: pair 8 i + lane / 8 (output lane / 8 of run i), 4 channels from 4 (lane % 8)
+  const int lq = (lane % 8) * 4;
+  f32x4 next[8];
+  const auto fetch = [&](int eight) {
+    const int ln = eight * 8 + lane / 8;
+    const float* wp = W + (size_t)min(ln, N - 1) * ldw;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = (wave * PR + i) * L + lq;
+      next[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (lq < L && k < K && ln < N) next[i] = LINES ? __builtin_nontemporal_load((const f32x4*)(wp + k)) : *(const f32x4*)(wp + k);
+    }
+  };
+  if (from < to) fetch(from);
+  f32x4 a[MR][CHUNK / 4];                         // (what lies past the run or past K is 0 times 0)
+#pragma unroll
+  for (int q = 0; q < CHUNK / 4; ++q)
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+      a[m][q] = 4 * q < L && k0 + 4 * q < K ? *(const f32x4*)(A + (size_t)m * lda + k0 + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int eight = from; eight < to; ++eight) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *(f32x4*)&stage[wave][i * 8 + lane / 8][lq] = next[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (eight + 1 < to) fetch(eight + 1);
+    float acc[MR];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) acc[m] = 0.f;
+#pragma unroll
+    for (int q = 0; q < CHUNK / 4; ++q) {
+      const f32x4 w = *(const f32x4*)&stage[wave][run * 8 + lane % 8][4 * q];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int m = 0; m < MR; ++m) acc[m] = fmaf(a[m][q][j], w[j], acc[m]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // the runs of a group in order, then the groups
+    float (*mine)[MR][8] = sums[(eight - from) % 2];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      float g = 0.f;
+#pragma unroll
+      for (int i = 0; i < PR; ++i) g += __shfl(acc[m], i * 8 + lane % 8, WAVE);
+      if (lane < 8) mine[wave][m][lane] = g;
+    }
+    __syncthreads();
+    const int m = threadIdx.x / 8, n = eight * 8 + threadIdx.x % 8;
+    if (m < MR && n < N) {
+      float t = 0.f;
+#pragma unroll
+      for (int g = 0; g < PG; ++g) t += mine[g][m][threadIdx.x % 8];
+      float* c = C + (size_t)m * ldc + n;
+      *c = ACCUMULATE ? *c + t : t;
+    }
   }
 }
 
@@ -211,11 +289,32 @@ template <int MR>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                        int accumulate, hipStream_t st) {
   const long groups = ((long)N + 7) / 8;
+  if constexpr (MR <= 2) {
+    // (a run that is no multiple of 32 channels, or rows off whole lines, would take lines in halves: those are to stay in the caches)
+    const bool lines = ldw % 32 == 0 && run_length(K) % 32 == 0 && (uintptr_t)W % 128 == 0;
+    if (run_length(K) <= CHUNK && groups > ROWS_WORKGROUPS) {
+#define TL_SHORT(ACC, LN) gemm_plain_short_kernel<MR, ACC, LN><<<ROWS_WORKGROUPS, 512, 0, st>>>(A, W, C, N, K, lda, ldw, ldc)
+      if (accumulate && lines) TL_SHORT(true, true);
+      else if (accumulate) TL_SHORT(true, false);
+      else if (lines) TL_SHORT(false, true);
+      else TL_SHORT(false, false);
+#undef TL_SHORT
+      TL_LAUNCH_CHECK("gemm_plain_short");
+      return 0;
+    }
+    if (lines) {
+      const dim3 grid((unsigned)(groups < GRID_X ? groups : GRID_X), 1, (unsigned)((groups + GRID_X - 1) / GRID_X));
+      if (accumulate) gemm_plain_rows_kernel<MR, true, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+      else gemm_plain_rows_kernel<MR, false, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+      TL_LAUNCH_CHECK("gemm_plain_rows");
+      return 0;
+    }
+  }
   const dim3 grid((unsigned)(groups < GRID_X ? groups : GRID_X), (M + MR - 1) / MR, (unsigned)((groups + GRID_X - 1) / GRID_X));
   if (accumulate)
-    gemm_plain_rows_kernel<MR, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+    gemm_plain_rows_kernel<MR, true, false><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   else
-    gemm_plain_rows_kernel<MR, false><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
+    gemm_plain_rows_kernel<MR, false, false><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
   TL_LAUNCH_CHECK("gemm_plain_rows");
   return 0;
 }
