@@ -127,11 +127,11 @@ def test_pairs_by_fours_are_those_one_by_one(ops, dtype, nq, nkv, d):
 
 
 @pytest.mark.parametrize("accumulate", [False, True])
-@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("N,K", [(4096, 2048), (4097, 2048), (4104, 2048), (9001, 1028), (16384, 2044), (5000, 1024), (4500, 64), (12345, 4), (3000, 2052),
                                  (2048, 4096), (4103, 132)])
 def test_few_rows_by_many_outputs(ops, M, N, K, accumulate):
-    """One or two rows: the bits of the same rows among eight, whose kernel adds in the same order, and float64 within the order's
+    """One to four rows: the bits of the same rows among eight, whose kernel adds in the same order, and float64 within the order's
     rounding: a sum in runs, groups and their sum is a chain of K / 64 + 16 additions, each off by 2^-24 of the sum of the sizes."""
     g = torch.Generator(device=DEV).manual_seed(N + K)
     a, w = torch.randn(8, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)

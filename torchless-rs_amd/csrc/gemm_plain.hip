@@ -103,10 +103,11 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
   }
 }
 
-// The same bits for one or two rows, K up to 2,048 and many outputs: a workgroup goes through a run of eights of outputs, the next
+// The same bits for one to four rows, K up to 2,048 and many outputs: a workgroup goes through a run of eights of outputs, the next
 // eight's pieces under way while it sums the last's, and a lane keeps its run of A, one piece long, in registers.  With an
 // eight a workgroup every workgroup waited for memory once and did nothing meanwhile, and read A from L1 for each.  One / two rows,
-// before and now: 16,384 x 2,048 28.5 / 32.8 and 24.5 / 25.9 us, 32,000 x 2,048 52.2 / 60.0 and 42.9 / 44.0 (5.95 TB/s).  With fewer
+// before and now: 16,384 x 2,048 28.5 / 32.8 and 24.5 / 25.9 us, 32,000 x 2,048 52.2 / 60.0 and 42.9 / 44.0 (5.95 TB/s); three / four rows, which
+// took tiles, 39.9 / 38.6 and 26.6 / 29.5, 75.3 / 69.0 and 45.4 / 47.4.  With fewer
 // eights than workgroups there is nothing to go on to (3,072 x 2,048 9.0 us at two rows, 10.1 so).
 constexpr int ROWS_WORKGROUPS = 512;              // two a compute unit (74 KB of LDS each), so that all run at once
 template <int MR, bool ACCUMULATE, bool LINES>
@@ -285,14 +286,17 @@ static int launch_tiles(const TA* A, const TW* W, float* C, int M, int N, int K,
   return 0;
 }
 
+// gemm_plain_short_kernel's sizes (of one to four rows)
+static bool goes_on(int N, int K) { return run_length(K) <= CHUNK && ((long)N + 7) / 8 > ROWS_WORKGROUPS; }
+
 template <int MR>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                        int accumulate, hipStream_t st) {
   const long groups = ((long)N + 7) / 8;
-  if constexpr (MR <= 2) {
+  if constexpr (MR <= 4) {
     // (a run that is no multiple of 32 channels, or rows off whole lines, would take lines in halves: those are to stay in the caches)
     const bool lines = ldw % 32 == 0 && run_length(K) % 32 == 0 && (uintptr_t)W % 128 == 0;
-    if (run_length(K) <= CHUNK && groups > ROWS_WORKGROUPS) {
+    if (goes_on(N, K) && M == MR) {
 #define TL_SHORT(ACC, LN) gemm_plain_short_kernel<MR, ACC, LN><<<ROWS_WORKGROUPS, 512, 0, st>>>(A, W, C, N, K, lda, ldw, ldc)
       if (accumulate && lines) TL_SHORT(true, true);
       else if (accumulate) TL_SHORT(true, false);
@@ -302,7 +306,7 @@ static int launch_rows(const float* A, const float* W, float* C, int M, int N, i
       TL_LAUNCH_CHECK("gemm_plain_short");
       return 0;
     }
-    if (lines) {
+    if (lines && MR <= 2) {
       const dim3 grid((unsigned)(groups < GRID_X ? groups : GRID_X), 1, (unsigned)((groups + GRID_X - 1) / GRID_X));
       if (accumulate) gemm_plain_rows_kernel<MR, true, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
       else gemm_plain_rows_kernel<MR, false, true><<<grid, 512, 0, st>>>(A, W, C, M, N, K, lda, ldw, ldc);
@@ -322,7 +326,7 @@ static int launch_rows(const float* A, const float* W, float* C, int M, int N, i
 // The kernel for few rows reads W once for every 8 rows and has a thread's chain 64 times shorter than K; the tiles read
 // it once for 32.  Measured (rows / tiles, microseconds): N x K = 2,048 x 8,192 at 8 rows 32 / 65, at 16 52 / 68, at 32
 // 96 / 72; 3,072 x 2,048 at 8 14.4 / 18.6, at 16 21 / 19; 4,096 x 14,336 at 8 110 / 126, at 16 197 / 123; 16,384 x
-// 2,048 at 2 31 / 36, at 4 41 / 36; 32,000 x 2,048 at 2 58 / 65, at 4 76 / 65.
+// 2,048 at 2 31 / 36, at 4 41 / 36; 32,000 x 2,048 at 2 58 / 65, at 4 76 / 65 (of up to four rows the latter two are `goes_on`'s now).
 static bool few_rows(int M, int N) { return M <= 2 || (M <= 16 && (long)M * N <= 32768); }
 
 template <typename TA, typename TW>
@@ -334,9 +338,10 @@ static int launch_plain(const void* Av, const void* Wv, float* C, int M, int N, 
                    (uintptr_t)W % (4 * sizeof(TW)) == 0;
   if (!vec) return launch_tiles<TA, TW, false>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
   if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4) {
-    if (few_rows(M, N)) {
+    if (few_rows(M, N) || (M <= 4 && goes_on(N, K))) {
       if (M == 1) return launch_rows<1>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       if (M == 2) return launch_rows<2>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+      if (M == 3) return launch_rows<3>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       if (M <= 4) return launch_rows<4>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       return launch_rows<8>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
     }
