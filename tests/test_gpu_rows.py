@@ -143,3 +143,14 @@ def test_few_rows_by_many_outputs(ops, M, N, K, accumulate):
     want = a[:M].double() @ w.double().t() + (start[:M].double() if accumulate else 0.0)
     size = a[:M].double().abs() @ w.double().abs().t() + (start[:M].double().abs() if accumulate else 0.0)
     assert bool(((few.double() - want).abs() <= (K / 64 + 18) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,H", [(1, 1), (1, 4096), (3, 1023), (2, 1028), (40, 2050), (300, 4100)])
+def test_rows_of_the_table(ops, dtype, n, H):
+    g = torch.Generator(device=DEV).manual_seed(H)
+    table = torch.randn(50, H, generator=g, device=DEV).to(dtype)
+    ids = torch.randint(0, 50, (n,), generator=g, device=DEV, dtype=torch.int32)
+    out = torch.full((n, H), float("nan"), device=DEV)
+    ops.embed(table, ids, out, 1.5)
+    assert torch.equal(out, table[ids.long()].float() * 1.5)

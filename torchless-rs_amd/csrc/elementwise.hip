@@ -16,13 +16,26 @@ void set_error(const char* fmt, ...) {
 
 // ---- embedding: out[n, :] = table[ids[n], :] * scale ---------------------------
 // src/model/modules/embedding.rs:15-21 of the reference (which has no scaling: scale 1).
+// Four channels a thread where rows are aligned for it, a row over several workgroups: a step of one row waits for one load of
+// the table and not for 16 in turn.  Bfloat16 rows of 4,096, before and now: one row 3.3 and 2.0 us
+// (a launch of nothing 1.9), 2,348 rows 14.8 and 9.6.
+__device__ __forceinline__ f32x4 row4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 row4(const bf16* p) {
+  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+  return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
 template <typename T>
-__global__ void embed_kernel(const T* __restrict__ table, const int* __restrict__ ids, int H, float scale,
-                             float* __restrict__ out) {
+__global__ void __launch_bounds__(256)
+embed_kernel(const T* __restrict__ table, const int* __restrict__ ids, int H, float scale, bool vec, float* __restrict__ out) {
   const int n = blockIdx.x;
   const T* row = table + (size_t)ids[n] * H;
   float* o = out + (size_t)n * H;
-  for (int i = threadIdx.x; i < H; i += blockDim.x) o[i] = to_f32(row[i]) * scale;
+  const long at = blockIdx.y * 256 + threadIdx.x;
+  if (vec) {
+    for (long i = at * 4; i < H; i += gridDim.y * 1024) *reinterpret_cast<f32x4*>(o + i) = row4(row + i) * scale;
+  } else {
+    for (long i = at; i < H; i += gridDim.y * 256) o[i] = to_f32(row[i]) * scale;
+  }
 }
 
 // The same with a second table read by pairs of tokens, and a norm of the sum: row (previous * mul_prev + current * mul_cur)
@@ -37,11 +50,6 @@ struct PairTerms {
   int* last;
   long long buckets, mul_prev, mul_cur;
 };
-__device__ __forceinline__ f32x4 row4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-__device__ __forceinline__ f32x4 row4(const bf16* p) {
-  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
-  return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-}
 template <typename T, int IT>
 __global__ void __launch_bounds__(256)
 embed_pairs_kernel(const T* __restrict__ table, const int* __restrict__ ids, int H, float scale, const T* __restrict__ pairs, PairTerms k,
@@ -777,16 +785,17 @@ act_mul_kernel(const float* __restrict__ gu, int I, int act, ActConstants k, boo
   const int n = blockIdx.x;
   const float* row = gu + (size_t)n * 2 * I;
   TO* o = out + (size_t)n * I;
-  for (long i = (blockIdx.y * 256 + threadIdx.x) * 4; i < I; i += gridDim.y * 1024) {
-    if (vec) {
-      const f32x4 g = *reinterpret_cast<const f32x4*>(row + i), u = *reinterpret_cast<const f32x4*>(row + I + i);
-      __attribute__((ext_vector_type(4))) TO h;
+  const long at = blockIdx.y * 256 + threadIdx.x;
+  if (!vec) {
+    for (long i = at; i < I; i += gridDim.y * 256) o[i] = from_f32<TO>(gate_times_up(row[i], row[I + i], act, k));
+    return;
+  }
+  for (long i = at * 4; i < I; i += gridDim.y * 1024) {
+    const f32x4 g = *reinterpret_cast<const f32x4*>(row + i), u = *reinterpret_cast<const f32x4*>(row + I + i);
+    __attribute__((ext_vector_type(4))) TO h;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = from_f32<TO>(gate_times_up(g[e], u[e], act, k));
-      *reinterpret_cast<decltype(h)*>(o + i) = h;
-    } else {
-      for (int e = 0; e < 4 && i + e < I; ++e) o[i + e] = from_f32<TO>(gate_times_up(row[i + e], row[I + i + e], act, k));
-    }
+    for (int e = 0; e < 4; ++e) h[e] = from_f32<TO>(gate_times_up(g[e], u[e], act, k));
+    *reinterpret_cast<decltype(h)*>(o + i) = h;
   }
 }
 
@@ -924,11 +933,12 @@ int tl_embed(const void* table, int table_dt, const int* ids, int n, int H, floa
              hipStream_t st) {
   TL_REQUIRE(n >= 0 && H > 0, "embed: bad sizes n=%d H=%d", n, H);
   if (n == 0) return 0;
-  const int nt = H >= 256 ? 256 : 64;
+  const bool vec = H % 4 == 0 && (uintptr_t)table % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const dim3 grid(n, (unsigned)min(((long)H + 1023) / 1024, 1024l));
   if (table_dt == DT_F32)
-    embed_kernel<float><<<n, nt, 0, st>>>((const float*)table, ids, H, scale, out);
+    embed_kernel<float><<<grid, 256, 0, st>>>((const float*)table, ids, H, scale, vec, out);
   else if (table_dt == DT_BF16)
-    embed_kernel<bf16><<<n, nt, 0, st>>>((const bf16*)table, ids, H, scale, out);
+    embed_kernel<bf16><<<grid, 256, 0, st>>>((const bf16*)table, ids, H, scale, vec, out);
   else
     TL_REQUIRE(false, "embed: unknown dtype code %d", table_dt);
   TL_LAUNCH_CHECK("embed");
