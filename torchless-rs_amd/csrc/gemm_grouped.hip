@@ -119,6 +119,13 @@ __device__ __forceinline__ int group_size(const Grouped& g, int x) { return x < 
 constexpr int GG_BM = 224, GG_BN = 256, GG_WN = 4, GG_NA = 2, GG_NW = 3;
 constexpr int GG_LDS = tile_lds<GG_WN, GG_BM / 32, GG_NA, GG_NW>();
 static_assert(GG_LDS <= 160 * 1024, "a compute unit's LDS");
+// Tiles of few positions wait for the weights: what A's ring does not need of the LDS goes to another stage of W under way.
+// A decode step of 19 rows of the 1,792-channel design (5 positions an expert): 1,343 us with the four-wave tiles, 1,380 to 1,404
+// with these and the rings of the large ones, 1,304 so; of 40 rows 1,429 with the four-wave tiles and 1,386.
+template <int MU> struct GGRings {
+  static constexpr int A = MU == 1 ? 4 : MU == 2 ? 3 : GG_NA, W = MU <= 2 ? 4 : GG_NW;
+  static_assert(tile_lds<GG_WN, MU, A, W>() <= GG_LDS, "the workgroup's LDS");
+};
 
 // A tile and its place.
 struct Tile {
@@ -159,7 +166,7 @@ __device__ __forceinline__ void gg_tile(const Grouped& g, const Tile& t, unsigne
   for (int u = 0; u < MU; ++u)
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[u][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  tile_loop<GG_WN, MU, GG_NA, GG_NW, 0>(smem, [&](int x, unsigned at) { return asrc[x] + at; }, [&](int x, unsigned at) { return wsrc[x] + at; }, t.K, 0,
+  tile_loop<GG_WN, MU, GGRings<MU>::A, GGRings<MU>::W, 0>(smem, [&](int x, unsigned at) { return asrc[x] + at; }, [&](int x, unsigned at) { return wsrc[x] + at; }, t.K, 0,
                                         (t.K + TILE_K - 1) / TILE_K, t.first, acc);
 
   // acc[u][v][r]: position 16 (wm MU + u) + li of the tile, row 64 wn + 16 v + 4 kg + r of W's tile
