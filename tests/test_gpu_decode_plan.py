@@ -123,7 +123,7 @@ def test_attention_in_planned_parts(ops, lengths, nq, nkv, d, window):
     assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs()) + 1e-5).all())
 
 
-@pytest.mark.parametrize("lengths", LENGTHS[:3])
+@pytest.mark.parametrize("lengths", [[1, 4200], [64, 65, 1, 4500, 129], [4300] + [130] * 30])
 @pytest.mark.parametrize("kind", ["sinks", "logistic", "kept", "chunk"])
 def test_attention_with_terms_in_planned_parts(ops, lengths, kind):
     nq, nkv, d = 8, 2, 128

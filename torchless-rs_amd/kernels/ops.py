@@ -644,7 +644,8 @@ def attention_scored(q, k_new, v_new, pages, nkv: int, dv: int, table, ring_page
             most_pages = min(most_pages, -(-terms.window // PAGE) + 1 + -(-int(terms.keep_first or 0) // PAGE))
         if terms.chunk:
             most_pages = min(most_pages, -(-terms.chunk // PAGE) + 1)
-        plan = decode_plan(ctx, nq, nkv, dk, table.shape[1], terms.window, int(terms.keep_first or 0), terms.chunk)
+        # (layers with terms are often few and each sort has a plan of its own: two layers over 256 to 2,048 keys lose 1 % of a step)
+        plan = decode_plan(ctx, nq, nkv, dk, table.shape[1], terms.window, int(terms.keep_first or 0), terms.chunk, least=64)
         if plan is not None:
             attn_decode_planned(q, pages, table, ring_pages, ctx, plan, terms.window, terms.scale, out, terms, gate)
             return
@@ -2569,12 +2570,15 @@ def decode_rounds(B: int, nq: int, nkv: int, units: int, head_dim: int):
     return places, (1 if 3 * B <= places else 3)
 
 
-def decode_plan(ctx, nq: int, nkv: int, d: int, table_width: int, window: Optional[int], keep_first: int = 0, chunk: int = 0):
+def decode_plan(ctx, nq: int, nkv: int, d: int, table_width: int, window: Optional[int], keep_first: int = 0, chunk: int = 0,
+                least: int = SPLIT_PAGES):
     """The plan of a single-token step's parts for layers of these sizes, made by the first of them (one small kernel, 4 us) and kept
-    while the step runs: (plan int32 [places, 4], seqs int32 [B, 2]), or None."""
+    while the step runs: (plan int32 [places, 4], seqs int32 [B, 2]), or None.  Tables of up to `least` pages go without:
+    up to SPLIT_PAGES the keys stay whole and there is no merge (19 sequences of 58 to 221 keys: 10.6 us, in parts 8.9 and 4.8 for the
+    merge)."""
     B = ctx.row_pos.shape[0]
     shape = decode_rounds(B, nq, nkv, compute_units(ctx.row_pos.device), d)
-    if shape is None or not lib().tl_attn_decode_takes_plan(d, int(table_width)):
+    if shape is None or table_width <= least or not lib().tl_attn_decode_takes_plan(d, int(table_width)):
         return None
     key = (shape, int(window or 0), int(keep_first) if window else 0, int(chunk or 0))
     plans = ctx.host.setdefault("decode_plans", {})
