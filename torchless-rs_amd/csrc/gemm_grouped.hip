@@ -120,8 +120,8 @@ constexpr int GG_BM = 224, GG_BN = 256, GG_WN = 4, GG_NA = 2, GG_NW = 3;
 constexpr int GG_LDS = tile_lds<GG_WN, GG_BM / 32, GG_NA, GG_NW>();
 static_assert(GG_LDS <= 160 * 1024, "a compute unit's LDS");
 // Tiles of few positions wait for the weights: what A's ring does not need of the LDS goes to another stage of W under way.
-// A decode step of 19 rows of the 1,792-channel design (5 positions an expert): 1,343 us with the four-wave tiles, 1,380 to 1,404
-// with these and the rings of the large ones, 1,304 so; of 40 rows 1,429 with the four-wave tiles and 1,386.
+// A decode step of 19 rows of the 1,792-channel design (5 positions an expert): with the rings of the large tiles 3 % behind the
+// four-wave tiles (1,404 against 1,364 us in one run), so 3 % ahead (1,304 against 1,343 in another); of 40 rows 1,386 against 1,429.
 template <int MU> struct GGRings {
   static constexpr int A = MU == 1 ? 4 : MU == 2 ? 3 : GG_NA, W = MU <= 2 ? 4 : GG_NW;
   static_assert(tile_lds<GG_WN, MU, A, W>() <= GG_LDS, "the workgroup's LDS");
