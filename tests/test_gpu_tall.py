@@ -89,9 +89,9 @@ def test_paired(ops, act, M, I, K, plan):
 def test_plans_fit_what_they_are_for(ops):
     """Every plan of the rule can be launched: K's slices all have stages, whole tiles are rounds of workgroups, partial sums are
     made only where they are welcome, nothing is planned up to MID_ROWS rows or for sizes the tiles do not take."""
-    for N, K in ((28672, 4096), (4096, 14336), (5120, 14336), (18560, 4096), (64, 64), (12288, 4104), (4096, 4096), (2048, 8192)):
+    for N, K in ((28672, 4096), (4096, 14336), (5120, 14336), (18560, 4096), (64, 64), (12288, 4104), (4096, 4096), (2048, 8192), (65536, 16384)):
         for M in list(range(129, 700, 37)) + [1024, 1999, 2048, 4097, 16384]:
-            for kind, sums in (("store", False), ("add", False), ("add", True), ("pair", False)):
+            for kind, sums in (("store", False), ("add", False), ("add", True), ("pair", False), ("act", False)):
                 p = ops.tall_plan(M, N, K, 256, kind, sums)
                 if p is None:
                     continue
@@ -146,3 +146,18 @@ def test_an_experts_activation(ops, act, M, I, K, plan, weighted):
     out = torch.full((M, I), float("nan"), device=DEV, dtype=torch.bfloat16)
     ops.gemm_tall_act(a, w, out, ops.TallPlan(*plan), row_weight=factor, **kw)
     assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + top) * (1.0 + top)).all())
+
+
+@pytest.mark.parametrize("M,I,K,plan", [(513, 32768, 16384, (256, 256)), (130, 131072, 16384, (192, 128)), (130, 131072, 16384, (224, 256, 1, False, 512, 2))])
+def test_gate_and_up_rows_that_lie_gigabytes_apart(ops, M, I, K, plan):
+    """2^30 and 2^32 bytes between a gate row and its up row; the bound is `test_an_experts_activation`'s, checked at the ends and in the middle."""
+    g = torch.Generator(device=DEV).manual_seed(I)
+    a, w = (torch.randn(M, K, generator=g, device=DEV) * K ** -0.5).bfloat16(), torch.randn(2 * I, K, generator=g, device=DEV, dtype=torch.bfloat16)
+    out = torch.full((M, I), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.gemm_tall_act(a, w, out, ops.TallPlan(*plan), terms=ops.GateTerms(3.0, 1.0, 0.0, float("inf"), True))
+    for c in (0, I // 2 - 96, I - 96):
+        p, u = a.double() @ w[c:c + 96].double().t(), a.double() @ w[I + c:I + c + 96].double().t()
+        want = torch.nn.functional.silu(p) * u
+        top = float(torch.maximum(p.abs(), u.abs()).max())
+        assert bool(((out[:, c:c + 96].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + top) * (1.0 + top)).all())
+    assert bool(torch.isfinite(out.float()).all())

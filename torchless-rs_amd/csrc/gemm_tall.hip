@@ -35,17 +35,18 @@ __device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, li = lane % 16, kg = lane / 16;
   const int wm = wave / WN, wn = wave % WN, sub = lane / 8;
   const int t0 = blockIdx.y * g.stages, n_t = min((g.K + TILE_K - 1) / TILE_K - t0, g.stages);
-  // a lane's rows as distances from the tile's first: at most 256 rows of K
+  // a lane's rows as distances from the first of the tile's that its wave loads: at most 256 rows of K.  Gate and up rows that lie
+  // apart go by 32 in turn, four waves' loads each: of all its loads a wave has gate rows or up rows.
   const char* A0 = reinterpret_cast<const char*>(g.A + (size_t)m0 * g.lda);
   const bool apart = g.epi == TALL_GATED;
-  const char* W0 = reinterpret_cast<const char*>(g.W + (size_t)(apart ? n0 / 2 : n0) * g.ldw);
+  const char* W0 = reinterpret_cast<const char*>(g.W + (size_t)(apart ? n0 / 2 + (wave & 4 ? g.N / 2 : 0) : n0) * g.ldw);
   unsigned aoff[S::A_PER], woff[S::W_PER];
 #pragma unroll
   for (int x = 0; x < S::A_PER; ++x) aoff[x] = (unsigned)min(tile_load<S::A_LOADS>(wave, x) * 8 + sub, m_rows - 1) * (unsigned)g.lda * 2u;
 #pragma unroll
   for (int x = 0; x < S::W_PER; ++x) {
     const int c = min((wave + TILE_WAVES * x) * 8 + sub, g.N - 1 - n0);
-    woff[x] = (unsigned)(apart ? c / 64 * 32 + c % 32 + (c & 32 ? g.N / 2 : 0) : c) * (unsigned)g.ldw * 2u;
+    woff[x] = (unsigned)(apart ? c / 64 * 32 + c % 32 : c) * (unsigned)g.ldw * 2u;
   }
 
   f32x4 acc[MU][4];
@@ -202,7 +203,6 @@ static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipSt
   TL_REQUIRE(!stagger || (n_split == 1 && K % TILE_K == 0), "gemm_tall: stages in turn need K=%d uncut and a multiple of %d", K, TILE_K);
   TL_REQUIRE(parts == 0 || ((parts == 2 || parts == 4) && n_split == 1 && channels == 256 && !once && !stagger && whole >= 0),
              "gemm_tall: tiles in %d parts (2 or 4, of 256 channels, K not cut)", parts);
-  TL_REQUIRE(epilogue != TALL_GATED || (long)N * ldw < (1l << 30), "gemm_tall: gate and up rows of %d x %d lie too far apart", N, ldw);
   g.stages = per;
 #define TL_TALL(R, CH, WN, MU, NA, NW)                                                         \
   if (rows == R && channels == CH) {                                                           \
