@@ -318,3 +318,33 @@ def test_tiles_of_every_height(ops, positions, H, ff, gated):
     z = torch.empty(n, H, device=DEV)
     ops.grouped_down(h, down, E, 0, 0, 1, off, z)
     assert bool(((z.double() - z_want).abs() <= (ff + 8) * 2.0 ** -24 * z_size + 1e-30).all())
+
+
+@pytest.mark.parametrize("on_input", [False, True])
+@pytest.mark.parametrize("n,shared", [(40, 0), (300, 304), (700, 0)])
+def test_a_gated_experts_epilogue_has_the_bits_of_the_activation(ops, n, shared, on_input):
+    """What a tile does with its sums is what the activation's own kernel makes of the same sums stored (K's stages in one order in
+    both), far from 0 too: pre-activations reach 20 and the clamp is off for the experts."""
+    H, E, top, ff = 136, 4, 2, 264
+    slices = ops.shared_slices(ff, shared) if shared else 0
+    g = torch.Generator(device=DEV).manual_seed(n)
+    up = (torch.randn(2 * (E * ff + shared), H, generator=g, device=DEV) * 5.0 * H ** -0.5).bfloat16()
+    y = torch.randn(n, H, generator=g, device=DEV).bfloat16()
+    weights, sw = torch.rand(n, E, generator=g, device=DEV) + 0.5, torch.rand(n, generator=g, device=DEV)
+    off, order, place = grouped(ops, choose(n, E, top, n, False), E)
+    terms = ops.GateTerms(float("inf"), 1.702, 1.0, 7.0, on_input)
+    h = torch.zeros(n * (top + slices), ff, dtype=torch.bfloat16, device=DEV)
+    ops.grouped_up(y, up, ff, shared, slices, off, order, top, weights, h, terms=terms, shared_weight=sw)
+    bounds = off.tolist()
+    for e in range(E):
+        rows = order[bounds[e]:bounds[e + 1]].long() // top
+        u, want = torch.empty(len(rows), 2 * ff, device=DEV), torch.empty(len(rows), ff, dtype=torch.bfloat16, device=DEV)
+        ops.gemm_tall_bf16(y[rows].contiguous(), up[2 * e * ff:2 * (e + 1) * ff], u, ops.TallPlan(224, 256))
+        ops.expert_gated_act(u, weights[rows, e:e + 1].contiguous(), 1, ff, 0, terms, want)
+        assert torch.equal(h[bounds[e]:bounds[e + 1]], want)
+    if shared:
+        u, want = torch.empty(n, 2 * shared, device=DEV), torch.empty(n, shared, dtype=torch.bfloat16, device=DEV)
+        ops.gemm_tall_bf16(y, up[2 * E * ff:], u, ops.TallPlan(224, 256))
+        ops.expert_gated_act(u, None, 0, 0, shared, terms, want, sw)
+        mine = torch.cat([h[n * (top + j):n * (top + j + 1)] for j in range(slices)], dim=1)[:, :shared]
+        assert torch.equal(mine, want)

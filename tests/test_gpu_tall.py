@@ -161,3 +161,17 @@ def test_gate_and_up_rows_that_lie_gigabytes_apart(ops, M, I, K, plan):
         top = float(torch.maximum(p.abs(), u.abs()).max())
         assert bool(((out[:, c:c + 96].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + top) * (1.0 + top)).all())
     assert bool(torch.isfinite(out.float()).all())
+
+
+@pytest.mark.parametrize("limit,alpha,shift", [(7.0, 1.702, 1.0), (float("inf"), 1.0, 0.0)])
+@pytest.mark.parametrize("M,I,K,plan", [(129, 160, 136, (192, 128)), (520, 672, 128, (256, 256, 1, False, 8, 2)), (520, 672, 128, (192, 256, 1, False, 8, 4))])
+def test_a_gated_epilogue_has_the_bits_of_the_activation(ops, M, I, K, plan, limit, alpha, shift):
+    """As the activation's own kernel makes of the same sums stored, far from 0 too (pre-activations reach 20)."""
+    a, w, _, _ = operands(M, 2 * I, K)
+    a = (a.float() * 4.0 * K ** -0.5).bfloat16()
+    terms, sw = ops.GateTerms(limit, alpha, shift, None, False), torch.rand(M, device=DEV)
+    u, want, out = torch.empty(M, 2 * I, device=DEV), *(torch.empty(M, I, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.gemm_tall_bf16(a, w.contiguous(), u, ops.TallPlan(*plan[:2]))
+    ops.expert_gated_act(u, None, 0, 0, I, terms, want, sw)
+    ops.gemm_tall_act(a, w.contiguous(), out, ops.TallPlan(*plan), terms=terms, row_weight=sw)
+    assert torch.equal(out, want)

@@ -39,17 +39,4 @@ __device__ __forceinline__ float gated_value(float g, float u, float s, float li
   return k.on_input ? a : a * s;
 }
 
-// The same where the result is rounded to bfloat16 (2^-9 of it) and a lane has many: the logistic function by the exponential and
-// reciprocal instructions, 2^-20 of the value or nearer.
-__device__ __forceinline__ float gated_value_near(float g, float u, float s, float limit, const GateTerms& k) {
-  if (k.on_input) {
-    g *= s;
-    u *= s;
-  }
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  const float a = g * __builtin_amdgcn_rcpf(1.0f + __expf(-k.alpha * g)) * (u + k.shift);
-  return k.on_input ? a : a * s;
-}
-
 }  // namespace tl

@@ -214,7 +214,7 @@ __device__ __forceinline__ void gg_tile(const Grouped& g, const Tile& t, unsigne
           if (n >= t.N) continue;
           bf16x4 h;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) h[r] = (bf16)(gated_value_near(acc[u][v][r], acc[u][v + 1][r], s[u], slice ? g.gate.limit_shared : g.gate.limit, g.gate) * after[u]);
+          for (int r = 0; r < 4; ++r) h[r] = (bf16)(gated_value(acc[u][v][r], acc[u][v + 1][r], s[u], slice ? g.gate.limit_shared : g.gate.limit, g.gate) * after[u]);
           *reinterpret_cast<bf16x4*>(out + n) = h;
         }
       }

@@ -73,7 +73,7 @@ __device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int
         bf16x4 h;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          h[r] = (bf16)(apart ? gated_value_near(acc[u][v][r], acc[u][v + 2][r], 1.f, g.gate.limit_shared, g.gate) * after
+          h[r] = (bf16)(apart ? gated_value(acc[u][v][r], acc[u][v + 2][r], 1.f, g.gate.limit_shared, g.gate) * after
                               : pair_value_near(acc[u][v][r], acc[u][v + 2][r], g.epi));
         *reinterpret_cast<bf16x4*>(out + n) = h;
       }
