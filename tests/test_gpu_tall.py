@@ -175,3 +175,14 @@ def test_a_gated_epilogue_has_the_bits_of_the_activation(ops, M, I, K, plan, lim
     ops.expert_gated_act(u, None, 0, 0, I, terms, want, sw)
     ops.gemm_tall_act(a, w.contiguous(), out, ops.TallPlan(*plan), terms=terms, row_weight=sw)
     assert torch.equal(out, want)
+
+
+def test_a_product_stored_in_bfloat16_is_the_librarys(ops):
+    """Products above MID_ROWS rows may be stored in bfloat16, also where float32 ones go in tiles: each sum, within `bound`, rounded
+    once to 8 bits."""
+    M, N, K = 1000, 14340, 2048
+    assert ops.tall_plan(M, N, K, 256, "store") is not None
+    a, w, want, size = operands(M, N, K)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.gemm(a, w.contiguous(), out)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 * bound(K, size)).all())

@@ -2235,7 +2235,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     if bf16_gemm_ok(a, w):
         if a.shape[0] > own_rows(a.shape[1]):
             plan = tall_plan(a.shape[0], w.shape[0], a.shape[1], compute_units(a.device), "add" if accumulate else "store")
-            if plan is not None and out.data_ptr() % 16 == 0:
+            if plan is not None and out.dtype == torch.float32 and out.data_ptr() % 16 == 0:
                 gemm_tall_bf16(a, w, out, plan, accumulate)
             else:
                 gemm_library(a, w, out, accumulate)
