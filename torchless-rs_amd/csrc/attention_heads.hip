@@ -177,10 +177,13 @@ int tl_head_prepare(const float* proj, int proj_stride, const int* row_pos, cons
   const Rotation rot{inv_freq, rotary_dim, 0};
   const HeadTerms t{bias, q_norm, k_norm, eps, mix, lambda, v_first, unit_norm, v_factor};
   const int units = nq + 2 * nkv + (ng + 255) / 256;
-  // units a wave: one up to 399 rows (32 + 8 + 8 heads at 200 rows 5.6 us, with two 4.9; at 64 rows 3.5 and 4.1), then a row in 200 more
-  // (600 rows 10.8 with three, 12.1 with one), at most 8 (2,348 rows 35.0, with four 36.2)
-  const int each = max(1, min(n / 200, 8));
-  const dim3 grid(n, (units + 4 * each - 1) / (4 * each));     // 8 workgroups a compute unit, or a head a wave
+  // units a wave: as many as leave 7 workgroups a compute unit, up to three; from 800 rows on a row in 200, at most 8.  32 + 8 + 8 heads of
+  // 128 with 32 gates, one / two / three units: 100 rows 3.8 / 4.2 / 4.5 us, 150 4.5 / 4.4 / 4.7, 200 5.4 / 4.8 / 5.1, 300 6.8 / 6.6 / 6.2, 600
+  // 11.4 / 10.3 / 9.9 (2,348 rows with three 34.8, with eight 33.1); 64 + 8 + 8 of 256 at 150 rows 10.6 / 8.8 / 9.2; 16 + 2 + 2 of 64
+  // at 256 rows 3.8 / 4.0 / 4.7; with 4,096 gates, whose units are short, at 130 rows 5.8 / 6.2 and at 256 8.9 / 9.0 / 8.0
+  const long workgroups = ((long)n * units + 3) / 4;
+  const int each = max((int)min((workgroups + 1791) / 1792, 3l), min(n / 200, 8));
+  const dim3 grid(n, (units + 4 * each - 1) / (4 * each));
 #define TL_HP(T, J)                                                                                                          \
   head_prepare_kernel<T, J><<<grid, 256, 0, st>>>(proj, proj_stride, row_pos, rot, t, nq, nkv, dk, dv, ng, (T*)q, (T*)k, (T*)v, gate, \
                                                   table, table_stride, ring_pages, (T*)pages)
