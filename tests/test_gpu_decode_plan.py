@@ -154,3 +154,47 @@ def test_who_goes_without_a_plan(ops):
         assert ops.decode_plan(ctx, 4, 2, 64, 8, None) is None
     finally:
         ops.decode_through_lds(was)
+
+
+@pytest.mark.parametrize("window", [None, 512])
+def test_replayed_steps_are_planned_by_their_own_lengths(tmp_path, ops, window):
+    """A captured step of two sequences over 11 pages makes its plan at every replay: the sequences change places in the batch and
+    grow over page boundaries, with eager work and synchronisations between the replays, and every step has the bits of an
+    engine that never captures, and float64's logits at the format's tolerance."""
+    import plain_mistral as plain
+    from torchless_rs_amd import write_random_model
+    from torchless_rs_amd.engine import Engine, SeqInput, load_model
+    from util import TOL, prompts, read_model_dir, rel_err
+    cfg = {"architectures": ["MistralForCausalLM"], "model_type": "mistral", "hidden_size": 256, "num_hidden_layers": 2, "num_attention_heads": 4, "num_key_value_heads": 2, "head_dim": 64,
+           "intermediate_size": 256, "vocab_size": 300, "rope_theta": 10000.0, "sliding_window": window, "rms_norm_eps": 1e-5,
+           "max_position_embeddings": 4096, "tie_word_embeddings": False, "hidden_act": "silu"}
+    mdir = write_random_model(str(tmp_path / "m"), cfg, seed=6, std=0.05, norm_std=0.1, dtype=torch.bfloat16)
+    cfgd, w = read_model_dir(mdir)
+    model = load_model(mdir, "bfloat16")
+    ids = prompts(cfg["vocab_size"], [700, 700, 700], seed=9)
+    at = [641, 20, 310]                                       # the first goes on inside its 11th page throughout
+    engines = [Engine(model, max_tokens=64 * 48, max_slots=4, use_graphs=g) for g in (True, False)]
+    for eng in engines:
+        eng.slots_ = [eng.alloc() for _ in ids]
+        eng.step([SeqInput(s, p[:n], []) for s, p, n in zip(eng.slots_, ids, at)])
+    planned = 0
+    for t in range(36):
+        pair = [(0, 1), (1, 0), (0, 2), (2, 0)][t % 4]
+        outs = []
+        for eng in engines:
+            outs.append(eng.step([SeqInput(eng.slots_[i], [ids[i][at[i]]], [0]) for i in pair]).clone())
+            if t % 5 == 0:
+                extra = eng.alloc()
+                eng.step([SeqInput(extra, ids[1][:100 + t], [0])])
+                eng.free(extra)
+            torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]), t
+        for row, i in enumerate(pair):
+            if t % 9 == 0:
+                assert rel_err(outs[0][row:row + 1], plain.forward(w, cfgd, ids[i][:at[i] + 1])[-1:]) < TOL["bfloat16"], (t, i)
+            at[i] += 1
+    for g in engines[0]._graphs.values():
+        planned += g.graph is not None and any(name.startswith("attn_plan_") for name in g.workspace._bufs)
+    assert planned and not engines[1]._graphs
+    for eng in engines:
+        eng.close()
