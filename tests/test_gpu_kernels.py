@@ -1521,3 +1521,31 @@ def test_products_into_the_stream_around_the_wide_rows(M, N, K, sliced):
     assert (ctx.pending is not None) == sliced
     flush_pending(ctx, x)
     assert bool(((x.double() - want).abs() <= 8 * K ** 0.5 * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("waves,kc", [(4, 128), (7, 128), (8, 128), (4, 64), (8, 64)])
+@pytest.mark.parametrize("M,N,K", [(17, 2100, 2048), (64, 520, 4096), (128, 4360, 2048), (40, 1096, 6144)])
+def test_gemm_ring_begins_with_other_stages(ops, waves, kc, M, N, K):
+    """K uncut and a multiple of 2,048: workgroups of other channels begin with other stages and go round, more workgroups than stages and
+    fewer, the last with channels missing; stored, accumulated and paired against float64.  The bound of a sum: as in
+    `test_wide_products_in_slices_of_K`; the paired results are rounded once more, by up to 2^-8 of themselves."""
+    a, w = rnd(M, K, seed=57, dtype=torch.bfloat16).to(DEV), rnd(N, K, seed=58, dtype=torch.bfloat16).to(DEV)
+    want, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    bound = 8 * K ** 0.5 * 2.0 ** -24 * size
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm_ring_bf16(a, w, out, waves=waves, kc=kc)
+    assert bool(((out.double() - want).abs() <= bound).all())
+    base = rnd(M, N, seed=59).to(DEV)
+    acc = base.clone()
+    ops.gemm_ring_bf16(a, w, acc, accumulate=True, waves=waves, kc=kc)
+    total = want + base.double()
+    assert bool(((acc.double() - total).abs() <= bound + 2.0 ** -23 * total.abs()).all())
+    if waves % 4 == 0:
+        wide = N // 64 * 64
+        w = (w[:wide].float() * K ** -0.5).bfloat16()
+        p = (a.double() @ w.double().t()).view(M, wide // 64, 2, 32)
+        gate, up = (t.reshape(M, wide // 2) for t in p.unbind(2))
+        h = torch.full((M, wide // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.gemm_ring_bf16(a, w, h, silu_pair=True, waves=waves, kc=kc)
+        ref = torch.nn.functional.silu(gate) * up
+        assert bool(((h.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * (1.0 + p.abs().max()) ** 2).all())
