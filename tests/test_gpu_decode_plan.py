@@ -111,7 +111,7 @@ LENGTHS = [[1, 700], [64, 65, 1, 1500, 129], [2048] + [130] * 30, [3000, 1, 500,
 @pytest.mark.parametrize("nq,nkv,d", [(8, 2, 128), (32, 8, 64), (12, 3, 128), (4, 1, 256), (40, 2, 64)])
 @pytest.mark.parametrize("window", [None, 300])
 def test_attention_in_planned_parts(ops, lengths, nq, nkv, d, window):
-    """The weights go to the second product with 8 bits and so does the result: 2^-9 of the sum of sizes and of itself; twice that."""
+    """The weights go to the second product with 8 bits and so does the result: up to 2^-8 of the sum of sizes and of itself."""
     q, pages, table, ctx = step(ops, lengths, nq, nkv, d)
     out = torch.full_like(q, float("nan"))
     planned = ops.decode_plan(ctx, nq, nkv, d, table.shape[1], window)

@@ -77,7 +77,7 @@ def test_heads_of_many_rows_are_those_of_few(ops, dtype, dk, dv, rotary):
             x = torch.cat([u * angle.cos() - w * angle.sin(), u * angle.sin() + w * angle.cos(), x[..., rotary:]], -1)
         if kw.get("unit_norm"):
             x = x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt()
-        # float32: a few roundings of 2^-24 of the two products of a rotated channel; bfloat16: one of 2^-9 of the result
+        # float32: a few roundings of 2^-24 of the two products of a rotated channel; bfloat16: one of up to 2^-8 of the result
         tol = 4e-6 * (1.0 + x.abs().amax(-1, keepdim=True)) + (2.0 ** -8 * x.abs() if dtype == torch.bfloat16 else 0.0)
         assert bool(((torch.cat(many[:2], 1).double() - x).abs() <= tol).all())
 

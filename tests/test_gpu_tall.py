@@ -64,8 +64,8 @@ def test_last_tiles_in_parts(ops, tile, parts, M, N):
 @pytest.mark.parametrize("M,I,K,plan", [(129, 32, 64, (192, 128)), (300, 96, 264, (160, 256)), (520, 672, 128, (256, 256, 1, False, 8, 2)),
                                         (520, 672, 128, (192, 256, 1, False, 8, 4))])
 def test_paired(ops, act, M, I, K, plan):
-    """act(gate) * up of the sums, rounded to bfloat16 once (2^-9 of itself); the sums' error and the exponential's, 2^-20, pass
-    through functions whose slope is near 1 or below, times the other factor: 1e-5 of the sums' sizes covers both."""
+    """act(gate) * up of the sums, rounded to bfloat16 once (up to 2^-8 of itself); the sums' error and the exponential's, (8 + 1.5 |g|) 2^-24
+    of the value, pass through functions whose slope is near 1 or below, times the other factor: 1e-5 of the sums' sizes covers both."""
     a, w, p, size = operands(M, 2 * I, K)
     a, p, size = a * K ** -0.5, p * K ** -0.5, size * K ** -0.5
     p = a.double() @ w.double().t()
@@ -186,3 +186,23 @@ def test_a_product_stored_in_bfloat16_is_the_librarys(ops):
     out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
     ops.gemm(a, w.contiguous(), out)
     assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 * bound(K, size)).all())
+
+
+def test_the_paired_silu_far_from_zero(ops):
+    """Gates down to -100 on sums that are exact (one product of each row counts): the exponential and reciprocal instructions are within
+    (8 + 1.5 |g|) 2^-24 of the value, whose rounding to 8 bits, half a unit of the last, is up to 2^-8 of itself; below -87 the value is under 2^-119 of the up sum and
+    may be 0."""
+    M, I, K = 256, 512, 64
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
+    a[torch.arange(M, device=DEV), torch.arange(M, device=DEV) % K] = 1.0
+    gate = (torch.rand(I, K, generator=g, device=DEV) * 140.0 - 100.0).bfloat16()
+    gate[:4] = torch.tensor([-20.0, -60.0, -87.0, -88.0], device=DEV)[:, None].bfloat16()
+    up = torch.randn(I, K, generator=g, device=DEV).bfloat16()
+    w = torch.stack([gate.view(I // 32, 32, K), up.view(I // 32, 32, K)], dim=1).reshape(2 * I, K).contiguous()
+    out = torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.gemm_tall_bf16(a, w, out, ops.TallPlan(256, 256), silu_pair=True)
+    p, u = a.double() @ gate.double().t(), a.double() @ up.double().t()
+    want = p / (1.0 + torch.exp(-p)) * u
+    bound = (2.0 ** -8 + (8.0 + 1.5 * p.abs()) * 2.0 ** -24) * want.abs() + torch.where(p < -87.0, 2.0 ** -118 * u.abs(), 0.0)
+    assert bool(((out.double() - want).abs() <= bound).all())

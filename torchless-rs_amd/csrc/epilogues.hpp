@@ -38,8 +38,11 @@ __device__ __forceinline__ float pair_value(float g, float u, const Epi& e) {
   return (g / (1.0f + expf(-g))) * u;
 }
 
-// The same where the result is rounded to bfloat16 (2^-9 of it) and a lane has many: the logistic function by the exponential and
-// reciprocal instructions, 2^-20 of the value or nearer.  A tile of 256 x 256 sums takes 2 us of them, 6 with the functions above.
+// The same where the result is rounded to bfloat16 (up to 2^-8 of it) and a lane has many: the logistic function by the exponential and
+// reciprocal instructions.  The exponent's product is rounded before the exponential, so that the error grows with a negative g:
+// within (8 + 1.5 |g|) 2^-24 of the value (2^-20.7 near 0, 2^-18.5 at -22, 2^-16.9 at -87), and below -87.3, where the reciprocal's
+// sum passes 2^126, the result may be 0 for a value under 2^-119 |u|.  A product of the library's that is stored in bfloat16 ahead of
+// the activation rounds g and u to 2^-8 of themselves besides.  A tile of 256 x 256 sums takes 2 us of them, 6 with the functions above.
 __device__ __forceinline__ float pair_value_near(float g, float u, const Epi& e) {
   if (e.code == EPI_SILU_PAIR) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
   return pair_value(g, u, e);

@@ -186,7 +186,7 @@ using namespace tl;
 // A [M, K] with rows lda apart, W [N, K] with rows ldw apart; K, lda, ldw multiples of 8, N of 4 (with a paired epilogue of 64).
 // n_split == 1: C as in tl_gemm_bf16; more: C float [n_split][M][N] receives partial sums (epilogue 0), every split with one
 // stage of 64 k at least.  rows, channels: the tile, one of 256, 224, 192, 160 x 256 and 256, 192, 128 x 128.  once: W is read by
-// one tile of rows only (its loads are marked non-temporal); stagger: tiles of other channels begin with other stages of K
+// one tile of rows only (tiles of 128 channels mark its loads non-temporal; the rule has no such product in wider ones); stagger: tiles of other channels begin with other stages of K
 // (K a multiple of 64, not cut).  parts: 0, or 2 or 4 (tiles of 256 channels, K not cut): the tiles behind the first `whole`, a
 // multiple of 8, are cut into so many.
 static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipStream_t st) {
@@ -207,7 +207,7 @@ static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipSt
 #define TL_TALL(R, CH, WN, MU, NA, NW)                                                         \
   if (rows == R && channels == CH) {                                                           \
     if (parts) return launch_tall<4, MU, 2, 3, 0, true>(g, n_split, st);                       \
-    return once ? launch_tall<WN, MU, NA, NW, 2>(g, n_split, st) : launch_tall<WN, MU, NA, NW, 0>(g, n_split, st); \
+    return launch_tall<WN, MU, NA, NW, 0>(g, n_split, st);                                     \
   }
   TL_TALL(256, 256, 4, 8, 2, 3)
   TL_TALL(224, 256, 4, 7, 2, 3)
