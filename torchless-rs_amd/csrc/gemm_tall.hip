@@ -59,27 +59,31 @@ __device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int
 
   // acc[u][v][r]: row 16 (wm MU + u) + li of the tile, channel 64 wn + 16 v + 4 kg + r
   const int c0 = n0 + wn * 64 + kg * 4;
-  if (apart || is_pair(g.epi)) {               // a wave's 64 channels are 32 gate rows and their 32 up rows
+  // a wave's 64 channels are 32 gate rows and their 32 up rows; value(gate, up, row)
+  const auto paired = [&](auto value) {
 #pragma unroll
     for (int u = 0; u < MU; ++u) {
       const int m = (wm * MU + u) * 16 + li;
       if (m >= m_rows) continue;
       bf16* out = reinterpret_cast<bf16*>(g.C) + (size_t)(m0 + m) * (g.N / 2);
-      const float after = g.row_weight ? g.row_weight[m0 + m] : 1.f;
 #pragma unroll
       for (int v = 0; v < 2; ++v) {
         const int n = (n0 + wn * 64) / 2 + v * 16 + kg * 4;
         if (n >= g.N / 2) continue;
         bf16x4 h;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          h[r] = (bf16)(apart ? gated_value(acc[u][v][r], acc[u][v + 2][r], 1.f, g.gate.limit_shared, g.gate) * after
-                              : pair_value_near(acc[u][v][r], acc[u][v + 2][r], g.epi));
+        for (int r = 0; r < 4; ++r) h[r] = (bf16)value(acc[u][v][r], acc[u][v + 2][r], m0 + m);
         *reinterpret_cast<bf16x4*>(out + n) = h;
       }
     }
-    return;
-  }
+  };
+  // (apart from each other: chosen for every value, the long ones cost the short one 3 us a tile)
+  if (g.epi == EPI_SILU_PAIR) return paired([&](float x, float y, int) { return pair_value_near(x, y, Epi(EPI_SILU_PAIR)); });
+  if (is_pair(g.epi)) return paired([&](float x, float y, int) { return pair_value(x, y, g.epi); });
+  if (apart)
+    return paired([&](float x, float y, int m) {
+      return gated_value(x, y, 1.f, g.gate.limit_shared, g.gate) * (g.row_weight ? g.row_weight[m] : 1.f);
+    });
   if (g.epi == TALL_UNARY) {
 #pragma unroll
     for (int u = 0; u < MU; ++u) {
