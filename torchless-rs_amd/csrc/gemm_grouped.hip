@@ -228,7 +228,7 @@ __device__ __forceinline__ void gg_tile(const Grouped& g, const Tile& t, unsigne
 // Bound by the products' rate with the chip full, and with few positions an expert by the weights (5.7 TB/s at 130 rows).  16
 // experts, 4 a row, microseconds, up / down, before with four waves of 160 x 64, a wave alone on its SIMD: 3,584 channels at 600 rows
 // 125 / 188 and 110 / 113 now, 2,312 rows 381 / 325 and 287 / 272 (0.95 and 1.0 PFLOP/s), 8,192 rows 1,144 / 1,081 and 862 / 891
-// (1.1); 1,792 gated ones at 2,312 rows 386 / 183 and 280 / 142; 130 and 300 rows as they were.
+// (1.1); 1,792 gated ones at 2,312 rows 386 / 183 and 292 / 153; 130 and 300 rows as they were.
 template <int EPI>
 __global__ void __launch_bounds__(TILE_WAVES * WAVE)
 gemm_grouped_kernel(Grouped g) {

@@ -1928,7 +1928,7 @@ LIBRARY_ROWS = 64   # where K is no such multiple, the BLAS library's product be
 
 def own_rows(K: int) -> int:
     """The most rows for which a bfloat16 product over K always runs in this package's own kernels (of more, those that
-    `wide_splits` takes do; the others go to the BLAS library)."""
+    `tall_plan` or `wide_splits` takes do; the others go to the BLAS library)."""
     return MID_ROWS if K % RING_K == 0 else LIBRARY_ROWS
 
 
@@ -1994,17 +1994,18 @@ def gemm_mid_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: 
     _check(lib().tl_gemm_mid_bf16(_p(a), _p(w), _p(out), M, N, K, int(n_split), epi, _stream()))
 
 
-WIDE_ROWS = 256      # most rows of the kernel that cuts a product of more than MID_ROWS rows along K
+WIDE_ROWS = 256      # most rows of a product that `wide_splits` cuts along K
 
 
 def wide_splits(M: int, N: int, K: int, units: int) -> int:
     """For MID_ROWS + 1 .. WIDE_ROWS rows: into how many slices `gemm_wide_bf16` cuts K, as many as make one round of
-    workgroups of 128 channels over the `units` compute units, each with four stages of 64 k at least; 1 where the BLAS
-    library's product is to be taken: sizes that are no multiples of 64, and two slices or fewer, where the
-    channels come near to filling the units by themselves (192 rows, with the partial sums added / the library's, microseconds:
-    16,384 x 4,096 in 2 slices 51 / 48, 12,288 x 2,048 in 2 30 / 27, 10,240 x 8,192 in 3 61 / 77, 7,168 x 5,120 in 4 34 / 43);
-    and partial sums, written and read, of more than one and a half times the weights' bytes (4,096 x 4,096 in 8, 192 rows
-    23 / 34, 256 rows 27 / 24; 8,192 x 1,024 in 4, 192 rows 24 / 21)."""
+    workgroups of 128 channels over the `units` compute units, each with four stages of 64 k at least; 1 where a product goes
+    without (`Linear.add_into` then asks `tall_plan`, and takes the library's product if that has no plan either): sizes that are no
+    multiples of 64; two slices or fewer, where the channels come near to filling the units by themselves; and partial sums, written and
+    read, of more than one and a half times the weights' bytes.  Product and the norm behind it, weights from memory, in slices /
+    the library's, microseconds: 192 rows of 4,096 x 4,096 in 8 25 / 38, of 4,096 x 14,336 in 8 40 / 107 (256 rows 50 / 72), of
+    6,144 x 4,096 in 5 28.5 / 39, of 7,168 x 5,120 in 4 35 / 48; 8,192 x 4,096 in 4 at 144, 200 and 256 rows 30 / 32, 34 / 36 and 36 / 48;
+    not taken: 8,192 x 1,024 in 4 24 / 22, 4,096 x 1,792 in 6 at 256 rows 26 / 17, 4,096 x 4,096 in 8 at 256 rows 28 / 27."""
     if not (MID_ROWS < M <= WIDE_ROWS and N % 64 == 0 and K % 64 == 0):
         return 1
     stages = K // 64
@@ -2016,7 +2017,7 @@ def wide_splits(M: int, N: int, K: int, units: int) -> int:
 
 def gemm_wide_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int) -> None:
     """Partial sums out float32 [n_split, M, N] of the product of up to WIDE_ROWS rows, N and K multiples of 64, in tiles of all of
-    the rows by 128 channels.  192 rows in 8 slices: 4,096 x 14,336 37 us, in 256 rows 40; 4,096 x 4,096 17."""
+    the rows by 128 channels."""
     M, K = a.shape
     N = w.shape[0]
     if not (0 < M <= WIDE_ROWS and N % 64 == 0 and K % 64 == 0):
@@ -2047,18 +2048,21 @@ def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False)
     """How the product of more than MID_ROWS rows, [M, K] by [N, K], goes in tiles of this package's own, or None where the BLAS
     library's product is to be taken.  `kind`: "store" (float32), "add" (to float32) or "pair" (the activation of a paired
     product, which the library's needs a kernel of its own for), "act" (the activation of an expert, for which a stored product's
-    float sums are written and read once more: 14,336 x 4,096 gated at 2,348 rows 302, here 238; at 1,024
-    115 and 98; 7,168 x 4,096 of one argument at 2,348 161 and 134, at 512 45, here 81: the library's).  `sums`: partial sums over slices of K are welcome (the
-    next norm adds them).
+    float sums are written and read once more: 14,336 x 4,096 gated at 2,348 rows 295, here 255; at 1,024
+    126 and 108; 7,168 x 4,096 of one argument at 2,348 164 and 136, at 513 58, here 81: the library's).  `sums`: partial sums over
+    slices of K are welcome (the next norm adds them).
 
     The time of every way is reckoned from what was measured: rounds of workgroups over the compute units, each a few microseconds
     and its stages of K (`TALL_STAGE`); what does not fill a last round goes in halves or quarters of tiles.  Reckoned and
-    measured, microseconds: 28,672 x 4,096 paired 2,048 rows 375 / 368 (halves), 3,000 561 / 552 (quarters), 600 148 / 139;
-    18,560 x 4,096 1,536 rows 189 / 191; 4,096 x 14,336 in slices 1,024 rows 101 / 101, 2,048 182 / 184.  The library's:
-    with the activation's kernel about 1.15 PFLOP/s, or 0.95 up to 640 rows, and no faster than 3.2 TB/s of weights (28,672 x
-    4,096 at 226 rows 73, here 67; 2,048 381; 3,000 579; 28,672 x 5,120 at 1,024 283, here 241, at 2,048 519 and 459); added
-    to the stream 3 us + 3.65 ns K + 1.5 PFLOP/s (4,096 x 14,336 at 512 rows 93, here 62 and 5 to 8 more in the norm; at
-    1,024 133, here 101 and 10; 4,096 x 4,096 at 2,048 65, here 62 and 12: the library's); more rows, or stored, up to 1.43 PFLOP/s
+    measured (weights from memory, one call after the other), microseconds: 28,672 x 4,096 paired 2,048 rows 375 / 355 (halves), 3,000
+    561 / 518 (quarters), 600 148 / 136; in slices, without the norm, 4,096 x 14,336 1,024 rows 101 / 101, 2,048 182 / 184.  The library's:
+    with the activation's kernel about 1.15 PFLOP/s, or 0.95 up to 640 rows, and no faster than 3.2 TB/s of weights; measured,
+    28,672 x 4,096 in tiles / by the library: 300 rows 74 / 81, 600 136 / 147, 1,024 187 / 202, 1,536 280 / 286, 2,048 355 / 377, 2,500
+    443 / 468, 4,096 668 / 704, 6,000 1,007 / 1,156; 28,672 x 5,120: 1,024 234 / 281, 2,048 436 / 515, 4,096 836 / 916; near the edges of
+    the tiles' rows the line is late (768 rows, left to the library, 151 to 156 / 167).  Added to the stream
+    3 us + 3.65 ns K + 1.5 PFLOP/s (4,096 x 14,336 at 512 rows 93, here 62 and 5 to 8 more in the norm; at
+    1,024 133, here 101 and 10; 4,096 x 4,096 at 200 to 240 rows, 8 slices, a step 0.6 to 1.3 % ahead of the library's, at 256 rows,
+    6 slices, 0.5 % behind; at 2,048 65, here 62 and 12: the library's); more rows, or stored, up to 1.43 PFLOP/s
     where both sizes are multiples of 256, less where rows are not, the least where channels are not (12,288 x 4,096 at 1,024
     rows 82, here 89: the library's; 6,144 x 4,096 at 2,034 85, here 97: the library's; 14,336 x 4,096 at 3,220 432, here
     314; 18,560 x 4,096 at 2,312 386, here 305; 5,120 x 14,336 at 2,500 456, here 302)."""
@@ -2230,7 +2234,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
          tiles: Optional[torch.Tensor] = None) -> None:
     """out[M,N] (+)= a[M,K] @ w[N,K]^T with float32 accumulation.  The kernel
     follows from the operand types: bfloat16 x bfloat16 goes to the matrix
-    cores (our kernels up to `own_rows(K)` rows, the library's above), anything
+    cores (our kernels up to `own_rows(K)` rows; above, with a float32 result, our
+    tiles where `tall_plan` has a plan, else the library's), anything
     with float32 in it to the plain FMA kernel.  `tiles`: see `gemm_bf16`."""
     if bf16_gemm_ok(a, w):
         if a.shape[0] > own_rows(a.shape[1]):

@@ -33,8 +33,8 @@ reads every expert's weights in every step, as a step of many rows does anyway, 
 A step of more rows than the kernels for few rows take (`GROUPED_ROWS`, `GROUPED_SIZE`), in bfloat16, sorts
 the (row, chosen expert) pairs by expert and runs every expert's two products over its own rows
 (`_grouped`): the chosen experts' multiplications alone, in one launch for all experts, which finds
-its tiles on the device; the shared expert runs along as slices of an expert's size, or in steps of very
-many rows by the library's products.
+its tiles on the device; the shared expert runs along as slices of an expert's size, or in steps of
+many rows by products of its own.
 
 A step of few rows (rows * top <= n_experts: the rows cannot use every expert) runs the chosen
 experts alone: per row two products of its experts' matrices with a vector
@@ -55,23 +55,28 @@ from .base import FeedForward, flush_pending, register_part
 from .linear import Linear
 
 
-# When experts run over their own rows.  Measured with both ways round (microseconds, grouped / side by side): 16 experts of
-# 3,584 channels, 4 a row, a shared one of 7,168: 16 rows 231 / 198, 24 rows 229 / 464, 64 rows 238 / 544, 128 rows 277 / 827,
-# 511 rows 367 / 758; gated ones of 1,792: 16 rows 216 / 166, 24 rows 221 / 337, 128 rows 294 / 568; 64 experts of 256, 2 a row:
-# 32 rows 62 / 51, 48 rows 63 / 140.
+# When experts run over their own rows.  Measured with both ways round (a whole layer with its router, microseconds, grouped / side by
+# side): 16 experts of 3,584 channels, 4 a row, a shared one of 7,168: 16 rows 227 / 197, 24 rows 228 / 445, 64 rows 235 / 525,
+# 128 rows 258 / 811, 511 rows 369 / 735; gated ones of 1,792: 16 rows 146 / 141, 24 rows 141 / 251, 128 rows 153 / 440; 64 experts
+# of 256, 2 a row: 32 rows 56 / 57, 48 rows 70 / 141.
 GROUPED_ROWS = 16                  # up to here the kernels for few rows stream all experts' weights as fast as they come
 GROUPED_SIZE = 600000              # above, from this many rows times hidden channels of all experts
 GROUPED_ROWS_PER_EXPERT = 128      # or, above the own product kernels' rows, from this many rows an expert on average
-# Above the own product kernels' rows the wide form is the library's, whose time goes with the channels of all experts, where a tile of
-# an expert's rows goes through all of a row's channels in a chain: the experts' own rows pay from GROUPED_WIDTH channels (a gated
-# one counts twice) a channel of the row.  And an expert of few channels leaves its tile of 256 empty: below GROUPED_FF it takes
+# Above the own product kernels' rows the wide form is two products of all experts' channels (`tall_plan`'s or the library's), where a
+# tile of an expert's rows goes through all of a row's channels in a chain: the experts' own rows pay from GROUPED_WIDTH channels (a
+# gated one counts twice) a channel of the row.  And an expert of few channels leaves its tile of 256 empty: below GROUPED_FF it takes
 # GROUPED_FEW rows an expert.  Microseconds, wide / grouped, 16 experts, 4 a row, 4,096 channels a row: experts of 256, 200 rows
-# 65 / 114, 400 rows 77 / 134; of 512 79 / 92, 103 / 123; of 1,024 and a shared one 209 / 140; 8,192 a row and experts of 512
-# 129 / 166, of 1,024 230 / 227, of 2,048 479 / 280; 512 a row and experts of 512 63 / 42.  512 experts of 32, 8 a row, 1,024 a row:
-# 200 rows 254 / 279, 511 rows 286 / 283, 800 rows 353 / 320; 128 experts of 128 132 / 107 at 200 rows.
+# 59 / 87, 400 rows 73 / 106; of 512 85 / 95, 111 / 113; of 1,024 140 / 115, and a shared one 215 / 159; 8,192 a row and experts of
+# 512 135 / 177, of 1,024 224 / 227 (400 rows 297 / 254: the line could lie at 2 there), of 2,048 491 / 274; 512 a row and experts of
+# 512 37 / 35.  512 experts of 32, 8 a row, 1,024 a row: 200 rows 266 / 275, 511 rows 308 / 283 (the line a little late), 800 rows
+# 365 / 319; 128 experts of 128 144 / 118 at 200 rows.  Narrow experts lose behind GROUPED_ROWS_PER_EXPERT too: of 256 with a shared
+# one, 600 rows 97 / 152.
 GROUPED_WIDTH = 2.5
 GROUPED_FF, GROUPED_FEW = 64, 8
-SLICED_ROWS = 512                  # up to here a shared expert runs along as slices (1,024 rows: 215 us against 140 by the library)
+# Up to here a shared expert runs along as slices.  Slices / a product of its own (`tall_plan`'s "act"), a whole layer, microseconds: 16
+# experts of 3,584 and a shared one of 7,168 200 rows 291 / 267, 512 365 / 343, 1,024 538 / 510; gated of 1,792 and 7,168 256 rows 258 / 267,
+# 512 308 / 324, 1,024 501 / 489, 2,048 819 / 773; of 1,024 and 1,024 512 167 / 174, 2,048 269 / 297: neither is ahead throughout.
+SLICED_ROWS = 512
 
 
 class PlainFeedForward(FeedForward):
@@ -289,7 +294,7 @@ class RoutedExperts(FeedForward):
         weights, chosen, sw = self._route(ctx, y, True)
         up_w, down_w = self.up.weight, self.down.weight
         act = {"terms": self.gate_terms} if self.gated else {"activation": self.activation}
-        # the shared expert's slices write and read a row of float sums each, which the library's product of many rows does not
+        # the shared expert's slices write and read a row of float sums each, which a product of its own does not
         slices = ops.shared_slices(ff, self.shared) if self.shared and (n <= SLICED_ROWS or self.up.own_kernels(n)) else 0
         offsets = ws.get("experts_offsets", (E + 1,), torch.int32)
         order = ws.get("experts_order", (n * top,), torch.int32)

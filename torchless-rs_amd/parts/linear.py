@@ -80,8 +80,10 @@ class Linear:
         return parts
 
     def wide_partial(self, a: torch.Tensor, ctx, name: str):
-        """The same for MID_ROWS + 1..WIDE_ROWS rows, where the sums go to the stream: the next norm adds them as it reads.
-        (q|k|v of a prompt would need a pass of its own for that: 24 + 6 us for 226 rows of 6,144 x 4,096, the library's 26.)"""
+        """The same for MID_ROWS + 1..WIDE_ROWS rows, where the sums go to the stream: whoever reads it next adds them, a norm as it
+        reads or a pass of its own.  (q|k|v of a prompt would need such a pass: 24 + 6 us for 226 rows of 6,144 x 4,096, the
+        library's 26.)  This rule comes before `tall_partial`'s: it asks for no norm, and takes 144 to 256 rows of wide outputs and short K
+        that the other, which reckons times, leaves to the library (8,192 x 4,096 at 256 rows 36 us in four slices, 48 there)."""
         M, N, K = a.shape[0], self.out_features, self.in_features
         if not (ops.MID_ROWS < M <= ops.WIDE_ROWS and ops.bf16_gemm_ok(a, self.weight)):
             return None
@@ -93,8 +95,9 @@ class Linear:
         return parts
 
     def tall_partial(self, a: torch.Tensor, ctx, name: str):
-        """The same for more rows than that, or fewer slices, where a norm that adds such sums is announced as the stream's next
-        reader (without one they would take a pass of their own)."""
+        """The same for more rows than that, and for what `wide_splits` leaves (4,096 x 4,096 at 200 to 240 rows; outputs of few channels:
+        1,024 x 4,096 at 226 rows 17 us with the norm, the library's 19), where a norm that adds such sums is announced as the
+        stream's next reader (without one they would take a pass of their own)."""
         norm = ctx.norm_ahead
         if a.shape[0] <= ops.MID_ROWS or norm is None or not getattr(norm, "takes_pending", False) or not ops.bf16_gemm_ok(a, self.weight):
             return None
