@@ -1,4 +1,4 @@
-"""Products over each expert's own rows (csrc/gemm_grouped.hip) against float64, at the edges of its tiles: 160 positions,
+"""Products over each expert's own rows (csrc/gemm_grouped.hip) against float64, at the edges of its tiles: 224 positions,
 256 channels (128 gated ones), stages of 64 k."""
 import pytest
 import torch
