@@ -529,6 +529,31 @@ def test_rows_without_a_distribution(ops):
         assert ids[4] == 11 and float(probs[4, 11]) == 1.0
 
 
+@pytest.mark.parametrize("V,k", [(65537, 1), (65537, 256), (65542, 64), (73729, 128), (131072, 50), (131072, 129), (131071, 256),
+                                 (262144, 17), (262144, 256)])
+def test_rows_in_parts(ops, monkeypatch, V, k):
+    """Top-k over rows that several workgroups look through gives the bits of one workgroup a row: values anywhere, all of the largest in one part, more equal ones than a part's list holds, a masked row, NaN, infinities."""
+    z = rnd(7, V, seed=V + k, scale=2.5)
+    z[1, V - 300:] += 20.0
+    z[2] = 1.5
+    z[3] = (z[3] * 4).round() / 4
+    z[4] = -float("inf")
+    z[4, V // 2] = 0.25
+    z[5, V // 3] = float("nan")
+    z[6, 0] = float("inf")
+    counters = [[b, 3] for b in range(7)]
+    ids, probs = run_sample(ops, z, 0.7, k, 0.9, 23, counters)
+    assert ops.sample_lists(7, V, 0.7, k, DEV) is not None
+    monkeypatch.setattr(ops, "sample_lists", lambda *a: None)
+    one_ids, one = run_sample(ops, z, 0.7, k, 0.9, 23, counters)
+    assert ids == one_ids
+    assert torch.equal(probs.view(torch.int32), one.view(torch.int32))
+    for b in (0, 1, 2, 3):
+        want = vector_distribution(z[b], torch.tensor(0.7).double(), k, 0.9)
+        assert abs(int((probs[b] > 0).sum()) - int((want > 0).sum())) <= 1
+        assert float((probs[b].double() - want).abs().max()) < 2e-6 + float(want[want > 0].min()) * 2
+
+
 def test_draws_do_not_depend_on_batch_mates_and_follow_the_probabilities(ops):
     V = 8
     z = torch.tensor([[2.0, 1.0, 0.0, -1.0, 0.5, 1.5, -2.0, 0.2]])

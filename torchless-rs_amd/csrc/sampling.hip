@@ -134,6 +134,7 @@ struct SampleShared {
   unsigned long long hist[2048];
   unsigned long long scan[SNT / WAVE];
   unsigned long long above;
+  int reached[2][SNT / WAVE][16];
   int digit;
   int count;
   int pick;
@@ -144,6 +145,42 @@ struct SampleShared {
 __device__ __forceinline__ float from_order_key(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
 }
+// The largest multiple of 2^12 that at least k of the block's NT values reach (0 if there is none above it), four bits and one
+// barrier a round: 3.3 us over 1,024 threads.
+template <int NT> __device__ __forceinline__ uint32_t bound_of_kth(uint32_t mine, int k, int (*reached)[SNT / WAVE][16]) {
+  const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  uint32_t bound = 0u;
+#pragma unroll
+  for (int round = 0; round < 5; ++round) {
+    const int shift = 28 - 4 * round;
+    int c = 0;
+#pragma unroll
+    for (int j = 1; j < 16; ++j) {
+      const int n = __popcll(__ballot(mine >= (bound | (uint32_t)j << shift)));
+      if (lane == j) c = n;
+    }
+    if (lane < 16) reached[round % 2][w][lane] = c;
+    __syncthreads();                                    // (the other half is written before the next one, so one a round is enough)
+    int all = 0;
+#pragma unroll
+    for (int i = 0; i < NT / WAVE; ++i) all += reached[round % 2][i][lane % 16];
+    const unsigned long long enough = __ballot(lane > 0 && lane < 16 && all >= k);
+    if (enough) bound |= (uint32_t)(63 - __clzll((long long)enough)) << shift;
+  }
+  return bound;
+}
+// The passes over logits go by the logits themselves (a division is 14 instructions, 12 us a pass over 131,072): two logits whose
+// quotients round to one number lie within 2 units in the last place of each other, so 4 are a margin.
+__device__ __forceinline__ uint32_t with_margin(uint32_t bound) { return bound > 4u ? bound - 4u : 0u; }
+// a candidate: by its quotient, of equal ones the smaller index first
+__device__ __forceinline__ unsigned long long candidate(float quotient, int i) { return (unsigned long long)order_key(quotient) << 32 | ~(uint32_t)i; }
+
+// Rows in parts: workgroups of their own look through PART_RUN logits each for what may be among the row's k largest. A part's
+// list: how many there are, then the first PART_KEEP of them in any order.
+constexpr int PART_NT = 512, PART_LOADS = 4, PART_RUN = PART_NT * PART_LOADS * 4, PART_KEEP = 511, PART_TOP_K = 256;
+static_assert(2 * PART_TOP_K <= PART_NT, "the k-th largest of the threads' maxima, which little more than k logits reach");
+typedef unsigned long long PartList[1 + PART_KEEP];
+
 // the short lists of the way by candidates
 constexpr int CANDIDATES = 2048;
 constexpr int MOST_TOP_K = 1024;
@@ -313,6 +350,53 @@ template <bool VEC> __device__ __forceinline__ void draw_row(const float* __rest
   if (threadIdx.x == 0) *out = r > 0.f ? sh.pick : 0;   // (index 0's running sum reaches a draw of 0)
 }
 
+// One part of a row, its logits in registers: the k-th largest of the threads' maxima bounds the part's k-th largest from below, and
+// the row's k largest are among their parts'.  What lies at or above the bound goes to the part's list, zeros to its probabilities.
+template <bool VEC>
+__global__ void __launch_bounds__(PART_NT)
+sample_part_kernel(const float* __restrict__ logits, int V, int run, float temperature, int top_k, float* __restrict__ probs, PartList* __restrict__ lists) {
+  __shared__ int reached[2][SNT / WAVE][16];
+  __shared__ int count;
+  const int b = blockIdx.x, tid = threadIdx.x, lo = blockIdx.y * run, hi = min(V, lo + run);
+  const float* z = logits + (size_t)b * V;
+  float* p = probs + (size_t)b * V;
+  unsigned long long* list = lists[(size_t)b * gridDim.y + blockIdx.y];
+  float v[PART_LOADS][4];
+  int n[PART_LOADS];
+#pragma unroll
+  for (int u = 0; u < PART_LOADS; ++u) n[u] = load4<VEC>(z, lo + (u * PART_NT + tid) * 4, hi, v[u]);
+  if (tid == 0) count = 0;
+  uint32_t mine = 0u;
+#pragma unroll
+  for (int u = 0; u < PART_LOADS; ++u)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < n[u]) mine = max(mine, order_key(v[u][j]));
+  const uint32_t bound = with_margin(bound_of_kth<PART_NT>(mine, top_k, reached));
+  const float zeros[4] = {0.f, 0.f, 0.f, 0.f};
+  int c = 0;
+#pragma unroll
+  for (int u = 0; u < PART_LOADS; ++u) {
+    store4<VEC>(p, lo + (u * PART_NT + tid) * 4, n[u], zeros);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c += j < n[u] && order_key(v[u][j]) >= bound;
+  }
+  const int upto = wave_incl_scan(c);                   // one request a wave for places: one a logit took 3.4 us of a part's 6.4
+  int at = 0;
+  if (tid % WAVE == WAVE - 1) at = atomicAdd(&count, upto);
+  at = __shfl(at, WAVE - 1, WAVE) + upto - c;
+#pragma unroll
+  for (int u = 0; u < PART_LOADS; ++u)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < n[u] && order_key(v[u][j]) >= bound) {
+        if (at < PART_KEEP) list[1 + at] = candidate(v[u][j] / temperature, lo + (u * PART_NT + tid) * 4 + j);
+        ++at;
+      }
+  __syncthreads();
+  if (tid == 0) list[0] = count;
+}
+
 // One workgroup of 1,024 threads a row.  What bounds it is one compute unit's work on a row (131,072 logits are
 // 512 KB, 3.5 us a pass at 64 bytes a cycle from L2, and more where an element costs a division or an exponential)
 // times the number of passes, so passes are what was taken out:
@@ -321,14 +405,15 @@ template <bool VEC> __device__ __forceinline__ void draw_row(const float* __rest
 //     there; softmax, top-p and the draw run over the list.
 //   * everything else: thresholds by a histogram of the key's bits, three passes whatever the row holds, where
 //     bisection took one a bit.  top-p adds probabilities as whole numbers of 2^-60.
-// Microseconds, the kernel alone (by bisection, a bit a pass, before): 16 rows of 131,072 logits at T = 0.7 with top-k 50
-// and top-p 0.95 36 (1,612), top-p 0.9 alone 135 (840), neither 81 (166), top-k 2,000 134 (939), greedy 12 (24);
-// 64 rows of 32,000 25 (443), 46 (238), 27 (54), 44 (257), 7 (9.1).
+// With `lists` the first way begins with the parts' candidates (sample_part_kernel) in place of its two passes.
+// Microseconds of the kernels (by bisection, a bit a pass, before): 16 rows of 131,072 logits at T = 0.7 with top-k 50
+// and top-p 0.95 22 in parts (1,612; 32 by one workgroup a row), top-p 0.9 alone 136 (840), neither 82 (166), top-k 2,000 134 (939),
+// greedy 12 (24); 64 rows of 32,000 18 (443), 46 (238), 27 (54), 44 (257), 7 (9.1).
 template <bool VEC>
 __global__ void __launch_bounds__(SNT)
 sample_kernel(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p,
               uint32_t seed_lo, uint32_t seed_hi, const int* __restrict__ counters,
-              float* __restrict__ probs, int* __restrict__ out) {
+              float* __restrict__ probs, int* __restrict__ out, const PartList* __restrict__ lists, int n_parts) {
   __shared__ SampleShared sh;
   __shared__ Lists li;
   const int b = blockIdx.x, tid = threadIdx.x, w = tid / WAVE, lane = tid % WAVE;
@@ -364,32 +449,39 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
   const auto bits = [](float v) { return __float_as_uint(v); };
 
   if (top_k > 0 && top_k < V && top_k <= MOST_TOP_K) {
-    uint32_t mine = 0u;
-    visit<VEC>(z_in, V, [&](int, float v) { mine = max(mine, order_key(v)); });
-    uint32_t bound = 0u;
-    for (int bit = 31; bit >= 12; --bit) {              // (a bound: its last bits may stay 0)
-      const uint32_t cand = bound | (1u << bit);
-      const int c = __popcll(__ballot(mine >= cand));
-      __syncthreads();
-      if (lane == 0) sh.wave_count[w] = c;
-      __syncthreads();
-      int all = 0;
-#pragma unroll
-      for (int i = 0; i < SNT / WAVE; ++i) all += sh.wave_count[i];
-      if (all >= top_k) bound = cand;
-    }
-    // the passes go by the logits themselves (a division is 14 instructions, 12 us a pass over 131,072); two logits
-    // whose quotients round to one number lie within 2 units in the last place of each other, so 4 are a margin
-    bound = bound > 4u ? bound - 4u : 0u;
+    const PartList* parts = lists ? lists + (size_t)b * n_parts : nullptr;
     if (tid == 0) sh.count = 0;
-    __syncthreads();
-    update<VEC>(z_in, p, V, [&](int i, float v) {
-      if (order_key(v) >= bound) {
-        const int at = atomicAdd(&sh.count, 1);
-        if (at < CANDIDATES) li.c[at] = (unsigned long long)order_key(v / temperature) << 32 | ~(uint32_t)i;
-      }
-      return 0.f;
-    });
+    // (a part with more than its list holds, equal logits for instance: as without parts)
+    if (parts && !__syncthreads_or(tid < n_parts && parts[min(tid, n_parts - 1)][0] > PART_KEEP)) {
+      const int per = max(1, SNT / WAVE / n_parts);      // waves a part
+      const auto each = [&](auto f) {
+        for (int s = w; s < n_parts * per; s += SNT / WAVE) {
+          const unsigned long long* l = parts[s / per];
+          const int n = (int)l[0];
+          for (int j = s % per * WAVE + lane; j < n; j += per * WAVE) f(l[1 + j]);
+        }
+      };
+      uint32_t mine = 0u;
+      each([&](unsigned long long c) { mine = max(mine, (uint32_t)(c >> 32)); });
+      const uint32_t bound = bound_of_kth<SNT>(mine, top_k, sh.reached);
+      each([&](unsigned long long c) {
+        if ((uint32_t)(c >> 32) >= bound) {
+          const int at = atomicAdd(&sh.count, 1);
+          if (at < CANDIDATES) li.c[at] = c;
+        }
+      });
+    } else {
+      uint32_t mine = 0u;
+      visit<VEC>(z_in, V, [&](int, float v) { mine = max(mine, order_key(v)); });
+      const uint32_t bound = with_margin(bound_of_kth<SNT>(mine, top_k, sh.reached));
+      update<VEC>(z_in, p, V, [&](int i, float v) {
+        if (order_key(v) >= bound) {
+          const int at = atomicAdd(&sh.count, 1);
+          if (at < CANDIDATES) li.c[at] = candidate(v / temperature, i);
+        }
+        return 0.f;
+      });
+    }
     __syncthreads();
     const int n = sh.count;
     if (n <= CANDIDATES) {
@@ -441,7 +533,14 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
         __syncthreads();
         if (kept) {
           double run = 0.0;
-          for (int o = 0; o < top_k; ++o) run += li.top_i[o] <= my_i ? (double)li.top_z[o] : 0.0;
+          for (int o = 0; o < top_k; o += 8) {          // (loads first: an addition that waits for its own takes 80 ns)
+            float z[8];
+            int i[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) { z[q] = li.top_z[o + q]; i[q] = li.top_i[o + q]; }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) run += o + q < top_k && i[q] <= my_i ? (double)z[q] : 0.0;
+          }
           if (run >= (double)r) atomicMin(&sh.pick, my_i);
           p[my_i] = e;                                  // (behind the zeros of the pass above: barriers lie between)
         }
@@ -513,15 +612,32 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
 
 using namespace tl;
 
+// The parts a row is looked through in, or 0: none, a row is one workgroup's.  Long rows, and not so many that one workgroup each fills
+// the chip.  Microseconds of the kernels, one workgroup a row / in parts, at T = 0.7 and top-k 50: 16 rows of 131,072
+// 28 / 20, 64 of them 30 / 31, 16 rows of 32,000 16 / 18.  lists: room for [B][parts] lists of tl_sample_list_bytes() each.
+extern "C" int tl_sample_parts(int B, int V, float temperature, int top_k) {
+  if (!(temperature > 0.f) || top_k <= 0 || top_k > PART_TOP_K || V <= 8 * PART_RUN || V > 32 * PART_RUN) return 0;
+  const int parts = (V + PART_RUN - 1) / PART_RUN;
+  return (long long)B * parts <= 512 ? parts : 0;
+}
+extern "C" int tl_sample_list_bytes() { return (int)sizeof(PartList); }
+
 extern "C" int tl_sample(const float* logits, int B, int V, float temperature, int top_k, float top_p,
-                         unsigned long long seed, const int* counters, float* probs, int* out,
+                         unsigned long long seed, const int* counters, float* probs, int* out, void* lists, int n_parts,
                          hipStream_t st) {
   TL_REQUIRE(B >= 0 && V > 0, "sample: bad sizes B=%d V=%d", B, V);
+  TL_REQUIRE(n_parts == 0 || (lists != nullptr && n_parts == tl_sample_parts(B, V, temperature, top_k)), "sample: %d parts of a row of %d", n_parts, V);
   if (B == 0) return 0;
   const bool vec = V % 4 == 0 && ((uintptr_t)logits | (uintptr_t)probs) % 16 == 0;
+  if (n_parts) {
+    const int run = ((V + n_parts - 1) / n_parts + 3) / 4 * 4;
+    const auto part = vec ? sample_part_kernel<true> : sample_part_kernel<false>;
+    part<<<dim3(B, n_parts), PART_NT, 0, st>>>(logits, V, run, temperature, top_k, probs, (PartList*)lists);
+    TL_LAUNCH_CHECK("sample_part");
+  }
   const auto kernel = vec ? sample_kernel<true> : sample_kernel<false>;
   kernel<<<B, SNT, 0, st>>>(logits, V, temperature, top_k, top_p, (uint32_t)(seed & 0xffffffffu),
-                            (uint32_t)(seed >> 32), counters, probs, out);
+                            (uint32_t)(seed >> 32), counters, probs, out, (const PartList*)(n_parts ? lists : nullptr), n_parts);
   TL_LAUNCH_CHECK("sample");
   return 0;
 }

@@ -1739,18 +1739,30 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: 
                                int(accumulate), _stream()))
 
 
+def sample_lists(B: int, V: int, temperature: float, top_k: int, device) -> Optional[torch.Tensor]:
+    """Room for the lists of a draw whose rows several workgroups look through, uint8 [B, parts, bytes of a list], or None: a row is
+    one workgroup's (the rule is `tl_sample_parts`)."""
+    parts = lib().tl_sample_parts(B, V, ctypes.c_float(temperature), int(top_k))
+    return torch.empty((B, parts, lib().tl_sample_list_bytes()), dtype=torch.uint8, device=device) if parts else None
+
+
 def sample(logits: torch.Tensor, temperature: float, top_k: int, top_p: float, seed: int,
-           counters: torch.Tensor, probs: torch.Tensor, out: torch.Tensor) -> None:
+           counters: torch.Tensor, probs: torch.Tensor, out: torch.Tensor, lists: Optional[torch.Tensor] = None) -> None:
     """One token per row.  counters[b] = (sequence, step) feeds the generator;
-    probs receives the distribution the draw was made from (when T > 0)."""
+    probs receives the distribution the draw was made from (when T > 0); lists: see `sample_lists`, which a caller may keep for
+    the draws that follow on the same stream."""
     B, V = logits.shape
+    if lists is None:
+        lists = sample_lists(B, V, temperature, top_k, logits.device)
+    if lists is not None:
+        _req(lists, "sample.lists", torch.uint8, (B, lists.shape[1], lib().tl_sample_list_bytes()))
     _req(logits, "sample.logits", torch.float32)
     _req(counters, "sample.counters", torch.int32, (B, 2))
     _req(probs, "sample.probs", torch.float32, (B, V))
     _req(out, "sample.out", torch.int32, (B,))
     _check(lib().tl_sample(_p(logits), B, V, ctypes.c_float(temperature), int(top_k),
                            ctypes.c_float(top_p), ctypes.c_ulonglong(seed & (2 ** 64 - 1)),
-                           _p(counters), _p(probs), _p(out), _stream()))
+                           _p(counters), _p(probs), _p(out), _p(lists), lists.shape[1] if lists is not None else 0, _stream()))
 
 
 EPI_STORE, EPI_ACCUMULATE, EPI_SILU_PAIR, EPI_GELU_PAIR = 0, 1, 2, 3
