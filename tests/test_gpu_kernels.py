@@ -554,6 +554,30 @@ def test_rows_in_parts(ops, monkeypatch, V, k):
         assert float((probs[b].double() - want).abs().max()) < 2e-6 + float(want[want > 0].min()) * 2
 
 
+def test_draws_through_pinned_memory(ops):
+    """The sampler's draws, one launched before the last is read, more rows and then fewer, sampler dropped with a draw under way:
+    the tokens that the kernel gives with its pairs on the device; host memory that is not pinned is refused."""
+    from torchless_rs_amd import SamplingConfig
+    from torchless_rs_amd.sampling.sampler import Sampler
+    z = rnd(80, 3000, seed=77, scale=2.0).to(DEV)
+    sampler, drawn, want = Sampler(SamplingConfig(0.9, 40, 0.9, 6), DEV), None, None
+    for t, B in enumerate((3, 3, 80, 2, 64, 64)):
+        ids, _ = run_sample(ops, z[:B], 0.9, 40, 0.9, 6, [[b + t, 10 * t] for b in range(B)])
+        now = sampler.draw(z[:B], [b + t for b in range(B)], [10 * t] * B)
+        if drawn is not None:
+            assert drawn.tokens() == want and drawn.tokens() == want
+        drawn, want = now, ids
+        assert now.device.tolist() == ids
+    del sampler, now
+    assert drawn.tokens() == want
+    out, probs = torch.empty(3, dtype=torch.int32, device=DEV), torch.empty(3, 3000, device=DEV)
+    pairs = torch.zeros(3, 2, dtype=torch.int32)
+    with pytest.raises(ops.KernelError):
+        ops.sample(z[:3], 0.9, 40, 0.9, 6, pairs, probs, out)
+    with pytest.raises(ops.KernelError):
+        ops.sample(z[:3], 0.9, 40, 0.9, 6, pairs.to(DEV), probs, out, host_out=torch.zeros(3, dtype=torch.int32))
+
+
 def test_draws_do_not_depend_on_batch_mates_and_follow_the_probabilities(ops):
     V = 8
     z = torch.tensor([[2.0, 1.0, 0.0, -1.0, 0.5, 1.5, -2.0, 0.2]])

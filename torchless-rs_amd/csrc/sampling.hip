@@ -300,8 +300,18 @@ __device__ __forceinline__ void keep_ties(float* __restrict__ p, int V, uint32_t
   __syncthreads();
 }
 
+// Where a row's token goes: device memory, and host memory that the device can write (or null).
+struct Tokens {
+  int* device;
+  int* host;
+  __device__ __forceinline__ void put(int b, int token) const {
+    device[b] = token;
+    if (host) __hip_atomic_store(host + b, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+
 // The draw over a whole row of probabilities: the first index whose running sum reaches r, else the last.
-template <bool VEC> __device__ __forceinline__ void draw_row(const float* __restrict__ p, int V, float r, SampleShared& sh, int* __restrict__ out) {
+template <bool VEC> __device__ __forceinline__ void draw_row(const float* __restrict__ p, int V, float r, SampleShared& sh, int b, Tokens out) {
   const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int run = ((V + SNT / WAVE - 1) / (SNT / WAVE) + 255) / 256 * 256;
   const int lo = min(V, w * run), hi = min(V, lo + run);
@@ -347,7 +357,7 @@ template <bool VEC> __device__ __forceinline__ void draw_row(const float* __rest
     if (lane == 0) sh.pick = pick;
   }
   __syncthreads();
-  if (threadIdx.x == 0) *out = r > 0.f ? sh.pick : 0;   // (index 0's running sum reaches a draw of 0)
+  if (threadIdx.x == 0) out.put(b, r > 0.f ? sh.pick : 0);   // (index 0's running sum reaches a draw of 0)
 }
 
 // One part of a row, its logits in registers: the k-th largest of the threads' maxima bounds the part's k-th largest from below, and
@@ -413,7 +423,7 @@ template <bool VEC>
 __global__ void __launch_bounds__(SNT)
 sample_kernel(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p,
               uint32_t seed_lo, uint32_t seed_hi, const int* __restrict__ counters,
-              float* __restrict__ probs, int* __restrict__ out, const PartList* __restrict__ lists, int n_parts) {
+              float* __restrict__ probs, Tokens out, const PartList* __restrict__ lists, int n_parts) {
   __shared__ SampleShared sh;
   __shared__ Lists li;
   const int b = blockIdx.x, tid = threadIdx.x, w = tid / WAVE, lane = tid % WAVE;
@@ -440,7 +450,7 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
         const int i2 = sh.wave_count[i];
         if (i2 >= 0 && (bi < 0 || v2 > best || (v2 == best && i2 > bi))) { best = v2; bi = i2; }
       }
-      out[b] = bi;
+      out.put(b, bi);
     }
     return;
   }
@@ -545,7 +555,7 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
           p[my_i] = e;                                  // (behind the zeros of the pass above: barriers lie between)
         }
         __syncthreads();
-        if (tid == 0) out[b] = r > 0.f ? sh.pick : 0;
+        if (tid == 0) out.put(b, r > 0.f ? sh.pick : 0);
         return;
       }
     }
@@ -580,7 +590,7 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
   update<VEC>(p, p, V, [&](int, float v) { return v / sum; });
   __syncthreads();
   if (!(sum > 0.f && sum < INFINITY)) {                 // infinities or NaN among the logits: no draw
-    if (tid == 0) out[b] = V - 1;
+    if (tid == 0) out.put(b, V - 1);
     return;
   }
 
@@ -605,7 +615,7 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
       keep_ties<VEC>(p, V, thr, room, 0.f, bits, scaled, sh);
     }
   }
-  draw_row<VEC>(p, V, r, sh, out + b);
+  draw_row<VEC>(p, V, r, sh, b, out);
 }
 
 }  // namespace tl
@@ -622,8 +632,10 @@ extern "C" int tl_sample_parts(int B, int V, float temperature, int top_k) {
 }
 extern "C" int tl_sample_list_bytes() { return (int)sizeof(PartList); }
 
+// counters [B][2] and host_out [B] (or null) may lie in pinned host memory: a row's workgroup reads 8 bytes of the one and writes 4 of the
+// other while it has half a megabyte of logits to go through, where a copy each costs the stream 8 us and the host 5.
 extern "C" int tl_sample(const float* logits, int B, int V, float temperature, int top_k, float top_p,
-                         unsigned long long seed, const int* counters, float* probs, int* out, void* lists, int n_parts,
+                         unsigned long long seed, const int* counters, float* probs, int* out, int* host_out, void* lists, int n_parts,
                          hipStream_t st) {
   TL_REQUIRE(B >= 0 && V > 0, "sample: bad sizes B=%d V=%d", B, V);
   TL_REQUIRE(n_parts == 0 || (lists != nullptr && n_parts == tl_sample_parts(B, V, temperature, top_k)), "sample: %d parts of a row of %d", n_parts, V);
@@ -637,7 +649,7 @@ extern "C" int tl_sample(const float* logits, int B, int V, float temperature, i
   }
   const auto kernel = vec ? sample_kernel<true> : sample_kernel<false>;
   kernel<<<B, SNT, 0, st>>>(logits, V, temperature, top_k, top_p, (uint32_t)(seed & 0xffffffffu),
-                            (uint32_t)(seed >> 32), counters, probs, out, (const PartList*)(n_parts ? lists : nullptr), n_parts);
+                            (uint32_t)(seed >> 32), counters, probs, Tokens{out, host_out}, (const PartList*)(n_parts ? lists : nullptr), n_parts);
   TL_LAUNCH_CHECK("sample");
   return 0;
 }

@@ -79,6 +79,11 @@ def _req(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
     raise KernelError(f"{name}: shape {tuple(t.shape)}, kernel needs {tuple(shape)}")
 
 
+def _req_pinned(t: torch.Tensor, name: str, dtype, shape) -> None:
+    if t.is_cuda or not t.is_pinned() or not t.is_contiguous() or t.dtype != dtype or t.shape != tuple(shape):
+        raise KernelError(f"{name}: must be contiguous pinned host memory, {dtype} {tuple(shape)}")
+
+
 def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0) -> None:
     """out[n, :] = table[ids[n], :] widened to float32, times `scale`."""
     n, H = ids.shape[0], table.shape[1]
@@ -1747,22 +1752,29 @@ def sample_lists(B: int, V: int, temperature: float, top_k: int, device) -> Opti
 
 
 def sample(logits: torch.Tensor, temperature: float, top_k: int, top_p: float, seed: int,
-           counters: torch.Tensor, probs: torch.Tensor, out: torch.Tensor, lists: Optional[torch.Tensor] = None) -> None:
+           counters: torch.Tensor, probs: torch.Tensor, out: torch.Tensor, lists: Optional[torch.Tensor] = None,
+           host_out: Optional[torch.Tensor] = None) -> None:
     """One token per row.  counters[b] = (sequence, step) feeds the generator;
     probs receives the distribution the draw was made from (when T > 0); lists: see `sample_lists`, which a caller may keep for
-    the draws that follow on the same stream."""
+    the draws that follow on the same stream.  counters may lie in pinned host memory, and host_out (int32 [B]), which does, receives
+    the tokens as `out` does: both have to stay as they are until the launch is over, and nothing but the caller sees to that."""
     B, V = logits.shape
     if lists is None:
         lists = sample_lists(B, V, temperature, top_k, logits.device)
     if lists is not None:
         _req(lists, "sample.lists", torch.uint8, (B, lists.shape[1], lib().tl_sample_list_bytes()))
     _req(logits, "sample.logits", torch.float32)
-    _req(counters, "sample.counters", torch.int32, (B, 2))
+    if counters.is_cuda:
+        _req(counters, "sample.counters", torch.int32, (B, 2))
+    else:
+        _req_pinned(counters, "sample.counters", torch.int32, (B, 2))
+    if host_out is not None:
+        _req_pinned(host_out, "sample.host_out", torch.int32, (B,))
     _req(probs, "sample.probs", torch.float32, (B, V))
     _req(out, "sample.out", torch.int32, (B,))
     _check(lib().tl_sample(_p(logits), B, V, ctypes.c_float(temperature), int(top_k),
                            ctypes.c_float(top_p), ctypes.c_ulonglong(seed & (2 ** 64 - 1)),
-                           _p(counters), _p(probs), _p(out), _p(lists), lists.shape[1] if lists is not None else 0, _stream()))
+                           _p(counters), _p(probs), _p(out), _p(host_out), _p(lists), lists.shape[1] if lists is not None else 0, _stream()))
 
 
 EPI_STORE, EPI_ACCUMULATE, EPI_SILU_PAIR, EPI_GELU_PAIR = 0, 1, 2, 3

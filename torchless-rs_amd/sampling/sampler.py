@@ -5,6 +5,7 @@ Philox4x32-10 gives for key = seed and counter = (t, s, 0, 0): it does not
 depend on which other sequences share the batch."""
 from __future__ import annotations
 
+import time
 from typing import List, Sequence
 
 import torch
@@ -13,16 +14,50 @@ from ..kernels import ops
 from .config import SamplingConfig
 
 
+LOOK_FOR = 1e-4       # seconds that the host looks at the tokens' memory before it waits for the draw's event instead: an event behind
+                      # a kernel is known 9 us after it, a token that the kernel wrote at once (16 rows of 131,072: 49 and 42 us a draw)
+
+
+class _Place:
+    """Pinned host memory of one draw: what its kernel reads, the (sequence, step) pairs, and writes, the tokens.  The kernel goes by
+    their addresses, of which torch's allocator knows nothing, so the memory is held until the draw is over."""
+
+    def __init__(self, cap: int):
+        self.counters = torch.empty((cap, 2), dtype=torch.int32, pin_memory=True)
+        self.tokens = torch.empty((cap,), dtype=torch.int32, pin_memory=True)
+        self.pairs, self.ids = self.counters.numpy(), self.tokens.numpy()
+        self.done = None                 # the event behind the draw that uses it, None once that is known to be over
+
+    def wait(self) -> None:
+        if self.done is not None:
+            self.done.synchronize()
+            self.done = None
+
+    def __del__(self):
+        self.wait()
+
+
 class Drawn:
     """The tokens of one draw: on the device at once (`device`, int32 [B], valid until the
-    sampler's next draw has been launched), on the host when `tokens()` is asked for."""
+    sampler's next draw has been launched), on the host when `tokens()` is asked for (until two
+    more draws have been launched)."""
 
-    def __init__(self, device: torch.Tensor, host: torch.Tensor, done: "torch.cuda.Event"):
-        self.device, self._host, self._done = device, host, done
+    def __init__(self, device: torch.Tensor, place: _Place):
+        self.device, self._place, self._done, self._tokens = device, place, place.done, None
 
     def tokens(self) -> List[int]:
-        self._done.synchronize()
-        return self._host.tolist()
+        if self._tokens is None:
+            place, ids = self._place, self._place.ids[:self.device.shape[0]]
+            # a row's token, never negative, is the last that its workgroup does with the memory: where all are there the draw is over
+            until = time.perf_counter() + LOOK_FOR
+            while ids.size and ids.min() < 0:
+                if time.perf_counter() > until:
+                    self._done.synchronize()
+                    break
+            if place.done is self._done:
+                place.done = None
+            self._tokens = ids.tolist()
+        return self._tokens
 
 
 class Sampler:
@@ -30,46 +65,38 @@ class Sampler:
         self.config = config
         self.device = device
         self._probs = None
-        self._stage = None               # pinned (sequence, step) pairs, and their copy on the device
-        self._counters = None
+        self._lists = None               # the lists of rows in parts, of the last shape drawn from
+        self._shape = None
         self._out = None
-        self._uploaded = None
-        self._host = None                # two pinned buffers for the tokens, used in turn
+        self._places = None              # two, used in turn: a draw may be launched while the one before is read
         self._turn = 0
 
     def draw(self, logits: torch.Tensor, seq_ids: Sequence[int], steps: Sequence[int]) -> Drawn:
         """logits: float32 [B, V] on the GPU -> B token ids, without waiting for them: the
-        kernel and the copy to the host are launched, `Drawn.tokens()` waits."""
+        kernel is launched, which takes the pairs from pinned memory and leaves the tokens there, `Drawn.tokens()` waits."""
         B, V = logits.shape
         c = self.config
-        if self._stage is None or self._stage.shape[0] < B:
+        if self._out is None or self._out.shape[0] < B:
             cap = max(B, 64)
-            self._stage = torch.empty((cap, 2), dtype=torch.int32).pin_memory()
-            self._counters = torch.empty((cap, 2), dtype=torch.int32, device=logits.device)
+            self._places = [_Place(cap) for _ in range(2)]
             self._out = torch.empty((cap,), dtype=torch.int32, device=logits.device)
-            self._host = [torch.empty((cap,), dtype=torch.int32).pin_memory() for _ in range(2)]
-            self._uploaded = None
-        if self._uploaded is not None:
-            self._uploaded.synchronize()             # the pinned pairs are free to be written again
-        stage = self._stage.numpy()
-        stage[:B, 0] = seq_ids
-        stage[:B, 1] = steps
-        counters = self._counters[:B]
-        counters.copy_(self._stage[:B], non_blocking=True)
-        if self._uploaded is None:
-            self._uploaded = torch.cuda.Event()
-        self._uploaded.record()
         if self._probs is None or self._probs.shape[0] < B or self._probs.shape[1] != V:
             self._probs = torch.empty((B, V), dtype=torch.float32, device=logits.device)
+        if self._shape != (B, V):
+            self._lists = ops.sample_lists(B, V, float(c.temperature), int(c.top_k or 0), logits.device)
+            self._shape = (B, V)
+        place = self._places[self._turn]
+        self._turn ^= 1
+        place.wait()                                 # the memory is free to be written again
+        place.pairs[:B, 0] = seq_ids
+        place.pairs[:B, 1] = steps
+        place.ids[:B] = -1
         out = self._out[:B]
         ops.sample(logits.contiguous(), float(c.temperature), int(c.top_k or 0), float(c.top_p or 0.0),
-                   int(c.seed), counters, self._probs[:B], out)
-        host = self._host[self._turn][:B]
-        self._turn ^= 1
-        host.copy_(out, non_blocking=True)
-        done = torch.cuda.Event()
-        done.record()
-        return Drawn(out, host, done)
+                   int(c.seed), place.counters[:B], self._probs[:B], out, self._lists, place.tokens[:B])
+        place.done = torch.cuda.Event()
+        place.done.record()
+        return Drawn(out, place)
 
     def sample(self, logits: torch.Tensor, seq_ids: Sequence[int], steps: Sequence[int]) -> List[int]:
         """logits: float32 [B, V] on the GPU -> B token ids."""
