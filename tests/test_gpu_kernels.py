@@ -1155,6 +1155,31 @@ def test_qkv_rope_commit_from_the_tiled_copy(ops, nq, nkv, d, K, lens):
     assert not torch.equal(out[1][1], torch.nan_to_num(c["pages"].float(), nan=-7.0))
 
 
+@pytest.mark.parametrize("nq,nkv,d,K,units", [(6, 2, 48, 64, 3), (6, 2, 48, 192, 4), (3, 1, 256, 128, 3), (5, 1, 16, 320, 4),
+                                               (8, 2, 128, 1024, 3), (32, 8, 128, 256, 0)])
+@pytest.mark.parametrize("share,interleaved", [(1.0, False), (0.5, False), (0.5, True)])
+def test_qkv_rope_commit_from_tiles_of_shares(ops, nq, nkv, d, K, units, share, interleaved):
+    """Tiles that are workgroups' shares of 24 or 32 rows, the last of them with fewer: the bits of the weights as stored."""
+    rot, _ = rotation_for(ops, d, 10000.0, share, interleaved)
+    lens = [0, 63, 64, 300, 9]
+    c = paged_case(ops, "bfloat16", nq, nkv, d, None, lens_cached=lens, lens_new=[1] * 5, seed=19, n_pages=60)
+    y = rnd(5, K, seed=20, dtype=torch.bfloat16).to(DEV)
+    w = rnd((nq + 2 * nkv) * d, K, seed=21, dtype=torch.bfloat16, scale=0.2).to(DEV)
+    rows = ops.qkv_tile_rows(nq, nkv, d, DEV, rot, shares=True)
+    assert sorted(rows.tolist()) == list(range((nq + 2 * nkv) * d))
+    tiles = ops.tile_weights(w, rows, 8 * units) if units else ops.qkv_tiles(w, nq, nkv, d, rot)
+    out = []
+    for t in (None, tiles):
+        q = torch.full((5, nq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        pages = c["pages"].clone()
+        ops.qkv_rope_commit(y, w, c["row_pos"], rot, c["table"], c["ring"], nq, nkv, d, q, pages, units=units, tiles=t)
+        out.append((q, torch.nan_to_num(pages.float(), nan=-7.0)))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    if units:
+        with pytest.raises(ops.KernelError, match="tiles of"):
+            ops.qkv_rope_commit(y, w, c["row_pos"], rot, c["table"], c["ring"], nq, nkv, d, q, pages, units=2, tiles=t)
+
+
 # ---- many channels against at most 16 rows: whole rows of the weights, 1 KB a load --------------
 
 @pytest.mark.parametrize("M", [1, 5, 16])

@@ -35,8 +35,8 @@ __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *reinterpret_cas
 // large buffer reaches 6.7 to 6.95 TB/s with such loads against 6.0 without (csrc/measure/ceilings.hip); gate|up
 // at 8 rows went from 41.6 to 38.0 us, down from 21.9 to 20.4, o from 9.0 to 8.3.  Not for the kernels
 // whose cache lines are shared between load instructions or waves (gemm_mid: a decode step at batch 64
-// 11.9 against 10.85 ms; the keys and values of decode attention: 11.56 against 10.85 ms), and the fused
-// q|k|v kernel gains nothing from it.
+// 11.9 against 10.85 ms; the keys and values of decode attention: 11.56 against 10.85 ms; the fused q|k|v kernel on
+// tiles that two workgroups share).
 __device__ __forceinline__ bf16x8 load8_once(const bf16* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
 }
@@ -473,11 +473,15 @@ static int launch_rows(const bf16* A, const bf16* W, float* C, int M, int N, int
 // (7B: 768 units are 3 for each of 256).
 // The sums and the rotation are those of the unfused kernels, bit for bit
 // (a' = a c - b s; b' = a s + b c; src/kernels/mod.rs:603-605 of the reference).
-// TILED: W is the tiled copy whose tile (head, t) holds units 2t and 2t+1 of the head, first
-// channels in its rows 0..7, second channels in 8..15 (`tl_qkv_tile_rows`).
+// COPY: W is a tiled copy.  QKV_HEAD_TILES: its tile (head, t) holds units 2t and 2t+1 of the head, first
+// channels in its rows 0..7, second channels in 8..15 (`tl_qkv_tile_rows`).  QKV_SHARES: a tile is a workgroup's share, its
+// units one after the other (`tl_qkv_share_rows`), so that what a workgroup reads is one run of memory: with three units a
+// workgroup a tile of 16 rows is two workgroups', on two XCDs, which both have its lines brought from memory (6,144 x 4,096 at 1 / 8 rows
+// 14.2 / 14.4 us, from shares 11.8 / 12.0, of which non-temporal loads are 0.7).
 constexpr int QKV_WAVES = 8;
+constexpr int QKV_STORED = 0, QKV_HEAD_TILES = 1, QKV_SHARES = 2;
 
-template <bool TILED, int NT>
+template <int COPY, int NT>
 __global__ void __launch_bounds__(QKV_WAVES * 64)
 gemm_qkv_rope_commit_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, int M, int K,
                             const int* __restrict__ row_pos, Rotation rot,
@@ -501,7 +505,10 @@ gemm_qkv_rope_commit_kernel(const bf16* __restrict__ A, const bf16* __restrict__
     const int g = g0 + (loads[t] ? u : 0);
     const int head = g / per_head, h = g % per_head;
     const bool rotated = head < nq + nkv;
-    if constexpr (TILED) {
+    if constexpr (COPY == QKV_SHARES) {
+      // (places of a share without a row hold zeros: no lane loads under a condition)
+      wrow[t] = W + (size_t)blockIdx.x * (8 * units) * K + kg * (64 * units) + min(16 * t + li, 8 * units - 1) * 8;
+    } else if constexpr (COPY == QKV_HEAD_TILES) {
       const int sub = h % 2;
       const int r = rotated ? (j < 4 ? 4 * sub + j : 8 + 4 * sub + j - 4) : 8 * sub + j;
       wrow[t] = W + (size_t)(head * (d / 16) + h / 2) * 16 * K + kg * 128 + r * 8;
@@ -528,7 +535,10 @@ gemm_qkv_rope_commit_kernel(const bf16* __restrict__ A, const bf16* __restrict__
     const bool ok0 = k + 8 <= K, ok1 = k + 16 <= K;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      if constexpr (TILED) {
+      if constexpr (COPY == QKV_SHARES) {
+        wv[t][0] = load8_once(wrow[t] + (size_t)s * (512 * units));
+        wv[t][1] = load8_once(wrow[t] + (size_t)s * (512 * units) + 256 * units);
+      } else if constexpr (COPY == QKV_HEAD_TILES) {
         wv[t][0] = loads[t] ? load8(wrow[t] + (size_t)s * TILE_STEP) : zero8();
         wv[t][1] = loads[t] ? load8(wrow[t] + (size_t)s * TILE_STEP + TILE_STEP / 2) : zero8();
       } else {
@@ -1105,14 +1115,22 @@ extern "C" int tl_gemm_ring_bf16(const void* A, const void* W, void* C, int M, i
   TL_REQUIRE(false, "gemm_ring: %d waves a workgroup (4, 7 or 8)", waves);
 }
 
+// The units of 8 rows of q|k|v a workgroup of the fused kernel owns: a whole number of rounds of workgroups over the compute units,
+// of at most 4 units each.
+static int qkv_units(int nq, int nkv, int d) {
+  const int cus = compute_units();
+  const long long n_units = (long long)(nq + 2 * nkv) * (d / 8), wgs = ((n_units + 4LL * cus - 1) / (4LL * cus)) * cus;
+  return (int)((n_units + wgs - 1) / wgs);
+}
+
 // q|k|v of a step with one token a sequence (row m is sequence m, at position row_pos[m]):
 // W is [(nq + 2 nkv) d, K]; q receives [M, nq, d], the pages k and v of the new position.
 // With ssq_in, row m's sums are multiplied by rsqrt(sum_j ssq_in[m][j] * inv_h + eps) first.
 // units: the units of 8 weight rows (see the kernel) a workgroup owns, 1 to 4; 0 lets the
 // launcher deal them in equal shares to the device's compute units.
-// Wt (or null): the tiled copy of W with the rows of `tl_qkv_tile_rows`, read instead of W
-// when K % 64 == 0.
-extern "C" int tl_gemm_qkv_rope_commit(const void* A, const void* W, const void* Wt, int M, int K, const int* row_pos,
+// Wt (or null): a tiled copy of W, read instead of W when K % 64 == 0: with tiles of 16 rows in the order of `tl_qkv_tile_rows`
+// (any `units`), or of 8 `units` rows, 24 or 32, in that of `tl_qkv_share_rows` (wt_height says which).
+extern "C" int tl_gemm_qkv_rope_commit(const void* A, const void* W, const void* Wt, int wt_height, int M, int K, const int* row_pos,
                                        const float* inv_freq, int rotary_dim, int interleaved,
                                        const int* table, int table_stride,
                                        int ring_pages, int nq, int nkv, int d, void* q, void* pages,
@@ -1133,26 +1151,24 @@ extern "C" int tl_gemm_qkv_rope_commit(const void* A, const void* W, const void*
   const Rotation rot{inv_freq, rotary_dim, interleaved != 0};
   if (M == 0) return 0;
   const long long n_units = (long long)(nq + 2 * nkv) * (d / 8);
-  if (units == 0) {
-    // a whole number of rounds of workgroups over the compute units, of at most 4 units each
-    const int cus = compute_units();
-    const long long wgs = ((n_units + 4LL * cus - 1) / (4LL * cus)) * cus;
-    units = (int)((n_units + wgs - 1) / wgs);
-  }
+  if (units == 0) units = qkv_units(nq, nkv, d);
   const int grid = (int)((n_units + units - 1) / units);
   NormSplit ns{};
   ns.ssq_in = ssq_in; ns.n_part = n_part; ns.inv_h = inv_h; ns.eps = eps;
   const bool tiled = Wt != nullptr && K % 64 == 0;
   TL_REQUIRE(!tiled || (uintptr_t)Wt % 16 == 0, "qkv_rope_commit: operands must be 16-byte aligned");
+  TL_REQUIRE(!tiled || wt_height == 16 || wt_height == 8 * units, "qkv_rope_commit: the tiled copy has tiles of %d rows, %d units a workgroup read "
+             "tiles of %d or 16", wt_height, units, 8 * units);
+  const bool shares = tiled && wt_height != 16;
   const bf16* w = tiled ? (const bf16*)Wt : (const bf16*)W;
-#define TL_QKV(TILED, NT)                                                                               \
-  gemm_qkv_rope_commit_kernel<TILED, NT><<<grid, QKV_WAVES * 64, 0, st>>>(                              \
+#define TL_QKV(COPY, NT)                                                                                \
+  gemm_qkv_rope_commit_kernel<COPY, NT><<<grid, QKV_WAVES * 64, 0, st>>>(                              \
       (const bf16*)A, w, M, K, row_pos, rot, table, table_stride, ring_pages, nq, nkv, d, (bf16*)q, \
       (bf16*)pages, ns, units)
   if (units <= 2) {
-    if (tiled) TL_QKV(true, 1); else TL_QKV(false, 1);
+    if (tiled) TL_QKV(QKV_HEAD_TILES, 1); else TL_QKV(QKV_STORED, 1);
   } else {
-    if (tiled) TL_QKV(true, 2); else TL_QKV(false, 2);
+    if (shares) TL_QKV(QKV_SHARES, 2); else if (tiled) TL_QKV(QKV_HEAD_TILES, 2); else TL_QKV(QKV_STORED, 2);
   }
 #undef TL_QKV
   TL_LAUNCH_CHECK("gemm_qkv_rope_commit");
@@ -1237,6 +1253,33 @@ extern "C" int tl_qkv_tile_rows(int nq, int nkv, int d, int rotary_dim, int inte
           ch = r < 8 ? ca : cb;
         }
         rows[(head * (d / 16) + t) * 16 + r] = head * d + ch;
+      }
+  return 0;
+}
+
+// The height of the tiles of the copy that the fused kernel reads fastest: a workgroup's share of rows where that is more than 16 (the
+// rows then in the order of tl_qkv_share_rows), else 16 (tl_qkv_tile_rows).
+extern "C" int tl_qkv_tile_height(int nq, int nkv, int d) {
+  const int units = qkv_units(nq, nkv, d);
+  return units > 2 ? 8 * units : 16;
+}
+
+// The order of W's rows in a copy whose tiles are workgroups' shares: unit after unit, a unit of a q or k head the first channels of its
+// four pairs and then their second channels, of a v head eight channels in a row.  rows: [(nq + 2 nkv) d], host.
+extern "C" int tl_qkv_share_rows(int nq, int nkv, int d, int rotary_dim, int interleaved, int* rows) {
+  TL_REQUIRE(nq > 0 && nkv > 0 && d >= 16 && d % 16 == 0, "qkv_share_rows: bad heads nq=%d nkv=%d d=%d", nq, nkv, d);
+  TL_REQUIRE(rotary_dim >= 0 && rotary_dim <= d && rotary_dim % 2 == 0,
+             "qkv_share_rows: %d rotated channels of a head of %d (even, at most the head)", rotary_dim, d);
+  for (int head = 0; head < nq + 2 * nkv; ++head)
+    for (int h = 0; h < d / 8; ++h)
+      for (int j = 0; j < 8; ++j) {
+        int ch = 8 * h + j;
+        if (head < nq + nkv) {
+          int ca, cb;
+          pair_channels(4 * h + j % 4, rotary_dim, interleaved != 0, ca, cb);
+          ch = j < 4 ? ca : cb;
+        }
+        rows[(head * (d / 8) + h) * 8 + j] = head * d + ch;
       }
   return 0;
 }

@@ -1836,15 +1836,24 @@ def tile_weights(w: torch.Tensor, rows: Optional[torch.Tensor] = None, height: O
     return out
 
 
-def qkv_tile_rows(nq: int, nkv: int, d: int, device, rotation=None) -> torch.Tensor:
+def qkv_tile_rows(nq: int, nkv: int, d: int, device, rotation=None, shares: bool = False) -> torch.Tensor:
     """The order of the rows of w = q|k|v in the tiled copy that `qkv_rope_commit` reads
     (a tile of a q or k head holds both channels of 8 pairs of `rotation`; None: the whole
-    head rotated in halves)."""
+    head rotated in halves).  `shares`: in the copy whose tiles are workgroups' shares of 24 or 32 rows (both channels
+    of 4 pairs, unit after unit)."""
     n = (nq + 2 * nkv) * d
     buf = (ctypes.c_int * n)()
     rotary_dim, interleaved = (d, False) if rotation is None else (rotation.rotary_dim, rotation.interleaved)
-    _check(lib().tl_qkv_tile_rows(int(nq), int(nkv), int(d), int(rotary_dim), int(interleaved), buf))
+    order = lib().tl_qkv_share_rows if shares else lib().tl_qkv_tile_rows
+    _check(order(int(nq), int(nkv), int(d), int(rotary_dim), int(interleaved), buf))
     return torch.tensor(list(buf), dtype=torch.int32, device=device)
+
+
+def qkv_tiles(w: torch.Tensor, nq: int, nkv: int, d: int, rotation=None) -> torch.Tensor:
+    """The tiled copy of w = q|k|v that `qkv_rope_commit` reads fastest on this device: tiles that are its workgroups' shares of the rows
+    where those are more than 16, else tiles of 16 (`qkv_tile_rows`)."""
+    height = int(lib().tl_qkv_tile_height(int(nq), int(nkv), int(d)))
+    return tile_weights(w, qkv_tile_rows(nq, nkv, d, w.device, rotation, shares=height > 16), height)
 
 
 def _req_tiles(tiles: Optional[torch.Tensor], N: int, K: int, height: Optional[int] = None) -> int:
@@ -2311,12 +2320,12 @@ def qkv_rope_commit(a: torch.Tensor, w: torch.Tensor, row_pos, rotation, table, 
     the rotation of q and k, q into its buffer and k, v into the pages, in one kernel; the
     same bits as `gemm` and then `rope_commit`.  `factor`: see `gemm_bf16_norm`.  `units`
     (tests): how many units of 8 weight rows a workgroup owns, 1 to 4; 0 leaves it to the launcher.
-    `tiles`: `tile_weights(w, qkv_tile_rows(nq, nkv, d, device, rotation))`, read instead of w.
+    `tiles`: `qkv_tiles(w, nq, nkv, d, rotation)` or `tile_weights(w, qkv_tile_rows(nq, nkv, d, device, rotation))`, read instead of w.
     `rotation`: see `rope_split`."""
     n, K = a.shape
     _req(a, "qkv_rope_commit.a", torch.bfloat16)
     _req(w, "qkv_rope_commit.w", torch.bfloat16, ((nq + 2 * nkv) * d, K))
-    _req_tiles(tiles, (nq + 2 * nkv) * d, K, height=16)
+    height = _req_tiles(tiles, (nq + 2 * nkv) * d, K)
     _req(row_pos, "qkv_rope_commit.row_pos", torch.int32, (n,))
     rot = _rotation(rotation, d, "qkv_rope_commit")
     _req(q, "qkv_rope_commit.q", torch.bfloat16, (n, nq, d))
@@ -2332,7 +2341,7 @@ def qkv_rope_commit(a: torch.Tensor, w: torch.Tensor, row_pos, rotation, table, 
         if factor.ssq.numel() < factor.n_part * 16 or factor.n_part < 1:
             raise KernelError(f"qkv_rope_commit.factor: {factor.ssq.numel()} floats for {factor.n_part} workgroups")
         ssq_in, n_part, inv_h, eps = factor.ssq, factor.n_part, 1.0 / factor.size, factor.eps
-    _check(lib().tl_gemm_qkv_rope_commit(_p(a), _p(w), _p(tiles), n, K, _p(row_pos), _p(rot.inv_freq),
+    _check(lib().tl_gemm_qkv_rope_commit(_p(a), _p(w), _p(tiles), height, n, K, _p(row_pos), _p(rot.inv_freq),
                                          rot.rotary_dim, int(rot.interleaved), _p(table),
                                          table.shape[1], int(ring_pages), nq, nkv, d, _p(q), _p(pages),
                                          _p(ssq_in), n_part, ctypes.c_float(inv_h), ctypes.c_float(eps),
