@@ -64,6 +64,21 @@ def test_a_plan_covers_every_page_once_in_the_smallest_parts(ops, lengths, round
     assert at <= places and all(e[0] == -1 for e in plan[at:places]) and plan[places:] == [[-7] * 4] * 8
 
 
+@pytest.mark.parametrize("lengths,first,resident", [([64 * (i % 33) + 5 for i in range(64)], 32, 64), ([700] * 64, 32, 64), ([9, 1000], 1, 2),
+                                                    (list(range(1, 5121, 10)), 32, 64), ([500, 40, 3000], 3, 3), ([100 * i + 1 for i in range(45)], 32, 64)])
+@pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (300, 0, 0), (4096, 100, 0), (0, 0, 256)])
+def test_an_order_has_every_sequence_once_the_longest_beside_the_shortest(ops, lengths, first, resident, window, keep, chunk):
+    B, pos = len(lengths), [x - 1 for x in lengths]
+    plan = torch.full((B + 8, 4), -7, dtype=torch.int32, device=DEV)
+    row_pos = torch.tensor(pos, dtype=torch.int32, device=DEV)
+    ops._check(ops.lib().tl_attn_decode_order(ops._p(row_pos), B, window, keep, chunk, first, resident, ops._p(plan), ops._stream()))
+    n = [n_pages(p, window, keep, chunk) for p in pos]
+    ranks = sorted(range(B), key=lambda b: (-n[b], b))
+    end = min(B, resident)
+    want = ranks[:first] + ranks[first:end][::-1] + ranks[end:]
+    assert plan.tolist() == [[4 * b + 3, 0, n[b], pos[b]] for b in want] + [[-7] * 4] * 8
+
+
 def step(ops, lengths, nq, nkv, d, seed=0):
     g = torch.Generator(device=DEV).manual_seed(seed)
     width = -(-max(lengths) // PAGE) + 1
@@ -142,7 +157,23 @@ def test_attention_with_terms_in_planned_parts(ops, lengths, kind):
     assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs()) + 1e-5).all())
 
 
+@pytest.mark.parametrize("nq,nkv,d,B", [(32, 8, 128, 64), (32, 8, 128, 128), (16, 16, 256, 32), (16, 8, 64, 64)])
+def test_attention_in_an_order_has_the_bits_of_the_batch_s_own(ops, nq, nkv, d, B):
+    lengths = [1 + (i * 613) % 900 for i in range(B)]
+    q, pages, table, ctx = step(ops, lengths, nq, nkv, d)
+    places, seqs = ops.decode_plan(ctx, nq, nkv, d, table.shape[1], None)
+    assert seqs is None and tuple(places.shape) == (B, 4)
+    out, own = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    ops.attention(q, None, None, pages, table, table.shape[1], ctx, None, None, d ** -0.5, out)
+    part = torch.empty(B * nq * (d + 2), device=DEV)
+    ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, d ** -0.5, 1, part, own)
+    assert torch.equal(out, own)
+
+
 def test_who_goes_without_a_plan(ops):
+    assert ops.decode_places(32, 32, 8, 33, 256, 128) is None and ops.decode_places(48, 32, 8, 33, 256, 128) is None
+    assert ops.decode_places(64, 32, 8, 33, 256, 128) == (32, 64) and ops.decode_places(64, 512, 512, 33, 256, 128) is None
+    assert ops.decode_places(513, 4, 1, 33, 256, 128) is None
     assert ops.decode_rounds(1, 32, 8, 256, 128) is None and ops.decode_rounds(33, 32, 8, 256, 128) is None
     assert ops.decode_rounds(8, 32, 8, 256, 128) == (64, 1) and ops.decode_rounds(22, 32, 8, 256, 128) == (64, 3)
     assert ops.decode_rounds(513, 4, 1, 2048, 128) is None and ops.decode_rounds(4, 32, 32, 256, 256) == (8, 3)

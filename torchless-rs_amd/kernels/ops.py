@@ -2520,10 +2520,12 @@ def _decode_args(q, pages, table, row_pos, part, out, n_splits: int) -> None:
         raise KernelError(f"attn.pages: shape {tuple(pages.shape)}, kernel needs [*, 2, nkv, {PAGE}, {d}]")
     _req(table, "attn.table", torch.int32)
     _req(row_pos, "attn.row_pos", torch.int32, (B,))
-    _req(part, "attn.part", torch.float32)
     _req(out, "attn.out", torch.bfloat16, (B, nq, d))
     if table.dim() != 2 or table.shape[0] != B:
         raise KernelError("attn.table: needs one row per sequence")
+    if part is None:                                 # (nothing to merge)
+        return
+    _req(part, "attn.part", torch.float32)
     if part.numel() < B * nq * n_splits * (d + 2):
         raise KernelError(f"attn.part: {part.numel()} elements, kernel needs {B * nq * n_splits * (d + 2)}")
 
@@ -2608,16 +2610,40 @@ def decode_rounds(B: int, nq: int, nkv: int, units: int, head_dim: int):
     return places, (1 if 3 * B <= places else 3)
 
 
+def decode_places(B: int, nq: int, nkv: int, max_pages: int, units: int, head_dim: int):
+    """(first, resident) of the order of a decode step's whole sequences (`tl_attn_decode_order`): places, of a workgroup for each KV head
+    (16 query heads of its group), that the units hold one each, and as many as they can; or None where the batch's own order does.  It is
+    for steps whose keys stay whole (`decode_splits`) and whose workgroups are more than the units, so that some share one."""
+    per = decode_groups(1, nq, nkv)
+    if (not (2 <= B <= PLAN_SEQS and per <= units < B * per) or decode_rounds(B, nq, nkv, units, head_dim) is not None
+            or decode_splits(B, nq, nkv, max_pages, units, head_dim) != 1):
+        return None
+    return units // per, units * decode_workgroups_per_unit(head_dim) // per
+
+
 def decode_plan(ctx, nq: int, nkv: int, d: int, table_width: int, window: Optional[int], keep_first: int = 0, chunk: int = 0,
                 least: int = SPLIT_PAGES):
     """The plan of a single-token step's parts for layers of these sizes, made by the first of them (one small kernel, 4 us) and kept
-    while the step runs: (plan int32 [places, 4], seqs int32 [B, 2]), or None.  Tables of up to `least` pages go without:
+    while the step runs: (plan int32 [places, 4], seqs int32 [B, 2]), for whole sequences in an order (plan int32 [B, 4], None), or None.
+    Tables of up to `least` pages go without:
     up to SPLIT_PAGES the keys stay whole and there is no merge (19 sequences of 58 to 221 keys: 10.6 us, in parts 8.9 and 4.8 for the
     merge)."""
-    B = ctx.row_pos.shape[0]
-    shape = decode_rounds(B, nq, nkv, compute_units(ctx.row_pos.device), d)
-    if shape is None or table_width <= least or not lib().tl_attn_decode_takes_plan(d, int(table_width)):
+    B, units = ctx.row_pos.shape[0], compute_units(ctx.row_pos.device)
+    shape = decode_rounds(B, nq, nkv, units, d)
+    if table_width <= least or not lib().tl_attn_decode_takes_plan(d, int(table_width)):
         return None
+    if shape is None:
+        order = decode_places(B, nq, nkv, table_width, units, d)
+        if order is None:
+            return None
+        key = (("order",) + order, int(window or 0), int(keep_first) if window else 0, int(chunk or 0))
+        plans = ctx.host.setdefault("decode_plans", {})
+        if key not in plans:
+            plan = ctx.workspace.get("attn_plan_" + "_".join(map(str, key[0] + key[1:])), (B, 4), torch.int32)
+            _req(ctx.row_pos, "attn_decode_order.row_pos", torch.int32, (B,))
+            _check(lib().tl_attn_decode_order(_p(ctx.row_pos), B, *key[1:], *order, _p(plan), _stream()))
+            plans[key] = plan, None
+        return plans[key]
     key = (shape, int(window or 0), int(keep_first) if window else 0, int(chunk or 0))
     plans = ctx.host.setdefault("decode_plans", {})
     if key not in plans:
@@ -2637,8 +2663,10 @@ def attn_decode_planned(q, pages, table, ring_pages: int, ctx, plan, window: Opt
     nkv = pages.shape[2]
     places, seqs = plan
     _req(places, "attn_decode_planned.plan", torch.int32)
-    _req(seqs, "attn_decode_planned.seqs", torch.int32, (B, 2))
-    part = ctx.workspace.get("attn_part", (places.shape[0] * nq * (d + 2),), torch.float32)
+    part = None
+    if seqs is not None:
+        _req(seqs, "attn_decode_planned.seqs", torch.int32, (B, 2))
+        part = ctx.workspace.get("attn_part", (places.shape[0] * nq * (d + 2),), torch.float32)
     _decode_args(q, pages, table, ctx.row_pos, part, out, 1)
     slopes, sinks, gt = _terms_args(terms, gate, B, nq) if terms is not None else (None, None, None)
     more = (1, int(terms.keep_first or 0), terms.chunk) if terms is not None else (0, 0, 0)
