@@ -1,5 +1,6 @@
 """Each kernel alone against a plain float64 computation, at sizes other than
 the engine's tests use."""
+import ctypes
 import math
 
 import numpy as np
@@ -340,6 +341,25 @@ def test_gemm_plain_adds_in_one_order(ops, N, K):
     out = torch.empty(9, N, device=DEV)
     ops.gemm_plain(a[:9].contiguous(), shifted, out)          # not aligned: tiles of 32 x 32, a channel a load
     assert torch.equal(out, base[:9])
+
+
+@pytest.mark.parametrize("N,K", [(33, 32), (70, 96), (65, 4128), (131, 12320), (2, 1024)])
+@pytest.mark.parametrize("M", [5, 17, 48, 65, 80, 129, 300])
+def test_gemm_plain_on_the_matrix_cores_has_the_bits_of_one_row(ops, N, K, M):
+    """Tiles of one to eight blocks of rows, with and without all groups of K in one workgroup, ends of tiles and of K, rows further
+    apart in memory than K, large and tiny numbers: the bits of the kernel for a row alone."""
+    a, w = rnd(M, K, seed=45).to(DEV), rnd(N, K, seed=46).to(DEV)
+    a[0] *= 1e-20
+    w[0] *= 1e-20
+    a[-1] *= 1e15
+    out, one = torch.empty(M, N, device=DEV), torch.empty(1, N, device=DEV)
+    ops.gemm_plain(a, w, out)
+    direct = torch.empty(M, N, device=DEV)               # no scratch: one workgroup goes through all of K
+    ops._check(ops.lib().tl_gemm_plain(ops._p(a), 0, ops._p(w), 0, ops._p(direct), None, ctypes.c_longlong(0), M, N, K, K, K, N, 0, ops._stream()))
+    assert torch.equal(out, direct)
+    for m in {0, 1, M // 2, M - 1}:
+        ops.gemm_plain(a[m:m + 1].contiguous(), w, one)
+        assert torch.equal(out[m:m + 1], one), m
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 70_000_000, 4), (2, 70_000_001, 3), (4_190_000, 2080, 4)])

@@ -98,6 +98,9 @@ __host__ __device__ __forceinline__ void pair_channels(int i, int rotary_dim, in
   }
 }
 
+// compute units of the device (gemm_bf16.hip)
+int compute_units();
+
 // ---- error channel -------------------------------------------------------
 void set_error(const char* fmt, ...);
 

@@ -308,7 +308,7 @@ static int launch_skinny(const bf16* A, const bf16* W, float* C, int M, int N, i
   return 0;
 }
 
-static int compute_units() {
+int compute_units() {
   static int cus = 0;
   if (cus == 0) {
     int dev = 0, n = 0;

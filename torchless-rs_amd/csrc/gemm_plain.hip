@@ -9,18 +9,9 @@
 // channels; a run is summed over k in ascending order, a group over its runs, the result over its groups.
 // (The runs are what lets few rows spread over the chip: a chain of 8,192 additions in one thread is the
 // whole time of a product of one row.)
-#include "common.hpp"
+#include "gemm_f32.hpp"
 
 namespace tl {
-
-constexpr int PG = 8, PR = 8;                     // groups of K, runs of a group
-constexpr int BK = 16;                            // runs are a multiple of this long
-
-// A launch has fewer than 2^32 threads along x (more are not refused: some are left out), here 512 a workgroup; what has more
-// workgroups goes on along another dimension.
-constexpr long GRID_X = 1l << 22;
-
-__host__ __device__ __forceinline__ int run_length(int K) { return (K + PG * PR * BK - 1) / (PG * PR * BK) * BK; }
 
 // Few rows of floats: a workgroup of 8 waves has 8 outputs' rows of W and up to MR rows of A.  A wave has a group
 // of K, its lanes the 64 pairs of an output and a run of the group; a lane's chain is one run long.  W comes in
@@ -323,14 +314,18 @@ static int launch_rows(const float* A, const float* W, float* C, int M, int N, i
   return 0;
 }
 
-// The kernel for few rows reads W once for every 8 rows and has a thread's chain 64 times shorter than K; the tiles read
-// it once for 32.  Measured (rows / tiles, microseconds): N x K = 2,048 x 8,192 at 8 rows 32 / 65, at 16 52 / 68, at 32
-// 96 / 72; 3,072 x 2,048 at 8 14.4 / 18.6, at 16 21 / 19; 4,096 x 14,336 at 8 110 / 126, at 16 197 / 123; 16,384 x
-// 2,048 at 2 31 / 36, at 4 41 / 36; 32,000 x 2,048 at 2 58 / 65, at 4 76 / 65 (of up to four rows the latter two are `goes_on`'s now).
-static bool few_rows(int M, int N) { return M <= 2 || (M <= 16 && (long)M * N <= 32768); }
+// The kernel for few rows reads W once for every 8 rows and has a thread's chain 64 times shorter than K.  Against it, microseconds
+// (rows / tiles): the tiles on the matrix cores (`fit`), N x K = 2,048 x 2,048 at 8 rows 10 / 11, 3,072 x 2,048 at 4 10 / 12, at 6 13.8 / 12.2,
+// 2,048 x 8,192 at 4 24 / 26, at 6 30 / 26, 4,096 x 14,336 at 4 66 / 62, at 8 109 / 62; the tiles on the vector pipes, 2,048 x 8,192 at 8 rows
+// 32 / 65, at 16 52 / 68, at 32 96 / 72; 3,072 x 2,048 at 8 14.4 / 18.6, at 16 21 / 19; 4,096 x 14,336 at 8 110 / 126, at 16 197 / 123;
+// 16,384 x 2,048 at 2 31 / 36, at 4 41 / 36 (of up to four rows wide outputs are `goes_on`'s).
+static bool few_rows(int M, int N, int K, bool fit) {
+  if (fit) return M <= 4 || (M <= 8 && (long)M * N <= 16384 && K <= 4096);
+  return M <= 2 || (M <= 16 && (long)M * N <= 32768);
+}
 
 template <typename TA, typename TW>
-static int launch_plain(const void* Av, const void* Wv, float* C, int M, int N, int K, int lda, int ldw,
+static int launch_plain(const void* Av, const void* Wv, float* C, float* parts, int M, int N, int K, int lda, int ldw,
                         int ldc, int accumulate, hipStream_t st) {
   const TA* A = (const TA*)Av;
   const TW* W = (const TW*)Wv;
@@ -338,13 +333,15 @@ static int launch_plain(const void* Av, const void* Wv, float* C, int M, int N, 
                    (uintptr_t)W % (4 * sizeof(TW)) == 0;
   if (!vec) return launch_tiles<TA, TW, false>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
   if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4) {
-    if (few_rows(M, N) || (M <= 4 && goes_on(N, K))) {
+    const bool fit = f32_tiles_fit(A, W, K, lda, ldw);
+    if (few_rows(M, N, K, fit) || (M <= 4 && goes_on(N, K))) {
       if (M == 1) return launch_rows<1>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       if (M == 2) return launch_rows<2>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       if (M == 3) return launch_rows<3>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       if (M <= 4) return launch_rows<4>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
       return launch_rows<8>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
     }
+    if (fit) return f32_tiles(A, W, C, parts, M, N, K, lda, ldw, ldc, accumulate, st);
   }
   return launch_tiles<TA, TW, true>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
 }
@@ -355,20 +352,28 @@ using namespace tl;
 
 constexpr int MOST_ROWS = 65535 * 64;      // what callers have always been held to; the tiles' own limit is `launch_tiles`'
 
-extern "C" int tl_gemm_plain(const void* A, int a_dt, const void* W, int w_dt, float* C, int M, int N,
+// The floats of scratch that a product of 32-bit operands of these sizes can use (it goes without, but slower).
+extern "C" long long tl_gemm_plain_parts(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || few_rows(M, N, K, true) || f32_tiles_split(M, N, K) == 1) return 0;
+  return (long long)PG * M * N;
+}
+
+// parts: scratch of n_parts floats (null or too few: none), see tl_gemm_plain_parts.
+extern "C" int tl_gemm_plain(const void* A, int a_dt, const void* W, int w_dt, float* C, float* parts, long long n_parts, int M, int N,
                              int K, int lda, int ldw, int ldc, int accumulate, hipStream_t st) {
   TL_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
   TL_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: leading dimensions lda=%d ldw=%d ldc=%d too small "
              "for K=%d N=%d", lda, ldw, ldc, K, N);
   TL_REQUIRE(M <= MOST_ROWS, "gemm: M=%d, products have at most %d rows", M, MOST_ROWS);
   if (M == 0) return 0;
+  if (n_parts < (long long)PG * M * N || (uintptr_t)parts % 16 != 0) parts = nullptr;
   if (a_dt == DT_F32 && w_dt == DT_F32)
-    return launch_plain<float, float>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+    return launch_plain<float, float>(A, W, C, parts, M, N, K, lda, ldw, ldc, accumulate, st);
   if (a_dt == DT_BF16 && w_dt == DT_BF16)
-    return launch_plain<bf16, bf16>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+    return launch_plain<bf16, bf16>(A, W, C, parts, M, N, K, lda, ldw, ldc, accumulate, st);
   if (a_dt == DT_BF16 && w_dt == DT_F32)
-    return launch_plain<bf16, float>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+    return launch_plain<bf16, float>(A, W, C, parts, M, N, K, lda, ldw, ldc, accumulate, st);
   if (a_dt == DT_F32 && w_dt == DT_BF16)
-    return launch_plain<float, bf16>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, st);
+    return launch_plain<float, bf16>(A, W, C, parts, M, N, K, lda, ldw, ldc, accumulate, st);
   TL_REQUIRE(false, "gemm: unknown dtype codes a=%d w=%d", a_dt, w_dt);
 }

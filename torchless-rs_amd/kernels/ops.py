@@ -34,6 +34,7 @@ def lib() -> ctypes.CDLL:
     L = load()
     if not _configured:
         L.tl_last_error.restype = ctypes.c_char_p
+        L.tl_gemm_plain_parts.restype = ctypes.c_longlong
         require_same(L.tl_page_size(), "the kernels' library")
         _configured = True
     return L
@@ -1740,7 +1741,12 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: 
     _req(a, "gemm.a")
     _req(w, "gemm.w", None, (N, K))
     _req(out, "gemm.out", torch.float32, (M, N))
-    _check(lib().tl_gemm_plain(_p(a), _code(a.dtype), _p(w), _code(w.dtype), _p(out), M, N, K, K, K, N,
+    n_parts, parts = 0, None
+    if a.dtype == torch.float32 and w.dtype == torch.float32 and M > 4:
+        n_parts = lib().tl_gemm_plain_parts(M, N, K)
+        if n_parts:                                      # the sums of eight groups of K, added up in their order
+            parts = torch.empty((n_parts,), dtype=torch.float32, device=a.device)
+    _check(lib().tl_gemm_plain(_p(a), _code(a.dtype), _p(w), _code(w.dtype), _p(out), _p(parts), ctypes.c_longlong(n_parts), M, N, K, K, K, N,
                                int(accumulate), _stream()))
 
 
