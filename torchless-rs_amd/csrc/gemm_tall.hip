@@ -14,7 +14,7 @@ struct Tall {
   int M, N, K, lda, ldw;
   int mt, nt;                  // tiles along the rows and the channels
   int share;                   // rows of a tile (the last may have fewer)
-  int stages;                  // of 64 k, a split's
+  int splits, stages;          // slices of K, and a slice's stages of 64 k
   int stagger;                 // tiles of other channels begin with other stages
   int whole, parts;            // the tiles behind the first `whole` ones are cut in `parts` (2 or 4); 0: none is
   Epi epi;
@@ -28,13 +28,13 @@ constexpr int TALL_UNARY = 6, TALL_GATED = 7;   // epilogues beside those of `Ep
 
 constexpr int TALL_GROUP = 8;  // tiles of rows that go side by side through the channels
 
-// m_rows rows from m0 by the channels from n0 on
+// m_rows rows from m0 by the channels from n0 on, slice `split` of K
 template <int WN, int MU, int NA, int NW, int W_AUX>
-__device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int n0, int first, unsigned char* smem) {
+__device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int n0, int split, int first, unsigned char* smem) {
   using S = TileShape<WN, MU>;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, li = lane % 16, kg = lane / 16;
   const int wm = wave / WN, wn = wave % WN, sub = lane / 8;
-  const int t0 = blockIdx.y * g.stages, n_t = min((g.K + TILE_K - 1) / TILE_K - t0, g.stages);
+  const int t0 = split * g.stages, n_t = min((g.K + TILE_K - 1) / TILE_K - t0, g.stages);
   // a lane's rows as distances from the first of the tile's that its wave loads: at most 256 rows of K.  Gate and up rows that lie
   // apart go by 32 in turn, four waves' loads each: of all its loads a wave has gate rows or up rows.
   const char* A0 = reinterpret_cast<const char*>(g.A + (size_t)m0 * g.lda);
@@ -103,7 +103,7 @@ __device__ __forceinline__ void tall_tile(const Tall& g, int m0, int m_rows, int
     }
     return;
   }
-  float* C = g.C + (size_t)blockIdx.y * g.M * g.N + (size_t)m0 * g.N;
+  float* C = g.C + (size_t)split * g.M * g.N + (size_t)m0 * g.N;
   if (g.epi == EPI_ACCUMULATE) {               // what is added to comes from memory for several blocks of rows at a time
     constexpr int UB = MU < 7 ? 4 : 2;                   // (in the registers that the operands had)
 #pragma unroll
@@ -137,13 +137,14 @@ gemm_tall_kernel(Tall g) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tall_smem[];
   constexpr int CHANNELS = TileShape<WN, MU>::CHANNELS;
   // each of the 8 XCDs (workgroups go round them) has a run of tiles of its own; the tiles go by groups of TALL_GROUP of rows, in
-  // a group from channels to channels, so that an XCD's workgroups share rows and channels in its L2
-  const int total = g.mt * g.nt, whole = PARTS ? g.whole : total;
+  // a group from channels to channels, so that an XCD's workgroups share rows and channels in its L2.  Where K is cut, a slice's tiles
+  // follow each other: an XCD then reads a slice or two of A instead of all of it.
+  const int total = g.mt * g.nt, whole = PARTS ? g.whole : total * g.splits;
   const bool cut = PARTS && (int)blockIdx.x >= whole;          // (whole is a multiple of 8 where tiles are cut)
   const int id = cut ? blockIdx.x - whole : blockIdx.x, count = cut ? (total - whole) * g.parts : whole;
   const int chunk = (count + 7) / 8, at = id % 8 * chunk + id / 8;
   if (id / 8 >= chunk || at >= count) return;
-  const int t = cut ? whole + at / g.parts : at;
+  const int split = PARTS ? 0 : at / total, t = cut ? whole + at / g.parts : at - split * total;
   const int group = t / (TALL_GROUP * g.nt), gm = group * TALL_GROUP, gs = min(TALL_GROUP, g.mt - gm), in = t - gm * g.nt;
   const int nb = in / gs, m0 = (gm + in % gs) * g.share, m_rows = min(g.share, g.M - m0), n0 = nb * CHANNELS;
   if constexpr (PARTS) {
@@ -151,21 +152,21 @@ gemm_tall_kernel(Tall g) {
       const int part = at % g.parts, n1 = n0 + part % 2 * (CHANNELS / 2);
       if (n1 >= g.N) return;
       if (g.parts == 2) {
-        tall_tile<WN / 2, 4, 4, 2, W_AUX>(g, m0, m_rows, n1, 0, tall_smem);
+        tall_tile<WN / 2, 4, 3, 4, W_AUX>(g, m0, m_rows, n1, 0, 0, tall_smem);
       } else {
         const int upper = (m_rows + 31) / 32 * 16, m1 = part / 2 * upper;
-        if (m1 < m_rows) tall_tile<WN / 2, 2, 5, 5, W_AUX>(g, m0 + m1, part / 2 ? m_rows - upper : upper, n1, 0, tall_smem);
+        if (m1 < m_rows) tall_tile<WN / 2, 2, 5, 5, W_AUX>(g, m0 + m1, part / 2 ? m_rows - upper : upper, n1, 0, 0, tall_smem);
       }
       return;
     }
   }
-  tall_tile<WN, MU, NA, NW, W_AUX>(g, m0, m_rows, n0, g.stagger ? nb : 0, tall_smem);
+  tall_tile<WN, MU, NA, NW, W_AUX>(g, m0, m_rows, n0, split, g.stagger ? nb : 0, tall_smem);
 }
 
 template <int WN, int MU, int NA, int NW, int W_AUX, bool PARTS = false> static int launch_tall(Tall g, int n_split, hipStream_t st) {
   using S = TileShape<WN, MU>;
   constexpr int LDS = PARTS ? 160 * 1024 : tile_lds<WN, MU, NA, NW>();
-  static_assert(LDS <= 160 * 1024 && tile_lds<2, 4, 4, 2>() <= 160 * 1024 && tile_lds<2, 2, 5, 5>() <= 160 * 1024, "a compute unit's LDS");
+  static_assert(LDS <= 160 * 1024 && tile_lds<2, 4, 3, 4>() <= 160 * 1024 && tile_lds<2, 2, 5, 5>() <= 160 * 1024, "a compute unit's LDS");
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tall_kernel<WN, MU, NA, NW, W_AUX, PARTS>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) {
@@ -175,11 +176,12 @@ template <int WN, int MU, int NA, int NW, int W_AUX, bool PARTS = false> static 
   g.mt = (int)(((long)g.M + S::ROWS - 1) / S::ROWS);
   g.nt = (int)(((long)g.N + S::CHANNELS - 1) / S::CHANNELS);
   g.share = ((g.M + g.mt - 1) / g.mt + 15) / 16 * 16;
+  g.splits = n_split;
   const long tiles = (long)g.mt * g.nt;
   TL_REQUIRE(!PARTS || (g.whole % 8 == 0 && g.whole >= 0 && g.whole <= tiles), "gemm_tall: %d of %ld tiles whole (a multiple of 8)", g.whole, tiles);
-  const long grid = PARTS ? g.whole + ((tiles - g.whole) * g.parts + 7) / 8 * 8 : (tiles + 7) / 8 * 8;
+  const long grid = PARTS ? g.whole + ((tiles - g.whole) * g.parts + 7) / 8 * 8 : (tiles * n_split + 7) / 8 * 8;
   TL_REQUIRE(grid * TILE_WAVES * WAVE < (1l << 32), "gemm_tall: M=%d N=%d have more tiles than a grid holds", g.M, g.N);
-  gemm_tall_kernel<WN, MU, NA, NW, W_AUX, PARTS><<<dim3((unsigned)grid, n_split), TILE_WAVES * WAVE, LDS, st>>>(g);
+  gemm_tall_kernel<WN, MU, NA, NW, W_AUX, PARTS><<<(unsigned)grid, TILE_WAVES * WAVE, LDS, st>>>(g);
   TL_LAUNCH_CHECK("gemm_tall");
   return 0;
 }
@@ -205,7 +207,7 @@ static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipSt
   TL_REQUIRE(!(is_pair(epilogue) || epilogue == TALL_GATED) || N % 64 == 0, "gemm_tall: the paired epilogue needs N=%d to be a multiple of 64", N);
   const int stages = (K + TILE_K - 1) / TILE_K, per = (stages + n_split - 1) / (n_split > 0 ? n_split : 1);
   TL_REQUIRE(n_split >= 1 && n_split <= 65535 && (long)(n_split - 1) * per < stages, "gemm_tall: %d splits of K=%d would leave one without a stage", n_split, K);
-  TL_REQUIRE(!stagger || (n_split == 1 && K % TILE_K == 0), "gemm_tall: stages in turn need K=%d uncut and a multiple of %d", K, TILE_K);
+  TL_REQUIRE(!stagger || K % TILE_K == 0, "gemm_tall: stages in turn need K=%d a multiple of %d", K, TILE_K);
   TL_REQUIRE(parts == 0 || ((parts == 2 || parts == 4) && n_split == 1 && channels == 256 && !once && !stagger && whole >= 0),
              "gemm_tall: tiles in %d parts (2 or 4, of 256 channels, K not cut)", parts);
   g.stages = per;
@@ -222,7 +224,8 @@ static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipSt
 #define TL_TALL(R, MU, NA, NW)                                                                 \
   if (rows == R && channels == 128)                                                            \
     return once ? launch_tall<2, MU, NA, NW, 2>(g, n_split, st) : launch_tall<2, MU, NA, NW, 0>(g, n_split, st);
-  TL_TALL(256, 4, 4, 2)
+  // (W, from memory, three stages ahead and A, from L2, two: 226 rows by 28,672, K = 4,096, 60 us; A three and W one ahead 71, A one and W five 70)
+  TL_TALL(256, 4, 3, 4)
   TL_TALL(192, 3, 4, 4)
   TL_TALL(128, 2, 5, 5)
 #undef TL_TALL
