@@ -362,6 +362,43 @@ def test_gemm_plain_on_the_matrix_cores_has_the_bits_of_one_row(ops, N, K, M):
         assert torch.equal(out[m:m + 1], one), m
 
 
+@pytest.mark.parametrize("K", [4, 100, 516, 1024, 1500, 2048])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+def test_products_with_what_stands_around_them_have_the_bits_of_the_kernels(ops, M, K):
+    """Few rows in 32 bits: the norm before a product, the gate or the rotation and commit behind it, more outputs than workgroups and fewer,
+    pairs of both kinds, heads turned in part or not at all; refused beyond the sizes."""
+    from torchless_rs_amd.parts.base import RmsForm
+    a = (rnd(M, K, seed=50) * 3.0).to(DEV)
+    norm = RmsForm(rnd(K, seed=51).to(DEV), K, 1e-5)
+    y = torch.empty_like(a)
+    ops.rmsnorm(a, norm.weight, norm.eps, y)
+    for I, act, consts in ((4, "silu", None), (36, "gelu_tanh", None), (2080, "swish_clamped", {"alpha": 1.7, "limit": 2.0, "shift": 1.0})):
+        w, gu = rnd(2 * I, K, seed=53, scale=0.3).to(DEV), torch.empty(M, 2 * I, device=DEV)
+        for n, src in ((norm, y), (None, a)):
+            want, got = torch.empty(M, I, device=DEV), torch.full((M, I), float("nan"), device=DEV)
+            ops.gemm_plain(src, w, gu)
+            ops.act_mul(gu, want, act, consts)
+            ops.gemm_plain_pair(a, w, got, act, consts, norm=n)
+            assert torch.equal(got, want), (I, act)
+    for nq, nkv, d, rotary, interleaved, window in ((6, 2, 48, 48, False, 70), (3, 1, 8, 4, True, None), (2, 2, 128, 64, False, None), (30, 2, 128, 0, False, None)):
+        c = paged_case(ops, "float32", nq, nkv, d, window, lens_cached=[0, 63, 64, 300][:M], lens_new=[1] * M, seed=54)
+        w, qkv = rnd((nq + 2 * nkv) * d, K, seed=55, scale=0.2).to(DEV), torch.empty(M, (nq + 2 * nkv) * d, device=DEV)
+        rot = ops.Rotation((777.0 ** -(torch.arange(rotary // 2) / max(rotary // 2, 1))).to(DEV) if rotary else None, rotary, interleaved)
+        for n, src in ((norm, y), (None, a)):
+            q1, q2 = torch.empty(M, nq, d, device=DEV), torch.full((M, nq, d), float("nan"), device=DEV)
+            pages1, pages2 = c["pages"].clone(), c["pages"].clone()
+            ops.gemm_plain(src, w, qkv)
+            ops.rope_commit(qkv, c["row_pos"], rot, c["table"], c["ring"], nq, nkv, d, q1, pages1)
+            ops.gemm_plain_rope(a, w, c["row_pos"], rot, c["table"], c["ring"], nq, nkv, d, q2, pages2, norm=n)
+            assert torch.equal(q1, q2)
+            assert torch.equal(torch.nan_to_num(pages1, nan=-7.0), torch.nan_to_num(pages2, nan=-7.0))
+    assert ops.plain_around_ok(a, w) and not ops.plain_around_ok(torch.zeros(5, K, device=DEV), w)
+    with pytest.raises(ops.KernelError, match="one to four rows"):
+        ops.gemm_plain_pair(torch.zeros(5, K, device=DEV), w, torch.empty(5, w.shape[0] // 2, device=DEV))
+    with pytest.raises(ops.KernelError, match="one to four rows"):
+        ops.gemm_plain_pair(torch.zeros(1, 2052, device=DEV), torch.zeros(8, 2052, device=DEV), torch.empty(1, 4, device=DEV))
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 70_000_000, 4), (2, 70_000_001, 3), (4_190_000, 2080, 4)])
 def test_gemm_plain_of_more_tiles_than_a_grid_is_wide(ops, M, N, K):
     """One launch has fewer than 2^32 threads along x: what lies behind them is there too."""

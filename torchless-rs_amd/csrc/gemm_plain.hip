@@ -9,6 +9,7 @@
 // channels; a run is summed over k in ascending order, a group over its runs, the result over its groups.
 // (The runs are what lets few rows spread over the chip: a chain of 8,192 additions in one thread is the
 // whole time of a product of one row.)
+#include "gated.hpp"
 #include "gemm_f32.hpp"
 
 namespace tl {
@@ -95,49 +96,153 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
 }
 
 // The same bits for one to four rows, K up to 2,048 and many outputs: a workgroup goes through a run of eights of outputs, the next
-// eight's pieces under way while it sums the last's, and a lane keeps its run of A, one piece long, in registers.  With an
+// eights' pieces under way while it sums the last's, and a lane keeps its run of A, one piece long, in registers.  With an
 // eight a workgroup every workgroup waited for memory once and did nothing meanwhile, and read A from L1 for each.  One / two rows,
-// before and now: 16,384 x 2,048 28.5 / 32.8 and 24.5 / 25.9 us, 32,000 x 2,048 52.2 / 60.0 and 42.9 / 44.0 (5.95 TB/s); three / four rows, which
-// took tiles, 39.9 / 38.6 and 26.6 / 29.5, 75.3 / 69.0 and 45.4 / 47.4.  With fewer
-// eights than workgroups there is nothing to go on to (3,072 x 2,048 9.0 us at two rows, 10.1 so).
-constexpr int ROWS_WORKGROUPS = 512;              // two a compute unit (74 KB of LDS each), so that all run at once
-template <int MR, bool ACCUMULATE, bool LINES>
-__global__ void __launch_bounds__(512)
+// an eight a workgroup and so: 16,384 x 2,048 28.5 / 32.8 and 25 / 26.2 us, 32,000 x 2,048 52.2 / 60.0 and 44.5 / 46 (5.8 TB/s); three / four rows, which
+// took tiles, 39.9 / 38.6 and 27.6 / 25.8, 75.3 / 69.0 and 48 / 45.  With fewer
+// eights than workgroups there is nothing to go on to (3,072 x 2,048 8.2 us at two rows, 9.3 so).
+// At one row two workgroups of 128 registers lie on a compute unit; with more rows' A it is one, of at most 256, which fetches two eights
+// ahead where the registers last (16,384 x 2,048: two rows 29.6 us with 512 workgroups and one eight ahead, 27.9 with 256, 26.2 with two
+// ahead; four rows 30.1 and 25.8 with 256, 45 with two ahead, which spills).
+//
+// Around the product it can do what stands next to it in a step of single tokens, with the bits of the kernels of their own:
+//   * the RMS norm of A's rows (`rmsnorm_reg_kernel`'s sums), by every workgroup for itself while its first weights are under way;
+//   * PAIR: act(gate) * up, an eight being four gates and the four ups that belong to them;
+//   * ROPE: the rotation of q and k, q into its rows and k, v into their pages (`rope_commit_kernel`); an eight is four pairs of channels.
+// Each of these was a launch that moved some KB.  Microseconds at one / two / four rows, launches of their own and so: norm, 16,384 x
+// 2,048 and gate 31.6 / 31.4 / 31.1 and 26.9 / 28.8 / 30.1; norm, 3,072 x 2,048 and rotation 12.5 / 14.0 / 17.8 and 9.8 / 11.1 / 13.0; at
+// K = 1,024, 8,192 outputs 14.3 / 17.0 / 17.1 and 11.5 / 14.2 / 15.0.
+constexpr int ROWS_WORKGROUPS = 512;
+constexpr int short_ahead(int mr) { return mr == 2 || mr == 3 ? 2 : 1; }
+constexpr int short_workgroups(int mr) { return mr == 1 ? ROWS_WORKGROUPS : ROWS_WORKGROUPS / 2; }
+enum { DO_STORE, DO_ADD, DO_PAIR, DO_ROPE };
+struct Around {
+  const float* norm_w;                            // [K], or null: A's rows as they are
+  float eps;
+  int act;                                        // PAIR: W is [gate | up] by rows, C [M, N / 2]
+  ActConstants constants;
+  const int* row_pos;                             // ROPE: W is [q | k | v] by rows
+  Rotation rot;
+  const int* table;
+  int table_stride, ring_pages, nq, nkv, d;
+  float *q, *pages;
+};
+template <int MR, int DO, bool LINES>
+__global__ void __launch_bounds__(512, MR == 1 ? 4 : 2)
 gemm_plain_short_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int N, int K, int lda, int ldw,
-                        int ldc) {
+                        int ldc, Around f) {
   __shared__ float stage[PG][64][CHUNK + 4];      // rows 144 bytes apart: 16-byte reads of 64 rows spread over the banks
   __shared__ float sums[2][PG][MR][8];            // of this eight, and of the one before, which others may still read
+  __shared__ float squares[MR][4];
+  constexpr int AHEAD = short_ahead(MR);
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const long eights = (N - 1) / 8 + 1;
   const int from = (int)(blockIdx.x * eights / gridDim.x), to = (int)((blockIdx.x + 1) * eights / gridDim.x);
   const int L = run_length(K);                    // at most CHUNK
   const int run = lane / 8;                       // of this lane's pair: output lane % 8, run lane / 8
   const int k0 = (wave * PR + run) * L;
+  // the row of W of an eight's output o; ROPE: pair 4 (eight % (d / 8)) + o % 4 of a head, its first channel or its second
+  const auto row_of = [&](int eight, int o) {
+    if constexpr (DO == DO_PAIR) return o < 4 ? 4 * eight + o : N / 2 + 4 * eight + o - 4;
+    if constexpr (DO == DO_ROPE) {
+      const int per = f.d / 8, head = eight / per;
+      int a, b;
+      pair_channels((eight - head * per) * 4 + o % 4, f.rot.rotary_dim, f.rot.interleaved, a, b);
+      return head * f.d + (o < 4 ? a : b);
+    }
+    return eight * 8 + o;
+  };
   // a load brings 128 bytes of 8 pairs: pair 8 i + lane / 8 (output lane / 8 of run i), 4 channels from 4 (lane % 8)
   const int lq = (lane % 8) * 4;
-  f32x4 next[8];
-  const auto fetch = [&](int eight) {
-    const int ln = eight * 8 + lane / 8;
+  f32x4 next[AHEAD][8];
+  const auto fetch = [&](f32x4 (&into)[8], int eight) {
+    const int ln = row_of(eight, lane / 8);
     const float* wp = W + (size_t)min(ln, N - 1) * ldw;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int k = (wave * PR + i) * L + lq;
-      next[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (lq < L && k < K && ln < N) next[i] = LINES ? __builtin_nontemporal_load((const f32x4*)(wp + k)) : *(const f32x4*)(wp + k);
+      into[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (lq < L && k < K && ln < N) into[i] = LINES ? __builtin_nontemporal_load((const f32x4*)(wp + k)) : *(const f32x4*)(wp + k);
     }
   };
-  if (from < to) fetch(from);
+#pragma unroll
+  for (int b = 0; b < AHEAD; ++b)
+    if (from + b < to) fetch(next[b], from + b);
+  // ROPE: the sine and cosine that the thread of output threadIdx.x % 8 of row threadIdx.x / 8 needs at the end of an eight
+  const int row = threadIdx.x / 8, out = threadIdx.x % 8;
+  float sn = 0.f, cs = 1.f;
+  int pos = 0, page = 0;
+  if (DO == DO_ROPE && row < MR) {
+    pos = f.row_pos[row];
+    page = f.table[(size_t)row * f.table_stride + (pos / PAGE) % f.ring_pages];
+  }
+  const auto angle = [&](int eight) {
+    if (row >= MR) return;
+    const int per = f.d / 8, head = eight / per, pair = (eight - head * per) * 4 + out % 4;
+    if (head < f.nq + f.nkv && 2 * pair < f.rot.rotary_dim) sincosf(f.rot.inv_freq[pair] * (float)pos, &sn, &cs);
+  };
+  const float* a_rows = A;
+  int a_stride = lda;
+  if (DO >= DO_PAIR && f.norm_w != nullptr) {      // four waves a row; the normed rows take the stage's place for a while
+    constexpr int MINE = (MR + 1) / 2;
+    const int t = threadIdx.x % 256, nv = K / 4;  // (K is at most 2,048)
+    const float4* wr = reinterpret_cast<const float4*>(f.norm_w);
+    float4 v[MINE][2], g[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (t + 256 * i < nv) g[i] = wr[t + 256 * i];
+#pragma unroll
+    for (int h = 0; h < MINE; ++h) {
+      const int m = 2 * h + wave / 4;
+      if (m >= MR) continue;
+      const float4* xr = reinterpret_cast<const float4*>(A + (size_t)m * lda);
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int c = t + 256 * i;
+        if (c < nv) {
+          v[h][i] = xr[c];
+          ss += v[h][i].x * v[h][i].x + v[h][i].y * v[h][i].y + v[h][i].z * v[h][i].z + v[h][i].w * v[h][i].w;
+        }
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) squares[m][wave % 4] = ss;
+    }
+    __syncthreads();
+    float* y = &stage[0][0][0];
+#pragma unroll
+    for (int h = 0; h < MINE; ++h) {
+      const int m = 2 * h + wave / 4;
+      if (m >= MR) continue;
+      float r = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r += squares[m][i];
+      const float rms = sqrtf(r / (float)K + f.eps);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int c = t + 256 * i;
+        if (c < nv)
+          *reinterpret_cast<float4*>(y + m * K + 4 * c) =
+              make_float4((v[h][i].x / rms) * g[i].x, (v[h][i].y / rms) * g[i].y, (v[h][i].z / rms) * g[i].z, (v[h][i].w / rms) * g[i].w);
+      }
+    }
+    __syncthreads();
+    a_rows = y;
+    a_stride = K;
+  }
   f32x4 a[MR][CHUNK / 4];                         // (what lies past the run or past K is 0 times 0)
 #pragma unroll
   for (int q = 0; q < CHUNK / 4; ++q)
 #pragma unroll
     for (int m = 0; m < MR; ++m)
-      a[m][q] = 4 * q < L && k0 + 4 * q < K ? *(const f32x4*)(A + (size_t)m * lda + k0 + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int eight = from; eight < to; ++eight) {
+      a[m][q] = 4 * q < L && k0 + 4 * q < K ? *(const f32x4*)(a_rows + (size_t)m * a_stride + k0 + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+  if (DO >= DO_PAIR && f.norm_w != nullptr) __syncthreads();
+  if (DO == DO_ROPE && from < to) angle(from);
+  const auto go = [&](f32x4 (&pieces)[8], int eight) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) *(f32x4*)&stage[wave][i * 8 + lane / 8][lq] = next[i];
+    for (int i = 0; i < 8; ++i) *(f32x4*)&stage[wave][i * 8 + lane / 8][lq] = pieces[i];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    if (eight + 1 < to) fetch(eight + 1);
+    if (eight + AHEAD < to) fetch(pieces, eight + AHEAD);
     float acc[MR];
 #pragma unroll
     for (int m = 0; m < MR; ++m) acc[m] = 0.f;
@@ -160,15 +265,38 @@ gemm_plain_short_kernel(const float* __restrict__ A, const float* __restrict__ W
       if (lane < 8) mine[wave][m][lane] = g;
     }
     __syncthreads();
-    const int m = threadIdx.x / 8, n = eight * 8 + threadIdx.x % 8;
-    if (m < MR && n < N) {
+    const int n = row_of(eight, out);
+    if (row < MR && n < N) {
       float t = 0.f;
 #pragma unroll
-      for (int g = 0; g < PG; ++g) t += mine[g][m][threadIdx.x % 8];
-      float* c = C + (size_t)m * ldc + n;
-      *c = ACCUMULATE ? *c + t : t;
+      for (int g = 0; g < PG; ++g) t += mine[g][row][out];
+      if constexpr (DO == DO_PAIR) {
+        const float up = __shfl_xor(t, 4, WAVE);
+        if (out < 4) C[(size_t)row * ldc + n] = gate_times_up(t, up, f.act, f.constants);
+      } else if constexpr (DO == DO_ROPE) {
+        const float other = __shfl_xor(t, 4, WAVE);
+        const int head = n / f.d, c = n - head * f.d, pair = (eight - head * (f.d / 8)) * 4 + out % 4;
+        if (head < f.nq + f.nkv && 2 * pair < f.rot.rotary_dim) {
+          float ra, rb;
+          rotate_pair(out < 4 ? t : other, out < 4 ? other : t, cs, sn, ra, rb);
+          t = out < 4 ? ra : rb;
+        }
+        float* kd = f.pages + (size_t)page * 2 * f.nkv * PAGE * f.d;
+        const int r = pos % PAGE;
+        if (head < f.nq) f.q[((size_t)row * f.nq + head) * f.d + c] = t;
+        else if (head < f.nq + f.nkv) kd[((size_t)(head - f.nq) * PAGE + r) * f.d + c] = t;
+        else kd[(size_t)f.nkv * PAGE * f.d + ((size_t)(head - f.nq - f.nkv) * f.d + c) * PAGE + r] = t;
+      } else {
+        float* c = C + (size_t)row * ldc + n;
+        *c = DO == DO_ADD ? *c + t : t;
+      }
     }
-  }
+    if (DO == DO_ROPE && eight + 1 < to) angle(eight + 1);
+  };
+  for (int eight = from; eight < to; eight += AHEAD)
+#pragma unroll
+    for (int b = 0; b < AHEAD; ++b)
+      if (eight + b < to) go(next[b], eight + b);
 }
 
 // 32 x 32 outputs a workgroup of 8 waves, each with a group of K and 4 x 4 outputs a lane, operands through the wave's
@@ -280,19 +408,43 @@ static int launch_tiles(const TA* A, const TW* W, float* C, int M, int N, int K,
 // gemm_plain_short_kernel's sizes (of one to four rows)
 static bool goes_on(int N, int K) { return run_length(K) <= CHUNK && ((long)N + 7) / 8 > ROWS_WORKGROUPS; }
 
+// (a run that is no multiple of 32 channels, or rows off whole lines, would take lines in halves: those are to stay in the caches)
+static bool whole_lines(const float* W, int K, int ldw) { return ldw % 32 == 0 && run_length(K) % 32 == 0 && (uintptr_t)W % 128 == 0; }
+
+// one to four rows of K up to 2,048 with what `f` does around the product
+template <int DO>
+static int launch_around(const char* what, const float* A, const float* W, float* C, int M, int N, int K, int ldc, const Around& f, hipStream_t st) {
+  TL_REQUIRE(M > 0 && M <= 4 && N > 0 && K > 0 && K % 4 == 0 && run_length(K) <= CHUNK, "%s: M=%d N=%d K=%d (one to four rows of at most %d channels)", what, M,
+             N, K, CHUNK * PG * PR);
+  TL_REQUIRE(A && W && ((uintptr_t)A | (uintptr_t)W | (uintptr_t)f.norm_w) % 16 == 0, "%s: operands must be 16-byte aligned", what);
+  const int grid = (int)min(((long)N + 7) / 8, (long)short_workgroups(M));
+  const bool lines = whole_lines(W, K, K);
+#define TL_AROUND(MR)                                                                                            \
+  do {                                                                                                           \
+    if (lines) gemm_plain_short_kernel<MR, DO, true><<<grid, 512, 0, st>>>(A, W, C, N, K, K, K, ldc, f);          \
+    else gemm_plain_short_kernel<MR, DO, false><<<grid, 512, 0, st>>>(A, W, C, N, K, K, K, ldc, f);               \
+  } while (0)
+  if (M == 1) TL_AROUND(1);
+  else if (M == 2) TL_AROUND(2);
+  else if (M == 3) TL_AROUND(3);
+  else TL_AROUND(4);
+#undef TL_AROUND
+  TL_LAUNCH_CHECK(what);
+  return 0;
+}
+
 template <int MR>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                        int accumulate, hipStream_t st) {
   const long groups = ((long)N + 7) / 8;
   if constexpr (MR <= 4) {
-    // (a run that is no multiple of 32 channels, or rows off whole lines, would take lines in halves: those are to stay in the caches)
-    const bool lines = ldw % 32 == 0 && run_length(K) % 32 == 0 && (uintptr_t)W % 128 == 0;
+    const bool lines = whole_lines(W, K, ldw);
     if (goes_on(N, K) && M == MR) {
-#define TL_SHORT(ACC, LN) gemm_plain_short_kernel<MR, ACC, LN><<<ROWS_WORKGROUPS, 512, 0, st>>>(A, W, C, N, K, lda, ldw, ldc)
-      if (accumulate && lines) TL_SHORT(true, true);
-      else if (accumulate) TL_SHORT(true, false);
-      else if (lines) TL_SHORT(false, true);
-      else TL_SHORT(false, false);
+#define TL_SHORT(DO, LN) gemm_plain_short_kernel<MR, DO, LN><<<short_workgroups(MR), 512, 0, st>>>(A, W, C, N, K, lda, ldw, ldc, Around{})
+      if (accumulate && lines) TL_SHORT(DO_ADD, true);
+      else if (accumulate) TL_SHORT(DO_ADD, false);
+      else if (lines) TL_SHORT(DO_STORE, true);
+      else TL_SHORT(DO_STORE, false);
 #undef TL_SHORT
       TL_LAUNCH_CHECK("gemm_plain_short");
       return 0;
@@ -376,4 +528,31 @@ extern "C" int tl_gemm_plain(const void* A, int a_dt, const void* W, int w_dt, f
   if (a_dt == DT_F32 && w_dt == DT_BF16)
     return launch_plain<float, bf16>(A, W, C, parts, M, N, K, lda, ldw, ldc, accumulate, st);
   TL_REQUIRE(false, "gemm: unknown dtype codes a=%d w=%d", a_dt, w_dt);
+}
+
+// out[m, i] = act(g_i) * u_i of g|u = norm(A[m]) W^T (norm_w null: of A itself), W [2 I, K]; the codes of `act` are tl_act_mul's
+extern "C" int tl_gemm_plain_pair(const float* A, const float* norm_w, float eps, const float* W, int act, float alpha, float limit, float shift,
+                                  float* out, int M, int I, int K, hipStream_t st) {
+  TL_REQUIRE(out && I > 0 && I % 4 == 0 && I < (1 << 30), "gemm_plain_pair: I=%d (a multiple of 4)", I);
+  TL_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || act == ACT_SWISH_CLAMPED || act == ACT_RELU, "gemm_plain_pair: no function of code %d", act);
+  TL_REQUIRE(act != ACT_SWISH_CLAMPED || limit > 0.f, "gemm_plain_pair: the clamp needs a positive limit");
+  Around f{};
+  f.norm_w = norm_w; f.eps = eps; f.act = act; f.constants = ActConstants{alpha, limit, shift};
+  return launch_around<DO_PAIR>("gemm_plain_pair", A, W, out, M, 2 * I, K, I, f, st);
+}
+
+// tl_rope_commit of q|k|v = norm(A) W^T (norm_w null: of A itself), W [(nq + 2 nkv) d, K]; pages of float
+extern "C" int tl_gemm_plain_rope(const float* A, const float* norm_w, float eps, const float* W, int M, int K, const int* row_pos,
+                                  const float* inv_freq, int rotary_dim, int interleaved, const int* table, int table_stride, int ring_pages,
+                                  int nq, int nkv, int d, float* q, float* pages, hipStream_t st) {
+  TL_REQUIRE(nq > 0 && nkv > 0 && d > 0 && d % 8 == 0 && d <= 256 && ring_pages > 0 && table_stride > 0 && (long)(nq + 2 * nkv) * d < (1 << 30),
+             "gemm_plain_rope: bad sizes nq=%d nkv=%d d=%d ring_pages=%d table_stride=%d", nq, nkv, d, ring_pages, table_stride);
+  TL_REQUIRE(rotary_dim >= 0 && rotary_dim <= d && rotary_dim % 2 == 0 && (rotary_dim == 0 || inv_freq != nullptr),
+             "gemm_plain_rope: %d rotated channels of a head of %d (even, at most the head, with their frequencies)", rotary_dim, d);
+  TL_REQUIRE(row_pos && table && q && pages, "gemm_plain_rope: a buffer is missing");
+  Around f{};
+  f.norm_w = norm_w; f.eps = eps;
+  f.row_pos = row_pos; f.rot = Rotation{inv_freq, rotary_dim, interleaved != 0};
+  f.table = table; f.table_stride = table_stride; f.ring_pages = ring_pages; f.nq = nq; f.nkv = nkv; f.d = d; f.q = q; f.pages = pages;
+  return launch_around<DO_ROPE>("gemm_plain_rope", A, W, nullptr, M, (nq + 2 * nkv) * d, K, 0, f, st);
 }

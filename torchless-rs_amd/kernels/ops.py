@@ -1750,6 +1750,67 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: 
                                int(accumulate), _stream()))
 
 
+AROUND_ROWS, AROUND_K = 4, 2048     # the rows and channels of products that do what stands around them (`plain_around_ok`)
+
+
+def plain_around_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Do `gemm_plain_pair` and `gemm_plain_rope` take these operands?  True 32-bit, a few rows, K short."""
+    K = w.shape[1]
+    return (a.is_cuda and a.dtype == torch.float32 and w.dtype == torch.float32 and 0 < a.shape[0] <= AROUND_ROWS
+            and K <= AROUND_K and K % 4 == 0 and a.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def row_norm_ok(norm, K: int) -> bool:
+    """Can those products do this norm (an object with `weight`, `size`, `eps`, or None) of their rows?"""
+    return (norm is not None and norm.weight is not None and norm.size == K and norm.weight.dtype == torch.float32
+            and norm.weight.data_ptr() % 16 == 0)
+
+
+def _row_norm(norm, K: int, what: str):
+    """(weight, eps) of the norm of a product's rows (an object with `weight` float32 [K], `eps`), or of none."""
+    if norm is None:
+        return None, ctypes.c_float(0.0)
+    _req(norm.weight, what + ".norm", torch.float32, (K,))
+    return norm.weight, ctypes.c_float(norm.eps)
+
+
+def gemm_plain_pair(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, activation: str = "silu", constants=None, norm=None) -> None:
+    """out = act(g) * u of g|u = norm(a) @ w^T in 32 bits, w = gate|up by rows, at most 4 rows: the bits of `rmsnorm` (with a `norm`),
+    `gemm_plain` and `act_mul`."""
+    M, K = a.shape
+    I = w.shape[0] // 2
+    if activation not in ACTIVATIONS:
+        raise KernelError(f"gemm_pair: no function {activation!r}; there are {sorted(ACTIVATIONS)}")
+    _req(a, "gemm_pair.a", torch.float32)
+    _req(w, "gemm_pair.w", torch.float32, (2 * I, K))
+    _req(out, "gemm_pair.out", torch.float32, (M, I))
+    weight, eps = _row_norm(norm, K, "gemm_pair")
+    _check(lib().tl_gemm_plain_pair(_p(a), _p(weight), eps, _p(w), ACTIVATIONS[activation], *_act_constants(activation, constants),
+                                    _p(out), M, I, K, _stream()))
+
+
+def gemm_plain_rope(a: torch.Tensor, w: torch.Tensor, row_pos, rotation, table, ring_pages: int, nq: int, nkv: int, d: int,
+                    q: torch.Tensor, pages: torch.Tensor, norm=None) -> None:
+    """`rope_commit` of q|k|v = norm(a) @ w^T in 32 bits, for a step with one token a sequence (at most 4): the bits of `rmsnorm` (with a
+    `norm`), `gemm_plain` and `rope_commit`."""
+    M, K = a.shape
+    _req(a, "gemm_rope.a", torch.float32)
+    _req(w, "gemm_rope.w", torch.float32, ((nq + 2 * nkv) * d, K))
+    _req(row_pos, "gemm_rope.row_pos", torch.int32, (M,))
+    rot = _rotation(rotation, d, "gemm_rope")
+    _req(q, "gemm_rope.q", torch.float32, (M, nq, d))
+    _req(table, "gemm_rope.table", torch.int32)
+    _req(pages, "gemm_rope.pages", torch.float32)
+    if pages.dim() != 5 or tuple(pages.shape[1:]) != (2, nkv, PAGE, d):
+        raise KernelError(f"gemm_rope.pages: shape {tuple(pages.shape)}, kernel needs [*, 2, {nkv}, {PAGE}, {d}]")
+    if table.dim() != 2 or table.shape[0] != M:
+        raise KernelError("gemm_rope.table: needs one row per sequence")
+    weight, eps = _row_norm(norm, K, "gemm_rope")
+    _check(lib().tl_gemm_plain_rope(_p(a), _p(weight), eps, _p(w), M, K, _p(row_pos), _p(rot.inv_freq), rot.rotary_dim,
+                                    int(rot.interleaved), _p(table), table.shape[1], int(ring_pages), nq, nkv, d, _p(q), _p(pages),
+                                    _stream()))
+
+
 def sample_lists(B: int, V: int, temperature: float, top_k: int, device) -> Optional[torch.Tensor]:
     """Room for the lists of a draw whose rows several workgroups look through, uint8 [B, parts, bytes of a list], or None: a row is
     one workgroup's (the rule is `tl_sample_parts`)."""

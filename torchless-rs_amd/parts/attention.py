@@ -28,7 +28,7 @@ import torch
 from ..cache.cache import KVRequest
 from ..kernels import ops
 from ..weights.binding import WeightSpec
-from .base import Mixer, PartSpec, make_part, register_part, take_row_factor
+from .base import Mixer, PartSpec, goes_as, make_part, register_part, take_row_factor, take_row_norm
 from .linear import Linear
 
 
@@ -105,6 +105,14 @@ class AttentionMixer(Mixer):
         self.qkv = Linear(fused, tiled=True, own_copy=copy)
         self.o = Linear(tensors[p + nm["o"]], tiled=True)
 
+    def norms_rows(self, ctx, norm, x: torch.Tensor, run) -> bool:
+        return goes_as(self, AttentionMixer) and self._around(ctx, x, run) and ops.row_norm_ok(norm.rms_form(), self.H)
+
+    def _around(self, ctx, y: torch.Tensor, run) -> bool:
+        """Does a step of single tokens do the norm, q|k|v, the rotation and the commit in one launch of the 32-bit path?"""
+        return (self.own_kv and ctx.all_single and not run.kv_read_later and self.d % 8 == 0 and self.d <= 256
+                and run.kv_group.storage[run.kv_layer].dtype == torch.float32 and ops.plain_around_ok(y, self.qkv.weight))
+
     def forward(self, ctx, run, y: torch.Tensor, x: torch.Tensor) -> None:
         n, nq, nkv, d = y.shape[0], self.nq, self.nkv, self.d
         ws = ctx.workspace
@@ -123,6 +131,9 @@ class AttentionMixer(Mixer):
                 ops.qkv_rope_commit(y, self.qkv.weight, ctx.row_pos, rotation, table, group.ring_pages,
                                     nq, nkv, d, q, pages, factor=factor,     # product, rotation and commit in one
                                     tiles=self.qkv.own_tiles)
+            elif self._around(ctx, y, run):
+                ops.gemm_plain_rope(y, self.qkv.weight, ctx.row_pos, rotation, table, group.ring_pages, nq, nkv, d, q, pages,
+                                    norm=take_row_norm(ctx))
             else:
                 qkv = self.qkv.partial(y, ctx, "attn_qkv_parts")     # partial sums, added up by the rotation
                 if qkv is None:

@@ -283,19 +283,38 @@ def take_row_factor(ctx: "StepContext", usable: bool):
     return f
 
 
-def read_through_norm(ctx: "StepContext", norm: "Norm", x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
+def goes_as(part: Part, kind: type) -> bool:
+    """Is `part`'s `forward` that of `kind`?  (A part made from `kind` with a `forward` of its own is run through that, whatever
+    shorter way `kind` has.)"""
+    return type(part).forward is kind.forward
+
+
+def take_row_norm(ctx: "StepContext"):
+    """For a part that has said `norms_rows`: the norm that its first product has to do (None: the input is normed already)."""
+    f, ctx.row_norm = ctx.row_norm, None
+    return f
+
+
+def read_through_norm(ctx: "StepContext", norm: "Norm", x: torch.Tensor, y: torch.Tensor, reader: Optional[Part] = None,
+                      run: Optional["RunBinding"] = None) -> torch.Tensor:
     """The stream `x` as `norm` gives it to the part behind it (a block calls this for every norm
     it runs; returns the buffer that holds the result, which is `y` or what a product left).
     Partial products that a part left pending are added first, by the norm itself if it can
     (`takes_pending`).  If the product that completed the stream did this norm's first half
     (`expect_norm` had announced it), the result is what that product left, and the factor per
     row goes to the part that reads it (`ctx.row_factor`; `ctx.settle` runs the plain norm into
-    the same buffer for a part that cannot apply it)."""
+    the same buffer for a part that cannot apply it).  `reader`: the part behind the norm, if the block
+    hands it nothing but what this returns; one whose first product does the norm itself at these sizes
+    (`norms_rows(ctx, norm, x, run)`) gets the stream and `ctx.row_norm`."""
     pre, ctx.prenormed = ctx.prenormed, None
     if pre is not None and pre[0] is norm:
         ctx.row_factor = pre[2]
         ctx.settle = lambda: norm.forward(ctx, x, pre[1])
         return pre[1]
+    can = getattr(reader, "norms_rows", None)
+    if can is not None and ctx.pending is None and can(ctx, norm, x, run):
+        ctx.row_norm = norm.rms_form()
+        return x
     if not getattr(norm, "takes_pending", False):
         flush_pending(ctx, x)
     norm.forward(ctx, x, y)
@@ -319,6 +338,8 @@ def part_done(ctx: "StepContext", part: Part) -> None:
     ctx.norm_ahead = None
     if ctx.row_factor is not None:
         raise RuntimeError(f"{type(part).__name__} declares takes_row_factor and left the factor untaken")
+    if ctx.row_norm is not None:
+        raise RuntimeError(f"{type(part).__name__} said that it norms its rows and did not")
 
 
 def splittable_entry(norm: "Norm", reader: Part) -> Optional["Norm"]:
@@ -413,4 +434,7 @@ class StepContext:
     prenormed: Any = None
     row_factor: Any = None
     settle: Any = None
+    # the norm (`RmsForm`) that the part that reads it does by itself, in its first product: what it is handed is the stream
+    # (`read_through_norm`), and it must take the norm (`take_row_norm`)
+    row_norm: Any = None
     host: Dict[str, Any] = field(default_factory=dict)     # the same data on the host

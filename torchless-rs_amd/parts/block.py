@@ -69,7 +69,7 @@ class PreNormBlock(Part):
         an arrangement needs for norms cut in two around the products."""
         ctx.host.pop("stream_copy", None)        # this block writes the stream: a copy of it goes stale
         y = ctx.workspace.get("block_y", tuple(x.shape), ctx.dtype)
-        y1 = read_through_norm(ctx, self.mixer_norm, x, y)
+        y1 = read_through_norm(ctx, self.mixer_norm, x, y, self.mixer, run)
         if self.ffn is None:
             expect_norm(ctx, self.mixer, norm_after)
         else:
@@ -78,7 +78,7 @@ class PreNormBlock(Part):
         part_done(ctx, self.mixer)
         if self.ffn is None:
             return
-        y2 = read_through_norm(ctx, self.ffn_norm, x, y)
+        y2 = read_through_norm(ctx, self.ffn_norm, x, y, self.ffn)
         expect_norm(ctx, self.ffn, norm_after)
         self.ffn.forward(ctx, y2, x)
         part_done(ctx, self.ffn)

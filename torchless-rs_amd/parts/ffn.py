@@ -15,7 +15,7 @@ import torch
 
 from ..kernels import ops
 from ..weights.binding import WeightSpec
-from .base import FeedForward, register_part, take_row_factor
+from .base import FeedForward, goes_as, register_part, take_row_factor, take_row_norm
 from .linear import Linear, interleave_pairs
 
 
@@ -75,6 +75,12 @@ class SwiGLU(FeedForward):
         self.gate_up = Linear(interleave_pairs(g, u) if self.paired else torch.cat([g, u], dim=0))
         self.down = Linear(tensors[p + nm["down"]], tiled=True)
 
+    def norms_rows(self, ctx, norm, x: torch.Tensor, run) -> bool:
+        return goes_as(self, SwiGLU) and ctx.dtype == torch.float32 and self._around(x) and ops.row_norm_ok(norm.rms_form(), self.H)
+
+    def _around(self, y: torch.Tensor) -> bool:
+        return self.I % 4 == 0 and ops.plain_around_ok(y, self.gate_up.weight)
+
     def forward(self, ctx, y: torch.Tensor, x: torch.Tensor) -> None:
         self.down.add_into(self._hidden(ctx, y), x, ctx, "ffn_down_parts")
 
@@ -100,6 +106,8 @@ class SwiGLU(FeedForward):
                 ops.silu_mul_pairs(gu, h, self.activation, self.constants)
             else:
                 ops.gemm_bf16(y, self.gate_up.weight, h, silu_pair=True, pair_act=self.pair)
+        elif h.dtype == torch.float32 and self._around(y):       # norm, product and activation in one
+            ops.gemm_plain_pair(y, self.gate_up.weight, h, self.activation, self.constants, norm=take_row_norm(ctx))
         else:
             gu = ctx.workspace.get("ffn_gu", (n, 2 * self.I), torch.float32)
             self.gate_up(y, gu)
