@@ -16,80 +16,91 @@ namespace tl {
 
 // Few rows of floats: a workgroup of 8 waves has 8 outputs' rows of W and up to MR rows of A.  A wave has a group
 // of K, its lanes the 64 pairs of an output and a run of the group; a lane's chain is one run long.  W comes in
-// coalesced pieces, 128 bytes of each of the 64 pairs at a time through the wave's own part of LDS, the next pieces
-// on their way in registers meanwhile.  Bound by the stream of W.  N / 8 workgroups fill the chip from N = 2,048 on;
-// tiles of 64 x 64 with a chain of all of K in a thread, which this replaced, made 32 workgroups there.
-// Microseconds at one row, tiles of 64 before: N x K = 2,048 x 8,192 19.4 and 525, 2,048 x 2,048 5.3 and 130,
-// 16,384 x 2,048 28.3 (4.7 TB/s; 24.5 by the kernel below) and 216.
-// LINES: W's loads take whole lines, each once, and are marked non-temporal (2,048 x 8,192 at 2 rows 20.0 us without, 18.2 with).
+// coalesced pieces, 128 bytes of each of the 64 pairs at a time through the wave's own part of LDS, and A's 128 bytes of the wave's 8
+// runs with them; the next pieces are on their way in registers meanwhile.  (Loads come back in the order they were asked for: when
+// a lane loaded its A where it used it, it waited for the next pieces of W with it.)  Bound by the stream of W.  N / 8 workgroups fill the
+// chip from N = 2,048 on; tiles of 64 x 64 with a chain of all of K in a thread, which this replaced, made 32 workgroups there.
+// Microseconds at one row, those tiles and so: N x K = 2,048 x 8,192 525 and 14.6, 2,048 x 2,048 130 and 5.6, 16,384 x 2,048 216 and
+// 24.  At one / two / four rows with A loaded by each lane, and through LDS: 2,048 x 8,192 17.6 / 18.8 / 24.4 and 14.6 / 15.3 / 17.1, 4,096 x 14,336
+// 45.7 / 52.2 / 66.2 and 39.6 / 40.3 / 47.6 (5.9 TB/s at one), 28,672 x 4,096 86.8 / 96.5 / 128.8 and 73.5 / 73.6 / 103 (6.4 TB/s), 3,072 x 2,048 7.3 / 8.4 /
+// 11.4 and 6.6 / 7.3 / 11.  Two pieces ahead: 2,048 x 8,192 16.2 at one row, 17.6 at two, whose registers then last for one workgroup a
+// compute unit only; three and four rows 19.1 and 18.6.
+// LINES: W's loads take whole lines, each once, and are marked non-temporal (2,048 x 8,192 at 2 rows 20.0 us without, 18.2 with, A loaded by each lane).
 constexpr int CHUNK = 32;                         // channels of a pair that a wave brings in at a time
+constexpr int UNITS = CHUNK / 4;                  // of 16 bytes
 template <int MR, bool ACCUMULATE, bool LINES>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, 4)
 gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc) {
-  __shared__ float stage[PG][64][CHUNK + 4];      // rows 144 bytes apart: 16-byte reads of 64 rows spread over the banks
+  // a wave's pieces, 64 rows of W and 8 MR of A; unit u of W's row p lies at u ^ (p / 2) % 8, of A's run r at u ^ r: reads of 16 rows spread
+  // over the banks.  Two rows' 80 KB are the most of which two workgroups lie on a compute unit
+  __shared__ f32x4 stage[PG][(64 + MR * PR) * UNITS];
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const long first_n = ((long)blockIdx.z * gridDim.x + blockIdx.x) * 8;
   if (first_n >= N) return;
   const int n0 = (int)first_n, m0 = blockIdx.y * MR;
   const int L = run_length(K);
-  const int run = lane / 8;                       // of this lane's pair: output lane % 8, run lane / 8
-  const int k0 = (wave * PR + run) * L;
   const int rows = min(MR, M - m0);
   float acc[MR];
 #pragma unroll
   for (int m = 0; m < MR; ++m) acc[m] = 0.f;
 
-  // a load brings 128 bytes of 8 pairs: pair 8 i + lane / 8 (output lane / 8 of run i), 4 channels from 4 (lane % 8)
-  const int ln = n0 + lane / 8, lq = (lane % 8) * 4;
+  // a load brings 128 bytes of 8 pairs: pair 8 i + lane / 8 (output lane / 8 of run i), 4 channels from 4 (lane % 8); of A those of run lane / 8
+  const int l8 = lane / 8, lu = lane % 8, lq = lu * 4, ln = n0 + l8;
   const float* wp = W + (size_t)min(ln, N - 1) * ldw;
-  f32x4 next[8];
+  f32x4 w[8], a[MR];
   const auto fetch = [&](int at) {
+    const int off = at + lq, ka = (wave * PR + l8) * L + off;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      a[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (off < L && ka < K) a[m] = *(const f32x4*)(A + (size_t)(m0 + min(m, rows - 1)) * lda + ka);     // (K is a multiple of 4)
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int off = at + lq, k = (wave * PR + i) * L + off;
-      next[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (off < L && k < K && ln < N) next[i] = LINES ? __builtin_nontemporal_load((const f32x4*)(wp + k)) : *(const f32x4*)(wp + k);
+      const int k = (wave * PR + i) * L + off;
+      w[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (off < L && k < K && ln < N) w[i] = LINES ? __builtin_nontemporal_load((const f32x4*)(wp + k)) : *(const f32x4*)(wp + k);
     }
   };
+  f32x4* mine = stage[wave];
+  f32x4* mine_a = mine + 64 * UNITS;
   fetch(0);
   for (int at = 0; at < L; at += CHUNK) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) *(f32x4*)&stage[wave][i * 8 + lane / 8][lq] = next[i];
+    for (int m = 0; m < MR; ++m) mine_a[(m * PR + l8) * UNITS + (lu ^ l8)] = a[m];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mine[(i * 8 + l8) * UNITS + (lu ^ ((i * 8 + l8) / 2 % 8))] = w[i];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (at + CHUNK < L) fetch(at + CHUNK);
-    const int todo = min(CHUNK, L - at);          // (a multiple of 16)
-#pragma unroll 4
-    for (int q = 0; q < todo; q += 4) {
-      const f32x4 w = *(const f32x4*)&stage[wave][run * 8 + lane % 8][q];
-      const int k = k0 + at + q;
-      if (k < K) {                                // (K is a multiple of 4)
-        f32x4 a[MR];
+    const int todo = min(UNITS, (L - at) / 4);    // (a run is a multiple of 16 long; what lies past K is 0 times 0)
+    const int p = l8 * 8 + lu;                    // this lane's pair: output lane % 8, run lane / 8
+#pragma unroll 2
+    for (int u = 0; u < todo; ++u) {
+      const f32x4 wv = mine[p * UNITS + (u ^ (p / 2 % 8))];
 #pragma unroll
-        for (int m = 0; m < MR; ++m) a[m] = *(const f32x4*)(A + (size_t)(m0 + min(m, rows - 1)) * lda + k);
+      for (int m = 0; m < MR; ++m) {
+        const f32x4 av = mine_a[(m * PR + l8) * UNITS + (u ^ l8)];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int m = 0; m < MR; ++m) acc[m] = fmaf(a[m][j], w[j], acc[m]);
+        for (int j = 0; j < 4; ++j) acc[m] = fmaf(av[j], wv[j], acc[m]);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
-  // the runs of a group in order, then the groups
-  __shared__ float sums[PG][MR][8];
+  // the runs of a group in order, then the groups, whose sums take the place of their wave's pieces
 #pragma unroll
   for (int m = 0; m < MR; ++m) {
     float g = 0.f;
 #pragma unroll
     for (int i = 0; i < PR; ++i) g += __shfl(acc[m], i * 8 + lane % 8, WAVE);
-    if (lane < 8) sums[wave][m][lane] = g;
+    if (lane < 8) reinterpret_cast<float*>(mine)[m * 8 + lane] = g;
   }
   __syncthreads();
   const int m = threadIdx.x / 8, n = n0 + threadIdx.x % 8;
   if (m < rows && n < N) {
     float t = 0.f;
 #pragma unroll
-    for (int g = 0; g < PG; ++g) t += sums[g][m][threadIdx.x % 8];
+    for (int g = 0; g < PG; ++g) t += reinterpret_cast<const float*>(stage[g])[m * 8 + threadIdx.x % 8];
     float* c = C + (size_t)(m0 + m) * ldc + n;
     *c = ACCUMULATE ? *c + t : t;
   }
@@ -97,10 +108,10 @@ gemm_plain_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
 
 // The same bits for one to four rows, K up to 2,048 and many outputs: a workgroup goes through a run of eights of outputs, the next
 // eights' pieces under way while it sums the last's, and a lane keeps its run of A, one piece long, in registers.  With an
-// eight a workgroup every workgroup waited for memory once and did nothing meanwhile, and read A from L1 for each.  One / two rows,
-// an eight a workgroup and so: 16,384 x 2,048 28.5 / 32.8 and 25 / 26.2 us, 32,000 x 2,048 52.2 / 60.0 and 44.5 / 46 (5.8 TB/s); three / four rows, which
-// took tiles, 39.9 / 38.6 and 27.6 / 25.8, 75.3 / 69.0 and 48 / 45.  With fewer
-// eights than workgroups there is nothing to go on to (3,072 x 2,048 8.2 us at two rows, 9.3 so).
+// eight a workgroup every workgroup waits for memory once and does nothing meanwhile, and brings A for each.  One / two rows,
+// an eight a workgroup and so: 16,384 x 2,048 24.0 / 25.3 and 24.4 / 25.2 us, 32,000 x 2,048 43.3 / 46.2 and 44.1 / 44.5 (5.9 TB/s), 16,384 x 1,024 16.6 / 17.3 and
+// 15.7 / 17.6; three / four rows, of which one workgroup lies on a compute unit, 37.8 / 40.7 and 26.6 / 26.1, 69.4 / 74.6 and 46.6 / 45.9.  With fewer
+// eights than workgroups there is nothing to go on to (3,072 x 2,048 7.3 us at two rows, 9.3 so).
 // At one row two workgroups of 128 registers lie on a compute unit; with more rows' A it is one, of at most 256, which fetches two eights
 // ahead where the registers last (16,384 x 2,048: two rows 29.6 us with 512 workgroups and one eight ahead, 27.9 with 256, 26.2 with two
 // ahead; four rows 30.1 and 25.8 with 256, 45 with two ahead, which spills).
@@ -467,12 +478,13 @@ static int launch_rows(const float* A, const float* W, float* C, int M, int N, i
 }
 
 // The kernel for few rows reads W once for every 8 rows and has a thread's chain 64 times shorter than K.  Against it, microseconds
-// (rows / tiles): the tiles on the matrix cores (`fit`), N x K = 2,048 x 2,048 at 8 rows 10 / 11, 3,072 x 2,048 at 4 10 / 12, at 6 13.8 / 12.2,
-// 2,048 x 8,192 at 4 24 / 26, at 6 30 / 26, 4,096 x 14,336 at 4 66 / 62, at 8 109 / 62; the tiles on the vector pipes, 2,048 x 8,192 at 8 rows
-// 32 / 65, at 16 52 / 68, at 32 96 / 72; 3,072 x 2,048 at 8 14.4 / 18.6, at 16 21 / 19; 4,096 x 14,336 at 8 110 / 126, at 16 197 / 123;
-// 16,384 x 2,048 at 2 31 / 36, at 4 41 / 36 (of up to four rows wide outputs are `goes_on`'s).
+// (rows / tiles): the tiles on the matrix cores (`fit`), N x K = 2,048 x 2,048 at 8 rows 8.9 / 11, 3,072 x 2,048 at 4 11 / 12, at 6 14.0 / 13.3,
+// 2,048 x 8,192 at 4 17 / 26, at 6 19.5 / 22.5, at 8 20.2 / 22.3, 4,096 x 4,096 at 6 22.8 / 22.5, at 8 23.0 / 22.6, 4,096 x 14,336 at 4 47 / 62, at 6 54 /
+// 62, at 8 56 / 62, 28,672 x 4,096 at 6 134 / 103; the tiles on the vector pipes, 2,048 x 8,192 at 16 rows 52 / 68, at 32 96 / 72 (with A loaded by
+// each lane); 3,072 x 2,048 at 16 21 / 19; 4,096 x 14,336 at 16 197 / 123; 16,384 x 2,048 at 4 41 / 36 (of up to four rows wide outputs are
+// `goes_on`'s).
 static bool few_rows(int M, int N, int K, bool fit) {
-  if (fit) return M <= 4 || (M <= 8 && (long)M * N <= 16384 && K <= 4096);
+  if (fit) return M <= 4 || (M <= 8 && (long)M * N <= (K <= 4096 ? 16384 : 32768));
   return M <= 2 || (M <= 16 && (long)M * N <= 32768);
 }
 
