@@ -399,6 +399,23 @@ def test_products_with_what_stands_around_them_have_the_bits_of_the_kernels(ops,
         ops.gemm_plain_pair(torch.zeros(1, 2052, device=DEV), torch.zeros(8, 2052, device=DEV), torch.empty(1, 4, device=DEV))
 
 
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("d,window", [(4, None), (20, 70), (64, None), (128, 100), (256, None)])
+def test_plain_attention_four_at_a_time_has_the_bits_of_one_at_a_time(ops, dt, d, window):
+    """Pages read four channels or four keys a load, and the same pages one element further, read one by one: keys that end within a page and
+    with it, tiles that begin within one (a window's), rings that have wrapped."""
+    a = paged_case(ops, dt, 6, 2, d, window, lens_cached=[0, 62, 63, 64, 131, 300], lens_new=[1] * 6, seed=56)
+    ops.kv_commit(a["k"], a["v"], a["row_seq"], a["row_pos"], a["after"], a["table"], a["ring"], a["pages"])
+    moved = torch.empty(a["pages"].numel() + 1, dtype=DT[dt], device=DEV)[1:].copy_(a["pages"].reshape(-1)).view(a["pages"].shape)
+    outs = []
+    for pages in (a["pages"], moved):
+        out = torch.full_like(a["q"], float("nan"))
+        ops.attn_plain(a["q"], None, None, pages, a["table"], a["ring"], a["row_seq"], a["row_pos"], a["cu"], a["after"], window, a["scale"], out)
+        outs.append(out)
+    assert torch.equal(*outs)
+    assert rel_err(outs[0], a["want"]) < KTOL[dt]
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 70_000_000, 4), (2, 70_000_001, 3), (4_190_000, 2080, 4)])
 def test_gemm_plain_of_more_tiles_than_a_grid_is_wide(ops, M, N, K):
     """One launch has fewer than 2^32 threads along x: what lies behind them is there too."""
