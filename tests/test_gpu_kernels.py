@@ -400,6 +400,22 @@ def test_products_with_what_stands_around_them_have_the_bits_of_the_kernels(ops,
 
 
 @pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H", [1028, 2048, 3076, 4096, 5120, 8192])
+def test_the_norm_of_few_rows_has_the_bits_of_many(ops, dt, H):
+    """Partial products added and normed by up to 1,024 threads a row, where rows are fewer than compute units, and by 256 where they are more."""
+    few = min(ops.compute_units(torch.device(DEV)), 200)
+    many = ops.compute_units(torch.device(DEV)) + 3
+    w = rnd(H, seed=57).to(DEV)
+    for S in (0, 1, 3, 8):
+        x, parts = rnd(many, H, seed=58).to(DEV), rnd(max(S, 1), many, H, seed=59).to(DEV)[:S]
+        x1, parts1 = x[:few].clone(), parts[:, :few].contiguous()
+        out, out1 = (torch.full((n, H), float("nan"), dtype=DT[dt], device=DEV) for n in (many, few))
+        ops.add_rmsnorm(x, parts, w, 1e-5, out)
+        ops.add_rmsnorm(x1, parts1, w, 1e-5, out1)
+        assert torch.equal(x[:few], x1) and torch.equal(out[:few], out1), S
+
+
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
 @pytest.mark.parametrize("d,window", [(4, None), (20, 70), (64, None), (128, 100), (256, None)])
 def test_plain_attention_four_at_a_time_has_the_bits_of_one_at_a_time(ops, dt, d, window):
     """Pages read four channels or four keys a load, and the same pages one element further, read one by one: keys that end within a page and

@@ -225,6 +225,67 @@ add_rmsnorm_reg_kernel(float* __restrict__ x, const float* __restrict__ parts, i
   }
 }
 
+// The same bits with 256 threads for every 1,024 channels (four times 256 at most), for steps of rows that are fewer than the chip can hold: a
+// thread of the kernel above waits for one vector's partial products after the other.  Eight / three partial products of 4,096 channels: 64
+// rows 4.4 / 4.4 us before, 4.1 / 3.4 now, 226 6.9 / 5.0 and 6.2 / 4.2; where every compute unit has more than a row they are equal or the
+// other is ahead (2,048 channels at 400 rows 4.4 and 4.6, three partial products at 2,048 rows 27.3 and 28.6).
+template <typename TO, int IT>
+__global__ void __launch_bounds__(256 * (IT < 4 ? IT : 4))
+add_rmsnorm_wide_kernel(float* __restrict__ x, const float* __restrict__ parts, int n_parts, size_t part_stride,
+                        const float* __restrict__ w, float eps, TO* __restrict__ out, int H) {
+  constexpr int G = IT < 4 ? IT : 4, MINE = IT / G;
+  __shared__ float squares[IT][256], sh[4];
+  const int n = blockIdx.x, t = threadIdx.x % 256, group = threadIdx.x / 256;
+  float4* xr = reinterpret_cast<float4*>(x + (size_t)n * H);
+  const float4* wr = reinterpret_cast<const float4*>(w);
+  const int nv = H / 4;
+  float4 v[MINE], g[MINE];
+#pragma unroll
+  for (int i = 0; i < MINE; ++i) {
+    const int c = t + 256 * (group + G * i);
+    float ss = 0.f;
+    if (c < nv) {
+      float4 a = xr[c];
+      g[i] = wr[c];
+#pragma unroll 8
+      for (int s = 0; s < n_parts; ++s) {
+        const float4 p = reinterpret_cast<const float4*>(parts + s * part_stride + (size_t)n * H)[c];
+        a.x += p.x; a.y += p.y; a.z += p.z; a.w += p.w;
+      }
+      xr[c] = a;
+      v[i] = a;
+      ss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
+    }
+    squares[group + G * i][t] = ss;
+  }
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) ss += squares[i][t];
+    ss = wave_sum(ss);
+    if (t % WAVE == 0) sh[t / WAVE] = ss;
+  }
+  __syncthreads();
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ss += sh[i];
+  const float rms = sqrtf(ss / (float)H + eps);
+  TO* o = out + (size_t)n * H;
+#pragma unroll
+  for (int i = 0; i < MINE; ++i) {
+    const int c = t + 256 * (group + G * i);
+    if (c < nv) {
+      __attribute__((ext_vector_type(4))) TO y;
+      y[0] = from_f32<TO>((v[i].x / rms) * g[i].x);
+      y[1] = from_f32<TO>((v[i].y / rms) * g[i].y);
+      y[2] = from_f32<TO>((v[i].z / rms) * g[i].z);
+      y[3] = from_f32<TO>((v[i].w / rms) * g[i].w);
+      *reinterpret_cast<decltype(y)*>(o + 4 * c) = y;
+    }
+  }
+}
+
 // (V: f32x4 where the pointers and the count allow it: 8 parts of 192 x 4,096 in 6.4 us, by floats 7.7)
 template <typename V>
 __global__ void __launch_bounds__(256)
@@ -984,9 +1045,14 @@ int tl_add_rmsnorm(float* x, const float* parts, int n_parts, const float* w, fl
              ((uintptr_t)parts % 16 == 0), "add_rmsnorm: H=%d must be a multiple of 4, at most 8192, rows 16-byte aligned", H);
   if (n == 0) return 0;
   const size_t stride = (size_t)n * H;
+  const bool wide = n <= compute_units() && H > 1024 && (uintptr_t)out % (out_dt == DT_F32 ? 16 : 8) == 0;
 #define TL_ARMS(IT)                                                                                        \
   do {                                                                                                     \
-    if (out_dt == DT_F32) add_rmsnorm_reg_kernel<float, IT><<<n, 256, 0, st>>>(x, parts, n_parts, stride, w, eps, (float*)out, H); \
+    if (wide && out_dt == DT_F32)                                                                          \
+      add_rmsnorm_wide_kernel<float, IT><<<n, 256 * min(IT, 4), 0, st>>>(x, parts, n_parts, stride, w, eps, (float*)out, H);  \
+    else if (wide)                                                                                         \
+      add_rmsnorm_wide_kernel<bf16, IT><<<n, 256 * min(IT, 4), 0, st>>>(x, parts, n_parts, stride, w, eps, (bf16*)out, H);    \
+    else if (out_dt == DT_F32) add_rmsnorm_reg_kernel<float, IT><<<n, 256, 0, st>>>(x, parts, n_parts, stride, w, eps, (float*)out, H); \
     else add_rmsnorm_reg_kernel<bf16, IT><<<n, 256, 0, st>>>(x, parts, n_parts, stride, w, eps, (bf16*)out, H);                   \
   } while (0)
   if (H <= 1024) TL_ARMS(1);
@@ -1172,7 +1238,9 @@ int tl_rope_commit(const float* qkv, int n_parts, const int* row_pos, const floa
   const Rotation rot{inv_freq, rotary_dim, interleaved != 0};
   if (n == 0) return 0;
   const size_t stride = (size_t)n * (nq + 2 * nkv) * d;
-  const dim3 grid(n, n >= 128 ? 1 : (n >= 32 ? 4 : 8));       // few rows: cut the heads over more workgroups
+  // few rows: the heads cut over more workgroups.  32 + 8 + 8 heads of 128, five partial sums, cut by 1 / 4 / 8: 32 rows - / 4.5 / 4.1 us, 64 - / 5.1 / 5.0,
+  // 128 11.5 / 7.2 / 7.2 (16 ways), 226 14.6 / 10.7 / 10.3, 512 21.6 / 20.7, 1,024 49.1 / 51.0; no partial sums: 100 rows 5.3 in 4, 6.0 in 8, 1,024 28.2 / 33.5
+  const dim3 grid(n, n > 512 ? 1 : (n >= 64 ? 4 : 8));
   if (dt == DT_F32)
     rope_commit_kernel<float><<<grid, 256, 0, st>>>(qkv, n_parts, stride, row_pos, rot, table, table_stride,
                                                   ring_pages, nq, nkv, d, (float*)q, (float*)pages);
