@@ -869,3 +869,36 @@ def test_a_block_of_another_arrangement_gets_the_split_norms_from_the_helpers(dt
         for name, fn in real.items():
             setattr(ops, name, fn)
         unregister_part("block", "three_norms")
+
+
+@pytest.mark.parametrize("rows,H", [(1, 64), (4, 64), (5, 64), (2, 2052), (2, 66)])
+@pytest.mark.parametrize("own_forward", [False, True])
+def test_who_norms_the_rows_of_a_feed_forward(rows, H, own_forward):
+    """In 32 bits a feed-forward of a few rows is handed the stream and the norm; more or longer rows, and a part with a `forward` of its own,
+    are handed the normed rows.  The results are the same bits either way."""
+    from types import SimpleNamespace
+    from torchless_rs_amd.kernels import ops
+    from torchless_rs_amd.parts.base import PartSpec, Workspace, make_part, read_through_norm
+    from torchless_rs_amd.parts.ffn import SwiGLU
+    kind = type("Seen", (SwiGLU,), {"forward": lambda self, ctx, y, x: SwiGLU.forward(self, ctx, y, x)}) if own_forward else SwiGLU
+    g = torch.Generator().manual_seed(60)
+    I = 48
+    ffn, norm = kind(H, I), make_part("norm", PartSpec("rmsnorm", {"size": H, "eps": 1e-5}))
+    ffn.load({"mlp.gate_proj.weight": torch.randn(I, H, generator=g).to(DEV), "mlp.up_proj.weight": torch.randn(I, H, generator=g).to(DEV),
+              "mlp.down_proj.weight": torch.randn(H, I, generator=g).to(DEV)}, torch.float32)
+    norm.load({"weight": torch.randn(H, generator=g).to(DEV)}, torch.float32)
+    x = torch.randn(rows, H, generator=g).to(DEV)
+    ctx = SimpleNamespace(prenormed=None, pending=None, row_factor=None, row_norm=None, settle=None, norm_ahead=None, dtype=torch.float32,
+                          workspace=Workspace(DEV))
+    y, want = torch.empty_like(x), x.clone()
+    got = read_through_norm(ctx, norm, x, y, ffn)
+    handed = not own_forward and rows <= 4 and H == 64
+    assert (got is x and ctx.row_norm is not None) if handed else (got is y and ctx.row_norm is None)
+    ffn.forward(ctx, got, x)
+    assert ctx.row_norm is None
+    norm.forward(ctx, want, y)
+    gu, h = torch.empty(rows, 2 * I, device=DEV), torch.empty(rows, I, device=DEV)
+    ops.gemm_plain(y, ffn.gate_up.weight, gu)
+    ops.act_mul(gu, h)
+    ops.gemm_plain(h, ffn.down.weight, want, True)
+    assert torch.equal(x, want)
