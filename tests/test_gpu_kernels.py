@@ -668,6 +668,17 @@ def test_draws_through_pinned_memory(ops):
         ops.sample(z[:3], 0.9, 40, 0.9, 6, pairs.to(DEV), probs, out, host_out=torch.zeros(3, dtype=torch.int32))
 
 
+def test_options_that_change_between_draws(ops):
+    """A sampler whose options are set anew between draws of one shape, with rows in parts and without: what a sampler of those options draws."""
+    from torchless_rs_amd import SamplingConfig
+    from torchless_rs_amd.sampling.sampler import Sampler
+    z = rnd(3, 70000, seed=78, scale=2.0).to(DEV)
+    sampler = Sampler(SamplingConfig(0.9, 40, 0.9, 6), DEV)
+    for T, k, p in ((0.9, 40, 0.9), (0.9, None, 0.9), (0.0, 40, None), (0.7, 5, None), (0.7, 257, 0.8), (0.9, 256, None)):
+        sampler.config.temperature, sampler.config.top_k, sampler.config.top_p = T, k, p
+        assert sampler.sample(z, [4, 5, 6], [1, 2, 3]) == Sampler(SamplingConfig(T, k, p, 6), DEV).sample(z, [4, 5, 6], [1, 2, 3])
+
+
 def test_draws_do_not_depend_on_batch_mates_and_follow_the_probabilities(ops):
     V = 8
     z = torch.tensor([[2.0, 1.0, 0.0, -1.0, 0.5, 1.5, -2.0, 0.2]])

@@ -38,8 +38,8 @@ class _Place:
 
 
 class Drawn:
-    """The tokens of one draw: on the device at once (`device`, int32 [B], valid until the
-    sampler's next draw has been launched), on the host when `tokens()` is asked for (until two
+    """The tokens of one draw: on the device at once (`device`, int32 [B], in the order of
+    the draw's stream, valid until the sampler's next draw has been launched), on the host when `tokens()` is asked for (until two
     more draws have been launched)."""
 
     def __init__(self, device: torch.Tensor, place: _Place):
@@ -65,8 +65,8 @@ class Sampler:
         self.config = config
         self.device = device
         self._probs = None
-        self._lists = None               # the lists of rows in parts, of the last shape drawn from
-        self._shape = None
+        self._lists = None               # the lists of rows in parts, of the last draw's shape and options
+        self._lists_for = None           # (the options may change between draws, and with them whether rows go in parts)
         self._out = None
         self._places = None              # two, used in turn: a draw may be launched while the one before is read
         self._turn = 0
@@ -82,9 +82,10 @@ class Sampler:
             self._out = torch.empty((cap,), dtype=torch.int32, device=logits.device)
         if self._probs is None or self._probs.shape[0] < B or self._probs.shape[1] != V:
             self._probs = torch.empty((B, V), dtype=torch.float32, device=logits.device)
-        if self._shape != (B, V):
-            self._lists = ops.sample_lists(B, V, float(c.temperature), int(c.top_k or 0), logits.device)
-            self._shape = (B, V)
+        wanted = (B, V, float(c.temperature), int(c.top_k or 0))
+        if self._lists_for != wanted:
+            self._lists = ops.sample_lists(*wanted, logits.device)
+            self._lists_for = wanted
         place = self._places[self._turn]
         self._turn ^= 1
         place.wait()                                 # the memory is free to be written again
