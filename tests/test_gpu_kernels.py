@@ -870,6 +870,57 @@ def test_attention_prefill_with_long_blocks_cut_into_runs(ops, monkeypatch, nq, 
                                                        for _, _, lo, w in fuller.items.cpu().tolist() if w >> 30))
 
 
+@pytest.mark.parametrize("cut", [False, True])
+@pytest.mark.parametrize("d", [64, 80, 128])
+def test_attention_prefill_of_scores_that_rise(ops, monkeypatch, cut, d):
+    """Maxima that rise from tile to tile, by steps of their own for the rows of a wave: by just under and just over 8 and by 2 and 4 with
+    2,000 earlier keys that still weigh, by 20, and past one earlier key with little else (row factors 1 to 1/8, a key alone at 7).  A row's
+    largest weight is 1 and needs no rounding; of the others each is rounded to 8 bits, and the result is."""
+    from torchless_rs_amd.cache import PAGE
+    nq, nkv, L, n_new = 2, 1, 2400, 150
+    T = L + n_new
+    g = torch.Generator().manual_seed(31)
+    v = torch.randn(T, nkv, d, generator=g).to(torch.bfloat16)
+    score = torch.empty(2, T).uniform_(-0.5, 0.5, generator=g)        # head 0: rises past many keys
+    for tile, top in ((32, 7.875), (33, 16.0), (34, 18.0), (35, 22.0), (36, 42.0)):
+        score[0, 64 * tile + 7 * (tile - 30)] = top
+    score[1] -= 300.0                                                  # head 1: one key, and one 7 above it
+    score[1, 70], score[1, 64 * 33 + 50] = 0.0, 7.0
+    score = score.to(torch.bfloat16)
+    k = torch.zeros(T, nkv, d, dtype=torch.bfloat16)
+    k[:, 0, 0], k[:, 0, 1] = score[0], score[1]
+    factor = torch.tensor([1.0, 0.5, 0.25, 0.125, 1.125, 0.75])[torch.arange(n_new) % 6]
+    q = torch.zeros(n_new, nq, d)
+    q[:, 0, 0], q[:, 1, 1] = factor, factor
+    q = q.to(torch.bfloat16)
+    perm = torch.randperm(40, generator=g)
+    table = perm[:-(-T // PAGE)].to(torch.int32).view(1, -1)
+    pages = torch.full((40, 2, nkv, PAGE, d), float("nan"), dtype=torch.bfloat16)
+    for p0 in range(0, L, PAGE):
+        n = min(PAGE, L - p0)
+        pages[table[0, p0 // PAGE], 0, :, :n] = k[p0:p0 + n].transpose(0, 1)
+        pages[table[0, p0 // PAGE], 1].view(nkv, d, PAGE)[:, :, :n] = v[p0:p0 + n].permute(1, 2, 0)
+    i32 = lambda l: torch.tensor(l, dtype=torch.int32, device=DEV)
+    off, cols = ops.aligned_columns([L], [n_new])
+    vt = torch.zeros(nkv, d, cols, dtype=torch.bfloat16)
+    vt[:, :, L % PAGE:L % PAGE + n_new] = v[L:].permute(1, 2, 0)
+    cuts = part = None
+    if cut:
+        monkeypatch.setattr(ops, "PREFILL_CUT_TILES", 3)
+        cuts = ops.prefill_cuts([n_new], [L], None, nq, 64, DEV)
+        part = torch.full((n_new * nq * cuts.ways * (d + 4),), float("nan"), device=DEV)
+    out = torch.empty(n_new, nq, d, dtype=torch.bfloat16, device=DEV)
+    ops.attn_prefill_bf16(q.to(DEV), k[L:].contiguous().to(DEV), vt.to(DEV), i32(off), pages.to(DEV), table.to(DEV), table.shape[1],
+                          i32(list(range(L, T))), i32([0, n_new]), i32([L]), -(-n_new // 128), None, 1.0, out, cuts=cuts, part=part)
+    got, v64 = out.cpu().double(), v[:, 0].double()
+    for h in range(nq):
+        s = factor.double()[:, None] * score[h].double()
+        w = torch.softmax(s.masked_fill(torch.arange(T)[None] > torch.arange(L, T)[:, None], -math.inf), 1)
+        want, others = w @ v64, w.scatter(1, w.argmax(1, keepdim=True), 0.0) @ v64.abs()
+        half_ulp = 2.0 ** (torch.floor(torch.log2(want.abs())) - 8)
+        assert bool(((got[:, h] - want).abs() <= half_ulp + 2.0 ** -8 * others + 2e-5 * (w @ v64.abs())).all()), h
+
+
 @pytest.mark.parametrize("through_lds", [True, False])
 @pytest.mark.parametrize("splits", [1, 3, 8])
 @pytest.mark.parametrize("nq,nkv,d,window", SHAPES)

@@ -77,11 +77,6 @@ struct PageSpan {
 constexpr int PF_BM = 128, PF_BN = 64, PF_VLD = PF_BN + 4;
 constexpr int PF_PART_HEAD = 4;       // floats before O in a half block's partial result: maximum, sum, two of padding
 
-// What the sums go by is a row's maximum when they last were scaled; they are scaled again only where a score passes it by more than this:
-// weights then reach e^8, which neither float sums nor a weight's 8 bits in bfloat16 notice, and the 64 products a lane of a scaling, which with 32
-// rows a wave had nearly every tile, become rare (one prompt of 2,048 / 8,192 tokens 80 / 746 us before, 77 / 716 so).
-constexpr float PF_SLACK = 8.f;
-
 // LEAN (d == DPAD, 256 % (DPAD / 8) == 0): whole tiles are fetched the short way.  DV > 0: values of another width than
 // keys, dv_arg channels padded to DV (0: as wide as keys).
 template <int DPAD, bool LEAN, bool TERMS = false, bool LOGI = false, int DV = 0>
@@ -398,8 +393,9 @@ attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_new,
 #pragma unroll
         for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[nb][r]);
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-      const float top = tmax * sc;                         // scale > 0: the maximum of the scaled scores
-      const float m_new = top > m + PF_SLACK ? top : m;
+      // scale > 0: the maximum of the scaled scores.  (O and l go by the maximum itself, not by one that may lag behind: then a row's
+      // largest weight is 1 and loses nothing as a bfloat16, where l, which sums the weights as they are, and O would part by up to 2^-8 of it)
+      const float m_new = fmaxf(m, tmax * sc);
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
       if (__ballot(m_new != m) != 0ull) {                  // the running maximum moved in some lane
         const float alpha = __expf(m - m_use);
