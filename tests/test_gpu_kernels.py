@@ -1332,6 +1332,27 @@ def test_qkv_rope_commit_from_tiles_of_shares(ops, nq, nkv, d, K, units, share, 
             ops.qkv_rope_commit(y, w, c["row_pos"], rot, c["table"], c["ring"], nq, nkv, d, q, pages, units=2, tiles=t)
 
 
+def test_qkv_rope_commit_refuses_copies_in_another_order(ops):
+    """A copy of the rows as stored has tiles of the same height as one of shares for 6,144 rows (24): refused, and so are shares made for other
+    heads or another rotation."""
+    nq, nkv, d, K = 32, 8, 128, 64
+    rot, _ = rotation_for(ops, d, 10000.0, 1.0, False)
+    other, _ = rotation_for(ops, d, 10000.0, 0.5, False)
+    c = paged_case(ops, "bfloat16", nq, nkv, d, None, lens_cached=[3, 64], lens_new=[1, 1], seed=19)
+    y = rnd(2, K, seed=20, dtype=torch.bfloat16).to(DEV)
+    w = rnd((nq + 2 * nkv) * d, K, seed=21, dtype=torch.bfloat16, scale=0.2).to(DEV)
+    call = lambda t: ops.qkv_rope_commit(y, w, c["row_pos"], rot, c["table"], c["ring"], nq, nkv, d, torch.empty(2, nq, d, dtype=y.dtype, device=DEV),
+                                         c["pages"], units=3, tiles=t)
+    stored = ops.tile_weights(w)
+    assert stored.shape == ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, rot, shares=True), 24).shape
+    swapped = torch.arange(w.shape[0] - 1, -1, -1, dtype=torch.int32, device=DEV)
+    for tiles in (stored, ops.tile_weights(w, swapped, 24), ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, other, shares=True), 24),
+                  ops.tile_weights(w, ops.qkv_tile_rows(40, 4, d, DEV, rot, shares=True), 24)):
+        with pytest.raises(ops.KernelError, match="tiles"):
+            call(tiles)
+    call(ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, rot, shares=True), 24))
+
+
 # ---- many channels against at most 16 rows: whole rows of the weights, 1 KB a load --------------
 
 @pytest.mark.parametrize("M", [1, 5, 16])

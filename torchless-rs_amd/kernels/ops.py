@@ -1900,6 +1900,7 @@ def tile_weights(w: torch.Tensor, rows: Optional[torch.Tensor] = None, height: O
     make = torch.empty if n_tiles * R == N else torch.zeros
     out = make((n_tiles, K // 64, 2, 4, R, 8), dtype=torch.bfloat16, device=w.device)
     _check(lib().tl_tile_weights(_p(w), _p(rows), N, K, R, _p(out), _stream()))
+    out.share_order = getattr(rows, "share_order", None)
     return out
 
 
@@ -1907,13 +1908,20 @@ def qkv_tile_rows(nq: int, nkv: int, d: int, device, rotation=None, shares: bool
     """The order of the rows of w = q|k|v in the tiled copy that `qkv_rope_commit` reads
     (a tile of a q or k head holds both channels of 8 pairs of `rotation`; None: the whole
     head rotated in halves).  `shares`: in the copy whose tiles are workgroups' shares of 24 or 32 rows (both channels
-    of 4 pairs, unit after unit)."""
+    of 4 pairs, unit after unit); these rows and the copy made by them carry what they are for as `share_order`."""
     n = (nq + 2 * nkv) * d
     buf = (ctypes.c_int * n)()
     rotary_dim, interleaved = (d, False) if rotation is None else (rotation.rotary_dim, rotation.interleaved)
     order = lib().tl_qkv_share_rows if shares else lib().tl_qkv_tile_rows
     _check(order(int(nq), int(nkv), int(d), int(rotary_dim), int(interleaved), buf))
-    return torch.tensor(list(buf), dtype=torch.int32, device=device)
+    rows = torch.tensor(list(buf), dtype=torch.int32, device=device)
+    rows.share_order = _share_order(nq, nkv, d, rotary_dim, interleaved) if shares else None
+    return rows
+
+
+def _share_order(nq: int, nkv: int, d: int, rotary_dim: int, interleaved: bool) -> tuple:
+    """What the order of rows in tiles of shares goes by."""
+    return int(nq), int(nkv), int(d), int(rotary_dim), bool(interleaved)
 
 
 def qkv_tiles(w: torch.Tensor, nq: int, nkv: int, d: int, rotation=None) -> torch.Tensor:
@@ -2395,14 +2403,19 @@ def qkv_rope_commit(a: torch.Tensor, w: torch.Tensor, row_pos, rotation, table, 
     the rotation of q and k, q into its buffer and k, v into the pages, in one kernel; the
     same bits as `gemm` and then `rope_commit`.  `factor`: see `gemm_bf16_norm`.  `units`
     (tests): how many units of 8 weight rows a workgroup owns, 1 to 4; 0 leaves it to the launcher.
-    `tiles`: `qkv_tiles(w, nq, nkv, d, rotation)` or `tile_weights(w, qkv_tile_rows(nq, nkv, d, device, rotation))`, read instead of w.
+    `tiles`: `qkv_tiles(w, nq, nkv, d, rotation)` or `tile_weights(w, qkv_tile_rows(nq, nkv, d, device, rotation))`, read instead of w (tiles of
+    more than 16 rows only with the `share_order` of these heads).
     `rotation`: see `rope_split`."""
     n, K = a.shape
     _req(a, "qkv_rope_commit.a", torch.bfloat16)
     _req(w, "qkv_rope_commit.w", torch.bfloat16, ((nq + 2 * nkv) * d, K))
-    height = _req_tiles(tiles, (nq + 2 * nkv) * d, K)
-    _req(row_pos, "qkv_rope_commit.row_pos", torch.int32, (n,))
     rot = _rotation(rotation, d, "qkv_rope_commit")
+    # a copy's height says nothing of the order of its rows: `tile_weights` of 6,144 rows as stored has tiles of 24 as well
+    share_order = getattr(tiles, "share_order", None)
+    height = _req_tiles(tiles, (nq + 2 * nkv) * d, K, height=16 if share_order is None else None)
+    if share_order is not None and share_order != _share_order(nq, nkv, d, rot.rotary_dim, rot.interleaved):
+        raise KernelError(f"qkv_rope_commit.tiles: rows in the order of (nq, nkv, d, rotated channels, interleaved) = {share_order}")
+    _req(row_pos, "qkv_rope_commit.row_pos", torch.int32, (n,))
     _req(q, "qkv_rope_commit.q", torch.bfloat16, (n, nq, d))
     _req(table, "qkv_rope_commit.table", torch.int32)
     _req(pages, "qkv_rope_commit.pages", torch.bfloat16)
