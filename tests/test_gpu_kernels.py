@@ -1334,7 +1334,7 @@ def test_qkv_rope_commit_from_tiles_of_shares(ops, nq, nkv, d, K, units, share, 
 
 def test_qkv_rope_commit_refuses_copies_in_another_order(ops):
     """A copy of the rows as stored has tiles of the same height as one of shares for 6,144 rows (24): refused, and so are shares made for other
-    heads or another rotation."""
+    heads or another rotation, or in tiles of 16, which are read in an order of their own."""
     nq, nkv, d, K = 32, 8, 128, 64
     rot, _ = rotation_for(ops, d, 10000.0, 1.0, False)
     other, _ = rotation_for(ops, d, 10000.0, 0.5, False)
@@ -1347,7 +1347,8 @@ def test_qkv_rope_commit_refuses_copies_in_another_order(ops):
     assert stored.shape == ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, rot, shares=True), 24).shape
     swapped = torch.arange(w.shape[0] - 1, -1, -1, dtype=torch.int32, device=DEV)
     for tiles in (stored, ops.tile_weights(w, swapped, 24), ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, other, shares=True), 24),
-                  ops.tile_weights(w, ops.qkv_tile_rows(40, 4, d, DEV, rot, shares=True), 24)):
+                  ops.tile_weights(w, ops.qkv_tile_rows(40, 4, d, DEV, rot, shares=True), 24),
+                  ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, rot, shares=True), 16)):
         with pytest.raises(ops.KernelError, match="tiles"):
             call(tiles)
     call(ops.tile_weights(w, ops.qkv_tile_rows(nq, nkv, d, DEV, rot, shares=True), 24))

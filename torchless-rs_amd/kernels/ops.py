@@ -2413,8 +2413,9 @@ def qkv_rope_commit(a: torch.Tensor, w: torch.Tensor, row_pos, rotation, table, 
     # a copy's height says nothing of the order of its rows: `tile_weights` of 6,144 rows as stored has tiles of 24 as well
     share_order = getattr(tiles, "share_order", None)
     height = _req_tiles(tiles, (nq + 2 * nkv) * d, K, height=16 if share_order is None else None)
-    if share_order is not None and share_order != _share_order(nq, nkv, d, rot.rotary_dim, rot.interleaved):
-        raise KernelError(f"qkv_rope_commit.tiles: rows in the order of (nq, nkv, d, rotated channels, interleaved) = {share_order}")
+    if share_order is not None and (height == 16 or share_order != _share_order(nq, nkv, d, rot.rotary_dim, rot.interleaved)):
+        raise KernelError(f"qkv_rope_commit.tiles: tiles of {height} rows in the order of shares of (nq, nkv, d, rotated channels, "
+                          f"interleaved) = {share_order}")
     _req(row_pos, "qkv_rope_commit.row_pos", torch.int32, (n,))
     _req(q, "qkv_rope_commit.q", torch.bfloat16, (n, nq, d))
     _req(table, "qkv_rope_commit.table", torch.int32)
