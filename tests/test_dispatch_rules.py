@@ -63,6 +63,22 @@ def test_rows_choose_the_kernel():
     assert [odd.own_kernels(m) for m in (64, 65)] == [True, False]
 
 
+def test_a_weight_takes_rows_in_an_order_of_its_own_for_its_copy(monkeypatch):
+    """`tile_rows` by name and third in order; the copy made by them is for the kernel that wants them alone."""
+    import torch
+    from types import SimpleNamespace
+    from torchless_rs_amd.parts import linear
+    made = []
+    monkeypatch.setattr(linear.ops, "tile_weights", lambda w, rows=None: made.append(rows) or "copy")
+    w, rows = torch.zeros(32, 64, dtype=torch.bfloat16), torch.arange(32, dtype=torch.int32)
+    assert linear.Linear(w, tiled=True, tile_rows=rows).own_tiles is None and not made      # (no device, no copy)
+    on_device = SimpleNamespace(dim=w.dim, contiguous=lambda: on_device, shape=w.shape, is_cuda=True, dtype=w.dtype)
+    for lin in (linear.Linear(on_device, tiled=True, tile_rows=rows), linear.Linear(on_device, True, rows)):
+        assert lin.own_tiles == "copy" and lin.tiles is None and made.pop() is rows
+    lin = linear.Linear(on_device, tiled=True)
+    assert lin.tiles == "copy" and lin.own_tiles is None and made.pop() is None
+
+
 def test_prefill_layout_cuts_long_blocks_of_small_launches_into_runs():
     """The host's layout for the multi-token attention of a step with fewer workgroups than compute
     units: every block's keys are covered once, by one entry or by consecutive runs, no run shorter

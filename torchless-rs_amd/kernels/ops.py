@@ -1884,8 +1884,8 @@ def tile_weights(w: torch.Tensor, rows: Optional[torch.Tensor] = None, height: O
     16 rows stream from: [ceil(N / R), K/64, 2, 4, R, 8] with element (T, s, c, g, r, e) =
     w[rows[R T + r], 64 s + 16 g + 8 c + e], so that what a workgroup reads is one run of memory (and
     with R = 16 what a wave loads at a time, lane after lane).  `rows` (int32 [N], on the device): a
-    permutation of the rows; None: none.  `height`: R; None: `tile_height(N)`, or 16 with `rows`
-    (the kernel that wants its own order reads tiles of 16).  Places of the last tile behind row N are
+    permutation of the rows; None: none.  `height`: R; None: `tile_height(N)`, or with `rows` what the kernel that
+    wants its own order reads fastest (16, or the shares of `qkv_tile_rows`).  Places of the last tile behind row N are
     zero."""
     N, K = w.shape
     _req(w, "tile_weights.w", torch.bfloat16)
@@ -1893,14 +1893,17 @@ def tile_weights(w: torch.Tensor, rows: Optional[torch.Tensor] = None, height: O
         raise KernelError(f"tile_weights: N={N} must be a multiple of 16 and K={K} of 64")
     if rows is not None:
         _req(rows, "tile_weights.rows", torch.int32, (N,))
-    R = int(height) if height is not None else (16 if rows is not None else tile_height(N))
+    share_order = getattr(rows, "share_order", None)
+    if height is None:
+        height = tile_height(N) if rows is None else 16 if share_order is None else lib().tl_qkv_tile_height(*share_order[:3])
+    R = int(height)
     if not 16 <= R <= 32:
         raise KernelError(f"tile_weights: tiles of {R} rows (16 to 32)")
     n_tiles = -(-N // R)
     make = torch.empty if n_tiles * R == N else torch.zeros
     out = make((n_tiles, K // 64, 2, 4, R, 8), dtype=torch.bfloat16, device=w.device)
     _check(lib().tl_tile_weights(_p(w), _p(rows), N, K, R, _p(out), _stream()))
-    out.share_order = getattr(rows, "share_order", None)
+    out.share_order = share_order
     return out
 
 
@@ -1924,11 +1927,15 @@ def _share_order(nq: int, nkv: int, d: int, rotary_dim: int, interleaved: bool) 
     return int(nq), int(nkv), int(d), int(rotary_dim), bool(interleaved)
 
 
+def qkv_in_shares(nq: int, nkv: int, d: int) -> bool:
+    """Does `qkv_rope_commit` read a copy fastest whose tiles are its workgroups' shares of the rows on this device?  (Where those are
+    more than 16 rows; else tiles of 16.)"""
+    return int(lib().tl_qkv_tile_height(int(nq), int(nkv), int(d))) > 16
+
+
 def qkv_tiles(w: torch.Tensor, nq: int, nkv: int, d: int, rotation=None) -> torch.Tensor:
-    """The tiled copy of w = q|k|v that `qkv_rope_commit` reads fastest on this device: tiles that are its workgroups' shares of the rows
-    where those are more than 16, else tiles of 16 (`qkv_tile_rows`)."""
-    height = int(lib().tl_qkv_tile_height(int(nq), int(nkv), int(d)))
-    return tile_weights(w, qkv_tile_rows(nq, nkv, d, w.device, rotation, shares=height > 16), height)
+    """The tiled copy of w = q|k|v that `qkv_rope_commit` reads fastest."""
+    return tile_weights(w, qkv_tile_rows(nq, nkv, d, w.device, rotation, shares=qkv_in_shares(nq, nkv, d)))
 
 
 def _req_tiles(tiles: Optional[torch.Tensor], N: int, K: int, height: Optional[int] = None) -> int:

@@ -98,11 +98,11 @@ class AttentionMixer(Mixer):
             fused = torch.cat(ws, dim=0)
         # single-token steps stream q|k|v and o from tiled copies; the fused q|k|v kernel has its own
         # order of rows, which follows the pairs of the rotation
-        copy = None
+        rows = None
         if self.own_kv and self.d % 16 == 0 and fused.is_cuda and fused.dtype == torch.bfloat16:
-            rotation = self.position.rotation(fused.device) or ops.NO_ROTATION
-            copy = lambda w: ops.qkv_tiles(w, self.nq, self.nkv, self.d, rotation)
-        self.qkv = Linear(fused, tiled=True, own_copy=copy)
+            rows = ops.qkv_tile_rows(self.nq, self.nkv, self.d, fused.device, self.position.rotation(fused.device) or ops.NO_ROTATION,
+                                     shares=ops.qkv_in_shares(self.nq, self.nkv, self.d))
+        self.qkv = Linear(fused, tiled=True, tile_rows=rows)
         self.o = Linear(tensors[p + nm["o"]], tiled=True)
 
     def norms_rows(self, ctx, norm, x: torch.Tensor, run) -> bool:

@@ -30,21 +30,22 @@ class Linear:
     """A weight [N, K] resident on the device in its stored width.  With `tiled` it
     also keeps the tiled copy (`ops.tile_weights`) that the products of steps of at
     most 16 rows read instead: memory spent for the rate at which decoding streams
-    the weights (a load under `loading_with(False)` makes none).  `own_copy`: makes the
-    copy of the weight for a kernel that wants an order of rows of its own; then only that kernel
+    the weights (a load under `loading_with(False)` makes none).  `tile_rows`: the
+    copy's own order of rows, for a kernel that wants one; then only that kernel
     reads it (`own_tiles`)."""
 
-    def __init__(self, weight: torch.Tensor, tiled: bool = False, own_copy=None):
+    def __init__(self, weight: torch.Tensor, tiled: bool = False, tile_rows: torch.Tensor = None):
         assert weight.dim() == 2
         self.weight = weight.contiguous()
         self.out_features, self.in_features = self.weight.shape
         self.tiles = self.own_tiles = None
         if (tiled and _tiled_copies.get() and self.weight.is_cuda and self.weight.dtype == torch.bfloat16
                 and ops.tiles_fit(self.out_features, self.in_features)):
-            if own_copy is None:
-                self.tiles = ops.tile_weights(self.weight)
+            copy = ops.tile_weights(self.weight, tile_rows)
+            if tile_rows is None:
+                self.tiles = copy
             else:
-                self.own_tiles = own_copy(self.weight)
+                self.own_tiles = copy
 
     def __call__(self, a: torch.Tensor, out: torch.Tensor, accumulate: bool = False, factor=None) -> None:
         """out[M, N] (+)= a[M, K] @ W^T; out is float32.  `factor` (`ops.RowFactor`): the
