@@ -902,3 +902,67 @@ def test_who_norms_the_rows_of_a_feed_forward(rows, H, own_forward):
     ops.act_mul(gu, h)
     ops.gemm_plain(h, ffn.down.weight, want, True)
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("what", ["nothing", "hidden", "forward on the part", "forward on the norm", "a norm derived", "a product of its own"])
+def test_parts_that_go_their_own_way_get_normed_rows(what):
+    """Few rows in 32 bits, and a method of the feed-forward, of the norm or of the weight that is not the package's: it runs, on what it
+    would be handed without the shorter way, and nothing fails.  (Two times the gate's rows or the norm, or one more than the product.)"""
+    from types import SimpleNamespace
+    from torchless_rs_amd.kernels import ops
+    from torchless_rs_amd.parts.base import Workspace, part_done, read_through_norm
+    from torchless_rs_amd.parts.ffn import SwiGLU
+    from torchless_rs_amd.parts.linear import Linear
+    from torchless_rs_amd.parts.norms import RMSNorm
+    rows, H, I = 3, 64, 48
+    calls = []
+
+    class Hidden(SwiGLU):
+        def _hidden(self, ctx, y):
+            calls.append(y.clone())
+            return SwiGLU._hidden(self, ctx, y * 2.0)
+
+    class Doubled(RMSNorm):
+        def forward(self, ctx, x, out):
+            calls.append(x.clone())
+            RMSNorm.forward(self, ctx, x, out)
+            out *= 2.0
+
+    class More(Linear):
+        def __call__(self, a, out, accumulate=False, factor=None):
+            calls.append(a.clone())
+            Linear.__call__(self, a, out, accumulate, factor)
+            out += 1.0
+
+    g = torch.Generator().manual_seed(61)
+    ffn = (Hidden if what == "hidden" else SwiGLU)(H, I)
+    norm = (Doubled if what == "a norm derived" else RMSNorm)(H, 1e-5)
+    ffn.load({"mlp.gate_proj.weight": torch.randn(I, H, generator=g).to(DEV), "mlp.up_proj.weight": torch.randn(I, H, generator=g).to(DEV),
+              "mlp.down_proj.weight": torch.randn(H, I, generator=g).to(DEV)}, torch.float32)
+    norm.load({"weight": torch.randn(H, generator=g).to(DEV)}, torch.float32)
+    x = torch.randn(rows, H, generator=g).to(DEV)
+    y, want = torch.empty_like(x), x.clone()
+    RMSNorm.forward(norm, None, x, y)
+    normed = y.clone()
+    if what == "forward on the part":
+        ffn.forward = lambda ctx, y, x: (calls.append(y.clone()), SwiGLU.forward(ffn, ctx, y * 2.0, x))
+    if what == "forward on the norm":
+        norm.forward = lambda ctx, x, out: (calls.append(x.clone()), RMSNorm.forward(norm, ctx, x, out), out.mul_(2.0))
+    if what == "a product of its own":
+        ffn.gate_up = More(ffn.gate_up.weight)
+    ctx = SimpleNamespace(prenormed=None, pending=None, row_factor=None, row_norm=None, settle=None, norm_ahead=None, dtype=torch.float32,
+                          workspace=Workspace(DEV))
+    got = read_through_norm(ctx, norm, x, y, ffn)
+    assert (got is x) == (what == "nothing")
+    ffn.forward(ctx, got, x)
+    part_done(ctx, ffn)
+    assert len(calls) == (what != "nothing")
+    if calls:
+        assert torch.equal(calls[0], want if "norm" in what else normed)
+    gu, h = torch.empty(rows, 2 * I, device=DEV), torch.empty(rows, I, device=DEV)
+    ops.gemm_plain(normed if what in ("nothing", "a product of its own") else normed * 2.0, ffn.gate_up.weight, gu)
+    if what == "a product of its own":
+        gu += 1.0
+    ops.act_mul(gu, h)
+    ops.gemm_plain(h, ffn.down.weight, want, True)
+    assert torch.equal(x, want)

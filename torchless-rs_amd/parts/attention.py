@@ -106,11 +106,12 @@ class AttentionMixer(Mixer):
         self.o = Linear(tensors[p + nm["o"]], tiled=True)
 
     def norms_rows(self, ctx, norm, x: torch.Tensor, run) -> bool:
-        return goes_as(self, AttentionMixer) and self._around(ctx, x, run) and ops.row_norm_ok(norm.rms_form(), self.H)
+        return goes_as(self, AttentionMixer, "forward") and self._around(ctx, x, run) and ops.row_norm_ok(norm.rms_form(), self.H)
 
     def _around(self, ctx, y: torch.Tensor, run) -> bool:
-        """Does a step of single tokens do the norm, q|k|v, the rotation and the commit in one launch of the 32-bit path?"""
-        return (self.own_kv and ctx.all_single and not run.kv_read_later and self.d % 8 == 0 and self.d <= 256
+        """Does a step of single tokens do the norm, q|k|v, the rotation and the commit in one launch of the 32-bit path?  (Not for a
+        weight with a product of its own.)"""
+        return (self.own_kv and ctx.all_single and not run.kv_read_later and self.d % 8 == 0 and self.d <= 256 and type(self.qkv) is Linear
                 and run.kv_group.storage[run.kv_layer].dtype == torch.float32 and ops.plain_around_ok(y, self.qkv.weight))
 
     def forward(self, ctx, run, y: torch.Tensor, x: torch.Tensor) -> None:

@@ -283,10 +283,24 @@ def take_row_factor(ctx: "StepContext", usable: bool):
     return f
 
 
-def goes_as(part: Part, kind: type) -> bool:
-    """Is `part`'s `forward` that of `kind`?  (A part made from `kind` with a `forward` of its own is run through that, whatever
-    shorter way `kind` has.)"""
-    return type(part).forward is kind.forward
+def goes_as(part: Part, kind: type, *methods: str) -> bool:
+    """Are these `methods` of `part` those of `kind`?  (A part made from `kind` with one of its own, or one set on the object, is run
+    through that, whatever shorter way `kind` has.)"""
+    own = getattr(part, "__dict__", ())
+    return all(m not in own and getattr(type(part), m) is getattr(kind, m) for m in methods)
+
+
+def norms_as_its_form(norm: "Norm") -> bool:
+    """Does `norm.forward` do what its `rms_form` says?  Not where it was set on the object, or by a class derived from the one that
+    says the form: such a norm is run by itself."""
+    if "forward" in getattr(norm, "__dict__", ()):
+        return False
+    for c in type(norm).__mro__:
+        if "rms_form" in vars(c):
+            return True
+        if "forward" in vars(c):
+            return False
+    return False
 
 
 def take_row_norm(ctx: "StepContext"):
@@ -305,14 +319,14 @@ def read_through_norm(ctx: "StepContext", norm: "Norm", x: torch.Tensor, y: torc
     row goes to the part that reads it (`ctx.row_factor`; `ctx.settle` runs the plain norm into
     the same buffer for a part that cannot apply it).  `reader`: the part behind the norm, if the block
     hands it nothing but what this returns; one whose first product does the norm itself at these sizes
-    (`norms_rows(ctx, norm, x, run)`) gets the stream and `ctx.row_norm`."""
+    (`norms_rows(ctx, norm, x, run)`) gets the stream and `ctx.row_norm`, if the norm does what its form says (`norms_as_its_form`)."""
     pre, ctx.prenormed = ctx.prenormed, None
     if pre is not None and pre[0] is norm:
         ctx.row_factor = pre[2]
         ctx.settle = lambda: norm.forward(ctx, x, pre[1])
         return pre[1]
     can = getattr(reader, "norms_rows", None)
-    if can is not None and ctx.pending is None and can(ctx, norm, x, run):
+    if can is not None and ctx.pending is None and norms_as_its_form(norm) and can(ctx, norm, x, run):
         ctx.row_norm = norm.rms_form()
         return x
     if not getattr(norm, "takes_pending", False):

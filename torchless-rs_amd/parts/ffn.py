@@ -76,10 +76,12 @@ class SwiGLU(FeedForward):
         self.down = Linear(tensors[p + nm["down"]], tiled=True)
 
     def norms_rows(self, ctx, norm, x: torch.Tensor, run) -> bool:
-        return goes_as(self, SwiGLU) and ctx.dtype == torch.float32 and self._around(x) and ops.row_norm_ok(norm.rms_form(), self.H)
+        return (goes_as(self, SwiGLU, "forward", "_hidden") and ctx.dtype == torch.float32 and self._around(x)
+                and ops.row_norm_ok(norm.rms_form(), self.H))
 
     def _around(self, y: torch.Tensor) -> bool:
-        return self.I % 4 == 0 and ops.plain_around_ok(y, self.gate_up.weight)
+        """Does the 32-bit path do the product and the activation in one launch?  (Not for a weight with a product of its own.)"""
+        return self.I % 4 == 0 and type(self.gate_up) is Linear and ops.plain_around_ok(y, self.gate_up.weight)
 
     def forward(self, ctx, y: torch.Tensor, x: torch.Tensor) -> None:
         self.down.add_into(self._hidden(ctx, y), x, ctx, "ffn_down_parts")
