@@ -201,3 +201,66 @@ def test_a_failing_step_leaves_nothing_held():
     with pytest.raises(ValueError, match="no room"):
         generate(eng, ArgmaxSampler(), [[1], [5, 6]], max_tokens=6)
     assert not eng.held
+
+
+# ---- how the host waits for a draw's tokens --------------------------------------------------
+
+class Place:
+    """Memory of a draw whose tokens are there from the `after`-th look on, or once its event has been waited for."""
+
+    def __init__(self, after):
+        import numpy as np
+        outer, self.waits, self.looks, self.mem = self, 0, 0, np.array([-1, -1, -1, 77], dtype=np.int32)
+
+        class Ids:
+            size = 3
+
+            def min(self):
+                outer.looks += 1
+                if outer.looks >= after:
+                    outer.mem[:3] = (4, 0, 6)
+                return outer.mem[:3].min()
+
+            def tolist(self):
+                return outer.mem[:3].tolist()
+
+        class Looked:
+            def __getitem__(self, rows):
+                assert rows == slice(None, 3)
+                return Ids()
+
+        class Event:
+            def synchronize(self):
+                outer.waits += 1
+                outer.mem[:3] = (4, 0, 6)
+
+        self.ids, self.done = Looked(), Event()
+
+
+def test_a_draw_with_a_step_behind_it_is_waited_for_without_looking():
+    """The interpreter is not kept from other threads: one wait, whatever lies in the memory, none the second time."""
+    from torchless_rs_amd.sampling.sampler import Drawn
+    for after in (1, 10 ** 9):
+        place = Place(after)
+        drawn = Drawn(torch.empty(3, dtype=torch.int32), place)
+        assert drawn.tokens() == [4, 0, 6] and drawn.tokens() == [4, 0, 6]
+        assert (place.waits, place.looks, place.done) == (1, 0, None)
+
+
+def test_tokens_wanted_at_once_are_looked_for_and_then_waited_for(monkeypatch):
+    from torchless_rs_amd.sampling import sampler
+    place = Place(after=3)
+    drawn = sampler.Drawn(torch.empty(3, dtype=torch.int32), place)
+    monkeypatch.setattr(sampler.Sampler, "draw", lambda self, *a: drawn)
+    assert sampler.Sampler(None, "cuda:0").sample(None, [], []) == [4, 0, 6]
+    assert (place.waits, place.looks, place.done) == (0, 3, None)
+    place = Place(after=10 ** 9)                             # late: the event is waited for
+    monkeypatch.setattr(sampler, "LOOK_FOR", 0.0)
+    drawn = sampler.Drawn(torch.empty(3, dtype=torch.int32), place)
+    assert sampler.Sampler(None, "cuda:0").sample(None, [], []) == [4, 0, 6]
+    assert place.waits == 1 and place.done is None
+    place = Place(after=10 ** 9)                             # the memory is another draw's by now: it stays taken
+    drawn = sampler.Drawn(torch.empty(3, dtype=torch.int32), place)
+    later = place.done = object()
+    drawn.tokens()
+    assert place.done is later

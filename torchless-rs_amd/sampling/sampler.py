@@ -14,19 +14,20 @@ from ..kernels import ops
 from .config import SamplingConfig
 
 
-LOOK_FOR = 1e-4       # seconds that the host looks at the tokens' memory before it waits for the draw's event instead: an event behind
-                      # a kernel is known 9 us after it, a token that the kernel wrote at once (16 rows of 131,072: 49 and 42 us a draw)
+LOOK_FOR = 1e-4       # seconds that the host looks at the memory of tokens that it wants at once (`Sampler.sample`) before it waits for the
+                      # draw's event instead: an event behind a kernel is known 9 us after it, a token that the kernel wrote at once (16 rows
+                      # of 131,072: 49 and 42 us a draw).  Looking keeps the interpreter, so a draw with a step behind it is only waited for
 
 
 class _Place:
     """Pinned host memory of one draw: what its kernel reads, the (sequence, step) pairs, and writes, the tokens.  The kernel goes by
     their addresses, of which torch's allocator knows nothing, so the memory is held until the draw is over."""
+    done = None                          # the event behind the draw that uses it, None once that is known to be over
 
     def __init__(self, cap: int):
         self.counters = torch.empty((cap, 2), dtype=torch.int32, pin_memory=True)
         self.tokens = torch.empty((cap,), dtype=torch.int32, pin_memory=True)
         self.pairs, self.ids = self.counters.numpy(), self.tokens.numpy()
-        self.done = None                 # the event behind the draw that uses it, None once that is known to be over
 
     def wait(self) -> None:
         if self.done is not None:
@@ -38,8 +39,8 @@ class _Place:
 
 
 class Drawn:
-    """The tokens of one draw: on the device at once (`device`, int32 [B], in the order of
-    the draw's stream, valid until the sampler's next draw has been launched), on the host when `tokens()` is asked for (until two
+    """The tokens of one draw: on the device at once (`device`, int32 [B], valid until the
+    sampler's next draw has been launched), on the host when `tokens()` is asked for (until two
     more draws have been launched)."""
 
     def __init__(self, device: torch.Tensor, place: _Place):
@@ -47,16 +48,25 @@ class Drawn:
 
     def tokens(self) -> List[int]:
         if self._tokens is None:
-            place, ids = self._place, self._place.ids[:self.device.shape[0]]
-            # a row's token, never negative, is the last that its workgroup does with the memory: where all are there the draw is over
+            self._done.synchronize()
+            self._take()
+        return self._tokens
+
+    def _take(self) -> None:
+        if self._place.done is self._done:
+            self._place.done = None
+        self._tokens = self._place.ids[:self.device.shape[0]].tolist()
+
+    def tokens_at_once(self) -> List[int]:
+        """`tokens()` for a caller that has nothing else to do meanwhile."""
+        if self._tokens is None:
+            ids = self._place.ids[:self.device.shape[0]]
+            # a row's token, never negative, is the last that its workgroup does with the memory: where all are there it may be used again
             until = time.perf_counter() + LOOK_FOR
             while ids.size and ids.min() < 0:
                 if time.perf_counter() > until:
-                    self._done.synchronize()
-                    break
-            if place.done is self._done:
-                place.done = None
-            self._tokens = ids.tolist()
+                    return self.tokens()
+            self._take()
         return self._tokens
 
 
@@ -101,7 +111,7 @@ class Sampler:
 
     def sample(self, logits: torch.Tensor, seq_ids: Sequence[int], steps: Sequence[int]) -> List[int]:
         """logits: float32 [B, V] on the GPU -> B token ids."""
-        return self.draw(logits, seq_ids, steps).tokens()
+        return self.draw(logits, seq_ids, steps).tokens_at_once()
 
     def last_distribution(self, B: int) -> torch.Tensor:
         """The probabilities the last draw was made from (temperature > 0)."""
