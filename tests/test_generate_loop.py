@@ -264,3 +264,10 @@ def test_tokens_wanted_at_once_are_looked_for_and_then_waited_for(monkeypatch):
     later = place.done = object()
     drawn.tokens()
     assert place.done is later
+
+
+def test_a_distribution_is_there_for_any_stream():
+    from torchless_rs_amd.sampling.sampler import Sampler
+    s, place = Sampler(None, "cuda:0"), Place(after=1)
+    s._probs, s._last = torch.eye(4), place.done
+    assert torch.equal(s.last_distribution(2), torch.eye(4)[:2]) and place.waits == 1

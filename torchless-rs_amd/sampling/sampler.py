@@ -58,7 +58,8 @@ class Drawn:
         self._tokens = self._place.ids[:self.device.shape[0]].tolist()
 
     def tokens_at_once(self) -> List[int]:
-        """`tokens()` for a caller that has nothing else to do meanwhile."""
+        """`tokens()` for a caller that has nothing else to do meanwhile.  What the draw leaves on the device is there for the draw's
+        own stream only when this returns."""
         if self._tokens is None:
             ids = self._place.ids[:self.device.shape[0]]
             # a row's token, never negative, is the last that its workgroup does with the memory: where all are there it may be used again
@@ -80,6 +81,7 @@ class Sampler:
         self._out = None
         self._places = None              # two, used in turn: a draw may be launched while the one before is read
         self._turn = 0
+        self._last = None                # the event behind the last draw
 
     def draw(self, logits: torch.Tensor, seq_ids: Sequence[int], steps: Sequence[int]) -> Drawn:
         """logits: float32 [B, V] on the GPU -> B token ids, without waiting for them: the
@@ -105,7 +107,7 @@ class Sampler:
         out = self._out[:B]
         ops.sample(logits.contiguous(), float(c.temperature), int(c.top_k or 0), float(c.top_p or 0.0),
                    int(c.seed), place.counters[:B], self._probs[:B], out, self._lists, place.tokens[:B])
-        place.done = torch.cuda.Event()
+        self._last = place.done = torch.cuda.Event()
         place.done.record()
         return Drawn(out, place)
 
@@ -114,5 +116,6 @@ class Sampler:
         return self.draw(logits, seq_ids, steps).tokens_at_once()
 
     def last_distribution(self, B: int) -> torch.Tensor:
-        """The probabilities the last draw was made from (temperature > 0)."""
+        """The probabilities the last draw was made from (temperature > 0), there for any stream."""
+        self._last.synchronize()
         return self._probs[:B]
