@@ -250,6 +250,7 @@ def test_a_draw_with_a_step_behind_it_is_waited_for_without_looking():
 def test_tokens_wanted_at_once_are_looked_for_and_then_waited_for(monkeypatch):
     from torchless_rs_amd.sampling import sampler
     place = Place(after=3)
+    monkeypatch.setattr(sampler, "LOOK_FOR", 60.0)           # (however slow this machine is)
     drawn = sampler.Drawn(torch.empty(3, dtype=torch.int32), place)
     monkeypatch.setattr(sampler.Sampler, "draw", lambda self, *a: drawn)
     assert sampler.Sampler(None, "cuda:0").sample(None, [], []) == [4, 0, 6]
