@@ -91,7 +91,7 @@ def step(ops, lengths, nq, nkv, d, seed=0):
     return q, pages, table, ctx
 
 
-def want(q, pages, table, lengths, scale, window=0, keep=0, chunk=0, logistic=False, bias=None, sinks=None, gate=None):
+def want(q, pages, table, lengths, scale, window=0, keep=0, chunk=0, logistic=False, bias=None, sinks=None, gate=None, slopes=None):
     B, nq, d = q.shape
     nkv = pages.shape[2]
     out, size = torch.empty(B, nq, d, dtype=torch.float64, device=DEV), torch.empty(B, nq, d, dtype=torch.float64, device=DEV)
@@ -101,6 +101,8 @@ def want(q, pages, table, lengths, scale, window=0, keep=0, chunk=0, logistic=Fa
         v = mine[:, 1].reshape(-1, nkv, d, PAGE).permute(1, 0, 3, 2).reshape(nkv, -1, d)[:, :L].repeat_interleave(nq // nkv, 0)
         s = (k * q[b].double()[:, None]).sum(-1) * scale
         j, p = torch.arange(L, device=DEV), L - 1
+        if slopes is not None:
+            s = s - slopes.double()[:, None] * (p - j)
         ok = torch.ones(L, dtype=torch.bool, device=DEV)
         if window:
             ok &= (p - j < window) | (j < keep)
@@ -170,6 +172,32 @@ def test_attention_in_an_order_has_the_bits_of_the_batch_s_own(ops, nq, nkv, d, 
     assert torch.equal(out, own)
 
 
+@pytest.mark.parametrize("kind", ["sinks", "logistic", "kept", "chunk", "slopes"])
+def test_attention_with_terms_in_an_order(ops, monkeypatch, kind):
+    """Whole sequences in an order with each of the terms, tables of more than 64 pages: the bits of the batch's own order, and float64's result at
+    the weights' and the result's 8 bits."""
+    nq, nkv, d, B = 16, 8, 64, 64
+    lengths = [1 + (i * 613) % 900 for i in range(B)]
+    lengths[5], lengths[40] = 4300, 2222
+    q, pages, table, ctx = step(ops, lengths, nq, nkv, d, 3)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    kw = {"sinks": {"sinks": torch.randn(nq, generator=g, device=DEV)}, "kept": {"window": 200, "keep_first": 70}, "chunk": {"chunk": 192},
+          "logistic": {"logistic": True, "score_bias": torch.randn(nq, generator=g, device=DEV) - 4.0},
+          "slopes": {"slopes": 0.02 * torch.rand(nq, generator=g, device=DEV)}}[kind]
+    ref_kw = {{"score_bias": "bias", "keep_first": "keep"}.get(k, k): v for k, v in kw.items()}
+    gate = torch.rand(B, nq, generator=g, device=DEV) if kind in ("sinks", "logistic") else None
+    ring = 1 << 20 if kind == "kept" else table.shape[1]
+    call = lambda out: ops.attention_scored(q, None, None, pages, nkv, d, table, ring, ctx, None, ops.ScoreTerms(d ** -0.5, **kw), gate, out)
+    out, own = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    call(out)
+    assert [seqs for _, seqs in ctx.host["decode_plans"].values()] == [None]
+    monkeypatch.setattr(ops, "decode_plan", lambda *a, **k: None)
+    call(own)
+    assert torch.equal(out, own)
+    ref, size = want(q, pages, table, lengths, d ** -0.5, gate=gate, **ref_kw)
+    assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs()) + 1e-5).all())
+
+
 def test_who_goes_without_a_plan(ops):
     assert ops.decode_places(32, 32, 8, 33, 256, 128) is None and ops.decode_places(48, 32, 8, 33, 256, 128) is None
     assert ops.decode_places(64, 32, 8, 33, 256, 128) == (32, 64) and ops.decode_places(64, 512, 512, 33, 256, 128) is None
@@ -227,5 +255,47 @@ def test_replayed_steps_are_planned_by_their_own_lengths(tmp_path, ops, window):
     for g in engines[0]._graphs.values():
         planned += g.graph is not None and any(name.startswith("attn_plan_") for name in g.workspace._bufs)
     assert planned and not engines[1]._graphs
+    for eng in engines:
+        eng.close()
+
+
+def test_replayed_steps_are_ordered_by_their_own_lengths(tmp_path, ops):
+    """A captured step of 64 sequences puts them in order at every replay: they change places in the batch and grow over page boundaries,
+    with eager work and synchronisations between the replays, and every step has the bits of an engine that never captures, and
+    float64's logits at the format's tolerance."""
+    import plain_mistral as plain
+    from torchless_rs_amd import write_random_model
+    from torchless_rs_amd.engine import Engine, SeqInput, load_model
+    from util import TOL, prompts, read_model_dir, rel_err
+    cfg = {"architectures": ["MistralForCausalLM"], "model_type": "mistral", "hidden_size": 256, "num_hidden_layers": 2, "num_attention_heads": 8, "num_key_value_heads": 8, "head_dim": 64,
+           "intermediate_size": 256, "vocab_size": 300, "rope_theta": 10000.0, "sliding_window": None, "rms_norm_eps": 1e-5,
+           "max_position_embeddings": 4096, "tie_word_embeddings": False, "hidden_act": "silu"}
+    mdir = write_random_model(str(tmp_path / "m"), cfg, seed=7, std=0.05, norm_std=0.1, dtype=torch.bfloat16)
+    cfgd, w = read_model_dir(mdir)
+    model = load_model(mdir, "bfloat16")
+    B = 64
+    ids = prompts(cfg["vocab_size"], [500] * B, seed=10)
+    at = [460 if i == 3 else 1 + (i * 53) % 300 for i in range(B)]       # the longest goes on inside its 8th page
+    engines = [Engine(model, max_tokens=64 * 8 * (B + 2), max_slots=B + 2, use_graphs=g) for g in (True, False)]
+    for eng in engines:
+        eng.slots_ = [eng.alloc() for _ in ids]
+        eng.step([SeqInput(s, p[:n], []) for s, p, n in zip(eng.slots_, ids, at)])
+    for t in range(20):
+        batch = sorted(range(B), key=lambda i: (i * (2 * t + 1) + 11 * t) % B)
+        outs = []
+        for eng in engines:
+            outs.append(eng.step([SeqInput(eng.slots_[i], [ids[i][at[i]]], [0]) for i in batch]).clone())
+            if t % 4 == 0:
+                extra = eng.alloc()
+                eng.step([SeqInput(extra, ids[1][:100 + t], [0])])
+                eng.free(extra)
+            torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]), t
+        for row, i in enumerate(batch):
+            if t % 9 == 0 and row % 13 == 0:
+                assert rel_err(outs[0][row:row + 1], plain.forward(w, cfgd, ids[i][:at[i] + 1])[-1:]) < TOL["bfloat16"], (t, i)
+            at[i] += 1
+    assert any(g.graph is not None and any(name.startswith("attn_plan_order") for name in g.workspace._bufs) for g in engines[0]._graphs.values())
+    assert not engines[1]._graphs
     for eng in engines:
         eng.close()

@@ -346,8 +346,8 @@ def test_gemm_plain_adds_in_one_order(ops, N, K):
 @pytest.mark.parametrize("N,K", [(33, 32), (70, 96), (65, 4128), (131, 12320), (2, 1024)])
 @pytest.mark.parametrize("M", [5, 17, 48, 65, 80, 129, 300])
 def test_gemm_plain_on_the_matrix_cores_has_the_bits_of_one_row(ops, N, K, M):
-    """Tiles of one to eight blocks of rows, with and without all groups of K in one workgroup, ends of tiles and of K, rows further
-    apart in memory than K, large and tiny numbers: the bits of the kernel for a row alone."""
+    """Tiles of two, three, five and seven blocks of rows, with and without all groups of K in one workgroup, ends of tiles and of K, large and
+    tiny numbers: the bits of the kernel for a row alone (5 rows are the kernel's for few)."""
     a, w = rnd(M, K, seed=45).to(DEV), rnd(N, K, seed=46).to(DEV)
     a[0] *= 1e-20
     w[0] *= 1e-20
@@ -360,6 +360,38 @@ def test_gemm_plain_on_the_matrix_cores_has_the_bits_of_one_row(ops, N, K, M):
     for m in {0, 1, M // 2, M - 1}:
         ops.gemm_plain(a[m:m + 1].contiguous(), w, one)
         assert torch.equal(out[m:m + 1], one), m
+
+
+def same_bits(a, b):
+    """Equal numbers of equal signs, NaN where the other has NaN."""
+    return bool(((a.view(torch.int32) == b.view(torch.int32)) | (a.isnan() & b.isnan())).all())
+
+
+@pytest.mark.parametrize("N,K", [(70, 96), (131, 4128), (33, 1024)])
+@pytest.mark.parametrize("M", [9, 16, 64, 96, 128, 177, 256])
+def test_gemm_plain_on_the_matrix_cores_strided_and_of_any_numbers(ops, M, N, K):
+    """Tiles of one, four, six and eight blocks of rows that lie further apart in memory than K, added to rows further apart than N, with and
+    without scratch; infinities, NaN, denormals and numbers 40 powers of two apart: the bits of the kernel for a row alone."""
+    a, w = rnd(M, K, seed=47), rnd(N, K, seed=48)
+    for k, v in ((3, float("inf")), (K // 2, -float("inf")), (K - 1, float("nan"))):
+        a[k % M, k] = v
+    w[5, 7], w[6, 9] = float("inf"), float("nan")
+    a[1 % M] *= 1e-38                                     # numbers and products that are denormals, or nearly
+    w[1] *= 2.0 ** -120
+    a[M - 2] *= 2.0 ** torch.randint(-20, 20, (K,), generator=torch.Generator().manual_seed(49)).float()
+    wide_a, wide_w = torch.full((M, K + 4), float("nan"), device=DEV), torch.full((N, K + 8), float("nan"), device=DEV)
+    wide_a[:, :K], wide_w[:, :K] = a.to(DEV), w.to(DEV)
+    base, want = rnd(M, N + 3, seed=50).to(DEV), torch.empty(M, N, device=DEV)
+    for m in range(M):
+        row = base[m:m + 1, :N].clone()
+        ops.gemm_plain(a[m:m + 1].to(DEV), w.to(DEV), row, True)
+        want[m] = row
+    n_parts = ops.lib().tl_gemm_plain_parts(M, N, K)
+    for parts in (None, torch.full((max(n_parts, 1),), float("nan"), device=DEV)):
+        out = base.clone()
+        ops._check(ops.lib().tl_gemm_plain(ops._p(wide_a), 0, ops._p(wide_w), 0, ops._p(out), ops._p(parts), ctypes.c_longlong(n_parts if parts is not None else 0),
+                                           M, N, K, K + 4, K + 8, N + 3, 1, ops._stream()))
+        assert same_bits(out[:, :N].contiguous(), want) and torch.equal(out[:, N:], base[:, N:])
 
 
 @pytest.mark.parametrize("K", [4, 100, 516, 1024, 1500, 2048])
