@@ -700,6 +700,20 @@ def test_draws_through_pinned_memory(ops):
         ops.sample(z[:3], 0.9, 40, 0.9, 6, pairs.to(DEV), probs, out, host_out=torch.zeros(3, dtype=torch.int32))
 
 
+@pytest.mark.parametrize("V", [3000, 131072])
+@pytest.mark.parametrize("T,k", [(0.0, None), (0.9, None), (0.9, 40)])
+def test_draws_of_no_rows(ops, V, T, k):
+    """No logits, no tokens, also where rows would go in parts; and the sampler draws rows afterwards."""
+    from torchless_rs_amd import SamplingConfig
+    from torchless_rs_amd.sampling.sampler import Sampler
+    empty = lambda *shape, dtype=torch.float32: torch.empty(*shape, dtype=dtype, device=DEV)
+    ops.sample(empty(0, V), T, k or 0, 0.9, 6, empty(0, 2, dtype=torch.int32), empty(0, V), empty(0, dtype=torch.int32))
+    sampler = Sampler(SamplingConfig(T, k, 0.9, 6), DEV)
+    assert sampler.sample(empty(0, V), [], []) == [] and sampler.draw(empty(0, V), [], []).tokens() == []
+    z = rnd(2, V, seed=79).to(DEV)
+    assert sampler.sample(z, [0, 1], [3, 4]) == Sampler(SamplingConfig(T, k, 0.9, 6), DEV).sample(z, [0, 1], [3, 4])
+
+
 def test_options_that_change_between_draws(ops):
     """A sampler whose options are set anew between draws of one shape, with rows in parts and without: what a sampler of those options draws."""
     from torchless_rs_amd import SamplingConfig

@@ -626,7 +626,7 @@ using namespace tl;
 // the chip.  Microseconds of the kernels, one workgroup a row / in parts, at T = 0.7 and top-k 50: 16 rows of 131,072
 // 28 / 20, 64 of them 30 / 31, 16 rows of 32,000 16 / 18.  lists: room for [B][parts] lists of tl_sample_list_bytes() each.
 extern "C" int tl_sample_parts(int B, int V, float temperature, int top_k) {
-  if (!(temperature > 0.f) || top_k <= 0 || top_k > PART_TOP_K || V <= 8 * PART_RUN || V > 32 * PART_RUN) return 0;
+  if (B <= 0 || !(temperature > 0.f) || top_k <= 0 || top_k > PART_TOP_K || V <= 8 * PART_RUN || V > 32 * PART_RUN) return 0;
   const int parts = (V + PART_RUN - 1) / PART_RUN;
   return (long long)B * parts <= 512 ? parts : 0;
 }
