@@ -587,6 +587,45 @@ def test_graph_replays_equal_eager_steps(zoo, dtype):
     assert rel_err(outs[0][:1], want) < TOL[dtype]
 
 
+def test_captured_steps_of_products_in_groups(tmp_path):
+    """32-bit steps of 16 sequences whose products go in groups of K, with scratch of each call's own: replays, with eager work of other sizes and
+    synchronizations between them, have the bits of an engine that never captures, and the plain logits."""
+    from torchless_rs_amd import write_random_model
+    from torchless_rs_amd.engine import Engine, SeqInput, load_model
+    from torchless_rs_amd.kernels import ops
+    cfg = {"architectures": ["MistralForCausalLM"], "model_type": "mistral", "hidden_size": 1024, "num_hidden_layers": 2, "num_attention_heads": 8,
+           "num_key_value_heads": 4, "head_dim": 64, "intermediate_size": 2048, "vocab_size": 300, "rope_theta": 10000.0, "sliding_window": 100,
+           "rms_norm_eps": 1e-5, "max_position_embeddings": 4096, "tie_word_embeddings": False, "hidden_act": "silu"}
+    mdir = write_random_model(str(tmp_path / "m"), cfg, seed=8, std=0.05, norm_std=0.1, dtype=torch.float32)
+    cfgd, w = read_model_dir(mdir)
+    model, B = load_model(mdir, "float32"), 16
+    assert all(ops.lib().tl_gemm_plain_parts(B, n, k) for n, k in ((1024, 1024), (4096, 1024), (1024, 2048)))
+    ids, at = prompts(cfg["vocab_size"], [120] * B, seed=11), [3 + 5 * i for i in range(B)]
+    engines = [Engine(model, max_tokens=128 * (B + 1), max_slots=B + 1, use_graphs=g) for g in (True, False)]
+    for eng in engines:
+        eng.slots_ = [eng.alloc() for _ in ids]
+        eng.step([SeqInput(s, p[:n], []) for s, p, n in zip(eng.slots_, ids, at)])
+    for t in range(12):
+        outs = []
+        for eng in engines:
+            outs.append(eng.step([SeqInput(s, [p[n]], [0]) for s, p, n in zip(eng.slots_, ids, at)]).clone())
+            if t % 3 == 0:
+                extra = eng.alloc()
+                eng.step([SeqInput(extra, ids[1][:20 + 3 * t], [0])])
+                eng.free(extra)
+            junk = torch.full((4 << 20,), float("nan"), device="cuda:0")     # (memory that the scratch was given back to, if it was)
+            del junk
+            torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]), t
+        for i in (0, 9, 15):
+            if t in (0, 11):
+                assert rel_err(outs[0][i:i + 1], plain.forward(w, cfgd, ids[i][:at[i] + 1])[-1:]) < TOL["float32"], (t, i)
+        at = [n + 1 for n in at]
+    assert any(g.graph is not None for g in engines[0]._graphs.values()) and not engines[1]._graphs
+    for eng in engines:
+        eng.close()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_steps_of_several_tokens_are_captured_when_their_shape_comes_again(zoo, dtype):
     """Chunks of the same numbers of tokens step after step (two sequences, 8 and 16 tokens a step, so that the
