@@ -17,10 +17,12 @@ namespace tl {
 constexpr int MAX_D = 256;
 
 // VEC (steps that read everything from the pages, heads of a multiple of 4, aligned): four channels of a key a load, and where a tile of
-// keys is one page's, as all but the first of a window are, four keys' values: the same sums in the same order, a quarter of the loads and
-// many of them under way at once, where a lane waited for each.  32 heads of 64 / 128, two rows: 50 keys 7.0 / 11.0 us before, 4.8 / 6.4 now,
-// 300 28.0 / 49.5 and 13.8 / 21.6, 2,000 194 / 363 and 99 / 175.  Steps with rows of their own read those, in whole lines, as before: of many
-// rows fewer waves of more registers were up to 6 percent slower (300 rows of 64 channels 63.0 and 66.7).
+// keys is one page's, four keys' values: the same sums in the same order, a quarter of the loads and many of them under way at once, where
+// a lane waited for each.  (Tiles begin at the first key that a row sees: they are pages' while that is the sequence's first, and for a row
+// past its window only where the window begins with a page; its values else come one by one.)  Without a window, 32 heads of 64 / 128, two
+// rows: 50 keys 7.0 / 11.0 us before, 4.8 / 6.4 now, 300 28.0 / 49.5 and 13.8 / 21.6, 2,000 194 / 363 and 99 / 175.  Steps with rows of their
+// own read those, in whole lines, as before: of many rows fewer waves of more registers were up to 6 percent slower (300 rows of 64 channels
+// 63.0 and 66.7).
 template <typename T, bool VEC>
 __global__ void __launch_bounds__(64)
 attn_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_new, const T* __restrict__ v_new,

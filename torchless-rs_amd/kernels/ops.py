@@ -1744,7 +1744,8 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: 
     n_parts, parts = 0, None
     if a.dtype == torch.float32 and w.dtype == torch.float32 and M > 4:
         n_parts = lib().tl_gemm_plain_parts(M, N, K)
-        if n_parts:                                      # the sums of eight groups of K, added up in their order
+        if n_parts:                                      # the sums of eight groups of K, added up in their order (at most 64 MB, in a
+                                                         # captured step of the graph's own pool)
             parts = torch.empty((n_parts,), dtype=torch.float32, device=a.device)
     _check(lib().tl_gemm_plain(_p(a), _code(a.dtype), _p(w), _code(w.dtype), _p(out), _p(parts), ctypes.c_longlong(n_parts), M, N, K, K, K, N,
                                int(accumulate), _stream()))
