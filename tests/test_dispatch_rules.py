@@ -63,6 +63,14 @@ def test_rows_choose_the_kernel():
     assert [odd.own_kernels(m) for m in (64, 65)] == [True, False]
 
 
+def test_products_in_slices_cut_k_while_units_are_left():
+    """Partial sums over slices of K (7B sizes, 256 units): the slices are as many as the units hold, since the sum of a longer one is further
+    from 64 bits; where they are the faster way they are taken up to 448 rows of the square weight."""
+    S = lambda M, K: getattr(ops.tall_plan(M, 4096, K, 256, "add", True), "n_split", None)
+    assert [S(M, 4096) for M in (129, 192, 226, 256, 300, 384, 448, 512)] == [8, 8, 8, 6, 6, 4, 4, None]
+    assert [S(M, 14336) for M in (144, 226, 256, 300, 384, 448, 512, 640, 1024)] == [8, 8, 8, 8, 8, 5, 8, 4, 4]
+
+
 def test_a_weight_takes_rows_in_an_order_of_its_own_for_its_copy(monkeypatch):
     """`tile_rows` by name and third in order; the copy made by them is for the kernel that wants them alone."""
     import torch

@@ -45,6 +45,25 @@ def test_tiles_and_slices(ops, tile, M, N, K, apart):
     assert bool(((x.double() - total).abs() <= bound(K, size) + 2.0 ** -23 * total.abs()).all())
 
 
+@pytest.mark.parametrize("tile", [(256, 256), (160, 256), (256, 128), (192, 128)])
+@pytest.mark.parametrize("M,K,S", [(226, 4096, 8), (513, 640, 3), (300, 1344, 4)])
+def test_a_slice_adds_its_stages_in_their_order(ops, tile, M, K, S):
+    """A slice's sums have the bits of the product of its columns alone, however the rule would go through a K that is not cut; and stages in
+    turn are refused where it is."""
+    N, stages = 772, -(-K // 64)
+    a, w, _, _ = operands(M, N, K)
+    out = torch.full((S, M, N), float("nan"), device=DEV)
+    ops.gemm_tall_bf16(a, w, out, ops.TallPlan(*tile, S))
+    per = -(-stages // S)
+    for s in range(S):
+        k = slice(64 * per * s, min(K, 64 * per * (s + 1)))
+        one = torch.empty(M, N, device=DEV)
+        ops.gemm_tall_bf16(a[:, k].contiguous(), w[:, k], one, ops.TallPlan(*tile))
+        assert torch.equal(out[s], one), s
+    with pytest.raises(ops.KernelError, match="uncut"):
+        ops.gemm_tall_bf16(a, w, out, ops.TallPlan(*tile, S, stagger=True))
+
+
 @pytest.mark.parametrize("tile", [t for t in TILES if t[1] == 256])
 @pytest.mark.parametrize("parts", [2, 4])
 @pytest.mark.parametrize("M,N", [(17, 4100), (257, 2176), (1000, 772), (1025, 640)])

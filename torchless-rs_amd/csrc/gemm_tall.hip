@@ -193,8 +193,8 @@ using namespace tl;
 // A [M, K] with rows lda apart, W [N, K] with rows ldw apart; K, lda, ldw multiples of 8, N of 4 (with a paired epilogue of 64).
 // n_split == 1: C as in tl_gemm_bf16; more: C float [n_split][M][N] receives partial sums (epilogue 0), every split with one
 // stage of 64 k at least.  rows, channels: the tile, one of 256, 224, 192, 160 x 256 and 256, 192, 128 x 128.  once: W is read by
-// one tile of rows only (tiles of 128 channels mark its loads non-temporal; the rule has no such product in wider ones); stagger: tiles of other channels begin with other stages of K,
-// or of their slice of it (K a multiple of 64).  parts: 0, or 2 or 4 (tiles of 256 channels, K not cut): the tiles behind the first `whole`, a
+// one tile of rows only (tiles of 128 channels mark its loads non-temporal; the rule has no such product in wider ones); stagger: tiles of other channels begin with other stages of K
+// (K a multiple of 64, not cut).  parts: 0, or 2 or 4 (tiles of 256 channels, K not cut): the tiles behind the first `whole`, a
 // multiple of 8, are cut into so many.
 static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipStream_t st) {
   const int M = g.M, N = g.N, K = g.K, lda = g.lda, ldw = g.ldw, stagger = g.stagger, whole = g.whole, parts = g.parts, epilogue = g.epi;
@@ -207,7 +207,7 @@ static int run_tall(Tall g, int rows, int channels, int n_split, int once, hipSt
   TL_REQUIRE(!(is_pair(epilogue) || epilogue == TALL_GATED) || N % 64 == 0, "gemm_tall: the paired epilogue needs N=%d to be a multiple of 64", N);
   const int stages = (K + TILE_K - 1) / TILE_K, per = (stages + n_split - 1) / (n_split > 0 ? n_split : 1);
   TL_REQUIRE(n_split >= 1 && n_split <= 65535 && (long)(n_split - 1) * per < stages, "gemm_tall: %d splits of K=%d would leave one without a stage", n_split, K);
-  TL_REQUIRE(!stagger || K % TILE_K == 0, "gemm_tall: stages in turn need K=%d a multiple of %d", K, TILE_K);
+  TL_REQUIRE(!stagger || (n_split == 1 && K % TILE_K == 0), "gemm_tall: stages in turn need K=%d uncut and a multiple of %d", K, TILE_K);
   TL_REQUIRE(parts == 0 || ((parts == 2 || parts == 4) && n_split == 1 && channels == 256 && !once && !stagger && whole >= 0),
              "gemm_tall: tiles in %d parts (2 or 4, of 256 channels, K not cut)", parts);
   g.stages = per;

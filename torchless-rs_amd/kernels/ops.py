@@ -2131,13 +2131,6 @@ def wide_splits(M: int, N: int, K: int, units: int) -> int:
     return -(-stages // -(-stages // S))            # (as many as have a stage)
 
 
-def slices_in_turn(M: int, K: int, S: int) -> bool:
-    """Do the tiles of a slice of K begin with different stages of it?  While an XCD's L2 holds the slice of A besides (microseconds in step /
-    in turn: 144 rows of 4,096 x 14,336 in 8 36.2 / 32.2, 384 of 4,096 x 4,096 in 4 24.0 / 21.5; 1,024 of 4,096 x 4,096 in 2, 4 MB of A
-    a slice, 36.8 / 39.2)."""
-    return S > 1 and K % 64 == 0 and M * K * 2 <= S * (2 << 20)
-
-
 def gemm_wide_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_split: int) -> None:
     """Partial sums out float32 [n_split, M, N] of the product of up to WIDE_ROWS rows, N and K multiples of 64, in tiles of all of
     the rows by 128 channels."""
@@ -2162,7 +2155,12 @@ class TallPlan:
 
 # microseconds that a stage of 64 k takes with every compute unit at work on tiles of so many rows and channels
 TALL_STAGE = {(256, 256): 1.45, (224, 256): 1.32, (192, 256): 1.15, (160, 256): 1.0, (256, 128): 0.85, (192, 128): 0.80, (128, 128): 0.68}
-TALL_ROUND, TALL_LAUNCH, TALL_SLICE = 8.0, 4.0, 0.3   # a round of workgroups besides its stages (first loads, results), the launch, a slice
+TALL_ROUND, TALL_LAUNCH = 8.0, 4.0        # a round of workgroups besides its stages (first loads, results), and the launch
+# In slices a stage of (256, 128) is reckoned longer than it takes, which cuts K in more slices where units are left for them: the sum of
+# a longer slice is further from 64 bits (4,096 x 4,096 at 226 rows in 8 / 6 1.37e-7 / 1.55e-7, 4,096 x 14,336 at 512 in 8 / 4 2.6e-7 / 3.7e-7)
+# and seldom ready sooner (with the norm behind it 28.4 / 26.9 and 71.8 / 67.4 us; 4,096 x 4,096 at 192 rows in 8 / 6 26.0 / 25.8, at 384 in 4
+# 26.9, by the library, which the shorter stage would take, 28.9)
+SLICE_STAGE = {**TALL_STAGE, (256, 128): 0.93}
 TALL_SHARED = 4 << 20                     # bytes of A that an XCD's L2 holds: up to there tiles may go through K out of step
 
 
@@ -2209,7 +2207,7 @@ def tall_plan(M: int, N: int, K: int, units: int, kind: str, sums: bool = False)
             if (S - 1) * per >= stages:
                 continue
             size = 4.0 * M * N                                       # of a partial sum, in bytes; the norm reads all, and writes one
-            t = TALL_LAUNCH + 2.0 + per * stage * fill(tiles * S) + S * (TALL_SLICE + size / 8e6) + max(1.0, ((S + 1) * size - 30e6) / 5e6)
+            t = TALL_LAUNCH + 2.0 + per * SLICE_STAGE[rows, channels] * fill(tiles * S) + S * size / 8e6 + max(1.0, ((S + 1) * size - 30e6) / 5e6)
             if t < best:
                 best, plan = t, TallPlan(rows, channels, S)
         full, rest = divmod(tiles, units)
@@ -2260,8 +2258,7 @@ def gemm_tall_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, plan: Ta
         _req(out, "gemm.out", torch.float32, (M, N))
         epi = EPI_ACCUMULATE if accumulate else EPI_STORE
     _check(lib().tl_gemm_tall(_p(a), K, _p(w), w.stride(0), _p(out), M, N, K, plan.rows, plan.channels, plan.n_split,
-                              int(M <= plan.rows and not plan.parts), int(plan.stagger or slices_in_turn(M, K, plan.n_split)), plan.whole,
-                              plan.parts, epi, _stream()))
+                              int(M <= plan.rows and not plan.parts), int(plan.stagger), plan.whole, plan.parts, epi, _stream()))
 
 
 def gemm_tall_act(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, plan: TallPlan, terms: Optional[GateTerms] = None,
