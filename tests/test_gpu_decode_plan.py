@@ -299,3 +299,18 @@ def test_replayed_steps_are_ordered_by_their_own_lengths(tmp_path, ops):
     assert not engines[1]._graphs
     for eng in engines:
         eng.close()
+
+
+@pytest.mark.parametrize("B,nq,nkv,d,splits", [(1, 32, 8, 128, 16), (1, 32, 8, 128, 2), (3, 40, 2, 64, 9), (2, 6, 6, 256, 5), (5, 17, 1, 128, 33), (8, 32, 8, 128, 8)])
+def test_parts_merged_by_the_last_of_them_have_the_bits_of_a_merge_of_its_own(ops, B, nq, nkv, d, splits):
+    lengths = [1 + (i * 977 + 700) % 2300 for i in range(B)]        # with fewer pages than parts among them
+    q, pages, table, ctx = step(ops, lengths, nq, nkv, d, seed=3)
+    part = torch.full((B * nq * splits * (d + 2),), float("nan"), device=DEV)
+    apart, met = torch.zeros_like(q), torch.zeros_like(q)
+    ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, apart)
+    arrived = ops.decode_counters(ctx, B, nq, nkv)
+    for _ in range(4):                                               # the counters are left as they were found
+        part.fill_(float("nan"))
+        met.zero_()
+        ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, met, arrived)
+        assert torch.equal(met, apart) and int(arrived.abs().max()) == 0

@@ -913,13 +913,20 @@ attn_decode_order_kernel(const int* __restrict__ row_pos, int B, int window, int
   plan[place] = make_int4(4 * b + 3, 0, n, pos);
 }
 
+// Numbers that workgroups of one launch leave for each other go past the XCDs' own caches in both directions (agent scope), so that
+// a counter behind them is all the order they need: a device-wide fence, which writes back and invalidates an L2, took a step of 32
+// layers at batch 8 from 4.0 to 4.7 ms.
+__device__ __forceinline__ void shared_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float shared_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 template <int D, int NS, bool TERMS = false, bool LOGI = false>
 __global__ void __launch_bounds__(DC_WAVES * 64)
 attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pages,
                         const int* __restrict__ table, int table_stride, int ring_pages,
                         const int* __restrict__ row_pos, int nq, int nkv, int window, float scale,
                         int n_splits, int head_groups, float* __restrict__ part, bf16* __restrict__ out,
-                        MoreTerms terms, const int4* __restrict__ plan = nullptr) {
+                        MoreTerms terms, const int4* __restrict__ plan = nullptr, const int2* __restrict__ seqs = nullptr,
+                        int* __restrict__ arrived = nullptr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char dr_smem[];
   constexpr int KB = D / 32, VB = D / 16;
   constexpr int K_BYTES = PAGE * D * 2, STAGE = 2 * K_BYTES;   // keys, then values, as many bytes each
@@ -1096,9 +1103,10 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
 #pragma unroll
     for (int r = 0; r < 4; ++r) red_o[wave * (VB * 4 * 64) + (vb * 4 + r) * 64 + lane] = o[vb][r] * f;
   __syncthreads();
-  for (int e = threadIdx.x; e < 16 * D; e += DC_WAVES * 64) {
-    const int hd = e / D, dv = e % D;
-    if (hg * 16 + hd >= g) continue;
+  // a wave takes a head (and every DC_WAVES-th behind it), a lane PER of its channels
+  constexpr int PER = D / WAVE;
+  const int heads = min(16, g - hg * 16);
+  for (int hd = wave; hd < heads; hd += DC_WAVES) {
     float mh = -INFINITY;
 #pragma unroll
     for (int w = 0; w < DC_WAVES; ++w) mh = fmaxf(mh, red_ml[(w * 2) * 16 + hd]);
@@ -1108,10 +1116,15 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
       const float mw = red_ml[(w * 2) * 16 + hd];
       ll += (mw == -INFINITY) ? 0.f : red_ml[(w * 2 + 1) * 16 + hd] * __expf(mw - mh);
     }
-    const int idx = ((dv / 16) * 4 + (dv % 4)) * 64 + ((dv % 16) / 4) * 16 + hd;
-    float osum = red_o[idx];
+    float osum[PER];
 #pragma unroll
-    for (int w = 1; w < DC_WAVES; ++w) osum += red_o[w * (VB * 4 * 64) + idx];
+    for (int i = 0; i < PER; ++i) {
+      const int dv = lane + WAVE * i;
+      const int idx = ((dv / 16) * 4 + (dv % 4)) * 64 + ((dv % 16) / 4) * 16 + hd;
+      osum[i] = red_o[idx];
+#pragma unroll
+      for (int w = 1; w < DC_WAVES; ++w) osum[i] += red_o[w * (VB * 4 * 64) + idx];
+    }
     const size_t bh = (size_t)b * nq + kvh * g + hg * 16 + hd;
     if constexpr (TERMS) {
       if (terms.sinks != nullptr && first_part) {     // the sink counts once: with the first split
@@ -1119,33 +1132,90 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
         const float ms = fmaxf(mh, sk);
         const float fs = (mh == -INFINITY) ? 0.f : __expf(mh - ms);
         ll = ll * fs + __expf(sk - ms);
-        osum *= fs;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) osum[i] *= fs;
         mh = ms;
       }
     }
     if constexpr (LOGI) ll = first_part ? 1.f : 0.f;  // the sum is a 1, once for a row
     if (alone) {
-      float res = osum / ll;
-      if constexpr (TERMS)
-        if (terms.gate != nullptr) res *= terms.gate[bh];
-      out[bh * D + dv] = (bf16)res;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        float res = osum[i] / ll;
+        if constexpr (TERMS)
+          if (terms.gate != nullptr) res *= terms.gate[bh];
+        out[bh * D + lane + WAVE * i] = (bf16)res;
+      }
       continue;
     }
     float* dst = part + (plan != nullptr ? (size_t)place * nq + kvh * g + hg * 16 + hd : bh * n_splits + blockIdx.y) * (D + 2);
-    dst[2 + dv] = osum;
-    if (dv == 0) {
-      dst[0] = mh;
-      dst[1] = ll;
+    const auto put = [&](int i, float v) { if (arrived != nullptr) shared_store(dst + i, v); else dst[i] = v; };
+#pragma unroll
+    for (int i = 0; i < PER; ++i) put(2 + lane + WAVE * i, osum[i]);
+    if (lane < 2) put(lane, lane == 0 ? mh : ll);
+  }
+  if (arrived == nullptr || alone || wave >= heads) return;
+  // Of the parts' waves with these heads the last to get here merges them, as attn_decode_combine_kernel does (the same bits).
+  // Nobody waits for anybody.  What bounds it is three trips past the L2s one after the other (stores, counter, loads), 3 us in place of
+  // a launch of 4.6: a step of 32 layers 2,913 and 2,888 us at batch 1 (1,024 keys), 3,600 and 3,588 to 3,565 at batch 8 (4,096 keys).
+  // A counter a workgroup, with its barriers and a thread's channels one after the other: no gain.
+  const int2 mine = plan != nullptr ? seqs[b] : make_int2(0, n_splits);
+  int* count = arrived + (((size_t)b * nkv + kvh) * head_groups + hg) * DC_WAVES + wave;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's results are where every XCD sees them
+  int before = 0;
+  if (lane == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(before) != mine.y - 1) return;
+  if (lane == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // for the next launch
+  const size_t stride = (size_t)(D + 2) * (plan != nullptr ? nq : 1);
+  for (int hd = wave; hd < heads; hd += DC_WAVES) {
+    const int head = kvh * g + hg * 16 + hd;
+    const size_t bh = (size_t)b * nq + head;
+    const float* src = part + (plan != nullptr ? (size_t)mine.x * nq + head : bh * n_splits) * (D + 2);
+    float acc[PER], ll = 0.f, mm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) acc[i] = 0.f;
+    constexpr int CH = 8;
+    for (int s0 = 0; s0 < mine.y; s0 += CH) {
+      float ms[CH], ls[CH], vs[CH][PER];
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const float* p = src + (size_t)min(s0 + c, mine.y - 1) * stride;
+        ms[c] = shared_load(p);
+        ls[c] = shared_load(p + 1);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) vs[c][i] = shared_load(p + 2 + lane + WAVE * i);
+      }
+      float mc = mm;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        if (s0 + c >= mine.y) ms[c] = -INFINITY;
+        mc = fmaxf(mc, ms[c]);
+      }
+      if (mc == -INFINITY) continue;                   // nothing visible so far
+      const float keep = (mm == -INFINITY) ? 0.f : __expf(mm - mc);
+      ll *= keep;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) acc[i] *= keep;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const float f = (ms[c] == -INFINITY) ? 0.f : __expf(ms[c] - mc);
+        ll += ls[c] * f;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) acc[i] += vs[c][i] * f;
+      }
+      mm = mc;
     }
+    float gt = 1.f;
+    if constexpr (TERMS)
+      if (terms.gate != nullptr) gt = terms.gate[bh];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) out[bh * D + lane + WAVE * i] = (bf16)(acc[i] / ll * gt);
   }
 }
 
 // Merge the splits of one (sequence, head): common maximum, weighted sums, in the order of the
-// splits.  (A second kernel and not the last workgroup of the first: what other XCDs wrote is
-// only sure to be seen across a kernel boundary or after a device-wide fence, and that fence
-// writes back and invalidates the XCD's L2.  Measured with the last workgroup merging behind a
-// counter: one fence a workgroup makes a step of 32 layers at batch 8 4.7 ms instead of 4.0, one
-// a thread 6.3.)
+// splits.  For callers without counters and for attn_decode_kernel; attn_decode_ring_kernel does it
+// itself where it has them.
 // One wave per (row, head).  Splits are taken 8 at a time with all their loads (maxima, sums and
 // this lane's elements) issued together, so that a usual split count costs one trip to memory;
 // chunks merge by the running-maximum rule.
@@ -1316,10 +1386,13 @@ constexpr int DR_MAX_PAGES = 2048;      // most pages of a sequence that the ker
 // single-token steps with more terms on the scores; LOGI: logistic weights
 // a step's parts as attn_decode_plan_kernel made them (null: n_splits for every sequence), over `places` places; without `seqs` every
 // sequence is one part and there is nothing to merge
+// arrived: DC_WAVES counters for each sequence, KV head and 16 heads of its group, all zero, which the kernel leaves at zero: the parts are then
+// merged by the last of them and not by a launch of their own.
 struct DecodePlan {
   const int4* plan = nullptr;
   const int2* seqs = nullptr;
   int places = 0;
+  int* arrived = nullptr;
 };
 
 template <int DPAD, bool LOGI>
@@ -1346,9 +1419,9 @@ static int launch_decode_terms(const bf16* q, const bf16* pages, const int* tabl
       if (plan.plan != nullptr) grid = dim3(plan.places * nkv * head_groups, 1);
       attn_decode_ring_kernel<DPAD, NS, true, LOGI><<<grid, DC_WAVES * 64, LDS, st>>>(q, pages, table, table_stride, ring_pages,
                                                                                       row_pos, nq, nkv, window, scale, n_splits,
-                                                                                      head_groups, part, out, *terms, plan.plan);
+                                                                                      head_groups, part, out, *terms, plan.plan, plan.seqs, plan.arrived);
       TL_LAUNCH_CHECK("attn_decode_ring with terms");
-      if (n_splits > 1 || plan.seqs != nullptr) {
+      if (plan.arrived == nullptr && (n_splits > 1 || plan.seqs != nullptr)) {
         attn_decode_combine_kernel<<<B * nq, 64, 0, st>>>(part, n_splits, d, out, terms->gate, plan.seqs, nq);
         TL_LAUNCH_CHECK("attn_decode_combine");
       }
@@ -1402,9 +1475,9 @@ static int launch_decode(const bf16* q, const bf16* pages, const int* table, int
       if (plan.plan != nullptr) grid = dim3(plan.places * nkv * head_groups, 1);
       attn_decode_ring_kernel<DPAD, NS><<<grid, DC_WAVES * 64, LDS, st>>>(q, pages, table, table_stride, ring_pages,
                                                                           row_pos, nq, nkv, window, scale, n_splits,
-                                                                          head_groups, part, out, MoreTerms{}, plan.plan);
+                                                                          head_groups, part, out, MoreTerms{}, plan.plan, plan.seqs, plan.arrived);
       TL_LAUNCH_CHECK("attn_decode_ring");
-      if (n_splits > 1 || plan.seqs != nullptr) {
+      if (plan.arrived == nullptr && (n_splits > 1 || plan.seqs != nullptr)) {
         attn_decode_combine_kernel<<<B * nq, 64, 0, st>>>(part, n_splits, d, out, nullptr, plan.seqs, nq);
         TL_LAUNCH_CHECK("attn_decode_combine");
       }
@@ -1589,10 +1662,21 @@ extern "C" int tl_attn_decode_bf16(const void* q, const void* pages, const int* 
                            part, out, st, nullptr);
 }
 
-// The same with more terms on the scores (slopes [nq], sinks [nq], gate [B, nq]; each may be null)
+// The same, whose parts the last of them merges where the kernel through LDS serves the head size.  arrived: as `DecodePlan` has it.
+extern "C" int tl_attn_decode_met_bf16(const void* q, const void* pages, const int* table, int table_stride,
+                                       int ring_pages, const int* row_pos, int B, int nq, int nkv, int d,
+                                       int window, float scale, int n_splits, float* part, int* arrived, void* out,
+                                       hipStream_t st) {
+  DecodePlan met;
+  met.arrived = arrived;
+  return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, n_splits,
+                           part, out, st, nullptr, met);
+}
+
+// The same with more terms on the scores (slopes [nq], sinks [nq], gate [B, nq]; each may be null); arrived may be null
 extern "C" int tl_attn_decode_terms_bf16(const void* q, const void* pages, const int* table, int table_stride,
                                          int ring_pages, const int* row_pos, int B, int nq, int nkv, int d,
-                                         int window, int keep_first, int chunk, float scale, int n_splits, float* part,
+                                         int window, int keep_first, int chunk, float scale, int n_splits, float* part, int* arrived,
                                          const float* slopes, const float* sinks, const float* gate, int logistic,
                                          const float* score_bias, void* out, hipStream_t st) {
   TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || window == 0 || (long long)ring_pages * PAGE >= (1LL << 24)),
@@ -1600,8 +1684,10 @@ extern "C" int tl_attn_decode_terms_bf16(const void* q, const void* pages, const
   TL_REQUIRE(chunk >= 0 && (!logistic || sinks == nullptr) && (logistic || score_bias == nullptr),
              "attn_decode: %d positions a chunk; logistic weights have no sink, a softmax no bias on the score", chunk);
   const MoreTerms terms{slopes, sinks, gate, window > 0 ? keep_first : 0, chunk, logistic, score_bias};
+  DecodePlan met;
+  met.arrived = arrived;
   return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, n_splits,
-                           part, out, st, &terms);
+                           part, out, st, &terms, met);
 }
 
 // Do single-token steps with heads of d and page tables of this width go through the kernel that stages the pages in LDS (the one
@@ -1635,17 +1721,17 @@ extern "C" int tl_attn_decode_order(const int* row_pos, int B, int window, int k
 }
 
 // tl_attn_decode_bf16, or with `more` tl_attn_decode_terms_bf16, with the parts of a plan over `places` places; part: float scratch of
-// places * nq * (d + 2) elements.  seqs null: the plan is an order, nothing is merged and part is not touched.
+// places * nq * (d + 2) elements.  seqs null: the plan is an order, nothing is merged and part is not touched.  arrived: see `DecodePlan`, or null.
 extern "C" int tl_attn_decode_planned_bf16(const void* q, const void* pages, const int* table, int table_stride, int ring_pages,
                                            const int* row_pos, int B, int nq, int nkv, int d, int window, float scale, const int* plan,
                                            const int* seqs, int places, int more, int keep_first, int chunk, const float* slopes,
                                            const float* sinks, const float* gate, int logistic, const float* score_bias, float* part,
-                                           void* out, hipStream_t st) {
+                                           int* arrived, void* out, hipStream_t st) {
   TL_REQUIRE(tl_attn_decode_takes_plan(d, table_stride), "attn_decode_planned: heads of %d with %d pages go without a plan", d, table_stride);
   TL_REQUIRE(plan && (part || !seqs) && (seqs ? places >= B : places == B) && (uintptr_t)plan % 16 == 0 && (uintptr_t)seqs % 8 == 0 &&
              nq > 0 && nkv > 0 && (long)places * nkv * ((nq / nkv + 15) / 16) * DC_WAVES * 64 < (1l << 31),
              "attn_decode_planned: %d places for %d sequences", places, B);
-  const DecodePlan dp{(const int4*)plan, (const int2*)seqs, places};
+  const DecodePlan dp{(const int4*)plan, (const int2*)seqs, places, arrived};
   if (!more) return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, 1, part, out, st, nullptr, dp);
   TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || window == 0 || (long long)ring_pages * PAGE >= (1LL << 24)),
              "attn_decode: first positions that stay visible beside a window need a cache that keeps every position");

@@ -659,9 +659,10 @@ def attention_scored(q, k_new, v_new, pages, nkv: int, dv: int, table, ring_page
         part = ctx.workspace.get("attn_part", (n * nq * splits * (dk + 2),), torch.float32)
         _decode_args(q, pages, table, ctx.row_pos, part, out, splits)
         slopes, sinks, gt = _terms_args(terms, gate, n, nq)
+        arrived = decode_counters(ctx, n, nq, nkv) if splits > 1 else None
         _check(lib().tl_attn_decode_terms_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(ctx.row_pos),
                                                n, nq, nkv, dk, int(terms.window or 0), int(terms.keep_first or 0),
-                                               terms.chunk, ctypes.c_float(terms.scale), int(splits), _p(part), slopes, sinks,
+                                               terms.chunk, ctypes.c_float(terms.scale), int(splits), _p(part), _p(arrived), slopes, sinks,
                                                gt, int(terms.logistic), _p(terms.score_bias), _p(out), _stream()))
     elif fast and k_new is not None and vt_new is not None:
         B = n_cached.shape[0]
@@ -2625,13 +2626,20 @@ def _decode_args(q, pages, table, row_pos, part, out, n_splits: int) -> None:
 
 
 def attn_decode_bf16(q, pages, table, ring_pages: int, row_pos, window: Optional[int], scale: float,
-                     n_splits: int, part, out) -> None:
+                     n_splits: int, part, out, arrived=None) -> None:
     """bfloat16 attention of one new token per sequence over its pages (the
     token's own key is already committed).  `part`: float32 scratch of at
-    least B * nq * n_splits * (d + 2) elements."""
+    least B * nq * n_splits * (d + 2) elements.  `arrived` (`decode_counters`): the
+    parts' merge needs no launch of its own."""
     B, nq, d = q.shape
     nkv = pages.shape[2]
     _decode_args(q, pages, table, row_pos, part, out, n_splits)
+    if arrived is not None:
+        _req(arrived, "attn.arrived", torch.int32, (DECODE_WAVES * decode_groups(B, nq, nkv),))
+        _check(lib().tl_attn_decode_met_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(row_pos),
+                                             B, nq, nkv, d, int(window or 0), ctypes.c_float(scale),
+                                             int(n_splits), _p(part), _p(arrived), _p(out), _stream()))
+        return
     _check(lib().tl_attn_decode_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(row_pos),
                                      B, nq, nkv, d, int(window or 0), ctypes.c_float(scale),
                                      int(n_splits), _p(part), _p(out), _stream()))
@@ -2648,6 +2656,14 @@ def decode_groups(B: int, nq: int, nkv: int) -> int:
     """Workgroups of a decode step's attention before splitting: one per
     (sequence, KV head, 16 query heads of its group)."""
     return B * nkv * (-(-(nq // nkv) // 16))
+
+
+DECODE_WAVES = 4            # waves of a workgroup of the decode attention
+
+
+def decode_counters(ctx, B: int, nq: int, nkv: int) -> torch.Tensor:
+    """The counters by which the parts of a decode step's attention find the last of them, which merges them: zero between launches."""
+    return ctx.workspace.get("attn_arrived", (DECODE_WAVES * decode_groups(B, nq, nkv),), torch.int32, zero=True)
 
 
 SPLIT_PAGES = 4             # fewest pages a part of the keys has
@@ -2757,9 +2773,10 @@ def attn_decode_planned(q, pages, table, ring_pages: int, ctx, plan, window: Opt
     nkv = pages.shape[2]
     places, seqs = plan
     _req(places, "attn_decode_planned.plan", torch.int32)
-    part = None
+    part = arrived = None
     if seqs is not None:
         _req(seqs, "attn_decode_planned.seqs", torch.int32, (B, 2))
+        arrived = decode_counters(ctx, B, nq, nkv)
         part = ctx.workspace.get("attn_part", (places.shape[0] * nq * (d + 2),), torch.float32)
     _decode_args(q, pages, table, ctx.row_pos, part, out, 1)
     slopes, sinks, gt = _terms_args(terms, gate, B, nq) if terms is not None else (None, None, None)
@@ -2767,7 +2784,7 @@ def attn_decode_planned(q, pages, table, ring_pages: int, ctx, plan, window: Opt
     _check(lib().tl_attn_decode_planned_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(ctx.row_pos), B, nq, nkv, d,
                                              int(window or 0), ctypes.c_float(scale), _p(places), _p(seqs), places.shape[0], *more, slopes,
                                              sinks, gt, int(terms.logistic) if terms is not None else 0,
-                                             _p(terms.score_bias) if terms is not None else None, _p(part), _p(out), _stream()))
+                                             _p(terms.score_bias) if terms is not None else None, _p(part), _p(arrived), _p(out), _stream()))
 
 
 def uses_transposed_values(dtype: torch.dtype, d: int, all_single: bool) -> bool:
@@ -2793,7 +2810,8 @@ def attention(q, k_new, v_new, pages, table, ring_pages: int, ctx, n_cached, win
             return
         splits = decode_splits(n, nq, nkv, table.shape[1], compute_units(q.device), d)   # by the table's width: fixed while a graph lives
         part = ctx.workspace.get("attn_part", (n * nq * splits * (d + 2),), torch.float32)
-        attn_decode_bf16(q, pages, table, ring_pages, ctx.row_pos, window, scale, splits, part, out)
+        attn_decode_bf16(q, pages, table, ring_pages, ctx.row_pos, window, scale, splits, part, out,
+                         decode_counters(ctx, n, nq, nkv) if splits > 1 else None)
     elif fast and k_new is not None and vt_new is not None:
         n_tiles = int(sum(-(-int(x) // PREFILL_BLOCK) for x in ctx.host["n_new"]))
         cuts = part = None
