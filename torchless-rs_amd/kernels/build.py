@@ -30,14 +30,16 @@ LIB_NAME = "libtorchless_hip.so"
 HOST_LIB_NAME = "libtorchless_host.so"
 MEASURE_LIB_NAME = "libtorchless_measure.so"
 _CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
-# Kernel arguments lie in host memory, a load over the bus before a wave's first address; with the preload the command
-# processor brings the leading ones (up to 16 registers, none of a struct's) with the dispatch.  A decode step of one sequence of
-# 160 launches 2,925 us without and 2,913 with, of eight 3,615 and 3,600, a prompt step of 226 rows 6,181 and 6,137.
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-               "-mllvm", "-amdgpu-kernarg-preload-count=16",
                "-Wno-unused-result"]
-
+# Kernel arguments lie in host memory, a load over the bus before a wave's first address; with the preload the command
+# processor brings the leading ones (up to 16 registers, none of a struct's) with the dispatch: the products of a decode step 1 to 5 % each,
+# a step of one sequence of 160 launches 2,925 us without and 2,913 with, of eight 3,615 and 3,600, a prompt step of 226 rows 6,181 and
+# 6,137.  Other kernels lose: norms and other short ones 0.2 us, and where the compiler orders loads otherwise more (the router
+# over 128 rows 10.0 and 14.0 us).  So it is for these sources.
+PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+PRELOADED = ("attention_bf16.hip", "gemm_bf16.hip", "gemm_plain.hip", "gemm_tall.hip")
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall"]
 
 _lib: Optional[ctypes.CDLL] = None
@@ -83,7 +85,7 @@ def _digest(files: List[str], flags: List[str]) -> str:
 
 
 def kernels_digest() -> str:
-    return _digest(sources() + _headers(), HIPCC_FLAGS)
+    return _digest(sources() + _headers(), [*HIPCC_FLAGS, *PRELOAD, *PRELOADED])
 
 
 def measure_digest() -> str:
@@ -220,7 +222,8 @@ def _build_hip(srcs: List[str], name: str, digest: str, verbose: bool) -> str:
     t0 = time.time()
 
     def one(i: int) -> None:
-        _run_with_progress([hipcc, *HIPCC_FLAGS, "-I", _CSRC, "-c", srcs[i], "-o", objs[i]],
+        extra = PRELOAD if os.path.basename(srcs[i]) in PRELOADED else []
+        _run_with_progress([hipcc, *HIPCC_FLAGS, *extra, "-I", _CSRC, "-c", srcs[i], "-o", objs[i]],
                            os.path.basename(srcs[i]))
         if verbose:
             _say(f"compiled {os.path.basename(srcs[i])} ({time.time() - t0:.0f} s)")
