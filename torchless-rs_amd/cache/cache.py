@@ -33,11 +33,9 @@ import ctypes
 
 import numpy as np
 
-from ..kernels.page import PAGE                  # noqa: F401  (positions in a page: csrc/page.h)
+from ..kernels.page import NO_RING, PAGE         # noqa: F401  (positions in a page: csrc/page.h)
 from . import native
 from .native import CacheFull, CacheMisuse      # noqa: F401
-
-NO_RING = 1 << 24          # "ring" of a group that keeps every position: never wraps
 
 
 @dataclass(frozen=True)

@@ -306,12 +306,24 @@ add_partials_kernel(V* __restrict__ x, const V* __restrict__ parts, int n_parts,
 // src/kernels/mod.rs:582-608, src/model/modules/attention.rs:68-78.
 constexpr int ROPE_MAX_HALF = 128;      // head sizes up to 256
 
+// Where a step's keys and values go in the cache (pages null: nowhere yet): the page of position p of sequence b.  Only for steps that
+// overwrite no position: the attention behind may then still read all that was there.
+template <typename T> struct Commit {
+  const int* table = nullptr;
+  int table_stride = 0, ring_pages = 1;
+  T* pages = nullptr;
+  __device__ __forceinline__ T* page(int b, int p, int nkv, int d) const {
+    return pages + (size_t)table[(size_t)b * table_stride + (p / PAGE) % ring_pages] * (2 * (size_t)nkv * PAGE * d);
+  }
+};
+
 template <typename TO>
 __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, const float* __restrict__ qkv,
                                                const int* __restrict__ row_pos, Rotation rot, int nq, int nkv, int d,
                                                TO* __restrict__ q, TO* __restrict__ k, TO* __restrict__ v,
                                                TO* __restrict__ vt, int vt_cols, const int* __restrict__ row_seq,
-                                               const int* __restrict__ tile_off, const int* __restrict__ n_cached) {
+                                               const int* __restrict__ tile_off, const int* __restrict__ n_cached,
+                                               const Commit<TO>& commit = Commit<TO>{}) {
   const int half = d / 2, rot_pairs = rot.rotary_dim / 2;
   const float pos = (float)row_pos[n];
   const float* src = qkv + (size_t)n * (nq + 2 * nkv) * d;
@@ -319,9 +331,10 @@ __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, cons
   // 2,048 rows of 32 + 8 heads of 128 with their 8 heads
   // of values (75 MB), a pair a thread and turn before: 19.8 us, 13.7 now; 226 rows 7.1 and 4.2.
   constexpr int TURNS = 3;
-  const bool quads = rot.rotary_dim == d && !rot.interleaved && d % 8 == 0 && ((uintptr_t)qkv | (uintptr_t)q | (uintptr_t)k) % 16 == 0;
+  const bool quads = rot.rotary_dim == d && !rot.interleaved && d % 8 == 0 && ((uintptr_t)qkv | (uintptr_t)q | (uintptr_t)k | (uintptr_t)commit.pages) % 16 == 0;
   const int per = half / 4, n_quads = (nq + nkv) * per;
   const auto pair_at = [&](int t) { return (t / per) * d + t % per * 4; };       // its first channel in the row
+  TO* kp = commit.pages ? commit.page(row_seq[n], row_pos[n], nkv, d) + (size_t)(row_pos[n] % PAGE) * d : nullptr;
   f32x4 a[TURNS], b[TURNS];
   if (quads) {
 #pragma unroll
@@ -351,6 +364,11 @@ __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, cons
       TO* dst = ((h < nq) ? q + ((size_t)n * nq + h) * d : k + ((size_t)n * nkv + (h - nq)) * d) + i;
       *reinterpret_cast<quad*>(dst) = ha;
       *reinterpret_cast<quad*>(dst + half) = hb;
+      if (kp != nullptr && h >= nq) {
+        TO* to = kp + (size_t)(h - nq) * PAGE * d + i;
+        *reinterpret_cast<quad*>(to) = ha;
+        *reinterpret_cast<quad*>(to + half) = hb;
+      }
     };
 #pragma unroll
     for (int u = 0; u < TURNS; ++u)
@@ -371,6 +389,11 @@ __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, cons
       TO* dst = (h < nq) ? q + ((size_t)n * nq + h) * d : k + ((size_t)n * nkv + (h - nq)) * d;
       dst[ia] = from_f32<TO>(ra);
       dst[ib] = from_f32<TO>(rb);
+      if (kp != nullptr && h >= nq) {
+        TO* to = kp + (size_t)(h - nq) * PAGE * d;
+        to[ia] = from_f32<TO>(ra);
+        to[ib] = from_f32<TO>(rb);
+      }
     }
   }
   const float* vs = src + (size_t)(nq + nkv) * d;
@@ -458,7 +481,7 @@ __device__ __forceinline__ void v_tile(int col_block, int kvh, int d_block, TO (
                                        const TS* __restrict__ qkv, int width, int v_off, int d,
                                        TO* __restrict__ vt, int vt_cols, int B, const int* __restrict__ cu_seqlens,
                                        const int* __restrict__ tile_off, const int* __restrict__ n_cached,
-                                       const int* __restrict__ len_after) {
+                                       const int* __restrict__ len_after, int nkv = 0, const Commit<TO>& commit = Commit<TO>{}) {
   const int col0 = col_block * PAGE;
   const ColumnTile t = column_tile(col0, B, tile_off, n_cached, len_after);
   if (t.lo >= t.hi) return;
@@ -492,12 +515,16 @@ __device__ __forceinline__ void v_tile(int col_block, int kvh, int d_block, TO (
       if (idx < PAGE * dc) tile[idx % dc][idx / dc] = from_f32<TO>(tmp[u]);
     }
   }
+  TO* vp = commit.pages ? commit.page(t.b, t.p0, nkv, d) + (size_t)nkv * PAGE * d + ((size_t)kvh * d + c0) * PAGE : nullptr;
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < 16; ++u) {
     const int idx = threadIdx.x + 256 * u;
     const int i = idx / PAGE, r = idx % PAGE, p = t.p0 + r;
-    if (i < dc && p >= t.lo && p < t.hi) vt[((size_t)kvh * d + c0 + i) * vt_cols + col0 + r] = tile[i][r];
+    if (i < dc && p >= t.lo && p < t.hi) {
+      vt[((size_t)kvh * d + c0 + i) * vt_cols + col0 + r] = tile[i][r];
+      if (vp != nullptr) vp[(size_t)i * PAGE + r] = tile[i][r];
+    }
   }
 }
 
@@ -513,26 +540,30 @@ v_tiles_kernel(const TS* __restrict__ qkv, int width, int v_off, int d, TO* __re
 
 // Both of the above in one launch, for a step with several rows a sequence: the first n workgroups
 // rotate a row each (q and k; the values are the tiles' business), the others transpose a tile of
-// values each.  The two read the same buffer and write different ones.
+// values each.  The two read the same buffer and write different ones.  With `commit` they put keys and values into their
+// pages as well, which kv_commit_tiles_kernel otherwise does behind
+// the attention (7 us a layer for 226 rows, 27 for 16,384): prompt steps of 226 rows 6,274 and 6,099 us, of 2,048 26,017 and 25,907, of 16,384
+// 260.3 and 258.1 ms.
 template <typename TO>
 __global__ void __launch_bounds__(256)
 rope_v_tiles_kernel(const float* __restrict__ qkv, const int* __restrict__ row_pos, Rotation rot, int n, int nq,
                     int nkv, int d, TO* __restrict__ q, TO* __restrict__ k, TO* __restrict__ vt, int vt_cols, int B,
                     const int* __restrict__ cu_seqlens, const int* __restrict__ tile_off,
-                    const int* __restrict__ n_cached, const int* __restrict__ len_after) {
+                    const int* __restrict__ n_cached, const int* __restrict__ len_after, const int* __restrict__ row_seq,
+                    Commit<TO> commit) {
   __shared__ __attribute__((aligned(16))) unsigned char sh[sizeof(TO) * 64 * (PAGE + 2) > 2 * sizeof(float) * ROPE_MAX_HALF
                                                             ? sizeof(TO) * 64 * (PAGE + 2)
                                                             : 2 * sizeof(float) * ROPE_MAX_HALF];
   if ((int)blockIdx.x < n) {
     float* cs = reinterpret_cast<float*>(sh);
     rope_split_row<TO>(blockIdx.x, cs, cs + ROPE_MAX_HALF, qkv, row_pos, rot, nq, nkv, d, q, k, (TO*)nullptr,
-                       (TO*)nullptr, 0, nullptr, nullptr, nullptr);
+                       (TO*)nullptr, 0, row_seq, nullptr, nullptr, commit);
     return;
   }
   const int item = blockIdx.x - n, d_blocks = (d + 63) / 64;
   const int d_block = item % d_blocks, kvh = (item / d_blocks) % nkv, col_block = item / (d_blocks * nkv);
   v_tile<TO>(col_block, kvh, d_block, reinterpret_cast<TO(*)[PAGE + 2]>(sh), qkv, (nq + 2 * nkv) * d, (nq + nkv) * d, d,
-             vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after);
+             vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after, nkv, commit);
 }
 
 // Commit of a step whose values lie transposed by tiles: the first blocks put the keys of 8 rows
@@ -1194,10 +1225,11 @@ int tl_v_tiles_rows(const void* v, int n, int nkv, int d, void* vt, int vt_cols,
   return 0;
 }
 
+// pages (or null): the cache, into which keys and values go at once; for steps after which every sequence fits its ring of pages
 int tl_rope_v_tiles(const float* qkv, const int* row_pos, const float* inv_freq, int rotary_dim, int interleaved,
                     int n, int nq, int nkv, int d, void* q, void* k, void* vt, int vt_cols, int B,
-                    const int* cu_seqlens, const int* tile_off, const int* n_cached, const int* len_after, int dt,
-                    hipStream_t st) {
+                    const int* cu_seqlens, const int* tile_off, const int* n_cached, const int* len_after, const int* row_seq,
+                    const int* table, int table_stride, int ring_pages, void* pages, int dt, hipStream_t st) {
   TL_REQUIRE(n >= 0 && nq > 0 && nkv > 0 && d > 0 && d % 2 == 0 && d <= 2 * ROPE_MAX_HALF && B > 0,
              "rope_v_tiles: bad sizes n=%d nq=%d nkv=%d d=%d B=%d (d even, at most %d)", n, nq, nkv, d, B,
              2 * ROPE_MAX_HALF);
@@ -1205,18 +1237,19 @@ int tl_rope_v_tiles(const float* qkv, const int* row_pos, const float* inv_freq,
   TL_REQUIRE(rotary_dim >= 0 && rotary_dim <= d && rotary_dim % 2 == 0 && (rotary_dim == 0 || inv_freq != nullptr),
              "rope_v_tiles: %d rotated channels of a head of %d (even, at most the head, with their frequencies)",
              rotary_dim, d);
+  TL_REQUIRE(pages == nullptr || (row_seq && table && table_stride > 0 && ring_pages > 0), "rope_v_tiles: pages without a page table");
   if (n == 0) return 0;
   const Rotation rot{inv_freq, rotary_dim, interleaved != 0};
   const long long blocks = (long long)n + (long long)(vt_cols / PAGE) * nkv * ((d + 63) / 64);
   TL_REQUIRE(blocks < 2147483647LL, "rope_v_tiles: %lld workgroups are too many", blocks);
   if (dt == DT_F32)
     rope_v_tiles_kernel<float><<<(unsigned)blocks, 256, 0, st>>>(qkv, row_pos, rot, n, nq, nkv, d, (float*)q, (float*)k,
-                                                                  (float*)vt, vt_cols, B, cu_seqlens, tile_off, n_cached,
-                                                                  len_after);
+                                                                  (float*)vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after,
+                                                                  row_seq, Commit<float>{table, table_stride, ring_pages, (float*)pages});
   else if (dt == DT_BF16)
     rope_v_tiles_kernel<bf16><<<(unsigned)blocks, 256, 0, st>>>(qkv, row_pos, rot, n, nq, nkv, d, (bf16*)q, (bf16*)k,
-                                                                 (bf16*)vt, vt_cols, B, cu_seqlens, tile_off, n_cached,
-                                                                 len_after);
+                                                                 (bf16*)vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after,
+                                                                 row_seq, Commit<bf16>{table, table_stride, ring_pages, (bf16*)pages});
   else
     TL_REQUIRE(false, "rope_v_tiles: unknown dtype code %d", dt);
   TL_LAUNCH_CHECK("rope_v_tiles");

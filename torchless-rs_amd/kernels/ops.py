@@ -16,7 +16,7 @@ from typing import Optional, Tuple
 import torch
 
 from .build import load, load_measure
-from .page import PAGE, require_same
+from .page import NO_RING, PAGE, require_same
 
 DT_F32, DT_BF16 = 0, 1
 _CODES = {torch.float32: DT_F32, torch.bfloat16: DT_BF16}
@@ -302,8 +302,9 @@ def v_tiles_rows(v: torch.Tensor, vt: torch.Tensor, cu_seqlens, tile_off, n_cach
 
 
 def rope_v_tiles(qkv: torch.Tensor, row_pos, rotation, nq: int, nkv: int, d: int, q: torch.Tensor, k: torch.Tensor,
-                 vt: torch.Tensor, cu_seqlens, tile_off, n_cached, len_after) -> None:
-    """`rope_split` (q and k) and `v_tiles` in one launch: the same bits as the two."""
+                 vt: torch.Tensor, cu_seqlens, tile_off, n_cached, len_after, commit=None) -> None:
+    """`rope_split` (q and k) and `v_tiles` in one launch: the same bits as the two.  `commit` (row_seq, table, ring_pages,
+    pages): `kv_commit_tiles` with it, for steps that `overwrite_nothing`."""
     n = qkv.shape[0]
     _req(qkv, "rope_v_tiles.qkv", torch.float32, (n, (nq + 2 * nkv) * d))
     _req(row_pos, "rope_v_tiles.row_pos", torch.int32, (n,))
@@ -317,9 +318,27 @@ def rope_v_tiles(qkv: torch.Tensor, row_pos, rotation, nq: int, nkv: int, d: int
     _tiles_args(B, cu_seqlens, tile_off, n_cached, len_after, "rope_v_tiles")
     if cu_seqlens is None:
         raise KernelError("rope_v_tiles.cu_seqlens: needed")
+    row_seq, table, ring_pages, pages = commit or (None, None, 1, None)
+    if commit:
+        _req(row_seq, "rope_v_tiles.row_seq", torch.int32, (n,))
+        _req(table, "rope_v_tiles.table", torch.int32)
+        _req(pages, "rope_v_tiles.pages", q.dtype)
+        if pages.dim() != 5 or tuple(pages.shape[1:]) != (2, nkv, PAGE, d):
+            raise KernelError(f"rope_v_tiles.pages: shape {tuple(pages.shape)}, kernel needs [*, 2, {nkv}, {PAGE}, {d}]")
+        if table.dim() != 2 or table.shape[0] != B:
+            raise KernelError("rope_v_tiles.table: needs one row per sequence")
     _check(lib().tl_rope_v_tiles(_p(qkv), _p(row_pos), _p(rot.inv_freq), rot.rotary_dim, int(rot.interleaved), n, nq,
                                  nkv, d, _p(q), _p(k), _p(vt), vt.shape[2], B, _p(cu_seqlens), _p(tile_off),
-                                 _p(n_cached), _p(len_after), _code(q.dtype), _stream()))
+                                 _p(n_cached), _p(len_after), _p(row_seq), _p(table), table.shape[1] if commit else 0, ring_pages, _p(pages),
+                                 _code(q.dtype), _stream()))
+
+
+def overwrite_nothing(ctx, ring_pages: int) -> bool:
+    """Do the step's new positions take the place of no older one in a ring of so many pages?  They may then lie in the cache before the
+    attention reads it.  (A captured step's lengths are other ones at every replay: only a ring that is none will do.)"""
+    if ctx.host.get("fixed_launches"):
+        return ring_pages >= NO_RING
+    return int(ctx.host["len_after"].max()) <= ring_pages * PAGE
 
 
 def kv_commit_tiles(k: torch.Tensor, vt: torch.Tensor, row_seq, row_pos, tile_off, n_cached, len_after,

@@ -17,6 +17,7 @@ def _read() -> int:
 
 
 PAGE = _read()
+NO_RING = 1 << 24          # "ring" of a group that keeps every position: never wraps
 
 
 def round_up(n_tokens: int) -> int:

@@ -118,6 +118,7 @@ class AttentionMixer(Mixer):
         n, nq, nkv, d = y.shape[0], self.nq, self.nkv, self.d
         ws = ctx.workspace
         group = run.kv_group
+        early = False                               # are this step's keys and values in the cache before its attention?
         pages = group.storage[run.kv_layer]
         table = ctx.tables[run.kv_group_index]
         rotation = self.position.rotation(y.device) or ops.NO_ROTATION
@@ -159,8 +160,10 @@ class AttentionMixer(Mixer):
                 # the matrix cores read values along the keys: only the transposed copy is made, by tiles
                 v = None
                 vt = ws.get("attn_vt" + tag, (nkv, d, ctx.host["aligned_cols"]), ctx.dtype)
+                early = not run.kv_read_later and ops.overwrite_nothing(ctx, group.ring_pages)
                 ops.rope_v_tiles(qkv, ctx.row_pos, rotation, nq, nkv, d, q, k, vt, ctx.cu_seqlens, ctx.tile_off,
-                                 ctx.len_before, ctx.len_after)       # rotation and transposition in one launch
+                                 ctx.len_before, ctx.len_after,       # rotation and transposition in one launch
+                                 commit=(ctx.row_seq, table, group.ring_pages, pages) if early else None)
             else:
                 vt = None
                 v = ws.get("attn_v" + tag, (n, nkv, d), ctx.dtype)
@@ -182,7 +185,7 @@ class AttentionMixer(Mixer):
         else:
             ops.attention(q, k, v, pages, table, group.ring_pages, ctx, ctx.len_before,
                           self.window, self.scale, out, vt_new=vt)
-            if self.own_kv:
+            if self.own_kv and not early:
                 def commit():
                     if vt is not None:
                         ops.kv_commit_tiles(k, vt, ctx.row_seq, ctx.row_pos, ctx.tile_off, ctx.len_before,
