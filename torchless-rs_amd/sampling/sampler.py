@@ -104,12 +104,11 @@ class Sampler:
         place.pairs[:B, 0] = seq_ids
         place.pairs[:B, 1] = steps
         place.ids[:B] = -1
-        out = self._out[:B]
-        ops.sample(logits.contiguous(), float(c.temperature), int(c.top_k or 0), float(c.top_p or 0.0),
-                   int(c.seed), place.counters[:B], self._probs[:B], out, self._lists, place.tokens[:B])
+        ops.sample_kept(logits.contiguous(), wanted[2], wanted[3], float(c.top_p or 0.0), int(c.seed), place.counters, self._probs, self._out,
+                        self._lists, place.tokens)
         self._last = place.done = torch.cuda.Event()
         place.done.record()
-        return Drawn(out, place)
+        return Drawn(self._out[:B], place)
 
     def sample(self, logits: torch.Tensor, seq_ids: Sequence[int], steps: Sequence[int]) -> List[int]:
         """logits: float32 [B, V] on the GPU -> B token ids."""
