@@ -461,14 +461,31 @@ sample_kernel(const float* __restrict__ logits, int V, float temperature, int to
   if (top_k > 0 && top_k < V && top_k <= MOST_TOP_K) {
     const PartList* parts = lists ? lists + (size_t)b * n_parts : nullptr;
     if (tid == 0) sh.count = 0;
+    // A wave takes parts w and w + 16: their counts and each lane's first candidate come in one trip, the others, which lists of more
+    // than a wave's lanes have, behind it
+    // (counts, candidates and again for the second pass: 16.4 us the kernel, 15.9 now).
+    constexpr int MINE = 2;
+    static_assert(MINE * (SNT / WAVE) >= 32, "tl_sample_parts gives at most 32");
+    int counts[MINE] = {};
+    unsigned long long first[MINE] = {};
+    if (parts) {
+#pragma unroll
+      for (int q = 0; q < MINE; ++q) {
+        const unsigned long long* l = parts[min(w + q * (SNT / WAVE), n_parts - 1)];
+        counts[q] = (int)l[0];
+        first[q] = l[1 + lane];
+      }
+#pragma unroll
+      for (int q = 0; q < MINE; ++q)
+        if (w + q * (SNT / WAVE) >= n_parts) counts[q] = 0;
+    }
     // (a part with more than its list holds, equal logits for instance: as without parts)
-    if (parts && !__syncthreads_or(tid < n_parts && parts[min(tid, n_parts - 1)][0] > PART_KEEP)) {
-      const int per = max(1, SNT / WAVE / n_parts);      // waves a part
+    if (parts && !__syncthreads_or(max(counts[0], counts[1]) > PART_KEEP)) {
       const auto each = [&](auto f) {
-        for (int s = w; s < n_parts * per; s += SNT / WAVE) {
-          const unsigned long long* l = parts[s / per];
-          const int n = (int)l[0];
-          for (int j = s % per * WAVE + lane; j < n; j += per * WAVE) f(l[1 + j]);
+#pragma unroll
+        for (int q = 0; q < MINE; ++q) {
+          if (lane < counts[q]) f(first[q]);
+          for (int j = lane + WAVE; j < counts[q]; j += WAVE) f(parts[w + q * (SNT / WAVE)][1 + j]);
         }
       };
       uint32_t mine = 0u;
