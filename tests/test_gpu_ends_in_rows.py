@@ -1,0 +1,103 @@
+"""A step's last block over the rows alone whose logits are wanted (`ENDS_IN_ROWS` of engine/model.py) against all of its rows: logits
+and everything that later steps read."""
+import copy
+import types
+
+import pytest
+import torch
+
+from util import TOL, make_model_dir, prompts, rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def models(tmp_path, name, dtype):
+    from torchless_rs_amd.engine import load_model
+    if name in ("A", "B"):
+        return load_model(make_model_dir(tmp_path, name, torch.bfloat16), dtype)
+    import importlib
+    t, plain = importlib.import_module(f"test_gpu_{name}"), importlib.import_module(f"plain_{name}")
+    cfg = copy.deepcopy(t.CONFIGS["mixed"])
+    return load_model(t.write_model(str(tmp_path / name), cfg, plain.random_weights(cfg, 7)), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", ["A", "B", "nepisun", "giforax"])
+def test_the_wanted_rows_alone_have_the_logits_of_all_rows(tmp_path, monkeypatch, name, dtype):
+    """Prompts in pieces (no logits wanted, the last row's, several), then tokens: 17 rows, and more than a tile; each step three times
+    over the same engines' lives, so that short ones come from a captured graph."""
+    from torchless_rs_amd.engine import Engine, SeqInput
+    from torchless_rs_amd.engine import model as m
+    model = models(tmp_path, name, dtype)
+    V = model.spec.vocab_size
+    ids = prompts(V, [150, 40, 33], 3)
+    engines = {all_rows: Engine(model, max_tokens=64 * 24, max_slots=4) for all_rows in (False, True)}
+    narrow = []
+    for block in model.blocks:
+        if hasattr(block, "forward_rows"):
+            real = block.forward_rows
+            monkeypatch.setattr(block, "forward_rows", lambda *a, _r=real, **k: (narrow.append(1), _r(*a, **k))[1])
+    for life in range(4):
+        got = {}
+        for all_rows, eng in engines.items():
+            monkeypatch.setattr(m, "ENDS_IN_ROWS", 1 << 30 if all_rows else 16)
+            slots = [eng.alloc() for _ in ids]
+            out, before = [], len(narrow)
+            steps = [[(0, 0, 17, [16])], [(0, 17, 60, []), (1, 0, 20, [])], [(0, 77, 73, [72]), (1, 20, 20, [19, 3]), (2, 0, 33, [32])]]
+            for step in steps:
+                out.append(eng.step([SeqInput(slots[s], ids[s][a:a + n], w) for s, a, n, w in step]).clone())
+            for t in range(2):
+                out.append(eng.step([SeqInput(s, [(5 * t + i) % V], [0]) for i, s in enumerate(slots)]).clone())
+            got[all_rows] = out
+            assert len(narrow) - before == (0 if all_rows else 3) or life > 1     # (a captured step runs once)
+            for s in slots:
+                eng.free(s)
+        for a, b in zip(got[False], got[True]):
+            assert a.shape == b.shape
+            if a.numel():
+                assert torch.isfinite(a).all() and rel_err(a, b.double()) < TOL[dtype]
+
+
+def test_who_may_end_in_rows():
+    from torchless_rs_amd.parts.base import rows_apart
+    from torchless_rs_amd.parts.ffn import SwiGLU
+
+    class Mixes(SwiGLU):
+        def forward(self, ctx, y, x):
+            x += y.sum(0)
+
+    class Says(Mixes):
+        row_wise = True
+
+    plain = types.SimpleNamespace
+    mk = lambda c: object.__new__(c)
+    assert rows_apart(mk(SwiGLU)) and not rows_apart(mk(Mixes)) and rows_apart(mk(Says)) and not rows_apart(plain())
+    patched = mk(SwiGLU)
+    patched.forward = lambda *a: None
+    assert not rows_apart(patched)
+
+
+@pytest.mark.parametrize("H", [64, 1000, 4096, 8192])
+@pytest.mark.parametrize("parts", [0, 1, 9])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_a_norm_of_some_rows_has_the_bits_of_adding_gathering_and_the_norm(H, parts, dt):
+    from torchless_rs_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(H + parts)
+    n, rows = 37, torch.tensor([36, 0, 0, 17], dtype=torch.int32, device=DEV)
+    x, w = torch.randn(n, H, generator=g, device=DEV), torch.randn(H, generator=g, device=DEV)
+    p = torch.randn(parts, n, H, generator=g, device=DEV) if parts else None
+    assert ops.rmsnorm_rows_ok(x, w, p) and not ops.rmsnorm_rows_ok(x[:, 1:], w, p) and not ops.rmsnorm_rows_ok(torch.zeros(2, 9000), w, None)
+    out, keep, was = torch.zeros(4, H, dtype=dt, device=DEV), torch.zeros(4, H, device=DEV), x.clone()
+    ops.rmsnorm(x, w, 1e-5, out, rows=rows, parts=p, keep=keep)
+    assert torch.equal(x, was)
+    if parts:
+        ops.add_partials(x, p)
+    xs, y = torch.zeros(4, H, device=DEV), torch.zeros(4, H, dtype=dt, device=DEV)
+    ops.gather_rows(x, rows, xs)
+    ops.rmsnorm(xs, w, 1e-5, y)
+    assert torch.equal(keep, xs) and torch.equal(out, y)
+    both = torch.stack([x, 2 * x])
+    many = torch.zeros(2, 4, H, device=DEV)
+    ops.gather_rows(both, rows, many)
+    assert torch.equal(many, both[:, rows.long()])

@@ -182,6 +182,46 @@ __global__ void __launch_bounds__(256) rmsnorm_reg_kernel(const float* __restric
   }
 }
 
+// The norm of some rows, each with its partial products (n_parts may be 0) added in their order, and (keep not null) those rows
+// themselves: what is read of the stream's end.  Adding, gathering and the norm were three launches, the first over all of a step's rows.
+template <typename TO, int IT>
+__global__ void __launch_bounds__(256)
+rmsnorm_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, const float* __restrict__ parts, int n_parts, size_t part_stride,
+                    const float* __restrict__ w, float eps, TO* __restrict__ out, float* __restrict__ keep, int H) {
+  __shared__ float sh[4];
+  const size_t at = (size_t)rows[blockIdx.x] * H;
+  const f32x4* xr = reinterpret_cast<const f32x4*>(x + at);
+  const f32x4* wr = reinterpret_cast<const f32x4*>(w);
+  const int nv = H / 4;
+  f32x4 v[IT], g[IT];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c < nv) {
+      v[i] = xr[c];
+      g[i] = wr[c];
+#pragma unroll 8
+      for (int s = 0; s < n_parts; ++s) v[i] += reinterpret_cast<const f32x4*>(parts + s * part_stride + at)[c];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < IT; ++i)
+    if ((int)threadIdx.x + 256 * i < nv) ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+  ss = block_sum<256>(ss, sh);
+  const float rms = sqrtf(ss / (float)H + eps);
+  TO* o = out + (size_t)blockIdx.x * H;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c < nv) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[4 * c + e] = from_f32<TO>((v[i][e] / rms) * g[i][e]);
+      if (keep != nullptr) reinterpret_cast<f32x4*>(keep + (size_t)blockIdx.x * H)[c] = v[i];
+    }
+  }
+}
+
 // x += sum of the partial products P[s][n][H] (in the order of s), then the norm of the new x.
 template <typename TO, int IT>
 __global__ void __launch_bounds__(256)
@@ -980,11 +1020,12 @@ __global__ void take_tokens_kernel(const int* __restrict__ src, const int* __res
   tokens[j] = (t >= 0 && t < vocab) ? t : 0;
 }
 
-__global__ void gather_rows_kernel(const float* __restrict__ x, const int* __restrict__ idx, int H,
+// blockIdx.y: one of several matrices of n rows, one behind the other
+__global__ void gather_rows_kernel(const float* __restrict__ x, const int* __restrict__ idx, int n, int H,
                                    float* __restrict__ out) {
   const int m = blockIdx.x;
-  const float* s = x + (size_t)idx[m] * H;
-  float* o = out + (size_t)m * H;
+  const float* s = x + ((size_t)blockIdx.y * n + idx[m]) * H;
+  float* o = out + ((size_t)blockIdx.y * gridDim.x + m) * H;
   for (int i = threadIdx.x; i < H; i += blockDim.x) o[i] = s[i];
 }
 
@@ -1065,8 +1106,30 @@ int tl_rmsnorm(const float* x, const float* w, float eps, void* out, int out_dt,
   return 0;
 }
 
-// vt (may be null): values also transposed, [nkv][d][vt_cols], row n in column
-// tile_off[row_seq[n]] + row_pos[n] - 64 * (n_cached[row_seq[n]] / 64)
+// out[m, H] = rmsnorm(x[rows[m]] + parts[0..n_parts)[rows[m]]), x and each of parts [n, H]; x stays as it is.  keep [m, H] (or null): those sums
+int tl_rmsnorm_rows(const float* x, int n, const int* rows, int m, const float* parts, int n_parts, const float* w, float eps, void* out, int out_dt,
+                    float* keep, int H, hipStream_t st) {
+  TL_REQUIRE(n > 0 && m >= 0 && n_parts >= 0, "rmsnorm_rows: bad sizes n=%d m=%d parts=%d", n, m, n_parts);
+  TL_REQUIRE(out_dt == DT_F32 || out_dt == DT_BF16, "rmsnorm_rows: unknown dtype code %d", out_dt);
+  TL_REQUIRE(x && rows && w && out && (parts || n_parts == 0), "rmsnorm_rows: a buffer is missing");
+  TL_REQUIRE(H > 0 && H % 4 == 0 && H <= 8192 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)parts | (uintptr_t)keep) % 16 == 0,
+             "rmsnorm_rows: H=%d must be a multiple of 4, at most 8192, rows 16-byte aligned", H);
+  if (m == 0) return 0;
+  const size_t stride = (size_t)n * H;
+#define TL_RMSR(IT)                                                                                                                  \
+  do {                                                                                                                               \
+    if (out_dt == DT_F32) rmsnorm_rows_kernel<float, IT><<<m, 256, 0, st>>>(x, rows, parts, n_parts, stride, w, eps, (float*)out, keep, H); \
+    else rmsnorm_rows_kernel<bf16, IT><<<m, 256, 0, st>>>(x, rows, parts, n_parts, stride, w, eps, (bf16*)out, keep, H);                     \
+  } while (0)
+  if (H <= 1024) TL_RMSR(1);
+  else if (H <= 2048) TL_RMSR(2);
+  else if (H <= 4096) TL_RMSR(4);
+  else TL_RMSR(8);
+#undef TL_RMSR
+  TL_LAUNCH_CHECK("rmsnorm_rows");
+  return 0;
+}
+
 // x[n, H] += parts[0..n_parts)[n, H]; out = rmsnorm(x)
 int tl_add_rmsnorm(float* x, const float* parts, int n_parts, const float* w, float eps, void* out, int out_dt,
                    int n, int H, hipStream_t st) {
@@ -1434,10 +1497,11 @@ int tl_take_tokens(const int* src, const int* idx, int n, int n_src, int vocab, 
   return 0;
 }
 
-int tl_gather_rows(const float* x, const int* idx, int m, int H, float* out, hipStream_t st) {
-  TL_REQUIRE(m >= 0 && H > 0, "gather_rows: bad sizes m=%d H=%d", m, H);
-  if (m == 0) return 0;
-  gather_rows_kernel<<<m, 256, 0, st>>>(x, idx, H, out);
+// x float [count][n][H] -> out [count][m][H]
+int tl_gather_rows(const float* x, const int* idx, int count, int n, int m, int H, float* out, hipStream_t st) {
+  TL_REQUIRE(m >= 0 && H > 0 && n >= 0 && count >= 0 && count <= 65535, "gather_rows: bad sizes m=%d H=%d n=%d of %d", m, H, n, count);
+  if (m == 0 || count == 0) return 0;
+  gather_rows_kernel<<<dim3(m, count), 256, 0, st>>>(x, idx, n, H, out);
   TL_LAUNCH_CHECK("gather_rows");
   return 0;
 }

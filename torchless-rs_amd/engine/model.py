@@ -14,10 +14,15 @@ import torch
 
 from ..cache.cache import Cache, KVRequest, StateRequest
 from ..config.base import ModelConfig
-from ..parts.base import ModelSpec, PartSpec, RunBinding, StepContext, flush_pending, make_part
+from ..parts.base import ModelSpec, PartSpec, RunBinding, StepContext, flush_pending, make_part, rows_through_norm
 from ..weights.binding import bind_weights
 
 
+# From how many rows on the model's last block runs its feed-forward over the rows alone whose logits are wanted (and over none
+# where none are): nobody reads the others, later steps only what the block's mixer keeps of them.  Steps of up to 16 rows have products
+# that the norms are cut around, and read their weights whatever the rows.  Prompt steps of 2,048 rows through 32 layers 25,907 us and
+# 25,502, of 226 6,099 and 5,994; through four layers with experts 2,312 rows 5,437 and 4,953, 2,348 rows 5,094 and 4,508.
+ENDS_IN_ROWS = 16
 EMBEDDING_RUN = -1            # the number under which the cache keeps the embedding's state, beside those of the runs
 
 
@@ -155,6 +160,7 @@ class Model:
         schedule = self.spec.schedule
         order = [self.blocks[run.layer] for run in schedule]
         handed = False                       # the block before saw to this run's stream part
+        narrow, ends = False, None           # what the last block left are the wanted rows alone
         for i, (block, binding) in enumerate(zip(order, runs)):
             if schedule[i].entry is not None and not handed:
                 part, t = schedule[i].entry
@@ -175,20 +181,28 @@ class Model:
                 kw["norm_after"] = after
             if handed:
                 kw["stream_after"] = (self.stream_parts[nxt[0]], nxt[1])
-            block.forward(ctx, binding, x, **kw)
+            if i + 1 == len(order) and n_want < ctx.n_rows > ENDS_IN_ROWS and (nxt is None or handed) \
+                    and hasattr(block, "ends_in_rows") and block.ends_in_rows(**kw):
+                ends = block.forward_rows(ctx, binding, x, want_rows if n_want else None, **kw)
+                narrow = True
+            else:
+                block.forward(ctx, binding, x, **kw)
         ctx.prenormed = None                 # nothing reads a norm's first half past the last block
         for commit in ctx.host.pop("deferred", []):
             commit()
-        flush_pending(ctx, x)
         if self.spec.exit is not None and not handed:
+            flush_pending(ctx, x)
             part, t = self.spec.exit
             self.stream_parts[part].forward(ctx, x, embedded, t)
         logits = ws.get("logits", (n_want, V), torch.float32)
         if n_want:
-            xs = ws.get("head_x", (n_want, H), torch.float32)
-            from ..kernels import ops
-            ops.gather_rows(x, want_rows, xs)
             y = ws.get("head_y", (n_want, H), ctx.dtype)
-            self.final_norm.forward(ctx, xs, y)
+            if narrow:
+                if not getattr(self.final_norm, "takes_pending", False):
+                    flush_pending(ctx, ends)
+                self.final_norm.forward(ctx, ends, y)
+            else:
+                rows_through_norm(ctx, self.final_norm, x, want_rows, None, y)
             self.head.forward(ctx, y, logits)
+        ctx.pending = None                   # (what rows that nobody wants would still have added)
         return logits

@@ -167,14 +167,35 @@ def scale_(x: torch.Tensor, s: float) -> None:
     _check(lib().tl_scale(_p(x), ctypes.c_float(s), ctypes.c_longlong(x.numel()), _stream()))
 
 
-def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor) -> None:
-    """out = x / sqrt(mean(x^2) + eps) * w, x float32 [n, H], w float32 [H]."""
+def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor, rows: Optional[torch.Tensor] = None,
+            parts: Optional[torch.Tensor] = None, keep: Optional[torch.Tensor] = None) -> None:
+    """out = x / sqrt(mean(x^2) + eps) * w, x float32 [n, H], w float32 [H].  `rows` (int32 [m], where `rmsnorm_rows_ok`): of these rows of
+    x alone, each with the sum of `parts` (float32 [S, n, H] or None) for it added, in one launch: the bits of `add_partials`,
+    `gather_rows` and the norm, but that x stays as it is.  `keep` (float32 [m, H]) receives those sums."""
     n, H = x.shape
     _req(x, "rmsnorm.x", torch.float32)
     _req(w, "rmsnorm.w", torch.float32, (H,))
-    _req(out, "rmsnorm.out", None, (n, H))
-    _check(lib().tl_rmsnorm(_p(x), _p(w), ctypes.c_float(eps), _p(out), _code(out.dtype), n, H,
-                            _stream()))
+    if rows is None:
+        _req(out, "rmsnorm.out", None, (n, H))
+        _check(lib().tl_rmsnorm(_p(x), _p(w), ctypes.c_float(eps), _p(out), _code(out.dtype), n, H,
+                                _stream()))
+        return
+    m = rows.shape[0]
+    _req(rows, "rmsnorm.rows", torch.int32, (m,))
+    _req(out, "rmsnorm.out", None, (m, H))
+    if parts is not None:
+        _req(parts, "rmsnorm.parts", torch.float32, (parts.shape[0], n, H))
+    if keep is not None:
+        _req(keep, "rmsnorm.keep", torch.float32, (m, H))
+    _check(lib().tl_rmsnorm_rows(_p(x), n, _p(rows), m, _p(parts), parts.shape[0] if parts is not None else 0, _p(w), ctypes.c_float(eps),
+                                 _p(out), _code(out.dtype), _p(keep), H, _stream()))
+
+
+def rmsnorm_rows_ok(x: torch.Tensor, w: torch.Tensor, parts: Optional[torch.Tensor]) -> bool:
+    """Does `rmsnorm` take rows of these?"""
+    H = x.shape[1]
+    return (H % 4 == 0 and H <= 8192 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (parts is None or (parts.data_ptr() % 16 == 0 and parts.shape[1:] == x.shape)))
 
 
 class Rotation:
@@ -1747,11 +1768,13 @@ def take_tokens(src: torch.Tensor, idx: torch.Tensor, vocab: int, tokens: torch.
 
 
 def gather_rows(x: torch.Tensor, idx: torch.Tensor, out: torch.Tensor) -> None:
-    m, H = idx.shape[0], x.shape[1]
+    """out[m] = x[idx[m]], float32 [n, H]; or the same rows of each of several matrices, x [count, n, H] and out [count, m, H]."""
+    m, H = idx.shape[0], x.shape[-1]
+    many = tuple(x.shape[:-2])
     _req(x, "gather.x", torch.float32)
     _req(idx, "gather.idx", torch.int32, (m,))
-    _req(out, "gather.out", torch.float32, (m, H))
-    _check(lib().tl_gather_rows(_p(x), _p(idx), m, H, _p(out), _stream()))
+    _req(out, "gather.out", torch.float32, many + (m, H))
+    _check(lib().tl_gather_rows(_p(x), _p(idx), many[0] if many else 1, x.shape[-2], m, H, _p(out), _stream()))
 
 
 def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool = False) -> None:

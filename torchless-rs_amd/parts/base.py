@@ -250,6 +250,8 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    row_wise = False          # does what it does to a row follow from that row alone? (asked through `rows_apart`)
+
     def forward(self, ctx: "StepContext", y: torch.Tensor, x: torch.Tensor) -> None:
         """y: normed input [n, H]; ADD the result to x (float32 [n, H])."""
         raise NotImplementedError
@@ -301,6 +303,32 @@ def norms_as_its_form(norm: "Norm") -> bool:
         if "forward" in vars(c):
             return False
     return False
+
+
+def rows_apart(part: "FeedForward") -> bool:
+    """Is `part` `row_wise`?  Not where its work was set on the object, or is that of a class derived from the one that says so."""
+    own = getattr(part, "__dict__", ())
+    if "forward" in own or "produce" in own:
+        return False
+    for c in type(part).__mro__:
+        if "row_wise" in vars(c):
+            return bool(vars(c)["row_wise"])
+        if "forward" in vars(c) or "produce" in vars(c):
+            return False
+    return False
+
+
+def rows_through_norm(ctx: "StepContext", norm: "Norm", x: torch.Tensor, rows: torch.Tensor, xs: Optional[torch.Tensor], y: torch.Tensor) -> None:
+    """`rows` of the stream, with the partial products that wait for it, in `xs` (None: nobody reads them so), and as `norm` gives
+    them in `y`.  Nobody reads the stream's other rows any more."""
+    if hasattr(norm, "forward_rows") and norms_as_its_form(norm) and norm.forward_rows(ctx, x, rows, y, xs):
+        return
+    from ..kernels import ops
+    flush_pending(ctx, x)
+    if xs is None:
+        xs = ctx.workspace.get("head_x", (rows.shape[0], x.shape[1]), torch.float32)
+    ops.gather_rows(x, rows, xs)
+    norm.forward(ctx, xs, y)
 
 
 def take_row_norm(ctx: "StepContext"):

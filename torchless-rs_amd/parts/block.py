@@ -13,8 +13,8 @@ import torch
 
 from ..weights.binding import WeightSpec
 from ..kernels import ops
-from .base import (LayerSpec, Part, expect_norm, flush_pending, make_part, part_done, read_through_norm,
-                   register_part, splittable_entry, take_row_factor)
+from .base import (LayerSpec, Part, expect_norm, flush_pending, goes_as, make_part, part_done, read_through_norm,
+                   register_part, rows_apart, rows_through_norm, splittable_entry, take_row_factor)
 
 
 class PreNormBlock(Part):
@@ -82,6 +82,29 @@ class PreNormBlock(Part):
         expect_norm(ctx, self.ffn, norm_after)
         self.ffn.forward(ctx, y2, x)
         part_done(ctx, self.ffn)
+
+    def ends_in_rows(self, stream_after=None) -> bool:
+        """Does `forward_rows` do what this block does to some of its rows?"""
+        return (stream_after is None and self.ffn is not None and rows_apart(self.ffn) and goes_as(self, PreNormBlock, "forward"))
+
+    def forward_rows(self, ctx, run, x: torch.Tensor, rows: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+        """The model's last block for a step of more than 16 rows of which only `rows` (None: none) are read behind it: the mixer runs as
+        ever, since later steps read what it keeps of every row, the feed-forward over the wanted rows alone.  Returns those of the stream."""
+        ctx.host.pop("stream_copy", None)
+        y = ctx.workspace.get("block_y", tuple(x.shape), ctx.dtype)
+        y1 = read_through_norm(ctx, self.mixer_norm, x, y, self.mixer, run)
+        expect_norm(ctx, self.mixer, self.ffn_norm, self.ffn)
+        self.mixer.forward(ctx, run, y1, x)
+        part_done(ctx, self.mixer)
+        if rows is None:
+            ctx.pending = None
+            return None
+        m = (rows.shape[0], x.shape[1])
+        xs, ys = ctx.workspace.get("rows_x", m, torch.float32), ctx.workspace.get("rows_y", m, ctx.dtype)
+        rows_through_norm(ctx, self.ffn_norm, x, rows, xs, ys)
+        self.ffn.forward(ctx, ys, xs)
+        part_done(ctx, self.ffn)
+        return xs
 
 
 class OutputNormBlock(Part):
@@ -250,6 +273,37 @@ class SandwichNormBlock(Part):
         take_row_factor(ctx, usable=False)
         bias = OutputNormBlock._result(ctx, self.ffn, z, y2)
         self._last_add(ctx, self.ffn_out_norm, z, x, bias, y, norm_after, stream_after)
+
+    def ends_in_rows(self, stream_after=None) -> bool:
+        """As `PreNormBlock.ends_in_rows`."""
+        return (self.ffn is not None and rows_apart(self.ffn) and goes_as(self, SandwichNormBlock, "forward", "_last_add")
+                and (stream_after is None or (hasattr(stream_after[0], "row_terms") and getattr(self.ffn_out_norm, "takes_between", False))))
+
+    def forward_rows(self, ctx, run, x: torch.Tensor, rows: Optional[torch.Tensor], stream_after=None) -> Optional[torch.Tensor]:
+        """As `PreNormBlock.forward_rows`; the mixer's norm too runs over the wanted rows alone."""
+        ctx.host.pop("stream_copy", None)
+        ws = ctx.workspace
+        y = ws.get("block_y", tuple(x.shape), ctx.dtype)
+        z = ws.get("block_z", tuple(x.shape), torch.float32)
+        y1 = read_through_norm(ctx, self.mixer_norm, x, y)
+        take_row_factor(ctx, usable=False)
+        bias = OutputNormBlock._result(ctx, self.mixer, z, run, y1)
+        if rows is None:
+            return None
+        m = (rows.shape[0], x.shape[1])
+        xs, zs, ys = ws.get("rows_x", m, torch.float32), ws.get("rows_z", m, torch.float32), ws.get("rows_y", m, ctx.dtype)
+        ops.gather_rows(x, rows, xs)
+        ops.gather_rows(z, rows, zs)
+        self.mixer_out_norm.add_to(ctx, zs, xs, bias=bias, then=(self.ffn_norm, ys))
+        y2 = read_through_norm(ctx, self.ffn_norm, xs, ys)
+        take_row_factor(ctx, usable=False)
+        bias = OutputNormBlock._result(ctx, self.ffn, zs, y2)
+        if stream_after is None:
+            self.ffn_out_norm.add_to(ctx, zs, xs, bias=bias)
+        else:
+            part, t = stream_after
+            self.ffn_out_norm.add_to(ctx, zs, xs, bias=bias, between=part.row_terms(ctx, x, rows, t))
+        return xs
 
 
 register_part("block", "pre_norm", PreNormBlock)

@@ -21,6 +21,7 @@ from .linear import Linear, interleave_pairs
 
 class SwiGLU(FeedForward):
     graph_safe = True
+    row_wise = True
     closes_stream = True          # its last write to the stream is `Linear.add_into`
     takes_row_factor = True       # its gate|up product can do the division of the norm before it
 

@@ -81,6 +81,7 @@ SLICED_ROWS = 512
 
 class PlainFeedForward(FeedForward):
     graph_safe = True
+    row_wise = True
     closes_stream = True
 
     NAMES = {"up": "up", "down": "down", "act": "act"}
@@ -135,6 +136,7 @@ class PlainFeedForward(FeedForward):
 
 class RoutedExperts(FeedForward):
     graph_safe = True
+    row_wise = True
     closes_stream = True
 
     # leaf names under `prefix`; "{e}" is the expert's number

@@ -69,6 +69,15 @@ class RMSNorm(Norm):
             ctx.pending = None
         ops.rmsnorm(x, self.weight, self.eps, out)
 
+    def forward_rows(self, ctx, x: torch.Tensor, rows: torch.Tensor, out: torch.Tensor, keep=None) -> bool:
+        """`forward` of the stream's `rows` alone, with their partial products waiting in `ctx.pending`, where nobody reads the stream's other
+        rows any more (x is not changed); the rows themselves go to `keep`.  False: not these sizes, nothing was done."""
+        if not ops.rmsnorm_rows_ok(x, self.weight, ctx.pending):
+            return False
+        ops.rmsnorm(x, self.weight, self.eps, out, rows=rows, parts=ctx.pending, keep=keep)
+        ctx.pending = None
+        return True
+
 
 class LayerNorm(Norm):
     """Mean and variance over the row; a weight and, with `bias_name`, a bias of the norm's own.

@@ -47,6 +47,14 @@ class DepthAverage(StreamPart):
         kept = ctx.workspace.get("depth_kept", (len(self.names) + 1,) + tuple(x.shape), torch.float32)
         return kept, (self.one if t == 0 else self.coef[t - 1]), t
 
+    def row_terms(self, ctx, x: torch.Tensor, rows: torch.Tensor, t: int):
+        """`mix_terms` for some of the stream's rows, whose versions so far are copied side by side."""
+        kept, coef, t = self.mix_terms(ctx, x, t)
+        few = ctx.workspace.get("depth_kept_rows", (kept.shape[0], rows.shape[0], self.H), torch.float32)
+        if t:
+            ops.gather_rows(kept[:t], rows, few[:t])
+        return few, coef, t
+
     def forward(self, ctx, x: torch.Tensor, embedded, t: int) -> None:
         ops.depth_average(x, *self.mix_terms(ctx, x, t))
 
