@@ -78,6 +78,22 @@ def test_who_may_end_in_rows():
     assert not rows_apart(patched)
 
 
+def test_who_gives_rows():
+    from torchless_rs_amd.parts.attention import AttentionMixer
+    from torchless_rs_amd.parts.attention_heads import HeadwiseAttentionMixer
+    from torchless_rs_amd.parts.base import Mixer, gives_rows
+    from torchless_rs_amd.parts.retention import RetentionMixer
+
+    class Other(AttentionMixer):
+        def forward(self, ctx, run, y, x):
+            pass
+
+    mk = lambda c: object.__new__(c)
+    assert gives_rows(mk(AttentionMixer), "forward_rows") and not gives_rows(mk(AttentionMixer), "produce_rows")
+    assert gives_rows(mk(HeadwiseAttentionMixer), "forward_rows") and gives_rows(mk(HeadwiseAttentionMixer), "produce_rows")
+    assert not gives_rows(mk(Other), "forward_rows") and not gives_rows(mk(RetentionMixer), "forward_rows") and not gives_rows(mk(Mixer), "forward_rows")
+
+
 @pytest.mark.parametrize("H", [64, 1000, 4096, 8192])
 @pytest.mark.parametrize("parts", [0, 1, 9])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])

@@ -19,9 +19,10 @@ from ..weights.binding import bind_weights
 
 
 # From how many rows on the model's last block runs its feed-forward over the rows alone whose logits are wanted (and over none
-# where none are): nobody reads the others, later steps only what the block's mixer keeps of them.  Steps of up to 16 rows have products
+# where none are), and its mixer's output product where the mixer can (`gives_rows`): nobody reads the others, later steps only what the
+# mixer keeps of them.  Steps of up to 16 rows have products
 # that the norms are cut around, and read their weights whatever the rows.  Prompt steps of 2,048 rows through 32 layers 25,907 us and
-# 25,502, of 226 6,099 and 5,994; through four layers with experts 2,312 rows 5,437 and 4,953, 2,348 rows 5,094 and 4,508.
+# 25,183, of 226 6,099 and 5,947; through four layers with experts 2,312 rows 5,437 and 4,809, 2,348 rows 5,094 and 4,419.
 ENDS_IN_ROWS = 16
 EMBEDDING_RUN = -1            # the number under which the cache keeps the embedding's state, beside those of the runs
 

@@ -28,7 +28,7 @@ import torch
 from ..cache.cache import KVRequest
 from ..kernels import ops
 from ..weights.binding import WeightSpec
-from .base import Mixer, PartSpec, goes_as, make_part, register_part, take_row_factor, take_row_norm
+from .base import Mixer, PartSpec, goes_as, make_part, register_part, take_row_factor, take_row_norm, take_rows
 from .linear import Linear
 
 
@@ -115,6 +115,15 @@ class AttentionMixer(Mixer):
                 and run.kv_group.storage[run.kv_layer].dtype == torch.float32 and ops.plain_around_ok(y, self.qkv.weight))
 
     def forward(self, ctx, run, y: torch.Tensor, x: torch.Tensor) -> None:
+        self.o.add_into(self._attended(ctx, run, y), x, ctx, "attn_o_parts")
+
+    def forward_rows(self, ctx, run, y: torch.Tensor, rows, xs) -> None:
+        out = self._attended(ctx, run, y)
+        if rows is not None:
+            self.o.add_into(take_rows(ctx, out, rows, "attn_out_rows"), xs, ctx, "attn_o_parts")
+
+    def _attended(self, ctx, run, y: torch.Tensor) -> torch.Tensor:
+        """The heads' weighted sums [n, nq * d], the step's keys and values in the cache."""
         n, nq, nkv, d = y.shape[0], self.nq, self.nkv, self.d
         ws = ctx.workspace
         group = run.kv_group
@@ -144,8 +153,7 @@ class AttentionMixer(Mixer):
                 ops.rope_commit(qkv, ctx.row_pos, rotation, table, group.ring_pages, nq, nkv, d, q, pages)
             ops.attention(q, None, None, pages, table, group.ring_pages, ctx, ctx.len_after,
                           self.window, self.scale, out)
-            self.o.add_into(out.view(n, nq * d), x, ctx, "attn_o_parts")
-            return
+            return out.view(n, nq * d)
         if self.own_kv:
             tag = f"_{run.index}" if run.kv_read_later else ""
             parts = self.qkv.partial(y, ctx, "attn_qkv_parts")
@@ -197,7 +205,7 @@ class AttentionMixer(Mixer):
                     ctx.host.setdefault("deferred", []).append(commit)
                 else:
                     commit()
-        self.o.add_into(out.view(n, nq * d), x, ctx, "attn_o_parts")
+        return out.view(n, nq * d)
 
 
 register_part("mixer", "attention", AttentionMixer)

@@ -229,5 +229,17 @@ class HeadwiseAttentionMixer(ProjectedMixer):
         z += self.produce(ctx, run, y, z)
         ops.add_partials(x, z.view(1, *z.shape))
 
+    def produce_rows(self, ctx, run, y: torch.Tensor, rows, out):
+        super().produce_rows(ctx, run, y, rows, out)
+        return self.o_bias
+
+    def forward_rows(self, ctx, run, y: torch.Tensor, rows, xs) -> None:
+        if rows is None or not self.has_o_bias:
+            super().forward_rows(ctx, run, y, rows, xs)
+            return
+        z = ctx.workspace.get("hattn_z_rows", tuple(xs.shape), torch.float32)
+        z += self.produce_rows(ctx, run, y, rows, z)
+        ops.add_partials(xs, z.view(1, *z.shape))
+
 
 register_part("mixer", "headwise_attention", HeadwiseAttentionMixer)

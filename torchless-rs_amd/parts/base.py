@@ -243,6 +243,10 @@ class Mixer(Part):
         """y: normed input [n, H] (compute dtype); ADD the result to x (float32 [n, H])."""
         raise NotImplementedError
 
+    # A mixer may also offer `forward_rows(ctx, run, y, rows, xs)` and `produce_rows(ctx, run, y, rows, out) -> Optional[bias]`, asked for through
+    # `gives_rows`: everything that `forward` (`produce`) leaves for later steps, of all rows, and the result of `rows` alone (int32 [m];
+    # None: of none), added to xs [m, H] (stored in out).
+
     # A mixer may also offer `produce(ctx, run, y, out) -> Optional[bias]`: STORE the result in
     # `out` (float32 [n, H]) instead of adding it to the stream, for an arrangement that norms a
     # sublayer's output before the sum.  What it returns (float32 [H] or None) is a bias that
@@ -316,6 +320,31 @@ def rows_apart(part: "FeedForward") -> bool:
         if "forward" in vars(c) or "produce" in vars(c):
             return False
     return False
+
+
+def gives_rows(mixer: "Mixer", method: str) -> bool:
+    """Does `mixer` offer `method` (`forward_rows` or `produce_rows`)?  Not where its work was set on the object, or is that of a class derived
+    from the one that offers it."""
+    own = getattr(mixer, "__dict__", ())
+    if "forward" in own or "produce" in own:
+        return False
+    for c in type(mixer).__mro__:
+        if method in vars(c):
+            return True
+        if "forward" in vars(c) or "produce" in vars(c):
+            return False
+    return False
+
+
+def take_rows(ctx: "StepContext", t: torch.Tensor, rows: torch.Tensor, name: str) -> torch.Tensor:
+    """`rows` of t [n, W], side by side."""
+    from ..kernels import ops
+    out = ctx.workspace.get(name, (rows.shape[0], t.shape[1]), t.dtype)
+    if t.dtype == torch.float32 or (t.shape[1] % 2 == 0 and t.data_ptr() % 4 == 0):
+        ops.gather_rows(t.view(torch.float32), rows, out.view(torch.float32))       # (bfloat16 by twos)
+    else:
+        torch.index_select(t, 0, rows, out=out)
+    return out
 
 
 def rows_through_norm(ctx: "StepContext", norm: "Norm", x: torch.Tensor, rows: torch.Tensor, xs: Optional[torch.Tensor], y: torch.Tensor) -> None:

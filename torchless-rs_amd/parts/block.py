@@ -13,7 +13,7 @@ import torch
 
 from ..weights.binding import WeightSpec
 from ..kernels import ops
-from .base import (LayerSpec, Part, expect_norm, flush_pending, goes_as, make_part, part_done, read_through_norm,
+from .base import (LayerSpec, Part, expect_norm, flush_pending, gives_rows, goes_as, make_part, part_done, read_through_norm,
                    register_part, rows_apart, rows_through_norm, splittable_entry, take_row_factor)
 
 
@@ -93,15 +93,27 @@ class PreNormBlock(Part):
         ctx.host.pop("stream_copy", None)
         y = ctx.workspace.get("block_y", tuple(x.shape), ctx.dtype)
         y1 = read_through_norm(ctx, self.mixer_norm, x, y, self.mixer, run)
-        expect_norm(ctx, self.mixer, self.ffn_norm, self.ffn)
-        self.mixer.forward(ctx, run, y1, x)
-        part_done(ctx, self.mixer)
-        if rows is None:
-            ctx.pending = None
-            return None
-        m = (rows.shape[0], x.shape[1])
-        xs, ys = ctx.workspace.get("rows_x", m, torch.float32), ctx.workspace.get("rows_y", m, ctx.dtype)
-        rows_through_norm(ctx, self.ffn_norm, x, rows, xs, ys)
+        xs = None
+        if rows is not None:
+            m = (rows.shape[0], x.shape[1])
+            xs, ys = ctx.workspace.get("rows_x", m, torch.float32), ctx.workspace.get("rows_y", m, ctx.dtype)
+        if gives_rows(self.mixer, "forward_rows"):
+            if rows is not None:
+                ops.gather_rows(x, rows, xs)
+                expect_norm(ctx, self.mixer, self.ffn_norm, self.ffn)
+            self.mixer.forward_rows(ctx, run, y1, rows, xs)
+            part_done(ctx, self.mixer)
+            if rows is None:
+                return None
+            ys = read_through_norm(ctx, self.ffn_norm, xs, ys, self.ffn)
+        else:
+            expect_norm(ctx, self.mixer, self.ffn_norm, self.ffn)
+            self.mixer.forward(ctx, run, y1, x)
+            part_done(ctx, self.mixer)
+            if rows is None:
+                ctx.pending = None
+                return None
+            rows_through_norm(ctx, self.ffn_norm, x, rows, xs, ys)
         self.ffn.forward(ctx, ys, xs)
         part_done(ctx, self.ffn)
         return xs
@@ -284,16 +296,22 @@ class SandwichNormBlock(Part):
         ctx.host.pop("stream_copy", None)
         ws = ctx.workspace
         y = ws.get("block_y", tuple(x.shape), ctx.dtype)
-        z = ws.get("block_z", tuple(x.shape), torch.float32)
         y1 = read_through_norm(ctx, self.mixer_norm, x, y)
         take_row_factor(ctx, usable=False)
-        bias = OutputNormBlock._result(ctx, self.mixer, z, run, y1)
+        zs = None
+        if rows is not None:
+            m = (rows.shape[0], x.shape[1])
+            xs, zs, ys = ws.get("rows_x", m, torch.float32), ws.get("rows_z", m, torch.float32), ws.get("rows_y", m, ctx.dtype)
+            ops.gather_rows(x, rows, xs)
+        if gives_rows(self.mixer, "produce_rows"):
+            bias = self.mixer.produce_rows(ctx, run, y1, rows, zs)
+        else:
+            z = ws.get("block_z", tuple(x.shape), torch.float32)
+            bias = OutputNormBlock._result(ctx, self.mixer, z, run, y1)
+            if rows is not None:
+                ops.gather_rows(z, rows, zs)
         if rows is None:
             return None
-        m = (rows.shape[0], x.shape[1])
-        xs, zs, ys = ws.get("rows_x", m, torch.float32), ws.get("rows_z", m, torch.float32), ws.get("rows_y", m, ctx.dtype)
-        ops.gather_rows(x, rows, xs)
-        ops.gather_rows(z, rows, zs)
         self.mixer_out_norm.add_to(ctx, zs, xs, bias=bias, then=(self.ffn_norm, ys))
         y2 = read_through_norm(ctx, self.ffn_norm, xs, ys)
         take_row_factor(ctx, usable=False)

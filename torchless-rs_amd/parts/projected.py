@@ -14,7 +14,7 @@ from typing import Dict, Tuple
 import torch
 
 from ..weights.binding import WeightSpec
-from .base import Mixer, PartSpec, make_part, register_part
+from .base import Mixer, PartSpec, make_part, register_part, take_rows
 from .linear import Linear
 
 ROW_STEP = 16           # input rows are padded with zeros to a multiple of this many channels where they are made up of odd parts
@@ -75,6 +75,16 @@ class ProjectedMixer(Mixer):
     def produce(self, ctx, run, y: torch.Tensor, out: torch.Tensor):
         """The result stored in `out` (float32 [n, H]) instead of added to the stream."""
         self.o(self._result(ctx, run, y), out)
+
+    def forward_rows(self, ctx, run, y: torch.Tensor, rows, xs) -> None:
+        res = self._result(ctx, run, y)
+        if rows is not None:
+            self.o.add_into(take_rows(ctx, res, rows, self.tag + "_rows"), xs, ctx, self.tag + "_o_parts")
+
+    def produce_rows(self, ctx, run, y: torch.Tensor, rows, out):
+        res = self._result(ctx, run, y)
+        if rows is not None:
+            self.o(take_rows(ctx, res, rows, self.tag + "_rows"), out)
 
 
 class ParallelMixer(ProjectedMixer):

@@ -27,7 +27,7 @@ import torch
 from ..cache.cache import StateRequest
 from ..kernels import ops
 from ..weights.binding import WeightSpec
-from .base import Mixer, register_part
+from .base import Mixer, register_part, take_rows
 from .linear import Linear
 
 
@@ -87,6 +87,14 @@ class StateSpaceMixer(Mixer):
         self.dt_bias, self.A_log, self.D, self.norm_w = f32("dt_bias"), f32("A_log"), f32("D"), f32("norm")
 
     def forward(self, ctx, run, y: torch.Tensor, x: torch.Tensor) -> None:
+        self.o.add_into(self._gated(ctx, run, y), x, ctx, "ssm_o_parts")
+
+    def forward_rows(self, ctx, run, y: torch.Tensor, rows, xs) -> None:
+        g = self._gated(ctx, run, y)
+        if rows is not None:
+            self.o.add_into(take_rows(ctx, g, rows, "ssm_g_rows"), xs, ctx, "ssm_o_parts")
+
+    def _gated(self, ctx, run, y: torch.Tensor) -> torch.Tensor:
         n = y.shape[0]
         ws = ctx.workspace
         block = run.state                               # [slots, conv rows | states] float32
@@ -103,7 +111,7 @@ class StateSpaceMixer(Mixer):
                      block[:, self.conv_elems:], ctx.cu_seqlens, ctx.slots, yy, span=span)
         g = ws.get("ssm_g", (n, self.inner), ctx.dtype)
         ops.ssm_gate_norm(yy, proj, self.parts, self.norm_w, self.eps, g)
-        self.o.add_into(g, x, ctx, "ssm_o_parts")
+        return g
 
 
 register_part("mixer", "state_space", StateSpaceMixer)
