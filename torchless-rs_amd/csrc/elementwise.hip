@@ -357,32 +357,71 @@ template <typename T> struct Commit {
   }
 };
 
-template <typename TO>
+// A projection that may come as `n` partial sums, `stride` elements apart (`SUMS`), added in their order as add_partials_kernel adds them.
+template <bool SUMS> struct Slices {
+  int n = 1;
+  size_t stride = 0;
+  template <typename V> __device__ __forceinline__ V at(const float* p) const {
+    V a = *reinterpret_cast<const V*>(p);
+    if constexpr (SUMS) {
+#pragma unroll 4
+      for (int s = 1; s < n; ++s) a += *reinterpret_cast<const V*>(p + s * stride);
+    }
+    return a;
+  }
+  // to COUNT sums at once; the loads of AHEAD slices are under way together
+  template <int COUNT> __device__ __forceinline__ void add_rest(const float* const (&p)[COUNT], f32x4 (&a)[COUNT]) const {
+    if constexpr (SUMS) {
+      constexpr int AHEAD = 4;
+      for (int s = 1; s < n; s += AHEAD) {
+        f32x4 more[AHEAD][COUNT];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+          for (int u = 0; u < COUNT; ++u) more[j][u] = *reinterpret_cast<const f32x4*>(p[u] + min(s + j, n - 1) * stride);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+          if (s + j < n) {
+#pragma unroll
+            for (int u = 0; u < COUNT; ++u) a[u] += more[j][u];
+          }
+      }
+    }
+  }
+};
+
+template <typename TO, bool SUMS = false>
 __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, const float* __restrict__ qkv,
                                                const int* __restrict__ row_pos, Rotation rot, int nq, int nkv, int d,
                                                TO* __restrict__ q, TO* __restrict__ k, TO* __restrict__ v,
                                                TO* __restrict__ vt, int vt_cols, const int* __restrict__ row_seq,
                                                const int* __restrict__ tile_off, const int* __restrict__ n_cached,
-                                               const Commit<TO>& commit = Commit<TO>{}) {
+                                               const Commit<TO>& commit = Commit<TO>{},
+                                               const Slices<SUMS>& slices = Slices<SUMS>{}, int share = 0, int shares = 1) {
+  const int tid = threadIdx.x + blockDim.x * share, step = blockDim.x * shares;      // of the row's workgroups
   const int half = d / 2, rot_pairs = rot.rotary_dim / 2;
   const float pos = (float)row_pos[n];
   const float* src = qkv + (size_t)n * (nq + 2 * nkv) * d;
   // Whole heads in halves: four pairs a thread and turn, the first turns' loads before the angles (which they do not wait for).
   // 2,048 rows of 32 + 8 heads of 128 with their 8 heads
   // of values (75 MB), a pair a thread and turn before: 19.8 us, 13.7 now; 226 rows 7.1 and 4.2.
-  constexpr int TURNS = 3;
+  constexpr int TURNS = SUMS ? 1 : 3;
   const bool quads = rot.rotary_dim == d && !rot.interleaved && d % 8 == 0 && ((uintptr_t)qkv | (uintptr_t)q | (uintptr_t)k | (uintptr_t)commit.pages) % 16 == 0;
   const int per = half / 4, n_quads = (nq + nkv) * per;
   const auto pair_at = [&](int t) { return (t / per) * d + t % per * 4; };       // its first channel in the row
   TO* kp = commit.pages ? commit.page(row_seq[n], row_pos[n], nkv, d) + (size_t)(row_pos[n] % PAGE) * d : nullptr;
-  f32x4 a[TURNS], b[TURNS];
+  f32x4 ab[2 * TURNS];
+  const float* from[2 * TURNS];
   if (quads) {
 #pragma unroll
     for (int u = 0; u < TURNS; ++u) {
-      const int at = pair_at(min((int)(threadIdx.x + blockDim.x * u), n_quads - 1));
-      a[u] = *reinterpret_cast<const f32x4*>(src + at);
-      b[u] = *reinterpret_cast<const f32x4*>(src + at + half);
+      const int at = pair_at(min(tid + step * u, n_quads - 1));
+      from[2 * u] = src + at;
+      from[2 * u + 1] = src + at + half;
     }
+#pragma unroll
+    for (int u = 0; u < 2 * TURNS; ++u) ab[u] = *reinterpret_cast<const f32x4*>(from[u]);
+    slices.add_rest(from, ab);
   }
   for (int i = threadIdx.x; i < rot_pairs; i += blockDim.x) {     // the row's angles, once
     const float ang = rot.inv_freq[i] * pos;
@@ -412,18 +451,18 @@ __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, cons
     };
 #pragma unroll
     for (int u = 0; u < TURNS; ++u)
-      if ((int)(threadIdx.x + blockDim.x * u) < n_quads) turn(threadIdx.x + blockDim.x * u, a[u], b[u]);
-    for (int t = threadIdx.x + blockDim.x * TURNS; t < n_quads; t += blockDim.x) {
+      if (tid + step * u < n_quads) turn(tid + step * u, ab[2 * u], ab[2 * u + 1]);
+    for (int t = tid + step * TURNS; t < n_quads; t += step) {
       const int at = pair_at(t);
-      turn(t, *reinterpret_cast<const f32x4*>(src + at), *reinterpret_cast<const f32x4*>(src + at + half));
+      turn(t, slices.template at<f32x4>(src + at), slices.template at<f32x4>(src + at + half));
     }
   } else {
     const int n_rot = (nq + nkv) * half;
-    for (int t = threadIdx.x; t < n_rot; t += blockDim.x) {
+    for (int t = tid; t < n_rot; t += step) {
       const int h = t / half, i = t % half;
       int ia, ib;
       pair_channels(i, rot.rotary_dim, rot.interleaved, ia, ib);
-      const float a = src[h * d + ia], b = src[h * d + ib];
+      const float a = slices.template at<float>(src + h * d + ia), b = slices.template at<float>(src + h * d + ib);
       float ra = a, rb = b;
       if (i < rot_pairs) rotate_pair(a, b, cs[i], sn[i], ra, rb);
       TO* dst = (h < nq) ? q + ((size_t)n * nq + h) * d : k + ((size_t)n * nkv + (h - nq)) * d;
@@ -439,12 +478,12 @@ __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, cons
   const float* vs = src + (size_t)(nq + nkv) * d;
   if (v != nullptr) {
     TO* vd = v + (size_t)n * nkv * d;
-    for (int t = threadIdx.x; t < nkv * d; t += blockDim.x) vd[t] = from_f32<TO>(vs[t]);
+    for (int t = tid; t < nkv * d; t += step) vd[t] = from_f32<TO>(slices.template at<float>(vs + t));
   }
   if (vt != nullptr) {      // the same values transposed: [kv head][d][column of this row]
     const int b = row_seq[n];
     const int col = tile_off[b] + row_pos[n] - (n_cached[b] / PAGE) * PAGE;
-    for (int t = threadIdx.x; t < nkv * d; t += blockDim.x) vt[(size_t)t * vt_cols + col] = from_f32<TO>(vs[t]);
+    for (int t = tid; t < nkv * d; t += step) vt[(size_t)t * vt_cols + col] = from_f32<TO>(slices.template at<float>(vs + t));
   }
 }
 
@@ -516,12 +555,14 @@ __device__ __forceinline__ ColumnTile column_tile(int col0, int B, const int* ti
 // vt[kv head][dv][column] = v of the row at that column, from the fused projection (float):
 // the transposed values of a step, written in whole lines (a row-by-row kernel writes them
 // two bytes at a time, a line apart).  grid: (columns / 64, kv heads, d / 64 rounded up).
-template <typename TO, typename TS = float>       // TS: the type of the rows the values are read from
+template <typename TO, typename TS = float, bool SUMS = false>       // TS: the type of the rows the values are read from
 __device__ __forceinline__ void v_tile(int col_block, int kvh, int d_block, TO (*tile)[PAGE + 2],
                                        const TS* __restrict__ qkv, int width, int v_off, int d,
                                        TO* __restrict__ vt, int vt_cols, int B, const int* __restrict__ cu_seqlens,
                                        const int* __restrict__ tile_off, const int* __restrict__ n_cached,
-                                       const int* __restrict__ len_after, int nkv = 0, const Commit<TO>& commit = Commit<TO>{}) {
+                                       const int* __restrict__ len_after, int nkv = 0, const Commit<TO>& commit = Commit<TO>{},
+                                       const Slices<SUMS>& slices = Slices<SUMS>{}) {
+  static_assert(!SUMS || sizeof(TS) == 4, "partial sums are floats");
   const int col0 = col_block * PAGE;
   const ColumnTile t = column_tile(col0, B, tile_off, n_cached, len_after);
   if (t.lo >= t.hi) return;
@@ -531,11 +572,22 @@ __device__ __forceinline__ void v_tile(int col_block, int kvh, int d_block, TO (
   const TS* src = qkv + v_off + kvh * d + c0;
   if (dc == 64 && sizeof(TS) == 4 && width % 4 == 0 && (uintptr_t)src % 16 == 0) {       // four channels at a time
     f32x4 four[4];
+    const auto mine = [&](int u) { return t.p0 + (int)threadIdx.x / 16 + 16 * u; };
+    if constexpr (SUMS) {
+      const float* from[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int p = t.p0 + (int)threadIdx.x / 16 + 16 * u;
-      four[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (p >= t.lo && p < t.hi) four[u] = *reinterpret_cast<const f32x4*>(src + (size_t)(row0 + p) * width + threadIdx.x % 16 * 4);
+      for (int u = 0; u < 4; ++u) {
+        from[u] = src + (size_t)(row0 + min(max(mine(u), t.lo), t.hi - 1)) * width + threadIdx.x % 16 * 4;
+        four[u] = *reinterpret_cast<const f32x4*>(from[u]);
+      }
+      slices.add_rest(from, four);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int p = mine(u);
+        four[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (p >= t.lo && p < t.hi) four[u] = *reinterpret_cast<const f32x4*>(src + (size_t)(row0 + p) * width + threadIdx.x % 16 * 4);
+      }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -547,7 +599,11 @@ __device__ __forceinline__ void v_tile(int col_block, int kvh, int d_block, TO (
     for (int u = 0; u < 16; ++u) {
       const int idx = threadIdx.x + 256 * u;
       const int r = idx / dc, i = idx % dc, p = t.p0 + r;
-      tmp[u] = (idx < PAGE * dc && p >= t.lo && p < t.hi) ? to_f32(src[(size_t)(row0 + p) * width + i]) : 0.f;
+      const TS* at = src + (size_t)(row0 + p) * width + i;
+      if constexpr (SUMS)
+        tmp[u] = (idx < PAGE * dc && p >= t.lo && p < t.hi) ? slices.template at<float>(at) : 0.f;
+      else
+        tmp[u] = (idx < PAGE * dc && p >= t.lo && p < t.hi) ? to_f32(*at) : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
@@ -584,26 +640,30 @@ v_tiles_kernel(const TS* __restrict__ qkv, int width, int v_off, int d, TO* __re
 // pages as well, which kv_commit_tiles_kernel otherwise does behind
 // the attention (7 us a layer for 226 rows, 27 for 16,384): prompt steps of 226 rows 6,274 and 6,099 us, of 2,048 26,017 and 25,907, of 16,384
 // 260.3 and 258.1 ms.
-template <typename TO>
+// A projection in partial sums (`SUMS`) is added up on the way in, by `shares` workgroups a row, so that a thread has two groups of four
+// channels and all their slices' loads are under way at once (by one workgroup a row, two slices ahead, 226 rows in five slices took 12.8 us):
+// with add_partials_kernel before it / here, 32 + 8 + 8 heads of 128 in five slices, 20 rows 6.3 / 4.8 us, 64 7.8 / 5.5, 128 9.2 / 7.2, 226
+// (28 MB of sums) 12.0 / 9.1.
+template <typename TO, bool SUMS>
 __global__ void __launch_bounds__(256)
 rope_v_tiles_kernel(const float* __restrict__ qkv, const int* __restrict__ row_pos, Rotation rot, int n, int nq,
                     int nkv, int d, TO* __restrict__ q, TO* __restrict__ k, TO* __restrict__ vt, int vt_cols, int B,
                     const int* __restrict__ cu_seqlens, const int* __restrict__ tile_off,
                     const int* __restrict__ n_cached, const int* __restrict__ len_after, const int* __restrict__ row_seq,
-                    Commit<TO> commit) {
+                    Commit<TO> commit, Slices<SUMS> slices, int shares) {
   __shared__ __attribute__((aligned(16))) unsigned char sh[sizeof(TO) * 64 * (PAGE + 2) > 2 * sizeof(float) * ROPE_MAX_HALF
                                                             ? sizeof(TO) * 64 * (PAGE + 2)
                                                             : 2 * sizeof(float) * ROPE_MAX_HALF];
-  if ((int)blockIdx.x < n) {
+  if ((int)blockIdx.x < n * shares) {
     float* cs = reinterpret_cast<float*>(sh);
-    rope_split_row<TO>(blockIdx.x, cs, cs + ROPE_MAX_HALF, qkv, row_pos, rot, nq, nkv, d, q, k, (TO*)nullptr,
-                       (TO*)nullptr, 0, row_seq, nullptr, nullptr, commit);
+    rope_split_row<TO, SUMS>(blockIdx.x / shares, cs, cs + ROPE_MAX_HALF, qkv, row_pos, rot, nq, nkv, d, q, k, (TO*)nullptr,
+                             (TO*)nullptr, 0, row_seq, nullptr, nullptr, commit, slices, blockIdx.x % shares, shares);
     return;
   }
-  const int item = blockIdx.x - n, d_blocks = (d + 63) / 64;
+  const int item = blockIdx.x - n * shares, d_blocks = (d + 63) / 64;
   const int d_block = item % d_blocks, kvh = (item / d_blocks) % nkv, col_block = item / (d_blocks * nkv);
-  v_tile<TO>(col_block, kvh, d_block, reinterpret_cast<TO(*)[PAGE + 2]>(sh), qkv, (nq + 2 * nkv) * d, (nq + nkv) * d, d,
-             vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after, nkv, commit);
+  v_tile<TO, float, SUMS>(col_block, kvh, d_block, reinterpret_cast<TO(*)[PAGE + 2]>(sh), qkv, (nq + 2 * nkv) * d, (nq + nkv) * d, d,
+                          vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after, nkv, commit, slices);
 }
 
 // Commit of a step whose values lie transposed by tiles: the first blocks put the keys of 8 rows
@@ -1289,12 +1349,13 @@ int tl_v_tiles_rows(const void* v, int n, int nkv, int d, void* vt, int vt_cols,
 }
 
 // pages (or null): the cache, into which keys and values go at once; for steps after which every sequence fits its ring of pages
-int tl_rope_v_tiles(const float* qkv, const int* row_pos, const float* inv_freq, int rotary_dim, int interleaved,
+// n_parts >= 1: qkv is [n_parts][n][(nq + 2 nkv) d], summed on the way in
+int tl_rope_v_tiles(const float* qkv, int n_parts, const int* row_pos, const float* inv_freq, int rotary_dim, int interleaved,
                     int n, int nq, int nkv, int d, void* q, void* k, void* vt, int vt_cols, int B,
                     const int* cu_seqlens, const int* tile_off, const int* n_cached, const int* len_after, const int* row_seq,
                     const int* table, int table_stride, int ring_pages, void* pages, int dt, hipStream_t st) {
-  TL_REQUIRE(n >= 0 && nq > 0 && nkv > 0 && d > 0 && d % 2 == 0 && d <= 2 * ROPE_MAX_HALF && B > 0,
-             "rope_v_tiles: bad sizes n=%d nq=%d nkv=%d d=%d B=%d (d even, at most %d)", n, nq, nkv, d, B,
+  TL_REQUIRE(n >= 0 && nq > 0 && nkv > 0 && d > 0 && d % 2 == 0 && d <= 2 * ROPE_MAX_HALF && B > 0 && n_parts > 0,
+             "rope_v_tiles: bad sizes n=%d nq=%d nkv=%d d=%d B=%d parts=%d (d even, at most %d)", n, nq, nkv, d, B, n_parts,
              2 * ROPE_MAX_HALF);
   TL_REQUIRE(vt_cols > 0 && vt_cols % PAGE == 0, "rope_v_tiles: %d columns are no multiple of %d", vt_cols, PAGE);
   TL_REQUIRE(rotary_dim >= 0 && rotary_dim <= d && rotary_dim % 2 == 0 && (rotary_dim == 0 || inv_freq != nullptr),
@@ -1303,18 +1364,22 @@ int tl_rope_v_tiles(const float* qkv, const int* row_pos, const float* inv_freq,
   TL_REQUIRE(pages == nullptr || (row_seq && table && table_stride > 0 && ring_pages > 0), "rope_v_tiles: pages without a page table");
   if (n == 0) return 0;
   const Rotation rot{inv_freq, rotary_dim, interleaved != 0};
-  const long long blocks = (long long)n + (long long)(vt_cols / PAGE) * nkv * ((d + 63) / 64);
+  const int shares = n_parts == 1 ? 1 : (int)min(8LL, ((long long)(nq + nkv) * d / 8 + 255) / 256);
+  const long long blocks = (long long)n * shares + (long long)(vt_cols / PAGE) * nkv * ((d + 63) / 64);
   TL_REQUIRE(blocks < 2147483647LL, "rope_v_tiles: %lld workgroups are too many", blocks);
+  const auto launch = [&](auto out, auto slices) {
+    using TO = decltype(out);
+    slices.n = n_parts;
+    slices.stride = (size_t)n * (nq + 2 * nkv) * d;
+    rope_v_tiles_kernel<TO><<<(unsigned)blocks, 256, 0, st>>>(qkv, row_pos, rot, n, nq, nkv, d, (TO*)q, (TO*)k, (TO*)vt, vt_cols, B,
+                                                              cu_seqlens, tile_off, n_cached, len_after, row_seq,
+                                                              Commit<TO>{table, table_stride, ring_pages, (TO*)pages}, slices, shares);
+  };
+  TL_REQUIRE(dt == DT_F32 || dt == DT_BF16, "rope_v_tiles: unknown dtype code %d", dt);
   if (dt == DT_F32)
-    rope_v_tiles_kernel<float><<<(unsigned)blocks, 256, 0, st>>>(qkv, row_pos, rot, n, nq, nkv, d, (float*)q, (float*)k,
-                                                                  (float*)vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after,
-                                                                  row_seq, Commit<float>{table, table_stride, ring_pages, (float*)pages});
-  else if (dt == DT_BF16)
-    rope_v_tiles_kernel<bf16><<<(unsigned)blocks, 256, 0, st>>>(qkv, row_pos, rot, n, nq, nkv, d, (bf16*)q, (bf16*)k,
-                                                                 (bf16*)vt, vt_cols, B, cu_seqlens, tile_off, n_cached, len_after,
-                                                                 row_seq, Commit<bf16>{table, table_stride, ring_pages, (bf16*)pages});
+    n_parts == 1 ? launch(float{}, Slices<false>{}) : launch(float{}, Slices<true>{});
   else
-    TL_REQUIRE(false, "rope_v_tiles: unknown dtype code %d", dt);
+    n_parts == 1 ? launch(bf16{}, Slices<false>{}) : launch(bf16{}, Slices<true>{});
   TL_LAUNCH_CHECK("rope_v_tiles");
   return 0;
 }

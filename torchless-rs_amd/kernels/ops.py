@@ -324,10 +324,11 @@ def v_tiles_rows(v: torch.Tensor, vt: torch.Tensor, cu_seqlens, tile_off, n_cach
 
 def rope_v_tiles(qkv: torch.Tensor, row_pos, rotation, nq: int, nkv: int, d: int, q: torch.Tensor, k: torch.Tensor,
                  vt: torch.Tensor, cu_seqlens, tile_off, n_cached, len_after, commit=None) -> None:
-    """`rope_split` (q and k) and `v_tiles` in one launch: the same bits as the two.  `commit` (row_seq, table, ring_pages,
+    """`rope_split` (q and k) and `v_tiles` in one launch: the same bits as the two.  qkv float32 [n, (nq + 2*nkv)*d], or partial sums of
+    it [S, n, (nq + 2*nkv)*d], added up in their order as `add_partials` does.  `commit` (row_seq, table, ring_pages,
     pages): `kv_commit_tiles` with it, for steps that `overwrite_nothing`."""
-    n = qkv.shape[0]
-    _req(qkv, "rope_v_tiles.qkv", torch.float32, (n, (nq + 2 * nkv) * d))
+    n_parts, n = (qkv.shape[0] if qkv.dim() == 3 else 1), qkv.shape[-2]
+    _req(qkv, "rope_v_tiles.qkv", torch.float32, (n_parts,) * (qkv.dim() == 3) + (n, (nq + 2 * nkv) * d))
     _req(row_pos, "rope_v_tiles.row_pos", torch.int32, (n,))
     rot = _rotation(rotation, d, "rope_v_tiles")
     _req(q, "rope_v_tiles.q", None, (n, nq, d))
@@ -348,7 +349,7 @@ def rope_v_tiles(qkv: torch.Tensor, row_pos, rotation, nq: int, nkv: int, d: int
             raise KernelError(f"rope_v_tiles.pages: shape {tuple(pages.shape)}, kernel needs [*, 2, {nkv}, {PAGE}, {d}]")
         if table.dim() != 2 or table.shape[0] != B:
             raise KernelError("rope_v_tiles.table: needs one row per sequence")
-    _check(lib().tl_rope_v_tiles(_p(qkv), _p(row_pos), _p(rot.inv_freq), rot.rotary_dim, int(rot.interleaved), n, nq,
+    _check(lib().tl_rope_v_tiles(_p(qkv), n_parts, _p(row_pos), _p(rot.inv_freq), rot.rotary_dim, int(rot.interleaved), n, nq,
                                  nkv, d, _p(q), _p(k), _p(vt), vt.shape[2], B, _p(cu_seqlens), _p(tile_off),
                                  _p(n_cached), _p(len_after), _p(row_seq), _p(table), table.shape[1] if commit else 0, ring_pages, _p(pages),
                                  _code(q.dtype), _stream()))

@@ -156,15 +156,17 @@ class AttentionMixer(Mixer):
             return out.view(n, nq * d)
         if self.own_kv:
             tag = f"_{run.index}" if run.kv_read_later else ""
-            parts = self.qkv.partial(y, ctx, "attn_qkv_parts")
-            if parts is not None:               # K cut into partial sums: the first slice takes the others
-                qkv = parts[0]
-                ops.add_partials(qkv, parts[1:])
+            tiles = ops.uses_transposed_values(ctx.dtype, d, ctx.all_single)
+            parts = (self.qkv.rotated_partial if tiles else self.qkv.partial)(y, ctx, "attn_qkv_parts")
+            if parts is not None:               # K cut into partial sums: the rotation adds them up, or the first slice takes the others
+                qkv = parts if tiles else parts[0]
+                if not tiles:
+                    ops.add_partials(qkv, parts[1:])
             else:
                 qkv = ws.get("attn_qkv", (n, (nq + 2 * nkv) * d), torch.float32)
                 self.qkv(y, qkv)
             k = ws.get("attn_k" + tag, (n, nkv, d), ctx.dtype)
-            if ops.uses_transposed_values(ctx.dtype, d, ctx.all_single):
+            if tiles:
                 # the matrix cores read values along the keys: only the transposed copy is made, by tiles
                 v = None
                 vt = ws.get("attn_vt" + tag, (nkv, d, ctx.host["aligned_cols"]), ctx.dtype)

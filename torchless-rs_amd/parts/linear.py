@@ -81,8 +81,7 @@ class Linear:
 
     def wide_partial(self, a: torch.Tensor, ctx, name: str):
         """The same for MID_ROWS + 1..WIDE_ROWS rows, where the sums go to the stream: whoever reads it next adds them, a norm as it
-        reads or a pass of its own.  (q|k|v of a prompt would need such a pass: 24 + 6 us for 226 rows of 6,144 x 4,096, the
-        library's 26.)  This rule comes before `tall_partial`'s: it asks for no norm, and takes 144 to 256 rows of wide outputs and short K
+        reads or a pass of its own; and where the rotation of a prompt's q|k|v adds them.  This rule comes before `tall_partial`'s: it asks for no norm, and takes 144 to 256 rows of wide outputs and short K
         that the other, which reckons times, leaves to the library (8,192 x 4,096 at 256 rows 36 us in four slices, 48 there)."""
         M, N, K = a.shape[0], self.out_features, self.in_features
         if not (ops.MID_ROWS < M <= ops.WIDE_ROWS and ops.bf16_gemm_ok(a, self.weight)):
@@ -92,6 +91,21 @@ class Linear:
             return None
         parts = ctx.workspace.get(name, (S, M, N), torch.float32)
         ops.gemm_wide_bf16(a, self.weight, parts, S)
+        return parts
+
+    def rotated_partial(self, a: torch.Tensor, ctx, name: str):
+        """`partial`, or `wide_partial` where the rotation of a prompt's q|k|v (`ops.rope_v_tiles`) adds the sums up sooner than the library
+        stores the product: K of 4,096 and more in 8 slices at most.  Product and rotation, weights from memory, in slices / by the
+        library, microseconds: 6,144 x 4,096 at 130, 192, 226 and 255 rows 28.5 / 32.2, 30.0 / 39.6, 31.1 / 32.8 and 32.1 / 33.7; 6,144 x 5,120
+        31.8 / 38.0 to 37.4 / 40.6; 8,192 x 4,096 30.7 / 32.2 to 37.4 / 37.8; 10,240 x 8,192 49 / 65 to 67 / 96; 4,096 x 4,096 at 130 to
+        192 rows 25.7 / 26.8 to 27.1 / 38.2; not taken: 6,144 x 3,072 26.7 / 26.2 to 30.3 / 27.7, 3,072 x 4,096 in 10 26.1 / 19.9.
+        Against 64 bits the sum of slices is off by 1.7e-7 of its norm where the library's product is by 4.0e-7 (K 4,096)."""
+        from .base import goes_as
+        parts = self.partial(a, ctx, name)
+        M, N, K = a.shape[0], self.out_features, self.in_features
+        if (parts is None and M > ops.MID_ROWS and K >= 4096 and goes_as(self, Linear, "__call__")
+                and ops.wide_splits(M, N, K, ops.compute_units(a.device)) <= 8):
+            parts = self.wide_partial(a, ctx, name)
         return parts
 
     def tall_partial(self, a: torch.Tensor, ctx, name: str):
