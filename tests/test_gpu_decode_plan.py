@@ -314,3 +314,15 @@ def test_parts_merged_by_the_last_of_them_have_the_bits_of_a_merge_of_its_own(op
         met.zero_()
         ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, met, arrived)
         assert torch.equal(met, apart) and int(arrived.abs().max()) == 0
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("splits", [9, 16, 20, 36])
+def test_merged_parts_have_those_bits_where_they_come_in_more_than_one_trip(ops, d, splits):
+    """Many channels: a sum that one of the two ways rounds elsewhere changes a bfloat16 in some hundred thousand."""
+    q, pages, table, ctx = step(ops, [2200 + i for i in range(64)], 64, 8, d, seed=splits)
+    part = torch.full((64 * 64 * splits * (d + 2),), float("nan"), device=DEV)
+    apart, met = torch.zeros_like(q), torch.zeros_like(q)
+    ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, apart)
+    ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, met, ops.decode_counters(ctx, 64, 64, 8))
+    assert torch.equal(met, apart)

@@ -919,6 +919,28 @@ attn_decode_order_kernel(const int* __restrict__ row_pos, int B, int window, int
 __device__ __forceinline__ void shared_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float shared_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+// The next MERGED parts of a head (maxima, sums of weights, weighted sums of N channels) into those so far.  Which product of a sum is
+// rounded by itself is written out: left to the compiler it went one way in one kernel and the other in another.
+constexpr int MERGED = 8;
+template <int N>
+__device__ __forceinline__ void merge_parts(const float (&ms)[MERGED], const float (&ls)[MERGED], const float (&vs)[MERGED][N], float& mm,
+                                            float& ll, float (&acc)[N]) {
+#pragma clang fp contract(off)
+  float mc = mm;
+#pragma unroll
+  for (int c = 0; c < MERGED; ++c) mc = fmaxf(mc, ms[c]);
+  if (mc == -INFINITY) return;                         // nothing visible so far
+  const float keep = (mm == -INFINITY) ? 0.f : __expf(mm - mc);
+#pragma unroll
+  for (int c = 0; c < MERGED; ++c) {
+    const float f = (ms[c] == -INFINITY) ? 0.f : __expf(ms[c] - mc);
+    ll = c == 0 ? __builtin_fmaf(ll, keep, ls[c] * f) : __builtin_fmaf(ls[c], f, ll);
+#pragma unroll
+    for (int v = 0; v < N; ++v) acc[v] = c == 0 ? __builtin_fmaf(acc[v], keep, vs[c][v] * f) : __builtin_fmaf(vs[c][v], f, acc[v]);
+  }
+  mm = mc;
+}
+
 template <int D, int NS, bool TERMS = false, bool LOGI = false>
 __global__ void __launch_bounds__(DC_WAVES * 64)
 attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pages,
@@ -1174,36 +1196,19 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
     float acc[PER], ll = 0.f, mm = -INFINITY;
 #pragma unroll
     for (int i = 0; i < PER; ++i) acc[i] = 0.f;
-    constexpr int CH = 8;
-    for (int s0 = 0; s0 < mine.y; s0 += CH) {
-      float ms[CH], ls[CH], vs[CH][PER];
+    for (int s0 = 0; s0 < mine.y; s0 += MERGED) {
+      float ms[MERGED], ls[MERGED], vs[MERGED][PER];
 #pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const float* p = src + (size_t)min(s0 + c, mine.y - 1) * stride;
+      for (int c = 0; c < MERGED; ++c) {
+        const bool ok = s0 + c < mine.y;
+        const float* p = src + (size_t)(ok ? s0 + c : s0) * stride;
         ms[c] = shared_load(p);
         ls[c] = shared_load(p + 1);
 #pragma unroll
         for (int i = 0; i < PER; ++i) vs[c][i] = shared_load(p + 2 + lane + WAVE * i);
+        if (!ok) ms[c] = -INFINITY;
       }
-      float mc = mm;
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        if (s0 + c >= mine.y) ms[c] = -INFINITY;
-        mc = fmaxf(mc, ms[c]);
-      }
-      if (mc == -INFINITY) continue;                   // nothing visible so far
-      const float keep = (mm == -INFINITY) ? 0.f : __expf(mm - mc);
-      ll *= keep;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) acc[i] *= keep;
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const float f = (ms[c] == -INFINITY) ? 0.f : __expf(ms[c] - mc);
-        ll += ls[c] * f;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) acc[i] += vs[c][i] * f;
-      }
-      mm = mc;
+      merge_parts(ms, ls, vs, mm, ll, acc);
     }
     float gt = 1.f;
     if constexpr (TERMS)
@@ -1222,7 +1227,7 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
 __global__ void __launch_bounds__(64)
 attn_decode_combine_kernel(const float* __restrict__ part, int n_splits, int d, bf16* __restrict__ out,
                            const float* __restrict__ gate = nullptr, const int2* __restrict__ seqs = nullptr, int nq = 1) {
-  constexpr int CH = 8, MAXV = 4;                      // d <= 256: at most 4 elements a lane
+  constexpr int MAXV = 4;                      // d <= 256: at most 4 elements a lane
   const size_t bh = blockIdx.x;
   const float* src = part + bh * n_splits * (d + 2);
   const int lane = threadIdx.x;
@@ -1237,10 +1242,10 @@ attn_decode_combine_kernel(const float* __restrict__ part, int n_splits, int d, 
   float mm = -INFINITY, ll = 0.f, acc[MAXV];
 #pragma unroll
   for (int v = 0; v < MAXV; ++v) acc[v] = 0.f;
-  for (int s0 = 0; s0 < n_splits; s0 += CH) {
-    float ms[CH], ls[CH], vs[CH][MAXV];
+  for (int s0 = 0; s0 < n_splits; s0 += MERGED) {
+    float ms[MERGED], ls[MERGED], vs[MERGED][MAXV];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
+    for (int c = 0; c < MERGED; ++c) {
       const bool ok = s0 + c < n_splits;
       const float* p = src + (size_t)(ok ? s0 + c : s0) * stride;
       ms[c] = ok ? p[0] : -INFINITY;
@@ -1248,22 +1253,7 @@ attn_decode_combine_kernel(const float* __restrict__ part, int n_splits, int d, 
 #pragma unroll
       for (int v = 0; v < MAXV; ++v) vs[c][v] = (lane + 64 * v < d) ? p[2 + lane + 64 * v] : 0.f;
     }
-    float mc = mm;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) mc = fmaxf(mc, ms[c]);
-    if (mc == -INFINITY) continue;                     // nothing visible so far
-    const float keep = (mm == -INFINITY) ? 0.f : __expf(mm - mc);
-    ll *= keep;
-#pragma unroll
-    for (int v = 0; v < MAXV; ++v) acc[v] *= keep;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const float f = (ms[c] == -INFINITY) ? 0.f : __expf(ms[c] - mc);
-      ll += ls[c] * f;
-#pragma unroll
-      for (int v = 0; v < MAXV; ++v) acc[v] += vs[c][v] * f;
-    }
-    mm = mc;
+    merge_parts(ms, ls, vs, mm, ll, acc);
   }
   const float gt = gate != nullptr ? gate[bh] : 1.f;       // a factor on the head's output (or none)
 #pragma unroll
