@@ -326,3 +326,24 @@ def test_merged_parts_have_those_bits_where_they_come_in_more_than_one_trip(ops,
     ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, apart)
     ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, splits, part, met, ops.decode_counters(ctx, 64, 64, 8))
     assert torch.equal(met, apart)
+
+
+def test_too_few_counters_are_refused(ops, monkeypatch):
+    """By every way in, before anything is launched."""
+    lengths = [900, 1400]
+    q, pages, table, ctx = step(ops, lengths, 40, 2, 64)         # 20 heads a group: two times 16
+    need = ops.decode_counters(ctx, 2, 40, 2).numel()
+    assert need == 2 * 2 * 2 * 4
+    out, part = torch.zeros_like(q), torch.zeros(2 * 40 * 4 * 66, device=DEV)
+    short = torch.zeros(need - 1, dtype=torch.int32, device=DEV)
+    plan = ops.decode_plan(ctx, 40, 2, 64, table.shape[1], None)
+    assert plan is not None and plan[1] is not None
+    terms = ops.ScoreTerms(0.125, sinks=torch.zeros(40, device=DEV))
+    monkeypatch.setattr(ops, "decode_counters", lambda *a: short)
+    for call in (lambda: ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, 4, part, out, short),
+                 lambda: ops.attn_decode_planned(q, pages, table, table.shape[1], ctx, plan, None, 0.1, out),
+                 lambda: ops.attn_decode_planned(q, pages, table, table.shape[1], ctx, plan, None, 0.1, out, terms=terms),
+                 lambda: ops.attention_scored(q, None, None, pages, 2, 64, table, table.shape[1], ctx, None, terms, None, out)):
+        with pytest.raises(ops.KernelError, match="counters"):
+            call()
+    assert not bool(out.any()) and not bool(short.any())

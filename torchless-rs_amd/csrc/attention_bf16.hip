@@ -1376,14 +1376,18 @@ constexpr int DR_MAX_PAGES = 2048;      // most pages of a sequence that the ker
 // single-token steps with more terms on the scores; LOGI: logistic weights
 // a step's parts as attn_decode_plan_kernel made them (null: n_splits for every sequence), over `places` places; without `seqs` every
 // sequence is one part and there is nothing to merge
-// arrived: DC_WAVES counters for each sequence, KV head and 16 heads of its group, all zero, which the kernel leaves at zero: the parts are then
-// merged by the last of them and not by a launch of their own.
+// arrived: counters (`counters_of`), all zero, which the kernel leaves at zero: the parts are then merged by the last of them and not by a
+// launch of their own.
 struct DecodePlan {
   const int4* plan = nullptr;
   const int2* seqs = nullptr;
   int places = 0;
   int* arrived = nullptr;
+  long n_arrived = 0;
 };
+
+// Of every wave of a workgroup one, for each sequence, KV head and 16 heads of its group
+static long counters_of(int B, int nq, int nkv) { return (long)B * nkv * ((nq / nkv + 15) / 16) * DC_WAVES; }
 
 template <int DPAD, bool LOGI>
 static int launch_decode_terms(const bf16* q, const bf16* pages, const int* table, int table_stride,
@@ -1639,6 +1643,8 @@ static int attn_decode_entry(const void* q, const void* pages, const int* table,
   TL_REQUIRE(ring_pages > 0 && table_stride > 0 && window >= 0 && n_splits > 0 && n_splits <= 4096,
              "attn_decode: bad geometry ring_pages=%d table_stride=%d window=%d splits=%d", ring_pages,
              table_stride, window, n_splits);
+  TL_REQUIRE(plan.arrived == nullptr || plan.n_arrived >= counters_of(B, nq, nkv), "attn_decode: %ld counters, needs %ld", plan.n_arrived,
+             counters_of(B, nq, nkv));
   TL_BY_DPAD(launch_decode, (const bf16*)q, (const bf16*)pages, table, table_stride, ring_pages, row_pos,
              B, nq, nkv, d, window, scale, n_splits, part, (bf16*)out, st, terms, plan);
   return 1;
@@ -1652,13 +1658,19 @@ extern "C" int tl_attn_decode_bf16(const void* q, const void* pages, const int* 
                            part, out, st, nullptr);
 }
 
-// The same, whose parts the last of them merges where the kernel through LDS serves the head size.  arrived: as `DecodePlan` has it.
+// How many counters such a step needs
+extern "C" long tl_attn_decode_counters(int B, int nq, int nkv) {
+  return B > 0 && nq > 0 && nkv > 0 && nq % nkv == 0 ? counters_of(B, nq, nkv) : 0;
+}
+
+// The same, whose parts the last of them merges where the kernel through LDS serves the head size.  arrived: n_arrived counters (`DecodePlan`).
 extern "C" int tl_attn_decode_met_bf16(const void* q, const void* pages, const int* table, int table_stride,
                                        int ring_pages, const int* row_pos, int B, int nq, int nkv, int d,
-                                       int window, float scale, int n_splits, float* part, int* arrived, void* out,
+                                       int window, float scale, int n_splits, float* part, int* arrived, long n_arrived, void* out,
                                        hipStream_t st) {
   DecodePlan met;
   met.arrived = arrived;
+  met.n_arrived = n_arrived;
   return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, n_splits,
                            part, out, st, nullptr, met);
 }
@@ -1667,7 +1679,7 @@ extern "C" int tl_attn_decode_met_bf16(const void* q, const void* pages, const i
 extern "C" int tl_attn_decode_terms_bf16(const void* q, const void* pages, const int* table, int table_stride,
                                          int ring_pages, const int* row_pos, int B, int nq, int nkv, int d,
                                          int window, int keep_first, int chunk, float scale, int n_splits, float* part, int* arrived,
-                                         const float* slopes, const float* sinks, const float* gate, int logistic,
+                                         long n_arrived, const float* slopes, const float* sinks, const float* gate, int logistic,
                                          const float* score_bias, void* out, hipStream_t st) {
   TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || window == 0 || (long long)ring_pages * PAGE >= (1LL << 24)),
              "attn_decode: first positions that stay visible beside a window need a cache that keeps every position");
@@ -1676,6 +1688,7 @@ extern "C" int tl_attn_decode_terms_bf16(const void* q, const void* pages, const
   const MoreTerms terms{slopes, sinks, gate, window > 0 ? keep_first : 0, chunk, logistic, score_bias};
   DecodePlan met;
   met.arrived = arrived;
+  met.n_arrived = n_arrived;
   return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, n_splits,
                            part, out, st, &terms, met);
 }
@@ -1716,12 +1729,12 @@ extern "C" int tl_attn_decode_planned_bf16(const void* q, const void* pages, con
                                            const int* row_pos, int B, int nq, int nkv, int d, int window, float scale, const int* plan,
                                            const int* seqs, int places, int more, int keep_first, int chunk, const float* slopes,
                                            const float* sinks, const float* gate, int logistic, const float* score_bias, float* part,
-                                           int* arrived, void* out, hipStream_t st) {
+                                           int* arrived, long n_arrived, void* out, hipStream_t st) {
   TL_REQUIRE(tl_attn_decode_takes_plan(d, table_stride), "attn_decode_planned: heads of %d with %d pages go without a plan", d, table_stride);
   TL_REQUIRE(plan && (part || !seqs) && (seqs ? places >= B : places == B) && (uintptr_t)plan % 16 == 0 && (uintptr_t)seqs % 8 == 0 &&
              nq > 0 && nkv > 0 && (long)places * nkv * ((nq / nkv + 15) / 16) * DC_WAVES * 64 < (1l << 31),
              "attn_decode_planned: %d places for %d sequences", places, B);
-  const DecodePlan dp{(const int4*)plan, (const int2*)seqs, places, arrived};
+  const DecodePlan dp{(const int4*)plan, (const int2*)seqs, places, arrived, n_arrived};
   if (!more) return attn_decode_entry(q, pages, table, table_stride, ring_pages, row_pos, B, nq, nkv, d, window, scale, 1, part, out, st, nullptr, dp);
   TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || window == 0 || (long long)ring_pages * PAGE >= (1LL << 24)),
              "attn_decode: first positions that stay visible beside a window need a cache that keeps every position");

@@ -35,6 +35,7 @@ def lib() -> ctypes.CDLL:
     if not _configured:
         L.tl_last_error.restype = ctypes.c_char_p
         L.tl_gemm_plain_parts.restype = ctypes.c_longlong
+        L.tl_attn_decode_counters.restype = ctypes.c_long
         require_same(L.tl_page_size(), "the kernels' library")
         _configured = True
     return L
@@ -703,7 +704,7 @@ def attention_scored(q, k_new, v_new, pages, nkv: int, dv: int, table, ring_page
         arrived = decode_counters(ctx, n, nq, nkv) if splits > 1 else None
         _check(lib().tl_attn_decode_terms_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(ctx.row_pos),
                                                n, nq, nkv, dk, int(terms.window or 0), int(terms.keep_first or 0),
-                                               terms.chunk, ctypes.c_float(terms.scale), int(splits), _p(part), _p(arrived), slopes, sinks,
+                                               terms.chunk, ctypes.c_float(terms.scale), int(splits), _p(part), *_counters_args(arrived), slopes, sinks,
                                                gt, int(terms.logistic), _p(terms.score_bias), _p(out), _stream()))
     elif fast and k_new is not None and vt_new is not None:
         B = n_cached.shape[0]
@@ -2689,10 +2690,9 @@ def attn_decode_bf16(q, pages, table, ring_pages: int, row_pos, window: Optional
     nkv = pages.shape[2]
     _decode_args(q, pages, table, row_pos, part, out, n_splits)
     if arrived is not None:
-        _req(arrived, "attn.arrived", torch.int32, (DECODE_WAVES * decode_groups(B, nq, nkv),))
         _check(lib().tl_attn_decode_met_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(row_pos),
                                              B, nq, nkv, d, int(window or 0), ctypes.c_float(scale),
-                                             int(n_splits), _p(part), _p(arrived), _p(out), _stream()))
+                                             int(n_splits), _p(part), *_counters_args(arrived), _p(out), _stream()))
         return
     _check(lib().tl_attn_decode_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(row_pos),
                                      B, nq, nkv, d, int(window or 0), ctypes.c_float(scale),
@@ -2712,12 +2712,16 @@ def decode_groups(B: int, nq: int, nkv: int) -> int:
     return B * nkv * (-(-(nq // nkv) // 16))
 
 
-DECODE_WAVES = 4            # waves of a workgroup of the decode attention
-
-
 def decode_counters(ctx, B: int, nq: int, nkv: int) -> torch.Tensor:
     """The counters by which the parts of a decode step's attention find the last of them, which merges them: zero between launches."""
-    return ctx.workspace.get("attn_arrived", (DECODE_WAVES * decode_groups(B, nq, nkv),), torch.int32, zero=True)
+    return ctx.workspace.get("attn_arrived", (lib().tl_attn_decode_counters(B, nq, nkv),), torch.int32, zero=True)
+
+
+def _counters_args(arrived: Optional[torch.Tensor]):
+    """`arrived` and how many there are, as the entry points take them (they refuse too few)."""
+    if arrived is not None:
+        _req(arrived, "attn.arrived", torch.int32)
+    return _p(arrived), ctypes.c_long(arrived.numel() if arrived is not None else 0)
 
 
 SPLIT_PAGES = 4             # fewest pages a part of the keys has
@@ -2838,7 +2842,8 @@ def attn_decode_planned(q, pages, table, ring_pages: int, ctx, plan, window: Opt
     _check(lib().tl_attn_decode_planned_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(ctx.row_pos), B, nq, nkv, d,
                                              int(window or 0), ctypes.c_float(scale), _p(places), _p(seqs), places.shape[0], *more, slopes,
                                              sinks, gt, int(terms.logistic) if terms is not None else 0,
-                                             _p(terms.score_bias) if terms is not None else None, _p(part), _p(arrived), _p(out), _stream()))
+                                             _p(terms.score_bias) if terms is not None else None, _p(part), *_counters_args(arrived), _p(out),
+                                             _stream()))
 
 
 def uses_transposed_values(dtype: torch.dtype, d: int, all_single: bool) -> bool:
