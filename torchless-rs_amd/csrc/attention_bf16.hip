@@ -914,8 +914,11 @@ attn_decode_order_kernel(const int* __restrict__ row_pos, int B, int window, int
 }
 
 // Numbers that workgroups of one launch leave for each other go past the XCDs' own caches in both directions (agent scope), so that
-// a counter behind them is all the order they need: a device-wide fence, which writes back and invalidates an L2, took a step of 32
-// layers at batch 8 from 4.0 to 4.7 ms.
+// a counter between them needs no fence of the whole device, which writes back and invalidates an L2 (it took a step of 32 layers at
+// batch 8 from 4.0 to 4.7 ms).  The order around the counter is the wave's own, not the language's: the writer waits until vmcnt is
+// zero, which on gfx950 counts stores as well and for these stores means that they are past the L2 (an architecture with a count of
+// its own for stores needs another wait), and a reader's loads are not issued before the counter's value is there, for
+// a wave issues in order and the compiler is kept from moving them up.
 __device__ __forceinline__ void shared_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float shared_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
@@ -1187,6 +1190,7 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
   int before = 0;
   if (lane == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (__builtin_amdgcn_readfirstlane(before) != mine.y - 1) return;
+  asm volatile("" ::: "memory");                      // no load of the others' results above the counter
   if (lane == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // for the next launch
   const size_t stride = (size_t)(D + 2) * (plan != nullptr ? nq : 1);
   for (int hd = wave; hd < heads; hd += DC_WAVES) {
