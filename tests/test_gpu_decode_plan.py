@@ -333,7 +333,7 @@ def test_too_few_counters_are_refused(ops, monkeypatch):
     lengths = [900, 1400]
     q, pages, table, ctx = step(ops, lengths, 40, 2, 64)         # 20 heads a group: two times 16
     need = ops.decode_counters(ctx, 2, 40, 2).numel()
-    assert need == 2 * 2 * 2 * 4
+    assert need >= 2 * 2 * 2 * 4
     out, part = torch.zeros_like(q), torch.zeros(2 * 40 * 4 * 66, device=DEV)
     short = torch.zeros(need - 1, dtype=torch.int32, device=DEV)
     plan = ops.decode_plan(ctx, 40, 2, 64, table.shape[1], None)

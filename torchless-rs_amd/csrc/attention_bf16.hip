@@ -944,6 +944,11 @@ __device__ __forceinline__ void merge_parts(const float (&ms)[MERGED], const flo
   mm = mc;
 }
 
+// A counter has a line of memory to itself: side by side (a step's 32 of 8 KV heads in one line) they were taken one after the other, and
+// one sequence of 32 over 8 heads of 128 over 8,000 keys in 32 parts took 18.8 us, 14.5 now (16.9 with the launch), 16,000 keys
+// 25.4 and 21.6 (24.7); two sequences of 4,000 17.1 and 13.6 (15.3).
+constexpr int COUNTER_INTS = 32;
+
 template <int D, int NS, bool TERMS = false, bool LOGI = false>
 __global__ void __launch_bounds__(DC_WAVES * 64)
 attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pages,
@@ -1181,11 +1186,11 @@ attn_decode_ring_kernel(const bf16* __restrict__ q, const bf16* __restrict__ pag
   }
   if (arrived == nullptr || alone || wave >= heads) return;
   // Of the parts' waves with these heads the last to get here merges them, as attn_decode_combine_kernel does (the same bits).
-  // Nobody waits for anybody.  What bounds it is three trips past the L2s one after the other (stores, counter, loads), 3 us in place of
-  // a launch of 4.6: a step of 32 layers 2,913 and 2,888 us at batch 1 (1,024 keys), 3,600 and 3,588 to 3,565 at batch 8 (4,096 keys).
+  // Nobody waits for anybody.  What bounds it is three trips past the L2s one after the other (stores, counter, loads) and, for eight
+  // parts and each head of the wave more, one trip more.  For whom it pays: `meeting_counters` of kernels/ops.py.
   // A counter a workgroup, with its barriers and a thread's channels one after the other: no gain.
   const int2 mine = plan != nullptr ? seqs[b] : make_int2(0, n_splits);
-  int* count = arrived + (((size_t)b * nkv + kvh) * head_groups + hg) * DC_WAVES + wave;
+  int* count = arrived + ((((size_t)b * nkv + kvh) * head_groups + hg) * DC_WAVES + wave) * COUNTER_INTS;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's results are where every XCD sees them
   int before = 0;
   if (lane == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1391,7 +1396,7 @@ struct DecodePlan {
 };
 
 // Of every wave of a workgroup one, for each sequence, KV head and 16 heads of its group
-static long counters_of(int B, int nq, int nkv) { return (long)B * nkv * ((nq / nkv + 15) / 16) * DC_WAVES; }
+static long counters_of(int B, int nq, int nkv) { return (long)B * nkv * ((nq / nkv + 15) / 16) * DC_WAVES * COUNTER_INTS; }
 
 template <int DPAD, bool LOGI>
 static int launch_decode_terms(const bf16* q, const bf16* pages, const int* table, int table_stride,
