@@ -335,15 +335,32 @@ def test_too_few_counters_are_refused(ops, monkeypatch):
     need = ops.decode_counters(ctx, 2, 40, 2).numel()
     assert need >= 2 * 2 * 2 * 4
     out, part = torch.zeros_like(q), torch.zeros(2 * 40 * 4 * 66, device=DEV)
-    short = torch.zeros(need - 1, dtype=torch.int32, device=DEV)
-    plan = ops.decode_plan(ctx, 40, 2, 64, table.shape[1], None)
+    with pytest.raises(ops.KernelError, match="counters"):
+        ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, 4, part, out,
+                             torch.zeros(need - 1, dtype=torch.int32, device=DEV))
+    q, pages, table, ctx = step(ops, lengths, 8, 2, 64)
+    short = torch.zeros(ops.decode_counters(ctx, 2, 8, 2).numel() - 1, dtype=torch.int32, device=DEV)
+    out = torch.zeros_like(q)
+    plan = ops.decode_plan(ctx, 8, 2, 64, table.shape[1], None)
     assert plan is not None and plan[1] is not None
-    terms = ops.ScoreTerms(0.125, sinks=torch.zeros(40, device=DEV))
+    terms = ops.ScoreTerms(0.125, sinks=torch.zeros(8, device=DEV))
     monkeypatch.setattr(ops, "decode_counters", lambda *a: short)
-    for call in (lambda: ops.attn_decode_bf16(q, pages, table, table.shape[1], ctx.row_pos, None, 0.1, 4, part, out, short),
-                 lambda: ops.attn_decode_planned(q, pages, table, table.shape[1], ctx, plan, None, 0.1, out),
+    for call in (lambda: ops.attn_decode_planned(q, pages, table, table.shape[1], ctx, plan, None, 0.1, out),
                  lambda: ops.attn_decode_planned(q, pages, table, table.shape[1], ctx, plan, None, 0.1, out, terms=terms),
                  lambda: ops.attention_scored(q, None, None, pages, 2, 64, table, table.shape[1], ctx, None, terms, None, out)):
         with pytest.raises(ops.KernelError, match="counters"):
             call()
     assert not bool(out.any()) and not bool(short.any())
+
+
+@pytest.mark.parametrize("nq,nkv,meet", [(8, 8, True), (8, 2, True), (10, 2, False), (32, 2, False)])
+def test_parts_meet_where_a_wave_has_one_head(ops, monkeypatch, nq, nkv, meet):
+    real, asked = ops.decode_counters, []
+    monkeypatch.setattr(ops, "decode_counters", lambda *a: (asked.append(a[1:]), real(*a))[1])
+    for lengths in ([1400], [900, 1400]):            # uniform parts, and planned ones
+        q, pages, table, ctx = step(ops, lengths, nq, nkv, 64)
+        out = torch.zeros_like(q)
+        ops.attention(q, None, None, pages, table, table.shape[1], ctx, None, None, 0.1, out)
+        ops.attention_scored(q, None, None, pages, nkv, 64, table, table.shape[1], ctx, None, ops.ScoreTerms(0.1), None, out)
+        assert asked == [(len(lengths), nq, nkv)] * (2 * meet)
+        asked.clear()
