@@ -62,7 +62,7 @@ def test_which_steps_overwrite_nothing():
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("S", [2, 3, 5, 16])
-@pytest.mark.parametrize("nq,nkv,d,rotary,odd", [(4, 2, 16, 16, 0), (6, 3, 80, 40, 0), (40, 8, 256, 256, 0), (32, 8, 128, 128, 0), (4, 2, 128, 128, 1), (3, 1, 66, 66, 0)])
+@pytest.mark.parametrize("nq,nkv,d,rotary,odd", [(4, 2, 16, 16, 0), (6, 3, 80, 40, 0), (40, 8, 256, 256, 0), (32, 8, 128, 128, 0), (4, 2, 128, 128, 1), (3, 1, 66, 66, 0), (1, 1, 2, 2, 0), (2, 1, 2, 0, 0)])
 def test_partial_sums_are_added_with_the_rotation(dt, S, nq, nkv, d, rotary, odd):
     """Partial sums of q|k|v against `add_partials` and the rotation of their sum, bit by bit; buffers off 16 bytes (`odd`)."""
     from torchless_rs_amd.kernels import ops

@@ -1364,7 +1364,7 @@ int tl_rope_v_tiles(const float* qkv, int n_parts, const int* row_pos, const flo
   TL_REQUIRE(pages == nullptr || (row_seq && table && table_stride > 0 && ring_pages > 0), "rope_v_tiles: pages without a page table");
   if (n == 0) return 0;
   const Rotation rot{inv_freq, rotary_dim, interleaved != 0};
-  const int shares = n_parts == 1 ? 1 : (int)min(8LL, ((long long)(nq + nkv) * d / 8 + 255) / 256);
+  const int shares = n_parts == 1 ? 1 : (int)min(8LL, ((long long)(nq + nkv) * d + 2047) / 2048);     // (at least one)
   const long long blocks = (long long)n * shares + (long long)(vt_cols / PAGE) * nkv * ((d + 63) / 64);
   TL_REQUIRE(blocks < 2147483647LL, "rope_v_tiles: %lld workgroups are too many", blocks);
   const auto launch = [&](auto out, auto slices) {
