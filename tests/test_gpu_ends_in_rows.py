@@ -94,6 +94,52 @@ def test_who_gives_rows():
     assert not gives_rows(mk(Other), "forward_rows") and not gives_rows(mk(RetentionMixer), "forward_rows") and not gives_rows(mk(Mixer), "forward_rows")
 
 
+@pytest.mark.parametrize("name,what", [("A", "hidden"), ("A", "hidden on the object"), ("A", "down"), ("A", "add_into on the product"), ("A", "o"),
+                                       ("A", "norm"), ("giforax", "route"), ("giforax", "out norm"), ("giforax", "o")])
+def test_ways_of_a_callers_own_run_over_all_rows(tmp_path, name, what):
+    """A step of which one row is wanted, and in its last block a method or a product that is not the package's: it is handed every row."""
+    from torchless_rs_amd.engine import Engine, SeqInput
+    from torchless_rs_amd.parts.linear import Linear
+    model = models(tmp_path, name, "bfloat16")
+    block, rows = model.blocks[model.spec.schedule[-1].layer], []
+
+    def derived(part, method, of):
+        real = getattr(type(part), method)
+        part.__class__ = type("Own", (type(part),), {method: lambda self, *a, **k: (rows.append(a[of].shape[0]), real(self, *a, **k))[1]})
+
+    class Own(Linear):
+        def __call__(self, a, *rest, **kw):
+            rows.append(a.shape[0])
+            Linear.__call__(self, a, *rest, **kw)
+
+        def partial(self, *a):
+            return None
+
+        wide_partial = tall_partial = partial
+
+    if what == "hidden":
+        derived(block.ffn, "_hidden", 1)
+    elif what == "hidden on the object":
+        real = block.ffn._hidden
+        block.ffn._hidden = lambda ctx, y: (rows.append(y.shape[0]), real(ctx, y))[1]
+    elif what == "down":
+        block.ffn.down = Own(block.ffn.down.weight)
+    elif what == "add_into on the product":
+        real_add = block.ffn.down.add_into
+        block.ffn.down.add_into = lambda a, *rest: (rows.append(a.shape[0]), real_add(a, *rest))[1]
+    elif what == "o":
+        block.mixer.o = Own(block.mixer.o.weight)
+    elif what == "norm":
+        derived(block.ffn_norm, "forward", 1)
+    elif what == "route":
+        derived(block.ffn, "_route", 1)
+    else:
+        derived(block.ffn_out_norm, "add_to", 1)
+    eng = Engine(model, max_tokens=512, max_slots=2, use_graphs=False)
+    eng.step([SeqInput(eng.alloc(), prompts(model.spec.vocab_size, [40], 3)[0], [39])])
+    assert rows == [40]
+
+
 @pytest.mark.parametrize("H", [64, 1000, 4096, 8192])
 @pytest.mark.parametrize("parts", [0, 1, 9])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])

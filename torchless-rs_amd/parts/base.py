@@ -17,6 +17,7 @@ parts themselves.
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass, field
 from typing import Any, Callable, Dict, List, Optional, Tuple
 
@@ -127,6 +128,9 @@ class Part:
     # arguments whatever the step's values are (everything that varies is read on the
     # device): such a step can be captured once as a HIP graph and replayed.
     graph_safe = False
+
+    # Does what a feed-forward, a norm or a stream part does to a row follow from that row alone? (asked through `rows_apart`)
+    row_wise = False
 
     def may_capture(self, n_rows: int) -> bool:
         """May a single-token step of `n_rows` rows through this part go into a captured graph?
@@ -254,8 +258,6 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
-    row_wise = False          # does what it does to a row follow from that row alone? (asked through `rows_apart`)
-
     def forward(self, ctx: "StepContext", y: torch.Tensor, x: torch.Tensor) -> None:
         """y: normed input [n, H]; ADD the result to x (float32 [n, H])."""
         raise NotImplementedError
@@ -309,24 +311,40 @@ def norms_as_its_form(norm: "Norm") -> bool:
     return False
 
 
-def rows_apart(part: "FeedForward") -> bool:
-    """Is `part` `row_wise`?  Not where its work was set on the object, or is that of a class derived from the one that says so."""
-    own = getattr(part, "__dict__", ())
-    if "forward" in own or "produce" in own:
+@functools.lru_cache(maxsize=256)
+def _ways(c: type) -> frozenset:
+    """The names of the methods of `c` but those that any `Part` has."""
+    return frozenset(n for k in c.__mro__ for n, v in vars(k).items()
+                     if callable(v) or isinstance(v, (staticmethod, classmethod, property))) - frozenset(dir(Part))
+
+
+def goes_as_declared(part: Part, c: type) -> bool:
+    """Does `part` work as its base `c` does?  Not where a method of `c` (but those that any `Part` has) was set on the object or is that
+    of a class derived from `c`, nor where a product is no plain `Linear`."""
+    from .linear import Linear
+    own = getattr(part, "__dict__", {})
+    derived = type(part).__mro__[:type(part).__mro__.index(c)]
+    ways = _ways(c)
+    if not ways.isdisjoint(own) or any(not ways.isdisjoint(vars(k)) for k in derived):
         return False
-    for c in type(part).__mro__:
-        if "row_wise" in vars(c):
-            return bool(vars(c)["row_wise"])
-        if "forward" in vars(c) or "produce" in vars(c):
-            return False
-    return False
+    return all(type(v) is Linear and not any(callable(f) for f in vars(v).values()) for v in own.values() if callable(v))
+
+
+def rows_apart(part: Part) -> bool:
+    """Is `part` `row_wise`, and does it work as the class that says so (`goes_as_declared`)?"""
+    c = next((c for c in type(part).__mro__ if "row_wise" in vars(c)), None)
+    return c is not None and bool(vars(c)["row_wise"]) and goes_as_declared(part, c)
 
 
 def gives_rows(mixer: "Mixer", method: str) -> bool:
     """Does `mixer` offer `method` (`forward_rows` or `produce_rows`)?  Not where its work was set on the object, or is that of a class derived
-    from the one that offers it."""
+    from the one that offers it, nor where its output product is no plain `Linear`."""
+    from .linear import Linear
     own = getattr(mixer, "__dict__", ())
     if "forward" in own or "produce" in own:
+        return False
+    o = getattr(mixer, "o", None)
+    if o is not None and (type(o) is not Linear or any(callable(f) for f in vars(o).values())):
         return False
     for c in type(mixer).__mro__:
         if method in vars(c):

@@ -85,7 +85,8 @@ class PreNormBlock(Part):
 
     def ends_in_rows(self, stream_after=None) -> bool:
         """Does `forward_rows` do what this block does to some of its rows?"""
-        return (stream_after is None and self.ffn is not None and rows_apart(self.ffn) and goes_as(self, PreNormBlock, "forward"))
+        return (stream_after is None and self.ffn is not None and rows_apart(self.ffn) and rows_apart(self.ffn_norm)
+                and goes_as(self, PreNormBlock, "forward"))
 
     def forward_rows(self, ctx, run, x: torch.Tensor, rows: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
         """The model's last block for a step of more than 16 rows of which only `rows` (None: none) are read behind it: the mixer runs as
@@ -288,8 +289,10 @@ class SandwichNormBlock(Part):
 
     def ends_in_rows(self, stream_after=None) -> bool:
         """As `PreNormBlock.ends_in_rows`."""
-        return (self.ffn is not None and rows_apart(self.ffn) and goes_as(self, SandwichNormBlock, "forward", "_last_add")
-                and (stream_after is None or (hasattr(stream_after[0], "row_terms") and getattr(self.ffn_out_norm, "takes_between", False))))
+        return (self.ffn is not None and all(rows_apart(p) for p in (self.ffn, self.mixer_out_norm, self.ffn_norm, self.ffn_out_norm))
+                and goes_as(self, SandwichNormBlock, "forward", "_last_add")
+                and (stream_after is None or (rows_apart(stream_after[0]) and hasattr(stream_after[0], "row_terms")
+                                              and getattr(self.ffn_out_norm, "takes_between", False))))
 
     def forward_rows(self, ctx, run, x: torch.Tensor, rows: Optional[torch.Tensor], stream_after=None) -> Optional[torch.Tensor]:
         """As `PreNormBlock.forward_rows`; the mixer's norm too runs over the wanted rows alone."""

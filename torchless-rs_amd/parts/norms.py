@@ -16,6 +16,7 @@ from .base import Norm, RmsForm, register_part
 
 class RMSNorm(Norm):
     graph_safe = True
+    row_wise = True
     takes_pending = True        # adds partial products left in ctx.pending while it reads the stream
 
     def __init__(self, size: int, eps: float, name: str = "weight", scalar: bool = False, around_zero: bool = False):
@@ -85,6 +86,7 @@ class LayerNorm(Norm):
     in one kernel that also leaves the new stream in the compute dtype for the product that reads
     it next, or (`then`) runs the layer norm that reads the stream next on the new row."""
     graph_safe = True
+    row_wise = True
 
     def __init__(self, size: int, eps: float, name: str = "weight", bias_name: str = None):
         """`name`: the weight's leaf name behind the norm's prefix ("" where the prefix is the tensor);

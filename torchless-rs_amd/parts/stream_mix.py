@@ -24,6 +24,7 @@ from .base import StreamPart, register_part
 
 class DepthAverage(StreamPart):
     graph_safe = True
+    row_wise = True
 
     def __init__(self, hidden_size: int, names: Sequence[str]):
         """`names`: the tensors of weights for t = 1, 2, ... (call t of a step uses names[t - 1], a
