@@ -140,6 +140,35 @@ def test_ways_of_a_callers_own_run_over_all_rows(tmp_path, name, what):
     assert rows == [40]
 
 
+@pytest.mark.parametrize("derived", [False, True])
+def test_a_last_norm_of_a_callers_own_reads_the_whole_stream(monkeypatch, derived):
+    """The last feed-forward's product over 20 wanted rows comes in slices of K: a norm that knows nothing of them is handed their sum."""
+    from torchless_rs_amd import config_from_dict
+    from torchless_rs_amd.engine import Engine, SeqInput, model_from_tensors
+    from torchless_rs_amd.engine import model as m
+    from torchless_rs_amd.kernels import ops
+    from torchless_rs_amd.models import model_spec_for
+    cfg = config_from_dict(dict(architectures=["MistralForCausalLM"], num_hidden_layers=2, hidden_size=512, num_attention_heads=4, num_key_value_heads=2,
+                                head_dim=128, intermediate_size=2048, vocab_size=1000, rope_theta=1e4, rms_norm_eps=1e-5))
+    g = torch.Generator(device=DEV).manual_seed(2)
+    specs = model_spec_for(cfg).weight_specs()
+    w = {k: torch.ones(v.shape, device=DEV) if len(v.shape) == 1 else torch.randn(tuple(v.shape), generator=g, device=DEV) * v.shape[-1] ** -0.5
+         for k, v in specs.items()}
+    model = model_from_tensors(cfg, {k: t.bfloat16() for k, t in w.items()}, "bfloat16", DEV)
+    norm = model.final_norm
+    plain = lambda self, ctx, x, out: ops.rmsnorm(x, norm.weight, norm.eps, out)
+    if derived:
+        norm.__class__ = type("Own", (type(norm),), {"forward": plain})
+    else:
+        norm.forward = lambda ctx, x, out: plain(norm, ctx, x, out)
+    got = []
+    for line in (16, 1 << 30):
+        monkeypatch.setattr(m, "ENDS_IN_ROWS", line)
+        eng = Engine(model, max_tokens=512, max_slots=2, use_graphs=False)
+        got.append(eng.step([SeqInput(eng.alloc(), prompts(1000, [200], 3)[0], list(range(0, 200, 10)))]).clone())
+    assert torch.isfinite(got[0]).all() and rel_err(got[0], got[1].double()) < TOL["bfloat16"]
+
+
 @pytest.mark.parametrize("H", [64, 1000, 4096, 8192])
 @pytest.mark.parametrize("parts", [0, 1, 9])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])

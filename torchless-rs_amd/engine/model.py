@@ -14,7 +14,7 @@ import torch
 
 from ..cache.cache import Cache, KVRequest, StateRequest
 from ..config.base import ModelConfig
-from ..parts.base import ModelSpec, PartSpec, RunBinding, StepContext, flush_pending, make_part, rows_through_norm
+from ..parts.base import ModelSpec, PartSpec, RunBinding, StepContext, flush_pending, make_part, norms_as_its_form, rows_through_norm
 from ..weights.binding import bind_weights
 
 
@@ -199,7 +199,7 @@ class Model:
         if n_want:
             y = ws.get("head_y", (n_want, H), ctx.dtype)
             if narrow:
-                if not getattr(self.final_norm, "takes_pending", False):
+                if not (getattr(self.final_norm, "takes_pending", False) and norms_as_its_form(self.final_norm)):
                     flush_pending(ctx, ends)
                 self.final_norm.forward(ctx, ends, y)
             else:
