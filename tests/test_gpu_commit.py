@@ -120,3 +120,38 @@ def test_which_prompts_leave_their_projection_in_partial_sums(N, K, rows):
         def __call__(self, a, out, accumulate=False, factor=None):
             out.zero_()
     assert Own(lin.weight).rotated_partial(torch.ones(192, K, device=DEV, dtype=torch.bfloat16), ctx, "parts") is None
+
+
+@pytest.mark.gpu
+def test_a_projection_that_is_no_linear_serves_prompts(tmp_path):
+    """A product of a caller's own that knows the parts of `Linear` which the mixer has asked for all along."""
+    from torchless_rs_amd.engine import Engine, SeqInput, load_model
+    from util import TOL, make_model_dir, prompts, rel_err
+    model = load_model(make_model_dir(tmp_path, "A", torch.bfloat16), "bfloat16")
+    ids = prompts(model.spec.vocab_size, [150], 3)[0]
+
+    class Product:
+        def __init__(self, real):
+            self.real, self.weight, self.own_tiles, self.calls = real, real.weight, None, 0
+
+        def own_kernels(self, n):
+            return False
+
+        def partial(self, a, ctx, name):
+            return None
+
+        def __call__(self, a, out):
+            self.calls += 1
+            self.real(a, out)
+
+    def logits():
+        eng = Engine(model, max_tokens=512, max_slots=2, use_graphs=False)
+        return eng.step([SeqInput(eng.alloc(), ids, [149])]).clone()
+
+    want = logits()
+    mixers = [b.mixer for b in model.blocks]
+    for m in mixers:
+        m.qkv = Product(m.qkv)
+    got = logits()
+    assert all(m.qkv.calls == 1 for m in mixers)
+    assert torch.isfinite(got).all() and rel_err(got, want.double()) < TOL["bfloat16"]

@@ -157,7 +157,8 @@ class AttentionMixer(Mixer):
         if self.own_kv:
             tag = f"_{run.index}" if run.kv_read_later else ""
             tiles = ops.uses_transposed_values(ctx.dtype, d, ctx.all_single)
-            parts = (self.qkv.rotated_partial if tiles else self.qkv.partial)(y, ctx, "attn_qkv_parts")
+            partial = getattr(self.qkv, "rotated_partial", self.qkv.partial) if tiles else self.qkv.partial
+            parts = partial(y, ctx, "attn_qkv_parts")
             if parts is not None:               # K cut into partial sums: the rotation adds them up, or the first slice takes the others
                 qkv = parts if tiles else parts[0]
                 if not tiles:
