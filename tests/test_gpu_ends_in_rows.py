@@ -140,6 +140,18 @@ def test_ways_of_a_callers_own_run_over_all_rows(tmp_path, name, what):
     assert rows == [40]
 
 
+@pytest.mark.parametrize("n,want,alone", [(17, 2, True), (17, 3, False), (16, 1, False), (40, 0, True), (40, 5, True), (40, 6, False), (40, 39, False), (40, 40, False)])
+def test_up_to_an_eighth_of_the_rows_end_alone(tmp_path, monkeypatch, n, want, alone):
+    from torchless_rs_amd.engine import Engine, SeqInput
+    model = models(tmp_path, "A", "bfloat16")
+    block, narrow = model.blocks[model.spec.schedule[-1].layer], []
+    real = block.forward_rows
+    monkeypatch.setattr(block, "forward_rows", lambda *a, **k: (narrow.append(1), real(*a, **k))[1])
+    eng = Engine(model, max_tokens=512, max_slots=2, use_graphs=False)
+    eng.step([SeqInput(eng.alloc(), prompts(model.spec.vocab_size, [n], 3)[0], list(range(want)))])
+    assert len(narrow) == alone
+
+
 @pytest.mark.parametrize("derived", [False, True])
 def test_a_last_norm_of_a_callers_own_reads_the_whole_stream(monkeypatch, derived):
     """The last feed-forward's product over 20 wanted rows comes in slices of K: a norm that knows nothing of them is handed their sum."""

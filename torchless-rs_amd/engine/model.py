@@ -21,9 +21,14 @@ from ..weights.binding import bind_weights
 # From how many rows on the model's last block runs its feed-forward over the rows alone whose logits are wanted (and over none
 # where none are), and its mixer's output product where the mixer can (`gives_rows`): nobody reads the others, later steps only what the
 # mixer keeps of them.  Steps of up to 16 rows have products
-# that the norms are cut around, and read their weights whatever the rows.  Prompt steps of 2,048 rows through 32 layers 25,907 us and
-# 25,183, of 226 6,099 and 5,947; through four layers with experts 2,312 rows 5,437 and 4,809, 2,348 rows 5,094 and 4,419.
+# that the norms are cut around, and read their weights whatever the rows.  A step of 226 rows through 32 layers of 4,096 channels 6,099 us
+# and 5,947, of 2,048 25,907 and 25,183, a row a sequence wanted.
 ENDS_IN_ROWS = 16
+# And up to what share of the rows (one in so many): gathering rows costs passes of its own, and fewer rows may meet a slower way through a
+# feed-forward than all of them.  Through four layers, wanted rows / all rows, microseconds: 4,096 channels, 2,048 rows of which 256 are
+# wanted 3,118 / 3,638, 226 of which 28 892 / 940; gated experts, 226 rows of which 28 1,839 / 1,864, 56 1,883 / 1,875, 113 1,944 / 1,894,
+# 2,048 of which 256 4,375 / 4,898, 2,047 5,300 / 5,199; 2,048 channels, 600 rows of which 75 834 / 874, 150 913 / 890.
+WANTED_SHARE = 8
 EMBEDDING_RUN = -1            # the number under which the cache keeps the embedding's state, beside those of the runs
 
 
@@ -182,7 +187,7 @@ class Model:
                 kw["norm_after"] = after
             if handed:
                 kw["stream_after"] = (self.stream_parts[nxt[0]], nxt[1])
-            if i + 1 == len(order) and n_want < ctx.n_rows > ENDS_IN_ROWS and (nxt is None or handed) \
+            if i + 1 == len(order) and ctx.n_rows > ENDS_IN_ROWS and WANTED_SHARE * n_want <= ctx.n_rows and (nxt is None or handed) \
                     and hasattr(block, "ends_in_rows") and block.ends_in_rows(**kw):
                 ends = block.forward_rows(ctx, binding, x, want_rows if n_want else None, **kw)
                 narrow = True
