@@ -204,3 +204,13 @@ def test_a_norm_of_some_rows_has_the_bits_of_adding_gathering_and_the_norm(H, pa
     many = torch.zeros(2, 4, H, device=DEV)
     ops.gather_rows(both, rows, many)
     assert torch.equal(many, both[:, rows.long()])
+
+
+def test_rows_are_gathered_of_one_matrix_or_several():
+    """More dimensions than that were taken and all but the first matrices left out."""
+    from torchless_rs_amd.kernels import ops
+    rows = torch.tensor([2, 0], dtype=torch.int32, device=DEV)
+    for shape in ((4,), (2, 3, 4, 8)):
+        x = torch.zeros(shape, device=DEV)
+        with pytest.raises(ops.KernelError, match="gather.x"):
+            ops.gather_rows(x, rows, torch.zeros(shape[:-2] + (2, shape[-1]), device=DEV))

@@ -1771,6 +1771,8 @@ def take_tokens(src: torch.Tensor, idx: torch.Tensor, vocab: int, tokens: torch.
 
 def gather_rows(x: torch.Tensor, idx: torch.Tensor, out: torch.Tensor) -> None:
     """out[m] = x[idx[m]], float32 [n, H]; or the same rows of each of several matrices, x [count, n, H] and out [count, m, H]."""
+    if x.dim() not in (2, 3):
+        raise KernelError(f"gather.x: shape {tuple(x.shape)}, kernel needs [n, H] or [count, n, H]")
     m, H = idx.shape[0], x.shape[-1]
     many = tuple(x.shape[:-2])
     _req(x, "gather.x", torch.float32)
