@@ -353,14 +353,21 @@ def test_too_few_counters_are_refused(ops, monkeypatch):
     assert not bool(out.any()) and not bool(short.any())
 
 
-@pytest.mark.parametrize("nq,nkv,meet", [(8, 8, True), (8, 2, True), (10, 2, False), (32, 2, False)])
-def test_parts_meet_where_a_wave_has_one_head(ops, monkeypatch, nq, nkv, meet):
+@pytest.mark.parametrize("nq,nkv,B,meet", [(8, 8, 1, True), (8, 2, 1, True), (8, 2, 2, True), (10, 2, 1, False), (32, 2, 2, False),
+                                           (8, 2, 60, True), (8, 2, 90, False), (8, 2, 300, False)])
+def test_parts_meet_where_a_wave_has_one_head_and_all_run_at_a_time(ops, monkeypatch, nq, nkv, B, meet):
+    """Uniform parts and planned ones; of 90 sequences in three rounds of places, and of 300 in two parts each, some wait for their places."""
+    assert ops.compute_units(torch.device(DEV)) == 256
     real, asked = ops.decode_counters, []
     monkeypatch.setattr(ops, "decode_counters", lambda *a: (asked.append(a[1:]), real(*a))[1])
-    for lengths in ([1400], [900, 1400]):            # uniform parts, and planned ones
-        q, pages, table, ctx = step(ops, lengths, nq, nkv, 64)
-        out = torch.zeros_like(q)
-        ops.attention(q, None, None, pages, table, table.shape[1], ctx, None, None, 0.1, out)
-        ops.attention_scored(q, None, None, pages, nkv, 64, table, table.shape[1], ctx, None, ops.ScoreTerms(0.1), None, out)
-        assert asked == [(len(lengths), nq, nkv)] * (2 * meet)
-        asked.clear()
+    lengths = [700] * B
+    q, pages, table, ctx = step(ops, lengths, nq, nkv, 64)
+    out = torch.zeros_like(q)
+    ops.attention(q, None, None, pages, table, table.shape[1], ctx, None, None, 0.1, out)
+    assert asked == [(B, nq, nkv)] * meet
+    asked.clear()
+    ops.attention_scored(q, None, None, pages, nkv, 64, table, table.shape[1], ctx, None, ops.ScoreTerms(0.1), None, out)
+    splits = ops.decode_splits(B, nq, nkv, table.shape[1], 256, 64)
+    assert asked == [(B, nq, nkv)] * (nq // nkv <= 4 and splits > 1 and splits * B * nkv <= 512)
+    ref, size = want(q, pages, table, lengths, 0.1)
+    assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs()) + 1e-5).all())

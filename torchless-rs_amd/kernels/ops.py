@@ -701,7 +701,7 @@ def attention_scored(q, k_new, v_new, pages, nkv: int, dv: int, table, ring_page
         part = ctx.workspace.get("attn_part", (n * nq * splits * (dk + 2),), torch.float32)
         _decode_args(q, pages, table, ctx.row_pos, part, out, splits)
         slopes, sinks, gt = _terms_args(terms, gate, n, nq)
-        arrived = meeting_counters(ctx, n, nq, nkv) if splits > 1 else None
+        arrived = meeting_counters(ctx, n, nq, nkv, dk, splits * decode_groups(n, nq, nkv)) if splits > 1 else None
         _check(lib().tl_attn_decode_terms_bf16(_p(q), _p(pages), _p(table), table.shape[1], ring_pages, _p(ctx.row_pos),
                                                n, nq, nkv, dk, int(terms.window or 0), int(terms.keep_first or 0),
                                                terms.chunk, ctypes.c_float(terms.scale), int(splits), _p(part), *_counters_args(arrived), slopes, sinks,
@@ -2722,13 +2722,18 @@ def decode_counters(ctx, B: int, nq: int, nkv: int) -> torch.Tensor:
 MEETING_HEADS = 4           # query heads a KV head up to which the parts' last one merges them: a head for each wave of its workgroup.  Merged so /
                             # by a launch, one sequence of heads of 128 over 1,000, 4,000, 16,000 and 130,000 keys, microseconds: 32 over 8 heads
                             # 10.7 / 11.6, 11.7 / 13.4, 21.6 / 24.6 and 88.1 / 91.9 (heads of 64 7 to 16 % less, of 256 1 to 10 %; 1 or 2 heads a group
-                            # 3 to 19 %, 32 sequences of 16,000 keys 0.4); eight sequences 12.4 / 14.1, 26.4 / 28.0 and 83.6 / 84.6.  Not taken, a wave has heads one after the other:
+                            # 3 to 19 %); eight sequences 12.4 / 14.1, 26.4 / 28.0 and 83.6 / 84.6.  Not taken, a wave has heads one after the other:
                             # 64 over 8 12.2 / 12.6, 14.1 / 14.2, 26.1 / 25.4 and 95.3 / 94.0; 16 over 1 14.7 / 13.5, 17.7 / 15.2, 30.5 / 22.1 and 68.7 / 46.3
 
 
-def meeting_counters(ctx, B: int, nq: int, nkv: int) -> Optional[torch.Tensor]:
-    """`decode_counters` where a merge by the last part pays, else None: by a launch of its own."""
-    return decode_counters(ctx, B, nq, nkv) if nq // nkv <= MEETING_HEADS else None
+def meeting_counters(ctx, B: int, nq: int, nkv: int, d: int, workgroups: int) -> Optional[torch.Tensor]:
+    """`decode_counters` where a merge by the last part pays, else None: by a launch of its own.  It pays while the units hold all
+    workgroups at a time; where others wait for their places, those waiting for their stores and the counter keep them: 72
+    sequences of 32 over 8 heads of 128 over 1,000 keys in 4 parts 63.1 us merged so, 60.1 by the launch, 150 over 400 keys in 2 62.2 and
+    58.7 (33 over 1,000 keys in 3, a round and a half, 32.0 and 32.8: not taken either)."""
+    if nq // nkv > MEETING_HEADS or workgroups > compute_units(ctx.row_pos.device) * decode_workgroups_per_unit(d):
+        return None
+    return decode_counters(ctx, B, nq, nkv)
 
 
 def _counters_args(arrived: Optional[torch.Tensor]):
@@ -2848,7 +2853,7 @@ def attn_decode_planned(q, pages, table, ring_pages: int, ctx, plan, window: Opt
     part = arrived = None
     if seqs is not None:
         _req(seqs, "attn_decode_planned.seqs", torch.int32, (B, 2))
-        arrived = meeting_counters(ctx, B, nq, nkv)
+        arrived = meeting_counters(ctx, B, nq, nkv, d, places.shape[0] * decode_groups(1, nq, nkv))
         part = ctx.workspace.get("attn_part", (places.shape[0] * nq * (d + 2),), torch.float32)
     _decode_args(q, pages, table, ctx.row_pos, part, out, 1)
     slopes, sinks, gt = _terms_args(terms, gate, B, nq) if terms is not None else (None, None, None)
@@ -2884,7 +2889,7 @@ def attention(q, k_new, v_new, pages, table, ring_pages: int, ctx, n_cached, win
         splits = decode_splits(n, nq, nkv, table.shape[1], compute_units(q.device), d)   # by the table's width: fixed while a graph lives
         part = ctx.workspace.get("attn_part", (n * nq * splits * (d + 2),), torch.float32)
         attn_decode_bf16(q, pages, table, ring_pages, ctx.row_pos, window, scale, splits, part, out,
-                         meeting_counters(ctx, n, nq, nkv) if splits > 1 else None)
+                         meeting_counters(ctx, n, nq, nkv, d, splits * decode_groups(n, nq, nkv)) if splits > 1 else None)
     elif fast and k_new is not None and vt_new is not None:
         n_tiles = int(sum(-(-int(x) // PREFILL_BLOCK) for x in ctx.host["n_new"]))
         cuts = part = None
