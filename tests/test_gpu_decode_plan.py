@@ -328,6 +328,44 @@ def test_merged_parts_have_those_bits_where_they_come_in_more_than_one_trip(ops,
     assert torch.equal(met, apart)
 
 
+@pytest.mark.parametrize("sort", ["plain", "sinks", "logistic", "window"])
+@pytest.mark.parametrize("nq,nkv,d", [(8, 2, 64), (8, 2, 128), (4, 2, 256), (34, 2, 128)])
+def test_planned_parts_and_terms_merge_to_the_same_bits_both_ways(ops, monkeypatch, sort, nq, nkv, d):
+    """Planned parts (counts that differ by sequence, one part among them) and uniform ones, with and without terms, merged by the last
+    part and by the launch; one buffer of counters for two numbers of sequences, zero behind every launch."""
+    from torchless_rs_amd.parts.base import Workspace
+    g = torch.Generator(device=DEV).manual_seed(d)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    kw = {"plain": None, "sinks": dict(sinks=rand(nq), slopes=rand(nq).abs() * 1e-3), "logistic": dict(logistic=True, score_bias=rand(nq)),
+          "window": dict(window=500, keep_first=64)}[sort]
+    terms = ops.ScoreTerms(0.1, **kw) if kw is not None else None
+    spaces = {meet: Workspace(torch.device(DEV)) for meet in (True, False)}
+    for lengths in ([6000, 1, 700, 2500, 64, 65, 1300], [900, 5000], [4100]):
+        q, pages, table, ctx = step(ops, lengths, nq, nkv, d, seed=len(lengths))
+        gate = torch.rand(len(lengths), nq, generator=g, device=DEV) if sort in ("sinks", "logistic") else None
+        got = {}
+        for meet, ws in spaces.items():
+            monkeypatch.setattr(ops, "meeting_counters", lambda ctx, B, nq, nkv, *rest, _m=meet: ops.decode_counters(ctx, B, nq, nkv) if _m else None)
+            ctx.workspace, ctx.host = ws, {}
+            if sort != "plain":
+                ways = [lambda out: ops.attention_scored(q, None, None, pages, nkv, d, table, 1 << 24, ctx, None, terms, gate, out)]
+            else:
+                ways = [lambda out: ops.attention(q, None, None, pages, table, 1 << 24, ctx, None, None, 0.1, out)]
+            plan = ops.decode_plan(ctx, nq, nkv, d, table.shape[1], terms.window if terms else None, terms.keep_first if terms else 0)
+            if plan is not None:
+                assert plan[1] is not None and int(plan[1][:, 1].max()) > 1
+                ways.append(lambda out: ops.attn_decode_planned(q, pages, table, 1 << 24, ctx, plan, terms.window if terms else None, 0.1, out, terms, gate))
+            for way in ways:
+                out = torch.zeros_like(q)
+                way(out)
+                got.setdefault(meet, []).append(out)
+                if meet:
+                    assert not bool(ops.decode_counters(ctx, len(lengths), nq, nkv).any())
+        assert len(got[True]) == len(got[False]) == 1 + (len(lengths) > 1)
+        for a, b in zip(got[True], got[False]):
+            assert torch.equal(a, b) and bool(a.any())
+
+
 def test_too_few_counters_are_refused(ops, monkeypatch):
     """By every way in, before anything is launched."""
     lengths = [900, 1400]
