@@ -559,33 +559,25 @@ gemm_qkv_rope_commit_kernel(const bf16* __restrict__ A, const bf16* __restrict__
   bf16x8 w0[NT][2], a0[2], w1[NT][2], a1[2];
   int s = s0;
   if (s < s1) load_step(s, w0, a0);
-  if (s + 1 < s1) load_step(s + 1, w1, a1);
   // the threads of the epilogue: 128 a unit; of a rotated unit 64 work, one a row and pair
   const int eu = tid / 128, et = tid % 128;
   const int eg = g0 + min(eu, mine - 1);
   const int ehead = eg / per_head, eh = eg % per_head;
   const bool e_on = eu < mine, e_rot = ehead < nq + nkv;
-  const int em = e_rot ? et / 4 : et / 8;              // its row
-  // Position, angle and page are looked up while the first two steps' weights are under way: behind the product they were two trips
-  // to memory one after the other.  6,144 x 4,096 at 1 / 8 rows 11.8 / 12.0 us and now 11.3 / 11.5, x 5,120 14.6 / 15.0 and 13.9 / 14.2, x 2,048 8.9 / 9.0
-  // and 8.0 / 8.1 (with one step under way before them they lost).
-  const int p = row_pos[min(em, M - 1)];
-  if (e_on && e_rot && et < 64) {
-    const int j = et % 4, i = 4 * eh + j;
-    if (em < M && 2 * i < rot.rotary_dim) sincosf(rot.inv_freq[i] * (float)p, &sn[eu][em][j], &cs[eu][em][j]);
+  if (e_on && e_rot && et < 64) {              // while the first loads are under way
+    const int m = et / 4, j = et % 4, i = 4 * eh + j;
+    if (m < M && 2 * i < rot.rotary_dim) sincosf(rot.inv_freq[i] * (float)row_pos[m], &sn[eu][m][j], &cs[eu][m][j]);
   }
-  const int page = table[(size_t)min(em, M - 1) * table_stride + (p / PAGE) % ring_pages];
   const bool scaled = ns.ssq_in != nullptr;
   RowFactors rf;
   if (scaled) rf.fetch(ns);
-  for (; s < s1; s += 2) {
+  for (; s + 1 < s1; s += 2) {
+    load_step(s + 1, w1, a1);
     mma_step(w0, a0);
     if (s + 2 < s1) load_step(s + 2, w0, a0);
-    if (s + 1 < s1) {
-      mma_step(w1, a1);
-      if (s + 3 < s1) load_step(s + 3, w1, a1);
-    }
+    mma_step(w1, a1);
   }
+  if (s < s1) mma_step(w0, a0);
   if (scaled) rf.finish(ns, rs);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -603,7 +595,7 @@ gemm_qkv_rope_commit_kernel(const bf16* __restrict__ A, const bf16* __restrict__
   if (!e_on) return;
   const size_t page_elems = 2 * (size_t)nkv * PAGE * d;
   if (e_rot) {
-    const int m = em, j = et % 4;
+    const int m = et / 4, j = et % 4;
     if (et < 64 && m < M) {
       const int i = 4 * eh + j;
       float ra = total(8 * eu + j, m), rb = total(8 * eu + 4 + j, m);
@@ -614,14 +606,18 @@ gemm_qkv_rope_commit_kernel(const bf16* __restrict__ A, const bf16* __restrict__
       if (ehead < nq) {
         dst = q + ((size_t)m * nq + ehead) * d;
       } else {
+        const int p = row_pos[m];
+        const int page = table[(size_t)m * table_stride + (p / PAGE) % ring_pages];
         dst = pages + (size_t)page * page_elems + ((size_t)(ehead - nq) * PAGE + p % PAGE) * d;
       }
       dst[ia] = (bf16)ra;
       dst[ib] = (bf16)rb;
     }
   } else {
-    const int m = em, nl = et % 8;
+    const int m = et / 8, nl = et % 8;
     if (m < M) {
+      const int p = row_pos[m];
+      const int page = table[(size_t)m * table_stride + (p / PAGE) % ring_pages];
       bf16* vd = pages + (size_t)page * page_elems + (size_t)nkv * PAGE * d;
       vd[((size_t)(ehead - nq - nkv) * d + 8 * eh + nl) * PAGE + p % PAGE] = (bf16)total(8 * eu + nl, m);
     }
