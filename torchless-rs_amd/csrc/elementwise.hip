@@ -475,15 +475,17 @@ __device__ __forceinline__ void rope_split_row(int n, float* cs, float* sn, cons
       }
     }
   }
-  const float* vs = src + (size_t)(nq + nkv) * d;
-  if (v != nullptr) {
-    TO* vd = v + (size_t)n * nkv * d;
-    for (int t = tid; t < nkv * d; t += step) vd[t] = from_f32<TO>(slices.template at<float>(vs + t));
-  }
-  if (vt != nullptr) {      // the same values transposed: [kv head][d][column of this row]
-    const int b = row_seq[n];
-    const int col = tile_off[b] + row_pos[n] - (n_cached[b] / PAGE) * PAGE;
-    for (int t = tid; t < nkv * d; t += step) vt[(size_t)t * vt_cols + col] = from_f32<TO>(slices.template at<float>(vs + t));
+  if constexpr (!SUMS) {    // (a projection in partial sums has its values in tiles, see v_tile)
+    const float* vs = src + (size_t)(nq + nkv) * d;
+    if (v != nullptr) {
+      TO* vd = v + (size_t)n * nkv * d;
+      for (int t = tid; t < nkv * d; t += step) vd[t] = from_f32<TO>(vs[t]);
+    }
+    if (vt != nullptr) {    // the same values transposed: [kv head][d][column of this row]
+      const int b = row_seq[n];
+      const int col = tile_off[b] + row_pos[n] - (n_cached[b] / PAGE) * PAGE;
+      for (int t = tid; t < nkv * d; t += step) vt[(size_t)t * vt_cols + col] = from_f32<TO>(vs[t]);
+    }
   }
 }
 

@@ -2714,9 +2714,14 @@ def decode_groups(B: int, nq: int, nkv: int) -> int:
     return B * nkv * (-(-(nq // nkv) // 16))
 
 
+@functools.lru_cache(maxsize=4096)
+def _n_counters(B: int, nq: int, nkv: int) -> int:
+    return lib().tl_attn_decode_counters(B, nq, nkv)
+
+
 def decode_counters(ctx, B: int, nq: int, nkv: int) -> torch.Tensor:
     """The counters by which the parts of a decode step's attention find the last of them, which merges them: zero between launches."""
-    return ctx.workspace.get("attn_arrived", (lib().tl_attn_decode_counters(B, nq, nkv),), torch.int32, zero=True)
+    return ctx.workspace.get("attn_arrived", (_n_counters(B, nq, nkv),), torch.int32, zero=True)
 
 
 MEETING_HEADS = 4           # query heads a KV head up to which the parts' last one merges them: a head for each wave of its workgroup.  Merged so /
@@ -2744,8 +2749,9 @@ def _counters_args(arrived: Optional[torch.Tensor]):
 
 
 SPLIT_PAGES = 4             # fewest pages a part of the keys has
-SPLIT_COST = 0.15           # what a part more costs in the merge, in pages of a workgroup's way (8 sequences of
-                            # 8 KV heads over 4,096 keys: 4 parts 3.91 ms a step, 8 parts 3.96, 6 parts 4.08)
+SPLIT_COST = 0.15           # what a part more costs in the merge, in pages of a workgroup's way (8 sequences of 32 over 8 heads of
+                            # 128 over 4,096 keys, microseconds, merged by the last part / by a launch: 4 parts 29.6 / 30.9, 6 27.8 /
+                            # 29.2, 8 27.5 / 28.8, 12 33.0 / 33.8, 16 31.9 / 33.0)
 FULL_UNIT_HEAD = 128        # the kernel that reads the pages into registers: the head size from which one workgroup
                             # has enough bytes under way to keep a compute unit streaming; smaller heads get
                             # FULL_UNIT_HEAD // head_dim workgroups a unit (heads of 48 ...)
@@ -2787,9 +2793,9 @@ PLAN_SEQS = 512             # most sequences that a plan is made for
 def decode_rounds(B: int, nq: int, nkv: int, units: int, head_dim: int):
     """(places, rounds) of the plan of a decode step's parts, or None where it goes without one: `decode_splits` then gives every
     sequence as many parts.  A place is one workgroup for each KV head (16 query heads of its group), a round as many places as the
-    units hold at a time.  One sequence has nothing to balance, and where more than half of a round are sequences the uniform parts
-    are so many that the units even out what they have by themselves (64 sequences of 140 to 2,048 keys: 60.5 us and 4.9 for the merge,
-    65.1 without parts; a step the same).  From a third of a round on, two or three rounds of smaller parts may divide better (20
+    units hold at a time.  One sequence has nothing to balance, and where more than half of a round are sequences whole ones in an
+    order (`decode_places`) or uniform parts even out by themselves (64 sequences of 140 to 2,048 keys: whole in an order 60.5 us, in 2 to 4
+    parts each 65.6 to 66.7).  From a third of a round on, two or three rounds of smaller parts may divide better (20
     sequences of one length in 64 places: 3 parts each, 60; 22: 2 parts each, or 5 each in two rounds)."""
     places = units * decode_workgroups_per_unit(head_dim) // decode_groups(1, nq, nkv)
     if not (2 <= B <= min(places // 2, PLAN_SEQS)):
@@ -2813,8 +2819,8 @@ def decode_plan(ctx, nq: int, nkv: int, d: int, table_width: int, window: Option
     """The plan of a single-token step's parts for layers of these sizes, made by the first of them (one small kernel, 4 us) and kept
     while the step runs: (plan int32 [places, 4], seqs int32 [B, 2]), for whole sequences in an order (plan int32 [B, 4], None), or None.
     Tables of up to `least` pages go without:
-    up to SPLIT_PAGES the keys stay whole and there is no merge (19 sequences of 58 to 221 keys: 10.6 us, in parts 8.9 and 4.8 for the
-    merge)."""
+    up to SPLIT_PAGES the keys stay whole and there is no merge (19 sequences of 58 to 221 keys: 9.9 us, in parts 9.9 merged by the last of
+    them and 11.3 by a launch; fewer sequences would gain by parts, 8 of 100 to 250 keys 9.5, 8.0 and 9.3)."""
     B, units = ctx.row_pos.shape[0], compute_units(ctx.row_pos.device)
     shape = decode_rounds(B, nq, nkv, units, d)
     if table_width <= least or not lib().tl_attn_decode_takes_plan(d, int(table_width)):
