@@ -1843,3 +1843,16 @@ def test_gemm_ring_begins_with_other_stages(ops, waves, kc, M, N, K):
         ops.gemm_ring_bf16(a, w, h, silu_pair=True, waves=waves, kc=kc)
         ref = torch.nn.functional.silu(gate) * up
         assert bool(((h.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * (1.0 + p.abs().max()) ** 2).all())
+
+
+@pytest.mark.parametrize("short", ["counters", "probs", "out", "lists", "host_out"])
+def test_a_draw_into_kept_buffers_without_room_is_refused(short):
+    from torchless_rs_amd.kernels import ops
+    B, V = 3, 131072
+    rows = {k: B - (k == short) for k in ("counters", "probs", "out", "lists", "host_out")}
+    i32 = lambda n, *more, **kw: torch.zeros((n, *more), dtype=torch.int32, **kw)
+    kept = dict(counters=i32(rows["counters"], 2, pin_memory=True), probs=torch.zeros(rows["probs"], V, device=DEV), out=i32(rows["out"], device=DEV),
+                lists=ops.sample_lists(rows["lists"], V, 0.7, 50, DEV), host_out=i32(rows["host_out"], pin_memory=True))
+    assert kept["lists"] is not None
+    with pytest.raises(ops.KernelError, match="no room"):
+        ops.sample_kept(torch.zeros(B, V, device=DEV), 0.7, 50, 0.9, 1, **kept)

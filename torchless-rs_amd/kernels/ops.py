@@ -1896,7 +1896,8 @@ def sample_kept(logits: torch.Tensor, temperature: float, top_k: int, top_p: flo
     are not looked at, which takes the host 7 us of the 17 before the launch (16 rows of 131,072: 42.9 us a draw, 36.4 so)."""
     B, V = logits.shape
     _req(logits, "sample.logits", torch.float32)
-    if counters.shape[0] < B or probs.shape[0] < B or probs.shape[1] != V or out.shape[0] < B or (host_out is not None and host_out.shape[0] < B):
+    if (counters.shape[0] < B or probs.shape[0] < B or probs.shape[1] != V or out.shape[0] < B or (host_out is not None and host_out.shape[0] < B)
+            or (lists is not None and lists.shape[0] < B)):
         raise KernelError(f"sample: the buffers have no room for {B} rows of {V}")
     _check(lib().tl_sample(_p(logits), B, V, ctypes.c_float(temperature), int(top_k),
                            ctypes.c_float(top_p), ctypes.c_ulonglong(seed & (2 ** 64 - 1)),
